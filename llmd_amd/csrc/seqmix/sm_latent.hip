@@ -376,9 +376,11 @@ __global__ __launch_bounds__(NT, 2) void latent_prompt_kernel(
 #pragma unroll
     for (int i = 1; i < 8; ++i) mx = fmaxf(mx, sc[i]);
     mx = row_max(mx);
-    if (__any(mx > m + 8.f)) {  // weights of up to 2^8 lose nothing in fp32
-      const float mn = fmaxf(m, mx);
-      const float corr = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+    // the reference moves only when a score of the row passes it by 2^8: weights of up to 2^8 lose nothing in fp32. The branch
+    // is the wave's, the move the row's own: other rows of the wave are multiplied by 1
+    if (__any(mx > m + 8.f)) {
+      const float mn = mx > m + 8.f ? mx : m;
+      const float corr = mn == m ? 1.f : __builtin_amdgcn_exp2f(m - mn);
       l *= corr;
       m = mn;
 #pragma unroll
