@@ -35,6 +35,14 @@ __device__ __forceinline__ float row_max(float v) {
   const auto t = __builtin_amdgcn_permlane32_swap(b, b, false, false);
   return fmaxf(__uint_as_float(t[0]), __uint_as_float(t[1]));
 }
+// The sum of those four values, the same in all of them: (own + 16 away) + (32 away + 48 away).
+__device__ __forceinline__ float row_sum(float v) {
+  const uint32_t a = __float_as_uint(v);
+  const auto s = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+  const uint32_t b = __float_as_uint(__uint_as_float(s[0]) + __uint_as_float(s[1]));
+  const auto t = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+}
 
 // Wave-wide copy of 1 KB to LDS without registers: lane i's 16 bytes at base + off land at dst + 16 i. Written as asm, so that
 // hipcc keeps counting its own LDS reads; the caller waits (vmcnt) before the barrier that publishes the tile.

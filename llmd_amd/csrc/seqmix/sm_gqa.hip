@@ -754,8 +754,8 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
       }
       qf[rb][ks] = __builtin_bit_cast(bf16x8_t, v);
     }
-  // o[rb][n][r] = this lane's row, column 16 n + 4 kq + r; m: what the weights are taken relative to (in base 2, the same in
-  // the row's four lanes); l: the sum of the weights of this lane's keys
+  // o[rb][n][r] = this lane's row, column 16 n + 4 kq + r; m, l: the row's maximum (base 2) and sum of weights so far, the same
+  // in its four lanes
   f32x4_t o[RB][NCB];
   float m[RB], l[RB];
 #pragma unroll
@@ -763,7 +763,7 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
     // a sink is a score that is already counted (by the first key range only)
     const bool sk = sinks != nullptr && blockIdx.z == 0;
     m[rb] = sk ? sinks[myhead[rb]] * 1.44269504088896341f : -INFINITY;
-    l[rb] = sk && kq == 0 ? 1.f : 0.f;
+    l[rb] = sk ? 1.f : 0.f;
 #pragma unroll
     for (int n = 0; n < NCB; ++n) o[rb][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
@@ -932,18 +932,15 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
 #pragma unroll
         for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[rb][kb][r]);
       mx = row_max(mx);
-      // the reference moves only when a score passes it by 2^8: until then weights are at most 2^8 and lose nothing in fp32
-      if (__any(mx > m[rb] + 8.f)) {
-        const float mn = fmaxf(m[rb], mx);
-        const float corr = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m[rb] - mn);
-        l[rb] *= corr;
-        m[rb] = mn;
+      const float mn = fmaxf(m[rb], mx), mref = mn == -INFINITY ? 0.f : mn;  // a row with no key yet
+      const float corr = __builtin_amdgcn_exp2f(m[rb] - mref);
+      if (__any(corr != 1.f)) {  // some row's maximum moved; a row whose own did not is multiplied by 1
 #pragma unroll
         for (int n = 0; n < NCB; ++n)
 #pragma unroll
           for (int r = 0; r < 4; ++r) o[rb][n][r] *= corr;
       }
-      const float mref = m[rb] == -INFINITY ? 0.f : m[rb];  // a row with no key yet
+      float psum = 0.f;
       u32x4_t hw, lw;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
@@ -953,7 +950,7 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
         for (int r = 0; r < 4; r += 2) {
           const float p0 = __builtin_amdgcn_exp2f(sc[rb][kb][r] - mref);
           const float p1 = __builtin_amdgcn_exp2f(sc[rb][kb][r + 1] - mref);
-          l[rb] += p0 + p1;
+          psum += p0 + p1;
           const uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
           const uint32_t r0 = __float_as_uint(p0 - __uint_as_float(u0 & 0xffff0000u));
           const uint32_t r1 = __float_as_uint(p1 - __uint_as_float(u1 & 0xffff0000u));
@@ -963,6 +960,8 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
       }
       pah[rb] = __builtin_bit_cast(bf16x8_t, hw);
       pal[rb] = __builtin_bit_cast(bf16x8_t, lw);
+      l[rb] = l[rb] * corr + row_sum(psum);
+      m[rb] = mn;
     }
 #pragma unroll
     for (int n0 = 0; n0 < NCB; n0 += 4) {
@@ -988,11 +987,6 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
       }
       __syncthreads();
     }
-  }
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {  // the row's sum over its four lanes
-    l[rb] += __shfl_xor(l[rb], 16, 64);
-    l[rb] += __shfl_xor(l[rb], 32, 64);
   }
   const bool fours = (vdim & 3) == 0;
   if (nsplit > 1) {  // RB == 1 (the host splits decode-only steps, whose items have at most 64 rows)
@@ -1049,8 +1043,10 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
 // A key row's 16-byte pieces lie in the order c ^ (the lane that reads the row), a value column's in c ^ (column / 4), so
 // the 16 lanes of a read meet all banks. Score rows are dealt like in the decode form: a lane's eight keys are
 // neighbours, one piece of a value column. Only a sequence's last tile may hold keys that were never written: its value
-// columns are cleared there. 2048 tokens, 32 heads x 128 over 4 kv heads, window 1024: 87 us with the general form, now 56 us;
-// 3 portions of 787 to 901 tokens after 333: 103 / 69 us. Two blocks of 16 rows per wave (half the LDS reads): 70 / 76 us.
+// columns are cleared there. 2048 tokens, 32 heads x 128 over 4 kv heads, window 1024: 87 us with the general form, now 61 us;
+// 3 portions of 787 to 901 tokens after 333: 103 / 74 us. Two blocks of 16 rows per wave (half the LDS reads): 70 / 76 us. A
+// reference that moved only when a row of the wave passed it by 2^8 took 57 / 69 us, but a row's rounding then depended on
+// the 15 rows beside it.
 template <int NKS, int NCB>
 __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache, const int* __restrict__ tables, int W, int bs,
@@ -1075,7 +1071,7 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
   const int mywlo = window > 0 ? max(0, mylen - window) : 0;                             // first key of the row's window
   const float myslope = slopes ? slopes[myhead] * 1.44269504088896341f : 0.f;
   float m = sinks ? sinks[myhead] * 1.44269504088896341f : -INFINITY;  // a sink is a score that is already counted
-  float l = sinks && kq == 0 ? 1.f : 0.f;
+  float l = sinks ? 1.f : 0.f;
   f32x4_t o[NCB];
 #pragma unroll
   for (int n = 0; n < NCB; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -1183,22 +1179,20 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
 #pragma unroll
     for (int i = 1; i < 8; ++i) mx = fmaxf(mx, sc[i]);
     mx = row_max(mx);
-    if (__any(mx > m + 8.f)) {  // weights of up to 2^8 lose nothing in fp32
-      const float mn = fmaxf(m, mx);
-      const float corr = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
-      l *= corr;
-      m = mn;
+    const float mn = fmaxf(m, mx), mref = mn == -INFINITY ? 0.f : mn;  // a row with no key yet
+    const float corr = __builtin_amdgcn_exp2f(m - mref);
+    if (__any(corr != 1.f)) {  // some row's maximum moved; a row whose own did not is multiplied by 1
 #pragma unroll
       for (int n = 0; n < NCB; ++n)
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[n][r] *= corr;
     }
-    const float mref = m == -INFINITY ? 0.f : m;  // a row with no key yet
+    float psum = 0.f;
     u32x4_t hw, lw;  // the weights in two bf16 parts, as in grouped_attention_mfma
 #pragma unroll
     for (int i = 0; i < 8; i += 2) {
       const float p0 = __builtin_amdgcn_exp2f(sc[i] - mref), p1 = __builtin_amdgcn_exp2f(sc[i + 1] - mref);
-      l += p0 + p1;
+      psum += p0 + p1;
       const uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
       const uint32_t r0 = __float_as_uint(p0 - __uint_as_float(u0 & 0xffff0000u));
       const uint32_t r1 = __float_as_uint(p1 - __uint_as_float(u1 & 0xffff0000u));
@@ -1206,6 +1200,8 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
       lw[i >> 1] = __builtin_amdgcn_perm(r1, r0, 0x07060302u);
     }
     const bf16x8_t pah = __builtin_bit_cast(bf16x8_t, hw), pal = __builtin_bit_cast(bf16x8_t, lw);
+    l = l * corr + row_sum(psum);
+    m = mn;
 #pragma unroll
     for (int n0 = 0; n0 < NCB; n0 += 4) {
       bf16x8_t v[4];
@@ -1218,8 +1214,6 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
     }
     arrive();
   }
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
   if (wave * 16 + r16 >= ntok * G) return;
   const float inv = 1.f / l;
   bf16_t* dst = out + ((int64_t)mytok * Hq + myhead) * vdim;

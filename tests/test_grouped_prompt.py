@@ -33,3 +33,29 @@ def test_grouped_prompt(Hq, Hkv, dim, bs, opts, runs):
     got = sm.grouped_attention(q.cuda(), cache.cuda(), dim, dim, dim ** -0.5, m, **kw("cuda", lambda x: x)).float().cpu()
     # bf16 results: 2^-9 of each; weights in two bf16 parts: 2^-16 of a mean of values up to about 5, and fp32 sums of dim products
     assert ((got - want).abs() <= 2 ** -8 * want.abs() + 2e-4).all()
+
+
+@pytest.mark.parametrize("bs,dim", [(64, 128), (64, 64), (64, 256), (16, 128), (16, 40)])  # whole sizes, general form
+@pytest.mark.parametrize("opts", [{}, {"window": 70, "keep_first": 3, "sinks": True}], ids=["causal", "window"])
+def test_rows_do_not_depend_on_the_cut(bs, dim, opts):
+    """A token's output has the same bits wherever its prompt is cut into portions, whatever its neighbours' scores are."""
+    from llmd_amd.ops import seqmix as sm
+
+    n, Hq, Hkv = 300, 6, 2
+    g = torch.Generator().manual_seed(dim)
+    whole, pages = _meta([(0, n)], bs, "cuda")
+    q = torch.randn(n, Hq, dim, generator=g) * 2.0 ** torch.randint(0, 6, (n, Hq, 1), generator=g)  # some rows' maxima jump
+    q, cache = q.bfloat16().cuda(), torch.randn(pages, Hkv, bs, 2 * dim, generator=g).bfloat16().cuda()
+    sinks = torch.randn(Hq, generator=g).cuda()
+    kw = {k: sinks if v is True else v for k, v in opts.items()}
+    out = []
+    for cuts in ((0, n), (0, 77, n), (0, 3, 130, 131, n)):
+        rows = []
+        for a, b in zip(cuts, cuts[1:]):
+            m, _ = _meta([(a, b - a)], bs, "cuda")
+            m.tables = whole.tables
+            if b - a == 1:
+                m.max_q = 2   # beside a portion: not a step of single tokens
+            rows.append(sm.grouped_attention(q[a:b], cache, dim, dim, dim ** -0.5, m, **kw))
+        out.append(torch.cat(rows))
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
