@@ -1041,12 +1041,14 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
 // of grouped_attention_mfma with less around them. Tiles are copied straight to LDS, the next one into the other buffer while
 // this one is multiplied, so a tile costs no registers, conversions or LDS writes; places of the copies are computed once.
 // A key row's 16-byte pieces lie in the order c ^ (the lane that reads the row), a value column's in c ^ (column / 4), so
-// the 16 lanes of a read meet all banks. Score rows are dealt like in the decode form: a lane's eight keys are
-// neighbours, one piece of a value column. Only a sequence's last tile may hold keys that were never written: its value
-// columns are cleared there. 2048 tokens, 32 heads x 128 over 4 kv heads, window 1024: 87 us with the general form, now 61 us;
-// 3 portions of 787 to 901 tokens after 333: 103 / 74 us. Two blocks of 16 rows per wave (half the LDS reads): 70 / 76 us. A
-// reference that moved only when a row of the wave passed it by 2^8 took 57 / 69 us, but a row's rounding then depended on
-// the 15 rows beside it.
+// the lanes of a read meet all banks. Keys enter every sum in the general form's order, so that both give the same bits and the
+// page size of a call does not decide which expert a near tie further on goes to: a lane holds keys 4 kq .. 4 kq + 3 of both
+// halves. It reads one piece of 16 bytes of a value column, eight neighbours, and lanes 16 apart exchange halves (two reads of
+// 8 bytes instead: 91 us where this takes 82). Only a sequence's last tile may hold keys that were never written: its value
+// columns are cleared there. 2048 tokens, 32 heads x 128 over 4 kv heads, window 1024: 67 us;
+// 3 portions of 787 to 901 tokens after 333: 75 us. With a reference that moved only when a row of the wave passed it by 2^8
+// (a row's rounding then depended on the 15 rows beside it) and eight neighbouring keys per lane: the general form 87 / 103 us,
+// this one 57 / 69, two blocks of 16 rows per wave (half the LDS reads) 70 / 76.
 template <int NKS, int NCB>
 __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache, const int* __restrict__ tables, int W, int bs,
@@ -1104,7 +1106,7 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
   for (int i = 0; i < NK; ++i) {
     const int e = (wave + 4 * i) * 64 + lane, row = e / PR;
     krow[i] = row;
-    const int f = NKS == 2 ? (row >> 3) * 2 + (row >> 1 & 1) : (row >> 3) * 4 + (row & 3);
+    const int f = NKS == 2 ? (row & 15) >> 1 : row & 15;
     kpiece[i] = ((e % PR) ^ f) * 16;
   }
 #pragma unroll
@@ -1126,12 +1128,12 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
     for (int i = 0; i < NV; ++i) copy_1k(base + bs * RBy + off * 2, vplace[i], at + KB + i * 4096);
   };
   auto arrive = [] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  // reads: the key row that lane r16 multiplies (block kb: 4 rows further), pieces of columns 16 n + r16
+  // reads: the key row that lane r16 multiplies (block kb: 16 rows further), pieces of columns 16 n + r16
   int ka[NKS <= 4 ? NKS : 4];
 #pragma unroll
   for (int ks = 0; ks < (NKS <= 4 ? NKS : 4); ++ks)
-    ka[ks] = (8 * (r16 >> 2) + (r16 & 3)) * RBy + ((4 * ks + kq) ^ (NKS == 2 ? r16 >> 1 : r16)) * 16;
-  const int va = KB + r16 * 64 + (kq ^ r16 >> 2) * 16;
+    ka[ks] = r16 * RBy + ((4 * ks + kq) ^ (NKS == 2 ? r16 >> 1 : r16)) * 16;
+  const int va = KB + r16 * 64 + ((kq >> 1 | (kq & 1) << 1) ^ r16 >> 2) * 16;
 
   if (kbase < vlen) copy(kbase, 0);
   arrive();
@@ -1150,14 +1152,14 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
     const bool plain = k0 >= full_lo && k0 + MKT <= full_hi;  // every key visible to every row: no masks
-    float sc[8];  // scores of this lane's rows against keys k0 + 8 kq + i
+    float sc[8];  // scores of this lane's row against keys k0 + 16 kb + 4 kq + r
     {
       f32x4_t a[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
-          const bf16x8_t k = *reinterpret_cast<const bf16x8_t*>(t + ka[ks & 3] + (ks >> 2) * 256 + kb * 4 * RBy);
+          const bf16x8_t k = *reinterpret_cast<const bf16x8_t*>(t + ka[ks & 3] + (ks >> 2) * 256 + kb * 16 * RBy);
           a[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qf[ks], a[kb], 0, 0, 0);
         }
 #pragma unroll
@@ -1166,14 +1168,14 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
     if (!plain) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int key = k0 + kq * 8 + i;
+        const int key = k0 + (i >> 2) * 16 + kq * 4 + (i & 3);
         const bool in = (key < mylen) & (key >= mylo) & ((key >= mywlo) | (key < keep));
         sc[i] = in ? sc[i] - myslope * (float)(mylen - 1 - key) : -INFINITY;
       }
     } else if (slopes != nullptr) {
-      const float dist = (float)(mylen - 1 - k0 - kq * 8);
+      const float dist = (float)(mylen - 1 - k0 - kq * 4);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) sc[i] -= myslope * (dist - (float)i);
+      for (int i = 0; i < 8; ++i) sc[i] -= myslope * (dist - (float)((i >> 2) * 16 + (i & 3)));
     }
     float mx = sc[0];
 #pragma unroll
@@ -1206,7 +1208,12 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
     for (int n0 = 0; n0 < NCB; n0 += 4) {
       bf16x8_t v[4];
 #pragma unroll
-      for (int n = 0; n < 4; ++n) v[n] = *reinterpret_cast<const bf16x8_t*>(t + va + (n0 + n) * 1024);
+      for (int n = 0; n < 4; ++n) {
+        const u32x4_t w = *reinterpret_cast<const u32x4_t*>(t + va + (n0 + n) * 1024);
+        const auto x = __builtin_amdgcn_permlane16_swap(w[0], w[2], false, false);
+        const auto y = __builtin_amdgcn_permlane16_swap(w[1], w[3], false, false);
+        v[n] = __builtin_bit_cast(bf16x8_t, u32x4_t{x[0], y[0], x[1], y[1]});
+      }
 #pragma unroll
       for (int n = 0; n < 4; ++n) o[n0 + n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[n], pah, o[n0 + n], 0, 0, 0);
 #pragma unroll

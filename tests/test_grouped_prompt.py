@@ -59,3 +59,31 @@ def test_rows_do_not_depend_on_the_cut(bs, dim, opts):
             rows.append(sm.grouped_attention(q[a:b], cache, dim, dim, dim ** -0.5, m, **kw))
         out.append(torch.cat(rows))
     assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("opts", [{}, {"window": 70, "keep_first": 3, "sinks": True}, {"chunk": 50, "slopes": True}, {"gate": True}],
+                         ids=["causal", "window", "chunk", "gate"])
+def test_bits_do_not_depend_on_the_form(dim, opts):
+    """Pages of whole tiles and smaller ones (the general form) give the same bits."""
+    from llmd_amd.ops import seqmix as sm
+
+    runs, Hq, Hkv = [(0, 300), (45, 1), (100, 77)], 6, 2
+    g = torch.Generator().manual_seed(dim)
+    T = sum(n for _, n in runs)
+    q = (torch.randn(T, Hq, dim, generator=g) * 2.0 ** torch.randint(0, 4, (T, Hq, 1), generator=g)).bfloat16().cuda()
+    vals = {"sinks": torch.randn(Hq, generator=g), "slopes": torch.rand(Hq, generator=g) * 0.05,
+            "gate": torch.randn(T, Hq * dim, generator=g).bfloat16()}
+    kw = {k: vals[k].cuda() if v is True else v for k, v in opts.items()}
+    keys, values = (torch.randn(len(runs), Hkv, 512, dim, generator=g).bfloat16() for _ in range(2))  # [sequence, head, key]
+    out = []
+    for bs in (64, 32, 16, 8):
+        m, pages = _meta(runs, bs, "cuda")
+        cache = torch.zeros(pages, Hkv, bs, 2 * dim).bfloat16()
+        for i, (e, n) in enumerate(runs):
+            for p in range(-(-(e + n) // bs)):
+                c = cache[int(m.tables[i, p])].view(Hkv, -1)
+                c[:, :bs * dim] = keys[i, :, p * bs:(p + 1) * bs].reshape(Hkv, -1)
+                c[:, bs * dim:] = values[i, :, p * bs:(p + 1) * bs].transpose(1, 2).reshape(Hkv, -1)
+        out.append(sm.grouped_attention(q, cache.cuda(), dim, dim, dim ** -0.5, m, **kw))
+    assert all(torch.equal(out[0], o) for o in out[1:])
