@@ -413,17 +413,23 @@ __device__ __forceinline__ f32x4_t mul_add4(const f32x4_t a, const f32x4_t b, f3
   return c;
 }
 
-// The chunk's values, transposed: vt[column][token], zeros past the chunk's end and past dv.
+// The chunk's values, transposed: vt[column][token], zeros past the chunk's end and past dv. Returns whether this lane's
+// are all finite.
 template <int NVT>
-__device__ __forceinline__ void stage_values(const bf16_t* row, bool there, int dv, bool vec, int kq, int tok, float* vt) {
+__device__ __forceinline__ bool stage_values(const bf16_t* row, bool there, int dv, bool vec, int kq, int tok, float* vt) {
+  float zero = 0.f;
 #pragma unroll
   for (int n = 0; n < NVT; ++n) {
     const int col = 16 * n + 4 * kq;
     f32x4_t v = {0.f, 0.f, 0.f, 0.f};
     if (there && col < dv) v = load4(row + col, dv - col, vec && col + 4 <= dv);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) vt[(col + j) * CS + tok] = v[j];
+    for (int j = 0; j < 4; ++j) {
+      vt[(col + j) * CS + tok] = v[j];
+      zero = __builtin_fmaf(v[j], 0.f, zero);  // NaN from an infinity or a NaN
+    }
   }
+  return zero == 0.f;
 }
 
 // Every chunk's own state contribution, transposed ([dv][KD], KD = 16 NKS, zeros past dk), and the product of its decays [KD].
@@ -560,7 +566,7 @@ __global__ __launch_bounds__(NT) void hgrn2_read_kernel(const bf16_t* __restrict
       for (int j = 0; j < 4; ++j) qh[ks][j] = Fn<bf16_t>::silu(raw[j]);
     }
   }
-  stage_values<NVT>(row + 2 * H * dk + h * dv, there, dv, vec != 0, kq, tok, vt);
+  const bool finite = stage_values<NVT>(row + 2 * H * dk + h * dv, there, dv, vec != 0, kq, tok, vt);
 
   // scores of query r16 against the keys 4 kq + r of the own block
   f32x4_t same = {0.f, 0.f, 0.f, 0.f}, at1 = same, at2 = same, at4 = same, at8 = same;
@@ -596,7 +602,32 @@ __global__ __launch_bounds__(NT) void hgrn2_read_kernel(const bf16_t* __restrict
     for (int m = 0; m < NVT; ++m)
       o[m] = mul_add4(*reinterpret_cast<const f32x4_t*>(vt + (16 * m + r16) * CS + 16 * b + 4 * kq), w, o[m]);
   };
-  values(wave, sc);
+  if (__all(finite)) {
+    values(wave, sc);
+  } else {
+    // the own block's later tokens have weight 0, and 0 times an infinity would spoil the earlier ones: finite values as
+    // above, the others token by token
+    auto usual = [](float v) { return __builtin_fabsf(v) < INFINITY; };
+#pragma unroll
+    for (int m = 0; m < NVT; ++m) {
+      f32x4_t v = *reinterpret_cast<const f32x4_t*>(vt + (16 * m + r16) * CS + 16 * wave + 4 * kq);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = usual(v[j]) ? v[j] : 0.f;
+      o[m] = mul_add4(v, sc, o[m]);
+    }
+#pragma unroll 1
+    for (int s = 0; s < 16; ++s) {
+      const float mine = (s & 2) ? ((s & 1) ? sc[3] : sc[2]) : ((s & 1) ? sc[1] : sc[0]);
+      const float w = __shfl(mine, (s >> 2) * 16 + r16, 64);
+#pragma unroll
+      for (int m = 0; m < NVT; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float v = vt[(16 * m + 4 * kq + r) * CS + 16 * wave + s];
+          if (s <= r16 && !usual(v)) o[m][r] += w * v;
+        }
+    }
+  }
   for (int b = wave - 1; b >= 0; --b) {  // qh: from here on with the decays back to the end of block b
     f32x4_t a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll

@@ -36,3 +36,26 @@ def test_hgrn2_prompts(H, dk, dv, lower, shift, lens, monkeypatch):
     scale = want.view(T, H, dv).abs().amax(-1, keepdim=True).expand(T, H, dv).reshape(T, H * dv)
     assert ((o - want).abs() <= 2 ** -8 * want.abs() + 2e-5 * (1 + scale)).all()
     assert (st - ws).abs().max() <= 2e-5 * ws.abs().max()  # up to 128 steps of one rounding each, hardware exponentials
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("at", [0, 7, 15, 16, 70, 98])
+def test_later_values_do_not_reach_earlier_tokens(at, bad):
+    """An infinite or undefined value changes its own token and those after it, in its head, and nothing else."""
+    from llmd_amd.ops import seqmix as sm
+
+    T, H, dk, dv = 99, 2, 64, 40
+    g = torch.Generator().manual_seed(at)
+    p = torch.randn(T, H * (2 * dk + dv), generator=g).bfloat16().cuda()
+    fb, low, nw = torch.randn(H * dk, generator=g).cuda(), torch.rand(H * dk, generator=g).cuda(), torch.ones(dv).bfloat16().cuda()
+    out = []
+    for v in (0.5, bad):
+        p[at, 2 * H * dk + dv + 3] = v  # head 1, column 3
+        m, _ = _meta([(0, T)], 64, "cuda")
+        st = torch.zeros(1, H, dk, dv, device="cuda")
+        out.append((sm.hgrn2_scan(p, H, dk, dv, fb, low, nw, 1e-5, st, m).view(T, H, dv), st))
+    (want, ws), (got, gs) = out
+    assert torch.equal(got[:at], want[:at]) and torch.equal(got[:, 0], want[:, 0]) and torch.equal(gs[:, 0], ws[:, 0])
+    assert not got[at:, 1, 3].isfinite().any() and not gs[0, 1, :, 3].isfinite().any()
+    other = torch.arange(dv) != 3
+    assert torch.equal(gs[0, 1][:, other], ws[0, 1][:, other])
