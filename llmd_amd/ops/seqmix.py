@@ -542,8 +542,8 @@ HGRN2_CHUNKED = os.environ.get("LLMD_HGRN2_CHUNKED", "1") == "1"
 # scanned one. 32 heads x 64 x 64, one run of 64 tokens: 31 us token by token, 29 in chunks on the matrix cores (beside 16
 # single tokens 41 / 45); of 100: 44 / 30 (beside 8: 52 / 41); of 128: 59 / 30, scanned chunks 74, which gain from 256 on
 HGRN2_CHUNK_FROM = int(os.environ.get("LLMD_HGRN2_CHUNK_FROM", "0"))
-# tokens per chunk: at most 64, the matrix-core form's four blocks of 16
-HGRN2_CHUNK_LEN = min(64, int(os.environ.get("LLMD_HGRN2_CHUNK_LEN", "64")))
+# tokens per chunk; the matrix-core form's chunks are four blocks of 16 at most, longer ones are for the scanned form
+HGRN2_CHUNK_LEN = int(os.environ.get("LLMD_HGRN2_CHUNK_LEN", "64"))
 
 
 def hgrn2_scan(p, H: int, dk: int, dv: int, f_bias, lower, norm_w, eps: float, state, seq):
@@ -565,9 +565,10 @@ def hgrn2_scan(p, H: int, dk: int, dv: int, f_bias, lower, norm_w, eps: float, s
         return ref.hgrn2_scan(p, H, dk, dv, f_bias, lower, norm_w, eps, state, seq.seq_start, seq.seq_slot,
                               seq.seq_init, out)
     chunks, nc, nd = None, 0, 0
-    chunk_from = HGRN2_CHUNK_FROM or (96 if p.dtype == torch.bfloat16 and dk <= 128 and dv <= 128 else 256)
+    matrix = p.dtype == torch.bfloat16 and dk <= 128 and dv <= 128
+    chunk_from = HGRN2_CHUNK_FROM or (96 if matrix else 256)
     if HGRN2_CHUNKED and seq.q_lens is not None and seq.max_q >= max(2, chunk_from):
-        chunks, nc = seq.scan_chunks(HGRN2_CHUNK_LEN)
+        chunks, nc = seq.scan_chunks(min(64, HGRN2_CHUNK_LEN) if matrix else HGRN2_CHUNK_LEN)
         nd = next(i for i, n in enumerate(seq.q_lens) if n != 1)
     native().hgrn2_scan(p, int(H), int(dk), int(dv), f_bias, lower, norm_w, float(eps), state, seq.seq_start,
                         seq.seq_slot, seq.seq_init, out, chunks, nc, nd)

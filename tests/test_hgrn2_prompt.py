@@ -59,3 +59,33 @@ def test_later_values_do_not_reach_earlier_tokens(at, bad):
     assert not got[at:, 1, 3].isfinite().any() and not gs[0, 1, :, 3].isfinite().any()
     other = torch.arange(dv) != 3
     assert torch.equal(gs[0, 1][:, other], ws[0, 1][:, other])
+
+
+@pytest.mark.parametrize("dtype,dk", [(torch.float32, 32), (torch.bfloat16, 32), (torch.bfloat16, 130)], ids=str)
+def test_chunk_length_option(dtype, dk):
+    """Chunks above 64 tokens (LLMD_HGRN2_CHUNK_LEN, read at import) for the scanned form; the matrix-core form keeps its 64."""
+    import os
+    import subprocess
+    import sys
+
+    code = f"""
+import torch
+from test_grouped_f32 import _meta
+from llmd_amd.ops import seqmix as sm
+T, H, dk, dv, dt = 300, 2, {dk}, 16, {dtype}
+g = torch.Generator().manual_seed(1)
+p = torch.randn(T, H * (2 * dk + dv), generator=g).to(dt)
+fb, low, nw = torch.randn(H * dk, generator=g), torch.rand(H * dk, generator=g), torch.ones(dv).to(dt)
+out = []
+for dev in ("cpu", "cuda"):
+    m, _ = _meta([(0, T)], 64, dev)
+    w = (lambda x: x.float()) if dev == "cpu" else (lambda x: x.cuda())
+    out.append(sm.hgrn2_scan(w(p), H, dk, dv, w(fb), w(low), w(nw), 1e-5, torch.zeros(1, H, dk, dv, device=dev), m).float().cpu())
+assert list(m._chunks) == [{100 if dtype == torch.float32 or dk > 128 else 64}], list(m._chunks)
+# bf16 results: 2^-9 of each; fp32 sums of up to 130 products of values of the size of the head's largest
+scale = out[0].abs().max()
+assert ((out[1] - out[0]).abs() <= ({2 ** -8 if dtype == torch.bfloat16 else 0.0}) * out[0].abs() + 2e-5 * (1 + scale)).all()
+"""
+    env = dict(os.environ, LLMD_HGRN2_CHUNK_LEN="100", PYTHONPATH=os.pathsep.join(sys.path))
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
