@@ -1093,7 +1093,7 @@ class ModelRunner:
             with torch.cuda.graph(g, pool=pool):
                 h = self.model(buf[:B], meta)
             self.graphs[B] = (g, h, buf, meta)
-        self._graph_constants = self._seq_constants
+        self._graph_constants = self._graph_warned = self._seq_constants
         torch.cuda.synchronize()
         log.info("captured %d decode graphs in %.1fs", len(buckets), time.time() - t0)
 
@@ -1116,8 +1116,15 @@ class ModelRunner:
 
     def _seq_graph_ok(self, pl: dict) -> bool:
         """A captured step of its size is there, made for contexts this long and with the model's present constants."""
-        return 0 < pl["nd"] == len(pl["ids"]) and self._graph_ok(pl["nd"]) and self._graph_constants == self._seq_constants and \
-            max(pl["pos"], default=0) < self.max_model_len
+        if not (0 < pl["nd"] == len(pl["ids"]) and self._graph_ok(pl["nd"]) and max(pl["pos"], default=0) < self.max_model_len):
+            return False
+        if self._graph_constants == self._seq_constants:
+            return True
+        if self._graph_warned != self._seq_constants:
+            self._graph_warned = self._seq_constants
+            log.warning("the model's constants were rebuilt after its decode steps were captured: steps run launch by launch "
+                        "until capture_graphs() is called again")
+        return False
 
     def _run_seq_graph(self, pl: dict) -> torch.Tensor:
         n = pl["nd"]

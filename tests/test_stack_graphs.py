@@ -68,3 +68,34 @@ def test_replayed_steps(name, dtype, tmp_path):
 
 def test_new_constants_are_not_replayed(tmp_path):
     assert _serve("tiny-kakalorn", "float32", False, tmp_path, lens=(5,), new=(6,), new_constants=True)[2] == 0
+
+
+def test_new_constants_are_reported(tmp_path, caplog):
+    """Steps that leave their graphs because the constants are newer say so once; captured again, they are replayed."""
+    import logging
+
+    from llmd_amd.engine.config import EngineConfig
+    from llmd_amd.engine.engine import LLMEngine
+    from llmd_amd.engine.request import SamplingParams
+
+    cfg = EngineConfig.create("tiny-koduzen", device="cuda", dtype="float32", block_size=64, num_gpu_blocks=8, max_num_seqs=1,
+                              max_model_len=100, max_num_batched_tokens=64, enable_prefix_caching=False)
+    eng = LLMEngine(cfg)
+    replays, replay = [], eng.runner._run_seq_graph
+    eng.runner._run_seq_graph = lambda pl: replays.append(1) or replay(pl)
+
+    def serve(name):
+        del replays[:]
+        caplog.clear()
+        with caplog.at_level(logging.WARNING):
+            r = eng.add_request(name, [3, 1, 2], SamplingParams(max_tokens=6, temperature=0.0, ignore_eos=True))
+            while eng.has_unfinished():
+                eng.step()
+        return r.output_token_ids, len(replays), sum("captured" in m.getMessage() for m in caplog.records)
+
+    toks, n, said = serve("a")
+    assert n == 5 and said == 0
+    eng.runner.model.finalize()
+    assert serve("b") == (toks, 0, 1) and serve("c") == (toks, 0, 0)
+    eng.runner.capture_graphs()
+    assert serve("d") == (toks, 5, 0)
