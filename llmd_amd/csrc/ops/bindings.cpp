@@ -7,6 +7,7 @@
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <pybind11/stl.h>
 
 #include <map>
@@ -886,7 +887,7 @@ void moe_group(torch::Tensor ids, int64_t E, torch::Tensor slot_pair, torch::Ten
   CHECK_CUDA(ids); CHECK_DT(ids, at::kInt); CHECK_DT(slot_pair, at::kInt); CHECK_DT(tiles, at::kInt); CHECK_DT(inv, at::kInt);
   const int64_t n = ids.numel(), mt = tiles.numel() / 3;
   TORCH_CHECK(ids.is_contiguous() && E >= 1 && E <= 4096 && inv.numel() >= n && slot_pair.numel() == mt * 128 &&
-                  mt * 128 >= n + E * 127, "moe_group buffers");
+                  mt >= (n + std::min(E, n) * 127) / 128, "moe_group buffers");
   torch::Tensor hist = torch::empty({llmd_moe_sort_scratch(n, E)}, ids.options());
   llmd_moe_group(ids.data_ptr<int>(), n, E, hist.data_ptr<int>(), slot_pair.data_ptr<int>(), tiles.data_ptr<int>(), inv.data_ptr<int>(),
                  cur_stream());

@@ -6,6 +6,7 @@
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
+#include <algorithm>
 
 extern "C" {
 void sm_embed_scale(const int64_t*, const void*, float, float*, float*, int, int, int64_t, int, hipStream_t);
@@ -624,7 +625,7 @@ void moe_group(Tensor ids, int64_t E, int64_t tm, Tensor slot_row, Tensor tiles,
   CHECK_I32(pair_slot);
   const int64_t n = ids.numel(), mt = tiles.numel() / 3;
   TORCH_CHECK((tm == 64 || tm == 128) && E >= 1 && E <= 8192, "tile rows, experts");
-  TORCH_CHECK(slot_row.numel() == mt * tm && pair_slot.numel() == n && mt * tm >= n + E * (tm - 1),
+  TORCH_CHECK(slot_row.numel() == mt * tm && pair_slot.numel() == n && mt >= (n + std::min(E, n) * (tm - 1)) / tm,
               "tile tables too small for n pairs over E experts");
   Tensor hist = torch::empty({sm_moe_sort_scratch(n, E)}, ids.options());
   sm_moe_group(ids.data_ptr<int>(), n, E, tm, hist.data_ptr<int>(), slot_row.data_ptr<int>(), tiles.data_ptr<int>(), pair_slot.data_ptr<int>(),

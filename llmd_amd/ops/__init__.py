@@ -1024,7 +1024,7 @@ def moe_experts(x, ids, wts, w1, w2, act=0, alpha=1.702, limit=7.0, out=None, b1
     if (MOE_SMALL and not v3 and act == ACT_SILU and b1 is None and b2 is None and C.moe_small_ok(x, w1)
             and C.moe_small_ok(w2[0], w2) and E <= 4096):
         # decode-sized steps: tiles of 128 slots, the weights' stream straight to the products' registers (csrc/ops/moe_tile.hip)
-        mt = (n + E * 127) // 128 + 1
+        mt = max(1, (n + min(E, n) * 127) // 128)  # every expert that has rows may leave one tile partly filled
         slot_pair = torch.empty(mt * 128, dtype=torch.int32, device=x.device)
         tiles = torch.empty(1 + 3 * mt, dtype=torch.int32, device=x.device)
         inv = torch.empty(n, dtype=torch.int32, device=x.device)  # -1 = not on this rank

@@ -204,7 +204,7 @@ def _moe_tables(C, ids, E: int, h, w1, w2):
     form takes."""
     n = ids.numel()
     tm = 128 if C.moe_tiled(h, w1) and C.moe_tiled(w2[0], w2) else 64
-    max_tiles = (n + E * (tm - 1)) // tm + 1
+    max_tiles = max(1, (n + min(E, n) * (tm - 1)) // tm)  # every expert that has rows may leave one tile partly filled
     slot_row = torch.empty(max_tiles * tm, dtype=torch.int32, device=h.device)
     tiles = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=h.device)
     pair_slot = torch.empty(n, dtype=torch.int32, device=h.device)   # -1: identity expert

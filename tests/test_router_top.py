@@ -84,3 +84,24 @@ def test_align_tables(bm):
     assert torch.equal(srt[inv[ok]], ok) and int((srt >= 0).sum()) == len(ok)
     first = offs[ids[ok].long()]
     assert (inv[ok] >= first).all() and (inv[ok] < first + cnt[ids[ok].long()]).all()
+
+
+@pytest.mark.parametrize("n,E", [(100, 1025), (4097, 1025), (100, 4096), (4097, 4096), (1, 4096)])
+def test_align_tables_of_many_experts(n, E):
+    """More experts than a workgroup has threads, on both sides of the line to many workgroups."""
+    from llmd_amd import ops
+
+    bm = 64
+    ids = torch.randint(-1, E, (n,), generator=torch.Generator().manual_seed(n + E)).int()
+    max_p = (n + E * (bm - 1) + bm - 1) // bm * bm
+    t = lambda m: torch.full((m,), 7, dtype=torch.int32, device="cuda")  # noqa: E731
+    srt, tile_e, offs, total, inv = t(max_p), t(max_p // bm), t(E + 1), t(1), t(n)
+    ops.native().moe_align(ids.cuda(), E, srt, tile_e, offs, total, inv, bm)
+    srt, tile_e, offs, inv = (x.cpu().long() for x in (srt, tile_e, offs, inv))
+    cnt = torch.bincount(ids[ids >= 0].long(), minlength=E)
+    seg = (cnt + bm - 1) // bm * bm
+    assert torch.equal(offs, torch.cat([torch.zeros(1, dtype=torch.long), seg.cumsum(0)])) and int(total) == int(seg.sum())
+    assert torch.equal(tile_e[:int(total) // bm], torch.repeat_interleave(torch.arange(E), seg // bm))
+    assert (tile_e[int(total) // bm:] == -1).all() and torch.equal(inv < 0, ids < 0)
+    ok = (ids >= 0).nonzero()[:, 0]
+    assert torch.equal(srt[inv[ok]], ok) and int((srt >= 0).sum()) == len(ok)
