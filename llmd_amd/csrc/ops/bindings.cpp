@@ -489,8 +489,8 @@ int64_t mla_v2_shape(int64_t R, bool fp8) { return llmd_mla_v2_shape((int)R, fp8
 
 bool skinny_supported(int64_t M, int64_t rb, int64_t occ) { return llmd_dgemm_supported((int)M, (int)rb, (int)occ); }
 
-// y [M, N] = x [M, K] . w [N, K]^T for 33 <= M <= 256 (decode batches of a P/D
-// decode replica): LDS-DMA staged tiles of 64 wrb W rows x all M, nsplit-way
+// y [M, N] = x [M, K] . w [N, K]^T for up to 256 rows (decode batches of a P/D
+// decode replica, smaller ones of unlisted shapes): LDS-DMA staged tiles of 64 wrb W rows x all M, nsplit-way
 // split-K, 3- or 4-stage ring (csrc/ops/mgemm.hip)
 // Split-K fixup counters of mgemm (csrc/ops/mgemm.hip): per device 256 slabs of 1024 zeroed ints, handed
 // out round-robin so kernels in flight on different streams (DBO, TP overlap) never share a slab; each

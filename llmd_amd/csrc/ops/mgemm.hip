@@ -1,6 +1,6 @@
-// Medium-M decode GEMM: Y[M, N] = X[M, K] . W[N, K]^T for M = 33..128 (a decode
-// batch on a P/D decode replica: 64-128 rows per step), bf16 in,
-// fp32 accumulate, bf16 out.
+// Medium-M decode GEMM: Y[M, N] = X[M, K] . W[N, K]^T for M = 33..256 (a decode
+// batch on a P/D decode replica: 64-128 rows per step), bf16 in, fp32 accumulate,
+// bf16 out. Shapes that no table lists come with 1..64 rows (ops.decode_rule).
 //
 // Why not skinny_gemm.hip's structure: there every wave streams its own K range
 // of W straight to VGPRs and loads X fragments itself, so X traffic is M / R of

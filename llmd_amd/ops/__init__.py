@@ -1216,8 +1216,8 @@ def dgemm_choice(M: int, N: int, K: int) -> Optional[tuple[int, int, int]]:
 
 
 def mgemm(x: torch.Tensor, w: torch.Tensor, plan: tuple[int, int, int]) -> torch.Tensor:
-    """Y = X W^T for 33 <= M <= 256 on the LDS-DMA medium-M decode GEMM
-    (csrc/ops/mgemm.hip); plan = (wrb: 64-row W tiles per workgroup, nsplit,
+    """Y = X W^T for up to 256 rows on the LDS-DMA medium-M decode GEMM
+    (csrc/ops/mgemm.hip, made for 33 and more: fewer fill a block of 32); plan = (wrb: 64-row W tiles per workgroup, nsplit,
     stages)."""
     M, K = x.shape
     N = w.shape[0]
@@ -1461,18 +1461,26 @@ def pgemm_wins(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, bool]]:
 
 def decode_rule(M: int, N: int, K: int):
     """Kernel and plan for a decode-sized projection that no measured table lists, or None for hipBLASLt.
-    1x MI355X, weights cold in HBM, hipBLASLt / here in us:
+    1x MI355X, weights cold in HBM, launches one behind the other, hipBLASLt / here in us:
 
     * M <= 16 and weights up to 32 MB: the stream kernel, whose workgroups of 16 rb weight rows are at most one
       per CU, and two K ranges where they would fill half of the CUs. (2048, 2048) 11.0 / 6.3 at M 8, 11.0 / 7.1
       at 16; (6144, 2048) 12.6 / 8.6 and 12.6 / 9.6; (4096, 4096) 15.8 / 9.7 and 15.7 / 11.1. Long rows of x cost
       it more than the weights: (2560, 8192) 13.6 / 15.2, (2048, 5632) 10.7 / 11.4 at 16, so from K 4096 on only
-      narrow outputs: (1024, 8192) 11.9 / 9.3.
+      narrow outputs, which it takes up to 64 MB: (1024, 8192) 11.9 / 9.3, (1024, 16384) 20.3 / 11.1 at M 1 and
+      21.1 / 13.8 at 16, (512, 32768) 66.5 / 12.3 and 66.5 / 15.0.
     * M 17 .. 64, and fewer rows on larger weights: the LDS-DMA kernel with 64-row tiles, four stages and K ranges
       of at least eight steps that make up to 256 workgroups; its time hardly depends on M. (2048, 2048) 11.0 / 7.7
-      at M 17, 11.7 / 8.9 at 64; (4096, 4096) 15.2 / 13.1 at 64; (16384, 4096) 32.6 / 24.2 and 33.9 / 26.5;
-      (32000, 2048) 34.2 / 24.0 and 33.9 / 28.4. Worst measured: (9216, 3072), whose 144 tiles leave CUs idle,
-      15.9 / 16.7 at 17, 20.7 / 19.6 at 64."""
+      at M 17, 11.7 / 8.9 at 64; (4096, 4096) 15.2 / 13.1 at 64; (16384, 4096) 32.4 / 24.0 at M 1, 32.6 / 24.2 at
+      17, 33.9 / 26.5 at 64; (32000, 2048) 32.3 / 24.0, 34.2 / 24.0, 33.9 / 28.4.
+    * 129 .. 170 tiles leave CUs idle: three K ranges, which still run two workgroups to a CU, where the rows of the
+      weights are long and the partial sums small (K >= 3072, M <= 32). (9216, 3072) 18.5 / 14.0 at M 1, 15.9 / 15.2
+      at 17, 16.9 / 17.0 at 32, with one range 16.3, 16.7 and 17.1; (9216, 4096) at 17 20.1 / 19.3, one range 20.8.
+    * 257 .. 415 tiles are a full round of the chip and a sparse one: from M 17 on hipBLASLt. (18432, 3072) 26.8 /
+      28.5 at 17, 30.7 / 36.6 at 64; (24576, 3072) 31.4 / 30.9 and 34.3 / 38.6; at M 16 64.4 / 28.4 and 49.4 / 30.6.
+      With 432 tiles, (27648, 2048), 28.9 / 22.0 at 17 and 29.5 / 27.0 at 64.
+
+    Worst measured: (28672, 3072) at 64 36.7 / 39.7 (46.5 / 36.7 at 48), (12800, 2560) at 64 18.9 / 19.7."""
     if N % 4 or K % 64 or K < 768 or not 1 <= M <= 64:  # (2048, 768), the smallest measured: 6.3 / 4.3 at M 8, 9.5 / 6.8 at 64
         return None
     if M <= 16 and N * K <= (1 << 25 if K > 4096 else 1 << 24):
@@ -1481,7 +1489,12 @@ def decode_rule(M: int, N: int, K: int):
         rb = min(8, -(-N // 4096))
         ns = max(1, min(256 // -(-N // (16 * rb)), K // 2048))
         return skinny_gemm, (rb, ns, 2 if native().skinny_supported(M, rb, 2) else 1)
-    return mgemm, (1, max(1, min(256 // -(-N // 64), K // 512)), 4)
+    tiles = -(-N // 64)
+    if M > 16 and 256 < tiles < 416:
+        return None
+    if 128 < tiles <= 170 and K >= 3072 and M <= 32:
+        return mgemm, (1, 3, 4)
+    return mgemm, (1, max(1, min(256 // tiles, K // 512)), 4)
 
 
 def _listed(M: int, N: int, K: int) -> bool:
@@ -1495,7 +1508,7 @@ def _listed(M: int, N: int, K: int) -> bool:
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Dense projection: decode-sized M on our decode GEMM kernels where their
     measured dispatch tables have them ahead of hipBLASLt - the medium-M LDS-DMA
-    kernel (csrc/ops/mgemm.hip, M 33..128, ops/mgemm_table.py) first, then the
+    kernel (csrc/ops/mgemm.hip, M 33..256, ops/mgemm_table.py) first, then the
     stream kernel (csrc/ops/skinny_gemm.hip, M <= 64, ops/dgemm_table.py), unlisted
     shapes by ``decode_rule`` (without a bias, which hipBLASLt adds for nothing) -
     prefill-sized M on the prefill GEMM where the shipped table (ops/pgemm_table.py)
