@@ -573,8 +573,8 @@ bool grouped_attention_mfma(Tensor q, Tensor cache, int64_t dim, int64_t vdim, T
     TORCH_CHECK(part_o && part_ml && split_keys > 0 && split_keys % 32 == 0, "split workspace");
     CHECK_F32(*part_o);
     CHECK_F32(*part_ml);
-    TORCH_CHECK(part_o->numel() >= n * Hkv * nsplit * 64 * vdim && part_ml->numel() >= n * Hkv * nsplit * 128,
-                "split workspace too small");
+    const int64_t rows = n * Hkv * nsplit * (is_f32(q) ? q.size(1) / Hkv : 64);
+    TORCH_CHECK(part_o->numel() >= rows * vdim && part_ml->numel() >= rows * 2, "split workspace too small");
     po = part_o->data_ptr<float>();
     pm = part_ml->data_ptr<float>();
   }

@@ -23,7 +23,8 @@
 //   blockIdx.z; a merge kernel joins them.
 // grouped_attention_f32 (fp32, sizes up to 256): the same structure on v_mfma_f32_16x16x4_f32.
 // All forms multiply the result by sigmoid(gate) when a gate is given. A row's result depends
-// only on its own keys and the fixed tile sizes.
+// only on its own keys and the fixed tile sizes; in bf16 steps of single tokens also on the ranges that the
+// step's size cuts the keys into.
 // Score options of all forms (each may be off): slopes [Hq] - the score of query i and key j loses
 // slopes[h] (i - j); chunk - query i sees only keys j >= (i / chunk) chunk; sinks [Hq] - one more
 // score per head that enters the softmax's denominator and has no value (the running maximum and
@@ -1469,13 +1470,43 @@ __global__ __launch_bounds__(NT, NKS <= 2 ? 3 : NKS <= 4 ? 2 : 1) void grouped_d
 // 16-byte piece of a (transposed) value column. Exponentials are expf, as in the FMA form. DkP = 16 NKS >= dim, VP = 16 NCB.
 // A 700-token prompt, 32 heads x 128 over 4 kv heads: 1537 us with the FMA form, now 112 us (128 matrix instructions of
 // 32 cycles per wave and tile).
+//
+// A row's result is the same in every step, whatever else the step holds. The softmax runs over ranges of FR keys at fixed places
+// of the sequence; a range's maximum, sum and products are joined to those of the ranges before it, in order. A step of few
+// single tokens runs the ranges as workgroups of their own (blockIdx.z) and joins them in a second kernel, with the same
+// operations in the same order. One token over 700 and 4000 keys, 32 heads x 128 over 4 kv heads: 30 and 37 us, in one
+// workgroup per kv head 100 and 517; 16 tokens over 700 38 us, over 4000 154. Ranges of 256 keys: 45, 49, 53 and 115 us.
+constexpr int FR = 128;
+
+// The ranges that a row (or an item, by its last one) of ``len`` keys meets, numbered without those that lie in the gap between
+// the kept first tokens and the window: ``kept`` ones from the sequence's start, then those from ``first`` on.
+struct Ranges {
+  int kept, first, count;
+  __device__ __forceinline__ Ranges(int len, int kbase, int keepT, int gap) {
+    const int all = (len - 1) / FR + 1;
+    kept = min((keepT + FR - 1) / FR, all);
+    first = max(kept, max(kbase, keepT + gap) / FR);
+    count = kept + max(0, all - first);
+  }
+  __device__ __forceinline__ int place(int z) const { return z < kept ? z : first + z - kept; }
+};
+
+// One more range (m, l): its weight against what is there (mt, lt), which is brought to the new maximum.
+__device__ __forceinline__ void join(float& mt, float& lt, float m, float l, float& was, float& now) {
+  const float M = fmaxf(mt, m), ref = M == -INFINITY ? 0.f : M;
+  was = expf(mt - ref);
+  now = expf(m - ref);
+  lt = __builtin_fmaf(lt, was, l * now);
+  mt = M;
+}
+
 template <int NKS, int NCB>
 __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ cache, const int* __restrict__ tables, int W, int bs,
     const int* __restrict__ items, const int* __restrict__ row_len, float scale, int Hq, int Hkv, int dim, int vdim,
-    const float* __restrict__ gate, int64_t gate_stride, float* __restrict__ out, int split_keys,
-    float* __restrict__ part_o, float* __restrict__ part_ml, const float* __restrict__ slopes, int chunk,
-    const float* __restrict__ sinks, int window, int keep, const int* __restrict__ longest) {
+    const float* __restrict__ gate, int64_t gate_stride, float* __restrict__ out, float* __restrict__ part_o,
+    float* __restrict__ part_ml, const float* __restrict__ slopes, int chunk, const float* __restrict__ sinks, int window,
+    int keep) {
   constexpr int DkP = 16 * NKS, VP = 16 * NCB;
   constexpr int KS = DkP + 4, VS = MKT + 4;      // LDS row strides: 16 rows' pieces take all banks
   constexpr int NBUF = NKS <= 8 ? 2 : 1;         // as in the bf16 form
@@ -1512,7 +1543,7 @@ __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_ke
   for (int e = threadIdx.x; e < NBUF * VP * VS; e += NT) sVt[e] = 0.f;
 
   const bool vec = (dim & 3) == 0;  // key and query rows are 16-byte multiples (value columns always: bs % 8 == 0)
-  f32x4_t qf[NKS], o[NCB];
+  f32x4_t qf[NKS], o[NCB], ot[NCB];  // o: the present range's, ot: those joined so far
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
@@ -1521,17 +1552,21 @@ __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_ke
       qf[ks][j] = (mylen > 0 && d < dim) ? q[((int64_t)mytok * Hq + myhead) * dim + d] * scale : 0.f;
     }
 #pragma unroll
-  for (int n = 0; n < NCB; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const bool sk = sinks != nullptr && blockIdx.z == 0;  // a sink is a score that is already counted (by the first key range only)
-  float m = sk ? sinks[myhead] : -INFINITY, l = sk ? 1.f : 0.f;
+  for (int n = 0; n < NCB; ++n) o[n] = ot[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  float mt = sinks ? sinks[myhead] : -INFINITY, lt = sinks ? 1.f : 0.f;  // a sink is a score that is already counted
   const int* bt = tables + (int64_t)seq * W;
-  const int nsplit = gridDim.z;
-  if (nsplit > 1) {
-    if ((int)blockIdx.z >= ranges_used(longest, nsplit, split_keys)) return;
-    split_keys = range_keys(longest, nsplit, split_keys);
+  const bool alone = gridDim.z > 1;  // this workgroup takes one range
+  int kbeg = kbase, kend = vlen;
+  if (alone) {
+    const Ranges rs(maxlen, kbase, keepT, gap);
+    if ((int)blockIdx.z >= rs.count) return;
+    // places of the sequence in the numbering without the gap
+    auto without_gap = [&](int p) { return p < keepT ? p : max(keepT, p - gap); };
+    const int at = rs.place(blockIdx.z) * FR;
+    kbeg = max(kbase, without_gap(at));
+    kend = min(vlen, without_gap(at + FR));
   }
-  const int kbeg = nsplit > 1 ? kbase + blockIdx.z * split_keys : kbase;
-  const int kend = nsplit > 1 ? min(vlen, kbeg + split_keys) : vlen;
   constexpr int CK = DkP / 4, NCK = (MKT * CK + NT - 1) / NT;  // pieces per key row, per thread
   constexpr int CV = MKT / 4, NCV = (VP * CV + NT - 1) / NT;   // pieces per value column (4 keys each), per thread
   const bool one_page = (bs % MKT) == 0;                       // a tile lies inside one page
@@ -1588,9 +1623,29 @@ __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_ke
     if (kbeg + MKT < kend) fetch(key_of(kbeg + MKT));
     __syncthreads();
   }
-  int it = 0;
+  auto next_range = [&] {
+    float was, now;
+    join(mt, lt, m, l, was, now);
+    // the accumulators hold rows 4 kq + r: their factors come from the lane that owns the row
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float a = __shfl(was, kq * 4 + r, 64), b = __shfl(now, kq * 4 + r, 64);
+#pragma unroll
+      for (int n = 0; n < NCB; ++n) {
+        ot[n][r] = __builtin_fmaf(ot[n][r], a, o[n][r] * b);
+        o[n][r] = 0.f;
+      }
+    }
+    m = -INFINITY;
+    l = 0.f;
+  };
+  int it = 0, range = kbeg < kend ? key_of(kbeg) / FR : 0;
   for (int v0 = kbeg; v0 < kend; v0 += MKT, ++it) {
     const int k0 = key_of(v0);
+    if (k0 / FR != range) {
+      range = k0 / FR;
+      if (any_row) next_range();
+    }
     const int cur = NBUF == 2 ? (it & 1) : 0;
     if (NBUF == 1) {
       __syncthreads();  // the previous tile is no longer read (first time: the zero fill is done)
@@ -1669,41 +1724,67 @@ __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_ke
     }
   }
   // o[n][r] = O[row 16 wave + 4 kq + r][column 16 n + r16]
-  const int64_t pbase = (((int64_t)item * Hkv + g) * nsplit + blockIdx.z) * 64;
-  if (nsplit > 1 && kq == 0) {
-    part_ml[(pbase + wave * 16 + r16) * 2] = m;
-    part_ml[(pbase + wave * 16 + r16) * 2 + 1] = l;
+  const int64_t pbase = (((int64_t)item * Hkv + g) * gridDim.z + blockIdx.z) * G;
+  if (!alone) next_range();
+  else if (kq == 0 && ok) {
+    part_ml[(pbase + myrow) * 2] = m;
+    part_ml[(pbase + myrow) * 2 + 1] = l;
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int row = wave * 16 + kq * 4 + r;
-    const float inv = 1.f / __shfl(l, kq * 4 + r, 64);
-    if (row >= ntok * G && nsplit == 1) continue;
+    const float inv = 1.f / __shfl(lt, kq * 4 + r, 64);
+    if (row >= ntok * G) continue;
     const int64_t tok = tok0 + row / G;
     const int h = g * G + row % G;
 #pragma unroll
     for (int n = 0; n < NCB; ++n) {
       const int col = n * 16 + r16;
       if (col >= vdim) continue;
-      if (nsplit > 1) {
+      if (alone) {
         part_o[(pbase + row) * vdim + col] = o[n][r];
         continue;
       }
-      float v = o[n][r] * inv;
+      float v = ot[n][r] * inv;
       if (gate) v *= 1.f / (1.f + expf(-gate[tok * gate_stride + h * vdim + col]));
       out[(tok * Hq + h) * vdim + col] = v;
     }
   }
 }
 
-// Merge the key-range partials of a split step: out = sum_z b^(m_z - M) o_z / sum_z b^(m_z - M) l_z; the maxima are in
-// base 2 (bf16 forms) or e (fp32).
-template <typename T>
+// Joins the ranges of a step of single tokens (item = token), as next_range does.
+__global__ __launch_bounds__(NT) void grouped_attention_f32_join_kernel(
+    const int* __restrict__ items, const int* __restrict__ row_len, int nsplit, const float* __restrict__ part_o,
+    const float* __restrict__ part_ml, int Hq, int Hkv, int vdim, const float* __restrict__ gate, int64_t gate_stride,
+    float* __restrict__ out, int chunk, const float* __restrict__ sinks, int window, int keep) {
+  const int item = blockIdx.x, g = blockIdx.y, row = blockIdx.z, G = Hq / Hkv;
+  const int64_t tok = items[item * 3 + 1];
+  const int h = g * G + row, len = row_len[tok];
+  const int kbase = chunk > 0 ? (((len - 1) / chunk) * chunk) / MKT * MKT : 0;
+  const int keepT = window > 0 ? (keep + MKT - 1) / MKT * MKT : 0;
+  const int gap = window > 0 ? max(0, max(0, len - window) / MKT * MKT - keepT) : 0;
+  const int nz = min(Ranges(len, kbase, keepT, gap).count, nsplit);
+  const int64_t p0 = ((int64_t)item * Hkv + g) * nsplit * G + row;
+  for (int c = threadIdx.x; c < vdim; c += NT) {
+    float mt = sinks ? sinks[h] : -INFINITY, lt = sinks ? 1.f : 0.f, ot = 0.f;
+    for (int z = 0; z < nz; ++z) {
+      const int64_t p = p0 + (int64_t)z * G;
+      float was, now;
+      join(mt, lt, part_ml[p * 2], part_ml[p * 2 + 1], was, now);
+      ot = __builtin_fmaf(ot, was, part_o[p * vdim + c] * now);
+    }
+    const float inv = 1.f / lt;
+    float v = ot * inv;
+    if (gate) v *= 1.f / (1.f + expf(-gate[tok * gate_stride + h * vdim + c]));
+    out[(tok * Hq + h) * vdim + c] = v;
+  }
+}
+
+// Merge the key-range partials of a split step (bf16): out = sum_z 2^(m_z - M) o_z / sum_z 2^(m_z - M) l_z.
 __global__ __launch_bounds__(NT) void grouped_attention_merge_kernel(
     const int* __restrict__ items, int nsplit, const float* __restrict__ part_o, const float* __restrict__ part_ml,
-    int Hq, int Hkv, int vdim, const T* __restrict__ gate, int64_t gate_stride, T* __restrict__ out, int split_keys,
+    int Hq, int Hkv, int vdim, const bf16_t* __restrict__ gate, int64_t gate_stride, bf16_t* __restrict__ out, int split_keys,
     const int* __restrict__ longest) {
-  auto power = [](float x) { return sizeof(T) == 4 ? expf(x) : exp2f(x); };
   const int item = blockIdx.x, g = blockIdx.y, row = blockIdx.z;
   const int G = Hq / Hkv;
   const int tok0 = items[item * 3 + 1], ntok = items[item * 3 + 2];
@@ -1712,7 +1793,7 @@ __global__ __launch_bounds__(NT) void grouped_attention_merge_kernel(
   const int64_t tok = tok0 + row / G;
   const int h = g * G + row % G;
   merge_ranges<NT>(part_ml + p0 * 2, 128, part_o + p0 * vdim, (int64_t)64 * vdim, ranges_used(longest, nsplit, split_keys), vdim,
-                   power, [&](int c, float v) {
+                   [](float x) { return exp2f(x); }, [&](int c, float v) {
     if (gate) v *= 1.f / (1.f + expf(-ld(gate + tok * gate_stride + h * vdim + c)));
     st(out + (tok * Hq + h) * vdim + c, v);
   });
@@ -1840,9 +1921,10 @@ int sm_grouped_attention(const void* q, const void* cache, const int* tables, in
 }
 
 // single: a step of single tokens (every item is one token): the waves of a workgroup share its rows (bf16).
-// longest: null, or the step's longest context on the device, which then sizes the key ranges (range_keys).
+// longest: null, or the step's longest context on the device, which then sizes the key ranges (range_keys, bf16).
 // Matrix cores, bf16 or (rb 1) fp32. ``rb`` (1 or 2): blocks of 16 rows per wave - items hold up to 64 rb rows;
-// key ranges (nsplit > 1) need rb = 1. Returns 0, or 1 when the sizes are outside the compiled forms
+// key ranges (nsplit > 1) need rb = 1. fp32: nsplit > 1 for single tokens only, with split_keys = FR and at least as many ranges
+// as any row meets; part_o [items, Hkv, nsplit, G, vdim], part_ml [items, Hkv, nsplit, G, 2]. Returns 0, or 1 when the sizes are outside the compiled forms
 // (dim > 256, vdim > 256, group size > 64).
 int sm_grouped_attention_mfma(const void* q, const void* cache, const int* tables, int W, int bs, const int* items,
                               int n_items, const int* row_len, float scale, int Hq, int Hkv, int dim, int vdim,
@@ -1856,21 +1938,19 @@ int sm_grouped_attention_mfma(const void* q, const void* cache, const int* table
   const int G = Hq / Hkv;
   if (f32) {
     const int wide = (std::max(dim, vdim) + 63) / 64;
-    if (rb != 1 || (((uintptr_t)q | (uintptr_t)cache) & 15)) return 1;
+    if (rb != 1 || (nsplit > 1 && (split_keys != FR || !single)) || (((uintptr_t)q | (uintptr_t)cache) & 15)) return 1;
     const dim3 fgrid(Hkv, n_items, nsplit);
-#define SM_GF(N)                                                                                                     \
+#define SM_GF(N)                                                                                                       \
   hipLaunchKernelGGL((grouped_attention_f32_kernel<N, N>), fgrid, dim3(NT), 0, stream, (const float*)q,                \
                      (const float*)cache, tables, W, bs, items, row_len, scale, Hq, Hkv, dim, vdim, (const float*)gate, \
-                     gate_stride, (float*)out, split_keys, part_o, part_ml, slopes, chunk, sinks, window, keep, \
-                     longest)
+                     gate_stride, (float*)out, part_o, part_ml, slopes, chunk, sinks, window, keep)
     if (wide <= 1) SM_GF(4);
     else if (wide <= 2) SM_GF(8);
     else SM_GF(16);
 #undef SM_GF
     if (nsplit > 1)
-      hipLaunchKernelGGL(grouped_attention_merge_kernel<float>, dim3(n_items, Hkv, G), dim3(NT), 0, stream, items, nsplit,
-                         part_o, part_ml, Hq, Hkv, vdim, (const float*)gate, gate_stride, (float*)out, split_keys,
-                         longest);
+      hipLaunchKernelGGL(grouped_attention_f32_join_kernel, dim3(n_items, Hkv, G), dim3(NT), 0, stream, items, row_len, nsplit,
+                         part_o, part_ml, Hq, Hkv, vdim, (const float*)gate, gate_stride, (float*)out, chunk, sinks, window, keep);
     return 0;
   }
   if (single && dim % 8 == 0 && bs % MKT == 0 && (((uintptr_t)q | (uintptr_t)cache) & 15) == 0) {
@@ -1885,7 +1965,7 @@ int sm_grouped_attention_mfma(const void* q, const void* cache, const int* table
     else SM_GD(8, 16);
 #undef SM_GD
     if (nsplit > 1)
-      hipLaunchKernelGGL(grouped_attention_merge_kernel<bf16_t>, dim3(n_items, Hkv, G), dim3(NT), 0, stream, items, nsplit,
+      hipLaunchKernelGGL(grouped_attention_merge_kernel, dim3(n_items, Hkv, G), dim3(NT), 0, stream, items, nsplit,
                          part_o, part_ml, Hq, Hkv, vdim, (const bf16_t*)gate, gate_stride, (bf16_t*)out, split_keys,
                          longest);
     return 0;
@@ -1917,7 +1997,7 @@ int sm_grouped_attention_mfma(const void* q, const void* cache, const int* table
 #undef SM_GO2
 #undef SM_GO
   if (nsplit > 1)
-    hipLaunchKernelGGL(grouped_attention_merge_kernel<bf16_t>, dim3(n_items, Hkv, 64), dim3(NT), 0, stream, items, nsplit,
+    hipLaunchKernelGGL(grouped_attention_merge_kernel, dim3(n_items, Hkv, 64), dim3(NT), 0, stream, items, nsplit,
                        part_o, part_ml, Hq, Hkv, vdim, (const bf16_t*)gate, gate_stride, (bf16_t*)out, split_keys,
                          longest);
   return 0;

@@ -306,6 +306,7 @@ def qkv_rope_cache(qkv, bias, positions, cos_sin, Hq, Hkv, dim, vdim, rot_dims, 
 
 
 GQA_MFMA = os.environ.get("LLMD_GQA_MFMA", "1") == "1"
+F32_RANGE = 128  # keys per range of the float32 form (FR in csrc/seqmix/sm_gqa.hip)
 # workgroups a decode-only step aims for. 64 sequences x 8 kv heads of 128 / 128 at context 2048, mean us per layer over
 # a full-context and a window-1024 stack (+ the kernel that merges the ranges): 512 workgroups 86, 1024 89 + 5,
 # 2048 97 + 6
@@ -332,7 +333,7 @@ def grouped_attention(q, cache, dim, vdim, scale: float, seq, gate=None, slopes=
 
     Sizes up to 256 run on the matrix cores, bfloat16 and float32 (work item = up to 64 (token, head-of-group) rows of one
     sequence and kv head; bfloat16 steps of single tokens have a kernel whose waves share an item's rows); larger ones on
-    the FMA kernel."""
+    the FMA kernel. A float32 row's result is the same in every step."""
     T, Hq, _ = q.shape
     Hkv = cache.shape[1]
     out = torch.empty(T, Hq * vdim, dtype=q.dtype, device=q.device)
@@ -354,7 +355,20 @@ def grouped_attention(q, cache, dim, vdim, scale: float, seq, gate=None, slopes=
         # workgroup ids run over the kv heads first: ids 256 apart (256 // Hkv items apart) share a CU
         items = seq.attention_items(max(1, 64 * rb // G), balance=max(1, 256 // Hkv) if seq.max_q > 1 else 0)
         nsplit, split, po, pm = 1, 0, None, None
-        if seq.max_q == 1 and span > 256:
+        if q.dtype == torch.float32:
+            # fixed ranges of R keys in every step: as workgroups of their own where one per item and kv head leaves CUs idle,
+            # with the same bits either way. s keys that start at a multiple of 32 meet at most (s + 2 R - 33) // R ranges
+            n, R = items.shape[0] * Hkv, F32_RANGE
+            nsplit = -(-seq.max_len // R)
+            if window or chunk:
+                nsplit = min(nsplit, -(-keep_first // R) + ((window or chunk) + 31 + 2 * R - 33) // R)
+            if seq.max_q > 1 or n >= GQA_DECODE_WGS or n * nsplit * G * vdim > 1 << 26:
+                nsplit = 1
+            if nsplit > 1:
+                split = R
+                po = torch.empty(n * nsplit * G * vdim, dtype=torch.float32, device=q.device)
+                pm = torch.empty(n * nsplit * G * 2, dtype=torch.float32, device=q.device)
+        elif seq.max_q == 1 and span > 256:
             # decode-only step of few sequences: key ranges so that items x kv heads x ranges fill the chip
             n = items.shape[0] * Hkv * -(-G // 16)
             nsplit = max(1, min(-(-GQA_DECODE_WGS // n), span // 128))

@@ -55,3 +55,40 @@ def test_grouped_attention_f32(Hq, Hkv, dim, vdim, bs, opts, runs):
         got[dev] = sm.grouped_attention(q.to(dev), c, dim, vdim, dim ** -0.5, m, **kw).cpu()
     # scores are sums of ``dim`` products of order 1, outputs weighted means of values of order 1: a few hundred fp32 roundings
     assert (got["cuda"] - got["cpu"]).abs().max() <= 2e-5
+
+
+@pytest.mark.parametrize("opts", [{}, {"window": 300, "keep_first": 3, "sinks": True}, {"window": 40, "keep_first": 290},
+                                  {"chunk": 270, "slopes": True}, {"gate": True, "window": 700}],
+                         ids=["causal", "window", "kept", "chunk", "gate"])
+@pytest.mark.parametrize("Hq,Hkv,dim,bs", [(8, 2, 128, 64), (3, 1, 30, 16), (6, 6, 200, 32)])
+def test_rows_do_not_depend_on_the_step(Hq, Hkv, dim, bs, opts, monkeypatch):
+    """A token's result has the same bits in a whole prompt, in portions of it, alone, in a batch of single tokens whose key
+    ranges run as workgroups of their own, and in one where they do not."""
+    from llmd_amd.ops import seqmix as sm
+
+    n, at = 900, [0, 30, 255, 256, 257, 511, 600, 899]
+    g = torch.Generator().manual_seed(dim)
+    whole, pages = _meta([(0, n)], bs, "cuda")
+    q = torch.randn(n, Hq, dim, generator=g) * 2.0 ** torch.randint(-1, 4, (n, Hq, 1), generator=g)
+    cache, gate = torch.randn(pages, Hkv, bs, 2 * dim, generator=g), torch.randn(n, Hq * dim, generator=g)
+    vals = {"sinks": torch.randn(Hq, generator=g), "slopes": torch.rand(Hq, generator=g) * 0.05}
+
+    def run(runs, rows, dev="cuda"):
+        m, _ = _meta(runs, bs, dev)
+        m.tables = whole.tables[:, :].expand(len(runs), -1).contiguous().to(dev)
+        kw = {k: (gate[rows] if k == "gate" else vals[k]).to(dev) if v is True else v for k, v in opts.items()}
+        return sm.grouped_attention(q[rows].to(dev), cache.to(dev), dim, dim, dim ** -0.5, m, **kw).cpu()
+
+    want = run([(0, n)], list(range(n)))
+    plain = run([(0, n)], list(range(n)), "cpu")
+    # scores are sums of ``dim`` products, up to 8 times their usual size, outputs weighted means of values of order 1
+    assert (want - plain).abs().max() <= 1e-4
+    cuts = (0, 250, 251, 519, n)
+    for a, b in zip(cuts, cuts[1:]):
+        assert torch.equal(run([(a, b - a)], list(range(a, b))), want[a:b])
+    singles = [(p, 1) for p in at]
+    for wgs in (512, 1):
+        monkeypatch.setattr(sm, "GQA_DECODE_WGS", wgs)
+        assert torch.equal(run(singles, at), want[at])
+        for p in at:
+            assert torch.equal(run([(p, 1)], [p]), want[p:p + 1])
