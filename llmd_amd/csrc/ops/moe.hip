@@ -6,7 +6,7 @@
 //                 (n_group / topk_group), renormalisation, routed scaling.
 //   moe_align     per-expert counts -> offsets padded to the GEMM M-tile ->
 //                 sorted_ids[P] (token*topk + slot, -1 for padding) and the
-//                 expert id of every M-tile; single workgroup (T*k <= 64k).
+//                 expert id of every M-tile; one workgroup, many above 4096 pairs (moe_sort.h).
 //   moe_gemm      grouped GEMM  Y[p, :] = X[tok(p), :] . W[e(tile)]^T
 //                 MFMA 16x16x32 bf16, 64x128 output tile per 256-thread
 //                 workgroup (2x2 waves of 32x64), K-step 64 double-buffered

@@ -12,8 +12,9 @@
 //               w * h for them.
 //
 // moe_route   : top-k of fp32 router logits (ties to the lower index), softmax over the chosen.
-// moe_group   : one workgroup sorts the (token, choice) pairs by expert into tiles of 64 or 128 rows
-//               (counts and ranks through LDS atomics; a tile holds rows of one expert only).
+// moe_group   : one workgroup, or two launches of many above 4096 pairs (moe_sort.h), sort the (token, choice)
+//               pairs by expert into tiles of 64 or 128 rows (counts and ranks through LDS atomics; a tile holds
+//               rows of one expert only).
 // moe_tile    : tile GEMM on the matrix cores, bf16 and fp32 (rows of 16-byte pieces).
 // moe_gemm    : the form for every other size, 64 rows x 64 columns per workgroup, K stepped by 16 through
 //               LDS, 4 x 4 outputs per thread. Both: fp32 accumulation in a fixed K order (a row's sums do

@@ -1461,7 +1461,8 @@ def pgemm_wins(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, bool]]:
 
 def decode_rule(M: int, N: int, K: int):
     """Kernel and plan for a decode-sized projection that no measured table lists, or None for hipBLASLt.
-    1x MI355X, weights cold in HBM, launches one behind the other, hipBLASLt / here in us:
+    1x MI355X, weights cold in HBM, products one behind the other in a graph (a split's reduce overlaps with the next
+    product: traced, (2048, 2048) at 64 is 7.6 + 4.9), hipBLASLt / here in us:
 
     * M <= 16 and weights up to 32 MB: the stream kernel, whose workgroups of 16 rb weight rows are at most one
       per CU, and two K ranges where they would fill half of the CUs. (2048, 2048) 11.0 / 6.3 at M 8, 11.0 / 7.1

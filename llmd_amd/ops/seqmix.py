@@ -221,8 +221,8 @@ UNGATED_ACTS = {"gelu": 1, "relu2": 4}
 def moe_ffn(h, ids, w, w1, w2, act: str = "gelu", extra=None, extra_gate=None):
     """sum_j w[t, j] * W2[e] act(W1[e] h_t), e = ids[t, j]: ungated experts with the exact (erf)
     GELU or the squared ReLU. w1 [E, F, d], w2 [E, d, F]. ``extra`` [T, d] (a shared expert's result)
-    is added times sigmoid(extra_gate [T] fp32). Rows are grouped by expert into tiles (one pass of a
-    single workgroup), two grouped GEMMs run over the tiles, and the combine sums each token's
+    is added times sigmoid(extra_gate [T] fp32). Rows are grouped by expert into tiles (by
+    one workgroup, or many above 4096 pairs), two grouped GEMMs run over the tiles, and the combine sums each token's
     rows in fp32; a row's sums do not depend on what else is in the step."""
     if not h.is_cuda:
         return ref.moe_ffn(h, ids, w, w1, w2, act, extra, extra_gate)
