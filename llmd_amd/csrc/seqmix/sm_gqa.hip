@@ -1468,20 +1468,21 @@ __global__ __launch_bounds__(NT, NKS <= 2 ? 3 : NKS <= 4 ? 2 : 1) void grouped_d
 // operands throughout. Pieces are 16 bytes = four elements, element j of a lane's piece belongs to product j: S^T = K Q^T over
 // dims 16 ks + 4 kq + j, then O += P V over keys 16 kb + 4 kq + j, for which a lane already holds its row's weights and a
 // 16-byte piece of a (transposed) value column. Exponentials are expf, as in the FMA form. DkP = 16 NKS >= dim, VP = 16 NCB.
-// A 700-token prompt, 32 heads x 128 over 4 kv heads: 1537 us with the FMA form, now 112 us (128 matrix instructions of
+// A 700-token prompt, 32 heads x 128 over 4 kv heads: 1537 us with the FMA form, now 113 us (128 matrix instructions of
 // 32 cycles per wave and tile).
 //
 // A row's result is the same in every step, whatever else the step holds. The softmax runs over ranges of FR keys at fixed places
 // of the sequence; a range's maximum, sum and products are joined to those of the ranges before it, in order. A step of few
-// single tokens runs the ranges as workgroups of their own (blockIdx.z) and joins them in a second kernel, with the same
-// operations in the same order. One token over 700 and 4000 keys, 32 heads x 128 over 4 kv heads: 30 and 37 us, in one
-// workgroup per kv head 100 and 517; 16 tokens over 700 38 us, over 4000 154. Ranges of 256 keys: 45, 49, 53 and 115 us.
+// single tokens deals a row's ranges to several workgroups (blockIdx.z), which store them apart, and joins them in a second
+// kernel, with the same operations in the same order. One token over 700 and 4000 keys, 32 heads x 128 over 4 kv heads: 30 and 38 us, in one
+// workgroup per kv head 100 and 520; 16 tokens over 700 38 us, over 4000 130. Ranges of 256 keys: 45, 49, 53 and 115 us.
+// At most 1024 workgroups: with one for each of the 1024 ranges of a step planned for 131072 keys, 16 tokens over 700 took 733 us.
 constexpr int FR = 128;
 
 // The ranges that a row (or an item, by its last one) of ``len`` keys meets, numbered without those that lie in the gap between
 // the kept first tokens and the window: ``kept`` ones from the sequence's start, then those from ``first`` on.
 struct Ranges {
-  int kept, first, count;
+  int kept, first, count;  // none of them is empty
   __device__ __forceinline__ Ranges(int len, int kbase, int keepT, int gap) {
     const int all = (len - 1) / FR + 1;
     kept = min((keepT + FR - 1) / FR, all);
@@ -1489,6 +1490,7 @@ struct Ranges {
     count = kept + max(0, all - first);
   }
   __device__ __forceinline__ int place(int z) const { return z < kept ? z : first + z - kept; }
+  __device__ __forceinline__ int number(int place) const { return place < kept ? place : place - first + kept; }
 };
 
 // One more range (m, l): its weight against what is there (mt, lt), which is brought to the new maximum.
@@ -1500,13 +1502,13 @@ __device__ __forceinline__ void join(float& mt, float& lt, float m, float l, flo
   mt = M;
 }
 
-template <int NKS, int NCB>
+template <int NKS, int NCB, bool APART>
 __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ cache, const int* __restrict__ tables, int W, int bs,
     const int* __restrict__ items, const int* __restrict__ row_len, float scale, int Hq, int Hkv, int dim, int vdim,
     const float* __restrict__ gate, int64_t gate_stride, float* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, const float* __restrict__ slopes, int chunk, const float* __restrict__ sinks, int window,
-    int keep) {
+    int keep, int nsplit) {
   constexpr int DkP = 16 * NKS, VP = 16 * NCB;
   constexpr int KS = DkP + 4, VS = MKT + 4;      // LDS row strides: 16 rows' pieces take all banks
   constexpr int NBUF = NKS <= 8 ? 2 : 1;         // as in the bf16 form
@@ -1537,6 +1539,17 @@ __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_ke
   const int full_lo = chunk > 0 ? ((maxlen - 1) / chunk) * chunk : (window > 0 ? max(0, maxlen - window) : 0);
   const int full_hi = row_len[tok0];
   auto key_of = [&](int v) { return v + (v >= keepT ? gap : 0); };
+  // APART: this workgroup's ranges are stored, not joined
+  const Ranges rs(maxlen, kbase, keepT, gap);
+  int kbeg = kbase, kend = vlen;
+  if (APART) {
+    const int per = (rs.count + gridDim.z - 1) / gridDim.z, z0 = blockIdx.z * per, z1 = min(rs.count, z0 + per);
+    if (z0 >= z1) return;
+    // places of the sequence in the numbering without the gap
+    auto without_gap = [&](int p) { return p < keepT ? p : max(keepT, p - gap); };
+    kbeg = max(kbase, without_gap(rs.place(z0) * FR));
+    kend = min(vlen, without_gap((rs.place(z1 - 1) + 1) * FR));
+  }
 
   // padding columns of the key tile and padding rows of the value tile stay zero for the whole kernel
   for (int e = threadIdx.x; e < NBUF * MKT * KS; e += NT) sK[e] = 0.f;
@@ -1556,17 +1569,6 @@ __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_ke
   float m = -INFINITY, l = 0.f;
   float mt = sinks ? sinks[myhead] : -INFINITY, lt = sinks ? 1.f : 0.f;  // a sink is a score that is already counted
   const int* bt = tables + (int64_t)seq * W;
-  const bool alone = gridDim.z > 1;  // this workgroup takes one range
-  int kbeg = kbase, kend = vlen;
-  if (alone) {
-    const Ranges rs(maxlen, kbase, keepT, gap);
-    if ((int)blockIdx.z >= rs.count) return;
-    // places of the sequence in the numbering without the gap
-    auto without_gap = [&](int p) { return p < keepT ? p : max(keepT, p - gap); };
-    const int at = rs.place(blockIdx.z) * FR;
-    kbeg = max(kbase, without_gap(at));
-    kend = min(vlen, without_gap(at + FR));
-  }
   constexpr int CK = DkP / 4, NCK = (MKT * CK + NT - 1) / NT;  // pieces per key row, per thread
   constexpr int CV = MKT / 4, NCV = (VP * CV + NT - 1) / NT;   // pieces per value column (4 keys each), per thread
   const bool one_page = (bs % MKT) == 0;                       // a tile lies inside one page
@@ -1623,28 +1625,46 @@ __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_ke
     if (kbeg + MKT < kend) fetch(key_of(kbeg + MKT));
     __syncthreads();
   }
-  auto next_range = [&] {
-    float was, now;
-    join(mt, lt, m, l, was, now);
-    // the accumulators hold rows 4 kq + r: their factors come from the lane that owns the row
+  auto end_range = [&](int range) {  // o[n][r] = O[row 16 wave + 4 kq + r][column 16 n + r16]
+    if (APART) {
+      const int64_t pbase = (((int64_t)item * Hkv + g) * nsplit + rs.number(range)) * G;
+      if (kq == 0 && ok) {
+        part_ml[(pbase + myrow) * 2] = m;
+        part_ml[(pbase + myrow) * 2 + 1] = l;
+      }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float a = __shfl(was, kq * 4 + r, 64), b = __shfl(now, kq * 4 + r, 64);
+      for (int r = 0; r < 4; ++r) {
+        const int row = wave * 16 + kq * 4 + r;
 #pragma unroll
-      for (int n = 0; n < NCB; ++n) {
-        ot[n][r] = __builtin_fmaf(ot[n][r], a, o[n][r] * b);
-        o[n][r] = 0.f;
+        for (int n = 0; n < NCB; ++n) {
+          const int col = n * 16 + r16;
+          if (row < ntok * G && col < vdim) part_o[(pbase + row) * vdim + col] = o[n][r];
+          o[n][r] = 0.f;
+        }
+      }
+    } else {
+      float was, now;
+      join(mt, lt, m, l, was, now);
+      // the accumulators hold rows 4 kq + r: their factors come from the lane that owns the row
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float a = __shfl(was, kq * 4 + r, 64), b = __shfl(now, kq * 4 + r, 64);
+#pragma unroll
+        for (int n = 0; n < NCB; ++n) {
+          ot[n][r] = __builtin_fmaf(ot[n][r], a, o[n][r] * b);
+          o[n][r] = 0.f;
+        }
       }
     }
     m = -INFINITY;
     l = 0.f;
   };
-  int it = 0, range = kbeg < kend ? key_of(kbeg) / FR : 0;
+  int it = 0, range = key_of(kbeg) / FR;
   for (int v0 = kbeg; v0 < kend; v0 += MKT, ++it) {
     const int k0 = key_of(v0);
     if (k0 / FR != range) {
+      if (any_row) end_range(range);
       range = k0 / FR;
-      if (any_row) next_range();
     }
     const int cur = NBUF == 2 ? (it & 1) : 0;
     if (NBUF == 1) {
@@ -1723,13 +1743,8 @@ __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_ke
       __syncthreads();
     }
   }
-  // o[n][r] = O[row 16 wave + 4 kq + r][column 16 n + r16]
-  const int64_t pbase = (((int64_t)item * Hkv + g) * gridDim.z + blockIdx.z) * G;
-  if (!alone) next_range();
-  else if (kq == 0 && ok) {
-    part_ml[(pbase + myrow) * 2] = m;
-    part_ml[(pbase + myrow) * 2 + 1] = l;
-  }
+  if (any_row) end_range(range);
+  if (APART) return;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int row = wave * 16 + kq * 4 + r;
@@ -1741,10 +1756,6 @@ __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_ke
     for (int n = 0; n < NCB; ++n) {
       const int col = n * 16 + r16;
       if (col >= vdim) continue;
-      if (alone) {
-        part_o[(pbase + row) * vdim + col] = o[n][r];
-        continue;
-      }
       float v = ot[n][r] * inv;
       if (gate) v *= 1.f / (1.f + expf(-gate[tok * gate_stride + h * vdim + col]));
       out[(tok * Hq + h) * vdim + col] = v;
@@ -1752,7 +1763,7 @@ __global__ __launch_bounds__(NT, NKS <= 8 ? 2 : 1) void grouped_attention_f32_ke
   }
 }
 
-// Joins the ranges of a step of single tokens (item = token), as next_range does.
+// Joins the ranges of a step of single tokens (item = token), as end_range does.
 __global__ __launch_bounds__(NT) void grouped_attention_f32_join_kernel(
     const int* __restrict__ items, const int* __restrict__ row_len, int nsplit, const float* __restrict__ part_o,
     const float* __restrict__ part_ml, int Hq, int Hkv, int vdim, const float* __restrict__ gate, int64_t gate_stride,
@@ -1939,14 +1950,19 @@ int sm_grouped_attention_mfma(const void* q, const void* cache, const int* table
   if (f32) {
     const int wide = (std::max(dim, vdim) + 63) / 64;
     if (rb != 1 || (nsplit > 1 && (split_keys != FR || !single)) || (((uintptr_t)q | (uintptr_t)cache) & 15)) return 1;
-    const dim3 fgrid(Hkv, n_items, nsplit);
-#define SM_GF(N)                                                                                                       \
-  hipLaunchKernelGGL((grouped_attention_f32_kernel<N, N>), fgrid, dim3(NT), 0, stream, (const float*)q,                \
+    // about two rounds of workgroups at most: ranges may be planned for contexts far longer than the step's
+    const dim3 fgrid(Hkv, n_items, std::min(nsplit, std::max(1, 1024 / (Hkv * n_items))));
+#define SM_GF(N, APART)                                                                                                \
+  hipLaunchKernelGGL((grouped_attention_f32_kernel<N, N, APART>), fgrid, dim3(NT), 0, stream, (const float*)q,         \
                      (const float*)cache, tables, W, bs, items, row_len, scale, Hq, Hkv, dim, vdim, (const float*)gate, \
-                     gate_stride, (float*)out, part_o, part_ml, slopes, chunk, sinks, window, keep)
-    if (wide <= 1) SM_GF(4);
-    else if (wide <= 2) SM_GF(8);
-    else SM_GF(16);
+                     gate_stride, (float*)out, part_o, part_ml, slopes, chunk, sinks, window, keep, nsplit)
+#define SM_GF2(N)                   \
+  if (nsplit > 1) SM_GF(N, true);   \
+  else SM_GF(N, false)
+    if (wide <= 1) { SM_GF2(4); }
+    else if (wide <= 2) { SM_GF2(8); }
+    else { SM_GF2(16); }
+#undef SM_GF2
 #undef SM_GF
     if (nsplit > 1)
       hipLaunchKernelGGL(grouped_attention_f32_join_kernel, dim3(n_items, Hkv, G), dim3(NT), 0, stream, items, row_len, nsplit,

@@ -356,13 +356,13 @@ def grouped_attention(q, cache, dim, vdim, scale: float, seq, gate=None, slopes=
         items = seq.attention_items(max(1, 64 * rb // G), balance=max(1, 256 // Hkv) if seq.max_q > 1 else 0)
         nsplit, split, po, pm = 1, 0, None, None
         if q.dtype == torch.float32:
-            # fixed ranges of R keys in every step: as workgroups of their own where one per item and kv head leaves CUs idle,
+            # fixed ranges of R keys in every step: dealt to several workgroups where one per item and kv head leaves CUs idle,
             # with the same bits either way. s keys that start at a multiple of 32 meet at most (s + 2 R - 33) // R ranges
             n, R = items.shape[0] * Hkv, F32_RANGE
             nsplit = -(-seq.max_len // R)
             if window or chunk:
                 nsplit = min(nsplit, -(-keep_first // R) + ((window or chunk) + 31 + 2 * R - 33) // R)
-            if seq.max_q > 1 or n >= GQA_DECODE_WGS or n * nsplit * G * vdim > 1 << 26:
+            if seq.max_q > 1 or n >= GQA_DECODE_WGS or n * nsplit * G * vdim > 1 << 28:
                 nsplit = 1
             if nsplit > 1:
                 split = R

@@ -92,3 +92,18 @@ def test_rows_do_not_depend_on_the_step(Hq, Hkv, dim, bs, opts, monkeypatch):
         assert torch.equal(run(singles, at), want[at])
         for p in at:
             assert torch.equal(run([(p, 1)], [p]), want[p:p + 1])
+
+
+def test_rows_do_not_depend_on_the_plan():
+    """Ranges planned for contexts far longer than the step's (a captured step), more of them than workgroups."""
+    from llmd_amd.ops import seqmix as sm
+
+    g = torch.Generator().manual_seed(1)
+    for B, n in ((1, 3000), (40, 700)):
+        m, pages = _meta([(n - 1 - i, 1) for i in range(B)], 64, "cuda")
+        q, cache = torch.randn(B, 8, 64, generator=g).cuda(), torch.randn(pages, 4, 64, 128, generator=g).cuda()
+        out = []
+        for m.max_len in (n, 9000, 131072):
+            for kw in ({}, {"window": 500, "keep_first": 200}):
+                out.append(sm.grouped_attention(q, cache, 64, 64, 0.125, m, **kw))
+        assert all(torch.equal(a, b) for a, b in zip(out, out[2:]))
