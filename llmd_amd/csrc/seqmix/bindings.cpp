@@ -62,8 +62,9 @@ void sm_moe_route(const float*, int64_t, int, int, int*, float*, int, int, hipSt
 int64_t sm_moe_sort_scratch(int, int);
 void sm_moe_group(const int*, int, int, int, int*, int*, int*, int*, hipStream_t);
 int sm_moe_tiled(const void*, int64_t, const void*, int64_t, int64_t, int);
-void sm_moe_gemm(const void*, int64_t, int64_t, int, const int*, const int*, const void*, int, int, void*, int, int, int, int, int,
+void sm_moe_gemm(const void*, int64_t, int, const int*, const int*, const void*, int, int, void*, int, int, int, int,
                  const float*, float, hipStream_t);
+int sm_moe_ring(const void*, int64_t, int64_t, const void*, int64_t, int64_t, int, int);
 int sm_retention(const void*, int64_t, int, int, int, int, const int64_t*, const float*, int, const float*, int, float,
                  float*, const int*, const int*, const int*, void*, int, int, int, int, int, const int*, const int*,
                  float*, float*, hipStream_t);
@@ -624,7 +625,7 @@ void moe_group(Tensor ids, int64_t E, int64_t tm, Tensor slot_row, Tensor tiles,
   CHECK_I32(tiles);
   CHECK_I32(pair_slot);
   const int64_t n = ids.numel(), mt = tiles.numel() / 3;
-  TORCH_CHECK((tm == 64 || tm == 128) && E >= 1 && E <= 8192, "tile rows, experts");
+  TORCH_CHECK((tm == 64 || tm == 120 || tm == 128) && E >= 1 && E <= 8192, "tile rows, experts");
   TORCH_CHECK(slot_row.numel() == mt * tm && pair_slot.numel() == n && mt >= (n + std::min(E, n) * (tm - 1)) / tm,
               "tile tables too small for n pairs over E experts");
   Tensor hist = torch::empty({sm_moe_sort_scratch(n, E)}, ids.options());
@@ -636,7 +637,11 @@ bool moe_tiled(Tensor A, Tensor W) {
   return sm_moe_tiled(A.data_ptr(), A.stride(0), W.data_ptr(), W.size(1), W.size(2), is_f32(A)) != 0;
 }
 
-void moe_gemm(Tensor A, int64_t kdiv, Tensor slot_row, Tensor tiles, Tensor W, Tensor C, int64_t act, int64_t tm, bool full,
+bool moe_ring(Tensor A, Tensor W, bool gated) {
+  return sm_moe_ring(A.data_ptr(), A.size(0), A.stride(0), W.data_ptr(), W.size(1), W.size(2), gated, is_f32(A)) != 0;
+}
+
+void moe_gemm(Tensor A, int64_t kdiv, Tensor slot_row, Tensor tiles, Tensor W, Tensor C, int64_t act, int64_t tm,
               std::optional<Tensor> row_w, double limit) {
   const c10::hip::OptionalHIPGuard g(dev_of(A));
   TORCH_CHECK(A.is_cuda() && act_ok(A) && A.dim() == 2 && A.stride(1) == 1, "A");
@@ -649,7 +654,9 @@ void moe_gemm(Tensor A, int64_t kdiv, Tensor slot_row, Tensor tiles, Tensor W, T
   const bool gated = act == 2 || act == 3 || act == 5;
   TORCH_CHECK(act >= 0 && act <= 5 && (!gated || W.size(1) % 2 == 0), "epilogue");
   const int64_t N = gated ? W.size(1) / 2 : W.size(1);  // gated: W holds [gate rows | up rows]
-  TORCH_CHECK(tm == 64 || (tm == 128 && moe_tiled(A, W)), "tile rows");
+  TORCH_CHECK(tm == 64 || (tm == 128 && moe_tiled(A, W)) ||
+                  (tm == 120 && moe_ring(A, W, gated) && mt * tm * 4 < (int64_t)1 << 31 && ((uintptr_t)C.data_ptr() & 15) == 0),
+              "tile rows");
   TORCH_CHECK(slot_row.numel() == mt * tm && C.is_contiguous() && C.dim() == 2 && C.size(0) == mt * tm &&
                   C.size(1) == N, "C [tiles * tm, N]");
   TORCH_CHECK(kdiv > 0 || A.size(0) == mt * tm, "A rows are the tile slots");
@@ -658,8 +665,8 @@ void moe_gemm(Tensor A, int64_t kdiv, Tensor slot_row, Tensor tiles, Tensor W, T
     TORCH_CHECK(gated && kdiv > 0 && row_w->numel() == A.size(0) * kdiv, "row_w [T, k] with a gated epilogue");
   }
   if (N == 0) return;
-  sm_moe_gemm(A.data_ptr(), A.size(0), A.stride(0), kdiv, slot_row.data_ptr<int>(), tiles.data_ptr<int>(), W.data_ptr(),
-              N, W.size(2), C.data_ptr(), mt, tm, full ? 1 : 0, (int)act, is_f32(A), row_w ? row_w->data_ptr<float>() : nullptr,
+  sm_moe_gemm(A.data_ptr(), A.stride(0), kdiv, slot_row.data_ptr<int>(), tiles.data_ptr<int>(), W.data_ptr(),
+              N, W.size(2), C.data_ptr(), mt, tm, (int)act, is_f32(A), row_w ? row_w->data_ptr<float>() : nullptr,
               (float)limit, cur());
 }
 
@@ -1026,6 +1033,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_route", &moe_route);
   m.def("moe_group", &moe_group);
   m.def("moe_tiled", &moe_tiled);
+  m.def("moe_ring", &moe_ring);
   m.def("moe_gemm", &moe_gemm);
   m.def("moe_combine", &moe_combine);
   m.def("bigram_embed", &bigram_embed);

@@ -13,9 +13,9 @@
 //
 // moe_route   : top-k of fp32 router logits (ties to the lower index), softmax over the chosen.
 // moe_group   : one workgroup, or two launches of many above 4096 pairs (moe_sort.h), sort the (token, choice)
-//               pairs by expert into tiles of 64 or 128 rows (counts and ranks through LDS atomics; a tile holds
+//               pairs by expert into tiles of 64, 120 or 128 rows (counts and ranks through LDS atomics; a tile holds
 //               rows of one expert only).
-// moe_tile    : tile GEMM on the matrix cores, bf16 and fp32 (rows of 16-byte pieces).
+// moe_tile    : tile GEMM on the matrix cores, bf16 and fp32 (rows of 16-byte pieces); moe_ring: bf16, more than a few rows.
 // moe_gemm    : the form for every other size, 64 rows x 64 columns per workgroup, K stepped by 16 through
 //               LDS, 4 x 4 outputs per thread. Both: fp32 accumulation in a fixed K order (a row's sums do
 //               not depend on its tile or on the rest of the step).
@@ -23,6 +23,7 @@
 //               has a gate) in fp32.
 #include <algorithm>
 
+#include "moe_ring.h"
 #include "moe_tile.h"
 #include "seqmix_common.h"
 #include "wave_top.h"
@@ -415,179 +416,27 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const T* __restrict__ 
   run_tile<T, GATED>(t, rows, wrow, out);
 }
 
-// bf16 steps that bring an expert many rows: the same tiles as one stream per workgroup. Two workgroups per CU walk the work
-// items, and the last steps of an item load the first ones of the next, so that the loads never stop. Both operands pass LDS,
-// the waves split a tile two by two. Needs an even number, at least four, of whole steps: the two sets of registers then
-// change places at the same point of every item. 16384 rows over the experts above: 64 x 256 tiles through one LDS buffer
-// 305 + 182 us, moe_tile_kernel 241 + 214, this 219 + 122 (453 TFLOP/s); 32768 rows 354 + 179. The weights alone are
-// 160 + 80 us; beyond that the tiles' products and LDS passes (1.2 us per step of both workgroups) overlap the loads only in part.
-// fp32 stays with moe_tile_kernel, whose matrix instructions are the limit either way (5600 rows: 412 + 210 against 461 + 235).
-template <typename T, int ACT>
-__global__ __launch_bounds__(256, 2) void moe_stream_kernel(const T* __restrict__ A, int64_t a_stride, int kdiv,
-                                                            const int* __restrict__ slot_row, const int* __restrict__ tiles,
-                                                            const T* __restrict__ Wt, int N, int K, T* __restrict__ Cout,
-                                                            const float* __restrict__ row_w, float limit, int NB) {
+// bf16 steps that bring an expert more than a few rows (moe_ring.h).
+template <int ACT>
+__global__ __launch_bounds__(moe_ring::NT, 2) void moe_ring_kernel(const bf16_t* __restrict__ A, int64_t a_stride, int kdiv,
+                                                                     const int* __restrict__ slot_row,
+                                                                     const int* __restrict__ tiles, const bf16_t* __restrict__ Wt,
+                                                                     int N, int K, bf16_t* __restrict__ Cout,
+                                                                     const float* __restrict__ row_w, float limit) {
+  __shared__ __attribute__((aligned(1024))) char lds[moe_ring::LDS];
   constexpr bool GATED = gated_act_code(ACT);
-  const int total = tiles[0] * NB, chunk = (total + 7) >> 3;  // one range of items per XCD
-  const int xcd = blockIdx.x & 7, step_items = gridDim.x >> 3;
-  const int end = min(total, (xcd + 1) * chunk);
-  int item = xcd * chunk + (blockIdx.x >> 3);
-  if (item >= end) return;
-  constexpr int EW = 16 * 64 * (int)sizeof(T);  // a wave's block of 16 rows on its way out
-  __shared__ __attribute__((aligned(128))) char lds[4 * TBUF + 4 * EW];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, kq = lane >> 4;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int nk = (K * (int)sizeof(T)) >> 7;
-  const int wr = lds_wr(tid), ra = wm * 64 * TLS + lds_rd(r16, kq);
-  // gated: blocks 0 and 1 of a wave are gate rows, 2 and 3 the matching up rows
-  const int rw = 2 * TBUF + (GATED ? wn * 32 : wn * 64) * TLS + lds_rd(r16, kq);
-  auto rwc = [&](int c) { return rw + (GATED ? (c & 1) * 16 + (c >> 1) * 64 : c * 16) * TLS; };
-
-  struct Item {
-    int rows, col0, tile;
-    const char* w;
-  };
-  auto look = [&](int it) {
-    const int* any = tiles + 1 + 3 * (it / NB);  // a tile of the item's expert
-    const int first = any[1], nt = any[2], j = it - first * NB;
-    Item t;
-    t.tile = first + j % nt;
-    t.col0 = (j / nt) * (GATED ? TBW / 2 : TBW);
-    t.rows = tiles[1 + 3 * t.tile] >> 16;
-    t.w = reinterpret_cast<const char*>(Wt + (int64_t)(any[0] & 0xffff) * (GATED ? 2 * N : N) * K);
-    return t;
-  };
-  // the pair or slot behind this thread's row i, -1 past the tile's rows: those read out of the buffer's range, zeros from nowhere
-  auto row_of = [&](const Item& t, int i) {
-    const int r = (tid >> 3) + i * 32, slot = t.tile * TBM + r;
-    return r >= t.rows ? -1 : kdiv > 0 ? slot_row[slot] : slot;
-  };
-  auto a_off = [&](int row) {
-    return row < 0 ? 0x80000000u : (uint32_t)(kdiv > 0 ? row / kdiv : row) * (uint32_t)(a_stride * (int)sizeof(T)) + (tid & 7) * 16;
-  };
-  const auto ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(A), 0, 0x7fffffff, 0x00020000);
-  auto w_off = [&](const Item& t, int i) {
-    const int j = (tid >> 3) + 32 * i, col = min(t.col0 + (GATED ? j & 63 : j), N - 1);
-    return (uint32_t)(col + (GATED && j >= 64 ? N : 0)) * (uint32_t)(K * (int)sizeof(T)) + (tid & 7) * 16;
-  };
-  f32x4_t acc[4][4];
-  u32x4_t wb[2][4], ab[2][4];
-  Item cur = look(item);
-  uint32_t ap[4], wp[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) ap[i] = a_off(row_of(cur, i)), wp[i] = w_off(cur, i);
-  auto load = [&](int s, const char* w, int kt) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      ab[s][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ar, ap[i], kt * 128, 0));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) wb[s][i] = *reinterpret_cast<const u32x4_t*>(w + kt * 128 + wp[i]);
-  };
-  auto store = [&](int s, int buf) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      *reinterpret_cast<u32x4_t*>(lds + buf * TBUF + wr + i * 32 * TLS) = ab[s][i];
-      *reinterpret_cast<u32x4_t*>(lds + (2 + buf) * TBUF + wr + i * 32 * TLS) = wb[s][i];
+  // the row's input weight scales both sums
+  auto scale = [&](int64_t slot) { return GATED && row_w != nullptr ? row_w[slot_row[slot]] : 1.f; };
+  auto act = [&](float g, float u, float sw) {
+    if constexpr (GATED) return gated_<bf16_t, ACT>(sw * g, sw * u, limit);
+    if (ACT == 1) return gelu_erf_(g);
+    if (ACT == 4) {
+      g = fmaxf(g, 0.f);
+      return g * g;
     }
+    return g;
   };
-  auto products = [&](int buf) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      __builtin_amdgcn_sched_barrier(0);
-      u32x4_t w[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) w[c] = *reinterpret_cast<const u32x4_t*>(lds + ((buf * TBUF + rwc(c)) ^ (h * 64)));
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const u32x4_t a = *reinterpret_cast<const u32x4_t*>(lds + ((buf * TBUF + ra + i * 16 * TLS) ^ (h * 64)));
-#pragma unroll
-        for (int c = 0; c < 4; ++c) mma16<T>(acc[c][i], w[c], a);
-      }
-    }
-  };
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[c][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  load(0, cur.w, 0);
-  load(1, cur.w, 1);
-  store(0, 0);
-  load(0, cur.w, 2);
-  // step kt: buffer kt & 1 holds it, set (kt + 1) & 1 the next step, the other set is on its way
-  while (true) {
-    const bool more = item + step_items < end;
-    // the last item "loads" its own first steps again
-    const Item nxt = more ? look(item + step_items) : cur;
-    int rn[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) rn[i] = row_of(nxt, i);
-    const bool mine = wm * 64 < cur.rows;
-    for (int kt = 0; kt < nk - 4; kt += 2) {
-      meet();
-      store(1, 1);
-      load(1, cur.w, kt + 3);
-      if (mine) products(0);
-      meet();
-      store(0, 0);
-      load(0, cur.w, kt + 4);
-      if (mine) products(1);
-    }
-    meet();
-    store(1, 1);
-    load(1, cur.w, nk - 1);
-    if (mine) products(0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ap[i] = a_off(rn[i]), wp[i] = w_off(nxt, i);
-    meet();
-    store(0, 0);
-    load(0, nxt.w, 0);
-    if (mine) products(1);
-    meet();
-    store(1, 1);
-    load(1, nxt.w, 1);
-    if (mine) products(0);
-    meet();
-    store(0, 0);
-    load(0, nxt.w, 2);
-    if (mine) products(1);
-    // acc[c][i][q] = C[row 64 wm + 16 i + r16][weight row 4 kq + q of the wave's block c]: 16 rows at a time through the wave's
-    // own LDS, so that a row leaves as 16-byte pieces of whole lines (stored straight from the registers, eight bytes of 16 rows
-    // per quarter of a wave: 170 us for the second product, now 122)
-    constexpr int NO = GATED ? 2 : 4, PIECES = NO * 16 * (int)sizeof(T) / 16;  // 16-byte pieces of a row
-    char* eb = lds + 4 * TBUF + wave * EW;
-    const int col = cur.col0 + (GATED ? wn * 32 : wn * 64);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (wm * 64 + i * 16 < cur.rows) {
-        float sw = 1.f;  // the row's input weight (gated forms with row_w): scales both sums
-        const int row = wm * 64 + i * 16 + r16;
-        if (GATED && row_w != nullptr && row < cur.rows) sw = row_w[slot_row[cur.tile * TBM + row]];
-#pragma unroll
-        for (int c = 0; c < NO; ++c) {
-          float v[4];
-          finish4<T, ACT>(v, acc[c][i], acc[(c + 2) & 3][i], sw, limit);
-          const int at = r16 * (NO * 16) + c * 16 + kq * 4;  // pieces of a row change places by the row, against bank conflicts
-          put4<T>(eb + ((at * (int)sizeof(T)) ^ ((r16 & (PIECES - 1)) * 16)), v);
-        }
-        // the wave's own writes: no other wave touches them
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int j = 0; j < 16 * PIECES / 64; ++j) {
-          const int r = (j * 64 + lane) / PIECES, pc = (j * 64 + lane) % PIECES;
-          const u32x4_t v = *reinterpret_cast<const u32x4_t*>(eb + r * (PIECES * 16) + (pc ^ (r & (PIECES - 1))) * 16);
-          const int n = col + pc * (16 / (int)sizeof(T));
-          if (wm * 64 + i * 16 + r < cur.rows && n < N)
-            *reinterpret_cast<u32x4_t*>(Cout + ((int64_t)cur.tile * TBM + wm * 64 + i * 16 + r) * N + n) = v;
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read before the next block is written
-      }
-#pragma unroll
-      for (int c = 0; c < 4; ++c) acc[c][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
-    if (!more) break;
-    item += step_items;
-    cur = nxt;
-  }
+  moe_ring::run<GATED ? moe_ring::HALVES : moe_ring::PLAIN>(A, a_stride, kdiv, slot_row, tiles, Wt, N, K, Cout, scale, act, lds);
 }
 
 template <typename T>
@@ -699,29 +548,47 @@ int sm_moe_tiled(const void* A, int64_t a_stride, const void* W, int64_t rows, i
   return K % per == 0 && rows * K * (f32 ? 4 : 2) < (int64_t)1 << 32 && a_stride % per == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0;
 }
 
+// Whether the form of many rows takes them: bf16, whole steps of K, whole 16-byte pieces of the output rows (``rows`` weight
+// rows, half of them columns in the gated forms), byte offsets below 2^31.
+int sm_moe_ring(const void* A, int64_t a_rows, int64_t a_stride, const void* W, int64_t rows, int64_t K, int gated, int f32) {
+  return !f32 && sm_moe_tiled(A, a_stride, W, rows, K, 0) && K % 64 == 0 && K >= 256 && rows % (gated ? 16 : 8) == 0 &&
+         rows * K * 2 < (int64_t)1 << 31 && a_stride >= 0 && a_rows * a_stride * 2 < (int64_t)1 << 31;
+}
+
 // act: 0 none, 1 erf-GELU, 2 tanh-GELU(gate) * up, 3 SiLU(gate) * up, 4 squared ReLU, 5 clamped units. N = output
 // columns (the gated forms read a weight of 2 N rows per expert). tm: slots per tile, 128 for the matrix-core form (operands
-// that sm_moe_tiled takes), 64 for the other. full: the experts get many rows each.
+// that sm_moe_tiled takes), 120 for its form of many rows (sm_moe_ring), 64 for the other.
 // row_w (gated forms): fp32 weight per (token, choice) pair that scales the row's INPUT, applied to
 // both fp32 sums before the activation; nullptr = 1.
-void sm_moe_gemm(const void* A, int64_t a_rows, int64_t a_stride, int kdiv, const int* slot_row, const int* tiles, const void* W,
-                 int N, int K, void* C, int max_tiles, int tm, int full, int act, int f32, const float* row_w,
+void sm_moe_gemm(const void* A, int64_t a_stride, int kdiv, const int* slot_row, const int* tiles, const void* W,
+                 int N, int K, void* C, int max_tiles, int tm, int act, int f32, const float* row_w,
                  float limit, hipStream_t stream) {
   const bool gated = gated_act_code(act);
+  if (tm == moe_ring::ROWS) {
+    const int cols = gated ? moe_ring::WROWS / 2 : moe_ring::WROWS;
+    const int64_t items = (int64_t)max_tiles * ((N + cols - 1) / cols);
+    const dim3 grid((unsigned)std::min<int64_t>((items + 7) / 8 * 8, 512));  // two workgroups per CU
+#define SM_RING(A_)                                                                                                        \
+  hipLaunchKernelGGL(moe_ring_kernel<A_>, grid, dim3(moe_ring::NT), 0, stream, (const bf16_t*)A, a_stride, kdiv, slot_row, \
+                     tiles, (const bf16_t*)W, N, K, (bf16_t*)C, row_w, limit)
+    if (act == 0) SM_RING(0);
+    else if (act == 1) SM_RING(1);
+    else if (act == 2) SM_RING(2);
+    else if (act == 3) SM_RING(3);
+    else if (act == 4) SM_RING(4);
+    else SM_RING(5);
+#undef SM_RING
+    return;
+  }
   if (tm == TBM) {
     const int NB = (N + (gated ? 63 : 127)) / (gated ? 64 : 128);
     const int64_t items = (int64_t)max_tiles * NB;
     const dim3 grid((unsigned)((items + 7) / 8 * 8));
-    // whole pairs of steps, whole 16-byte pieces of the output rows, and activations within a buffer's range
-    const bool flow = full && !f32 && K % 128 == 0 && K >= 256 && N % 8 == 0 && ((uintptr_t)C & 15) == 0 &&
-                      a_rows * a_stride * 2 < (int64_t)1 << 31;
-    const dim3 flow_grid((unsigned)std::min<int64_t>((items + 7) / 8 * 8, 512));  // two workgroups per CU
 #define SM_MT(KERN, TYPE, GRID)                                                                                       \
   hipLaunchKernelGGL(KERN, GRID, dim3(256), 0, stream, (const TYPE*)A, a_stride, kdiv, slot_row, tiles, (const TYPE*)W, \
                      N, K, (TYPE*)C, row_w, limit, NB)
 #define SM_MT2(A_)                                                                  \
   if (f32) SM_MT((moe_tile_kernel<float, A_>), float, grid);                        \
-  else if (flow) SM_MT((moe_stream_kernel<bf16_t, A_>), bf16_t, flow_grid);         \
   else SM_MT((moe_tile_kernel<bf16_t, A_>), bf16_t, grid)
     if (act == 0) { SM_MT2(0); }
     else if (act == 1) { SM_MT2(1); }

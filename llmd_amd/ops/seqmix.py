@@ -198,22 +198,25 @@ def moe_route(logits, k: int, sigmoid: bool = False):
     return ids, w
 
 
-def _moe_tables(C, ids, E: int, h, w1, w2):
+def _moe_tables(C, ids, E: int, h, w1, w2, gated: bool):
     """Pairs sorted by expert into tiles of rows: (slot -> pair, [number of tiles, three numbers of each], pair -> slot,
-    rows per tile, whether the tiles are well filled): 128 rows for the matrix-core GEMM, 64 for sizes that only the FMA
+    rows per tile): 128 rows for the matrix-core GEMM, 120 for its form of many rows, 64 for sizes that only the FMA
     form takes."""
     n = ids.numel()
     tm = 128 if C.moe_tiled(h, w1) and C.moe_tiled(w2[0], w2) else 64
+    if (n >= MOE_STREAM_FROM * E and C.moe_ring(h, w1, gated) and C.moe_ring(w2[0], w2, False)
+            and (n + E * 119) * w2.shape[2] < 1 << 30):
+        tm = 120
     max_tiles = max(1, (n + min(E, n) * (tm - 1)) // tm)  # every expert that has rows may leave one tile partly filled
     slot_row = torch.empty(max_tiles * tm, dtype=torch.int32, device=h.device)
     tiles = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=h.device)
     pair_slot = torch.empty(n, dtype=torch.int32, device=h.device)   # -1: identity expert
     C.moe_group(ids, E, tm, slot_row, tiles, pair_slot)
-    return slot_row, tiles, pair_slot, tm, tm == 128 and n >= MOE_STREAM_FROM * E
+    return slot_row, tiles, pair_slot, tm
 
 
-# rows per expert from which the bf16 GEMM runs as one stream per workgroup. 128 experts, both products, us against a workgroup
-# per tile: 25 rows 232 / 234, 44 rows 243 / 249, 62 rows 253 / 312; 4 rows 217 / 210
+# rows per expert from which the bf16 GEMM runs as one stream per workgroup (csrc/include/moe_ring.h). 128 experts, both products
+# with sorting and sum, us, against a workgroup per tile: 12 rows 234 / 250, 25 rows 259 / 290, 44 rows 268 / 320; 4 rows 217 / 210
 MOE_STREAM_FROM = int(os.environ.get("LLMD_MOE_STREAM_FROM", "24"))
 UNGATED_ACTS = {"gelu": 1, "relu2": 4}
 
@@ -230,11 +233,11 @@ def moe_ffn(h, ids, w, w1, w2, act: str = "gelu", extra=None, extra_gate=None):
     T, d = h.shape
     k = ids.shape[1]
     E, Fh, _ = w1.shape
-    slot_row, tiles, pair_slot, tm, full = _moe_tables(C, ids, E, h, w1, w2)
+    slot_row, tiles, pair_slot, tm = _moe_tables(C, ids, E, h, w1, w2, False)
     a = torch.empty(slot_row.numel(), Fh, dtype=h.dtype, device=h.device)
     y = torch.empty(slot_row.numel(), d, dtype=h.dtype, device=h.device)
-    C.moe_gemm(h, k, slot_row, tiles, w1, a, UNGATED_ACTS[act], tm, full, None, 0.0)
-    C.moe_gemm(a, 0, slot_row, tiles, w2, y, 0, tm, full, None, 0.0)
+    C.moe_gemm(h, k, slot_row, tiles, w1, a, UNGATED_ACTS[act], tm, None, 0.0)
+    C.moe_gemm(a, 0, slot_row, tiles, w2, y, 0, tm, None, 0.0)
     out = torch.empty_like(h)
     C.moe_combine(y, pair_slot, w, out, None, extra, extra_gate)
     return out
@@ -435,11 +438,11 @@ def moe_gated_ffn(h, ids, w, w1, w2, kind: str = "silu", scale_input: bool = Fal
     k = ids.shape[1]
     E, F2, _ = w1.shape
     Fh = F2 // 2
-    slot_row, tiles, pair_slot, tm, full = _moe_tables(C, ids, E, h, w1, w2)
+    slot_row, tiles, pair_slot, tm = _moe_tables(C, ids, E, h, w1, w2, True)
     a = torch.empty(slot_row.numel(), Fh, dtype=h.dtype, device=h.device)
     y = torch.empty(slot_row.numel(), d, dtype=h.dtype, device=h.device)
-    C.moe_gemm(h, k, slot_row, tiles, w1, a, GATED_ACTS[kind], tm, full, w if scale_input else None, float(limit))
-    C.moe_gemm(a, 0, slot_row, tiles, w2, y, 0, tm, full, None, 0.0)
+    C.moe_gemm(h, k, slot_row, tiles, w1, a, GATED_ACTS[kind], tm, w if scale_input else None, float(limit))
+    C.moe_gemm(a, 0, slot_row, tiles, w2, y, 0, tm, None, 0.0)
     out = torch.empty_like(h)
     C.moe_combine(y, pair_slot, None if scale_input else w, out, h, extra, None)
     return out
