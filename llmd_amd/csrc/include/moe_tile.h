@@ -10,6 +10,37 @@
 
 namespace moe_tile {
 
+// order (where it is asked for): the tiles by their number of 16-row blocks, most first. cnt, first: LDS, an expert's pairs and
+// its first tile, written by this workgroup.
+constexpr int SIZES = 8;  // blocks of 16 rows that a tile can have
+__device__ __forceinline__ void by_size(const int* cnt, const int* first, int E, int tm, int* __restrict__ order, int* sizes) {
+  const int tid = threadIdx.x;
+  if (tid < SIZES) sizes[tid] = 0;
+  __syncthreads();
+  auto last = [&](int e) { return cnt[e] - (cnt[e] - 1) / tm * tm; };  // rows of an expert's last tile
+  auto bin = [](int rows) { return SIZES - (rows + 15) / 16; };
+  for (int e = tid; e < E; e += blockDim.x)
+    if (cnt[e] > 0) {
+      atomicAdd(&sizes[bin(last(e))], 1);
+      if (cnt[e] > tm) atomicAdd(&sizes[bin(tm)], (cnt[e] - 1) / tm);
+    }
+  __syncthreads();
+  if (tid == 0)
+    for (int i = 0, at = 0; i < SIZES; ++i) {
+      const int n = sizes[i];
+      sizes[i] = at;
+      at += n;
+    }
+  __syncthreads();
+  for (int e = tid; e < E; e += blockDim.x)
+    if (cnt[e] > 0) {
+      const int full = (cnt[e] - 1) / tm;
+      order[atomicAdd(&sizes[bin(last(e))], 1)] = first[e] + full;
+      if (full > 0)
+        for (int i = 0, at = atomicAdd(&sizes[bin(tm)], full); i < full; ++i) order[at + i] = first[e] + i;
+    }
+}
+
 // Sorts the pairs by expert into tiles of ``tm`` slots. tiles[0] = number of tiles, then for each tile three numbers:
 // expert | rows << 16 (the tile's first ``rows`` slots hold pairs, slot_row says which), its expert's first tile and number
 // of tiles. A pair's rank inside its expert is what its LDS counter
@@ -17,9 +48,9 @@ namespace moe_tile {
 // scan over the workgroup. 512 pairs over 128 experts: 13.7 us with a serial scan by one thread and all slots marked, now 4 us.
 __global__ __launch_bounds__(1024) static void moe_group_kernel(const int* __restrict__ ids, int n, int E, int tm,
                                                          int* __restrict__ slot_row, int* __restrict__ tiles,
-                                                         int* __restrict__ pair_slot) {
+                                                         int* __restrict__ pair_slot, int* __restrict__ order) {
   extern __shared__ int sh[];  // cnt[E] | first tile[E]
-  __shared__ int wsum[16];
+  __shared__ int wsum[16], sizes[SIZES];
   int* cnt = sh;
   int* first = sh + E;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -66,6 +97,7 @@ __global__ __launch_bounds__(1024) static void moe_group_kernel(const int* __res
     }
   }
   if (tid == 1023) tiles[0] = at;
+  if (order != nullptr) by_size(cnt, first, E, tm, order, sizes);
   __syncthreads();
   for (int p0 = 0; p0 < n; p0 += 1024 * 8) {
     int r[8], e[8];
@@ -91,7 +123,9 @@ __global__ __launch_bounds__(moe_sort::NT) static void moe_group_place_kernel(co
                                                                               const int* __restrict__ hist,
                                                                               int* __restrict__ slot_row,
                                                                               int* __restrict__ tiles,
-                                                                              int* __restrict__ pair_slot) {
+                                                                              int* __restrict__ pair_slot,
+                                                                              int* __restrict__ order) {
+  __shared__ int sizes[SIZES];
   extern __shared__ int sh[];  // pairs[E] | first tile[E] | pairs in the blocks before[E]
   int *cnt = sh, *first = sh + E;
   const int total = moe_sort::plan(hist, gridDim.x, E, tm, cnt, first, sh + 2 * E);
@@ -106,21 +140,22 @@ __global__ __launch_bounds__(moe_sort::NT) static void moe_group_place_kernel(co
       t[2] = nt;
     }
   }
+  if (order != nullptr && blockIdx.x == 0) by_size(cnt, first, E, tm, order, sizes);
   moe_sort::place(ids, n, tm, first, sh + 2 * E, slot_row, pair_slot);
 }
 
 // ``hist`` (blocks(n) * E numbers): where moe_sort::many(n, E).
 static inline void launch_group(const int* ids, int n, int E, int tm, int* hist, int* slot_row, int* tiles, int* pair_slot,
-                                hipStream_t stream) {
+                                int* order, hipStream_t stream) {
   if (!moe_sort::many(n, E)) {
     hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), 2 * E * sizeof(int), stream, ids, n, E, tm, slot_row, tiles,
-                       pair_slot);
+                       pair_slot, order);
     return;
   }
   const dim3 grid(moe_sort::blocks(n)), wg(moe_sort::NT);
   hipLaunchKernelGGL(moe_sort::moe_count_kernel, grid, wg, E * sizeof(int), stream, ids, n, E, pair_slot, hist);
   hipLaunchKernelGGL(moe_group_place_kernel, grid, wg, 3 * E * sizeof(int), stream, ids, n, E, tm, hist, slot_row, tiles,
-                     pair_slot);
+                     pair_slot, order);
 }
 
 // On the matrix cores, both types: a workgroup owns one tile (up to 128 rows of one expert) and 128 weight rows.
@@ -133,13 +168,21 @@ static inline void launch_group(const int* ids, int n, int E, int tm, int* hist,
 //                   vector cache serves at 16 bytes per clock: above HBM's rate, but not above that of weights shared by
 //                   several tiles.)
 //   more rows     : weights pass LDS too, read from memory a whole 128-byte line per eight lanes. Up to 64 rows the waves
-//                   split the weight rows, beyond that two by two.
+//                   split the weight rows, beyond that two by two in bf16, where the reads of LDS count. In fp32 the products
+//                   do (256 FLOP per clock and CU): there the waves split the weight rows up to the end, and a tile costs
+//                   its blocks of 16 rows, not 128.
 // 128 gated experts of 2048 x 768, first + second product, us. bf16, 512 rows: 64 x 128 tiles through one LDS buffer 147 + 82,
 // this 138 + 73 (5.7 and 5.4 TB/s of weights). fp32, 5600 rows: FMA form 1707 + 905, this 412 + 210; 128 rows: 213 + 99.
 //
 // Work items are (expert, block of weight rows, tile), the tiles of one block side by side: they read the same weights at the
 // same time, once from memory (tile by tile, an expert's second tile came too late for L2: 1.65 GB for 0.8 GB of weights at
 // 32768 rows). The list is cut into eight ranges, one per XCD, so that an XCD's workgroups share an expert's rows too.
+// In fp32, from 16 rows per expert on, the tiles' products differ more than their weights' streams, and the XCDs' ranges with them:
+// the tiles go to the XCDs in turn, those with the most rows first. 128 gated experts of 2048 x 768, 8 chosen, by a
+// skewed router (700 tokens: 4 to 126 rows), both products with sorting and sum, us, before / rows by 16 / and by size:
+// 700 tokens 838 / 751 / 653, 1400 1380 / 1256 / 1020, 2048 1782 / 1701 / 1394 (118 of the 152 TFLOP/s that a large product
+// reaches); by size, 200 tokens 480 / 486, 64 436 / 458. Largest and smallest in turn, so that one's products pass beside the
+// other's weights: 665, 1037, 1449. Three steps of loads ahead instead of two: equal.
 // Gated forms: the 128 weight rows are 64 gate columns and the matching up columns.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -375,6 +418,12 @@ __device__ __forceinline__ void moe_tile_many(const MoeTile& t, WRow wrow, Out o
 // One tile of ``rows`` rows: the body for its size.
 template <typename T, bool GATED, typename WRow, typename Out>
 __device__ __forceinline__ void run_tile(const MoeTile& t, int rows, WRow wrow, Out out) {
+  if constexpr (sizeof(T) == 4) {
+    if (rows > 112) return moe_tile_many<T, GATED, 8, 1, 2>(t, wrow, out);
+    if (rows > 96) return moe_tile_many<T, GATED, 7, 1, 2>(t, wrow, out);
+    if (rows > 80) return moe_tile_many<T, GATED, 6, 1, 2>(t, wrow, out);
+    if (rows > 64) return moe_tile_many<T, GATED, 5, 1, 2>(t, wrow, out);
+  }
   if (rows > 64) moe_tile_many<T, GATED, 4, 2, 2>(t, wrow, out);
   else if (rows > 48) moe_tile_many<T, GATED, 4, 1, 2>(t, wrow, out);
   else if (rows > 32) moe_tile_many<T, GATED, 3, 1, 2>(t, wrow, out);
@@ -396,6 +445,19 @@ __device__ __forceinline__ bool find_work(const int* __restrict__ tiles, int NB,
   w.tile = any[1] + j % nt;
   w.e = any[0] & 0xffff;
   w.rows = tiles[1 + 3 * w.tile] >> 16;
+  return true;
+}
+
+// The same, the tiles with the most rows first (order: by_size above), a tile's blocks of weight rows on one XCD, the tiles to the
+// XCDs in turn.
+__device__ __forceinline__ bool find_work_by_size(const int* __restrict__ tiles, const int* __restrict__ order, int NB, Work& w) {
+  const int i = blockIdx.x >> 3, j = i / NB, rank = j * 8 + (blockIdx.x & 7);
+  if (rank >= tiles[0]) return false;
+  w.tile = order[rank];
+  w.nb = i - j * NB;
+  const int t = tiles[1 + 3 * w.tile];
+  w.e = t & 0xffff;
+  w.rows = t >> 16;
   return true;
 }
 

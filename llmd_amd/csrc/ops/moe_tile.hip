@@ -52,7 +52,7 @@ extern "C" {
 int64_t llmd_moe_sort_scratch(int n, int E) { return moe_sort::many(n, E) ? (int64_t)moe_sort::blocks(n) * E : 0; }
 
 void llmd_moe_group(const int* ids, int n, int E, int* hist, int* slot_pair, int* tiles, int* inv, hipStream_t st) {
-  moe_tile::launch_group(ids, n, E, moe_tile::TBM, hist, slot_pair, tiles, inv, st);
+  moe_tile::launch_group(ids, n, E, moe_tile::TBM, hist, slot_pair, tiles, inv, nullptr, st);
 }
 
 void llmd_moe_small(const void* A, int64_t a_stride, int topk, const int* slot_pair, const int* tiles, int max_tiles,

@@ -60,9 +60,9 @@ int sm_grouped_attention_mfma(const void*, const void*, const int*, int, int, co
 void sm_moe_route_scores(const float*, const float*, int, int, int*, float*, int, int, int, float, hipStream_t);
 void sm_moe_route(const float*, int64_t, int, int, int*, float*, int, int, hipStream_t);
 int64_t sm_moe_sort_scratch(int, int);
-void sm_moe_group(const int*, int, int, int, int*, int*, int*, int*, hipStream_t);
+void sm_moe_group(const int*, int, int, int, int*, int*, int*, int*, int*, hipStream_t);
 int sm_moe_tiled(const void*, int64_t, const void*, int64_t, int64_t, int);
-void sm_moe_gemm(const void*, int64_t, int, const int*, const int*, const void*, int, int, void*, int, int, int, int,
+void sm_moe_gemm(const void*, int64_t, int, const int*, const int*, const void*, int, int, void*, int, int, int, int, int,
                  const float*, float, hipStream_t);
 int sm_moe_ring(const void*, int64_t, int64_t, const void*, int64_t, int64_t, int, int);
 int sm_retention(const void*, int64_t, int, int, int, int, const int64_t*, const float*, int, const float*, int, float,
@@ -617,20 +617,23 @@ void moe_route(Tensor logits, int64_t k, Tensor ids, Tensor w, bool sigmoid) {
   sm_moe_route(logits.data_ptr<float>(), logits.stride(0), E, k, ids.data_ptr<int>(), w.data_ptr<float>(), T, sigmoid ? 1 : 0, cur());
 }
 
-// tiles [1 + 3 max_tiles]: their number, then three numbers of each (sm_moe.hip)
+// tiles [1 + 3 max_tiles]: their number, then three numbers of each (sm_moe.hip); [1 + 4 max_tiles] (tiles of 128 rows): the
+// tiles by size too
 void moe_group(Tensor ids, int64_t E, int64_t tm, Tensor slot_row, Tensor tiles, Tensor pair_slot) {
   const c10::hip::OptionalHIPGuard g(dev_of(ids));
   CHECK_I32(ids);
   CHECK_I32(slot_row);
   CHECK_I32(tiles);
   CHECK_I32(pair_slot);
-  const int64_t n = ids.numel(), mt = tiles.numel() / 3;
+  const int64_t n = ids.numel(), mt = slot_row.numel() / std::max<int64_t>(tm, 1);
+  const bool order = tiles.numel() == 1 + 4 * mt;
   TORCH_CHECK((tm == 64 || tm == 120 || tm == 128) && E >= 1 && E <= 8192, "tile rows, experts");
+  TORCH_CHECK(tiles.numel() == 1 + 3 * mt || (order && tm == 128), "tiles");
   TORCH_CHECK(slot_row.numel() == mt * tm && pair_slot.numel() == n && mt >= (n + std::min(E, n) * (tm - 1)) / tm,
               "tile tables too small for n pairs over E experts");
   Tensor hist = torch::empty({sm_moe_sort_scratch(n, E)}, ids.options());
   sm_moe_group(ids.data_ptr<int>(), n, E, tm, hist.data_ptr<int>(), slot_row.data_ptr<int>(), tiles.data_ptr<int>(), pair_slot.data_ptr<int>(),
-               cur());
+               order ? tiles.data_ptr<int>() + 1 + 3 * mt : nullptr, cur());
 }
 
 bool moe_tiled(Tensor A, Tensor W) {
@@ -650,13 +653,15 @@ void moe_gemm(Tensor A, int64_t kdiv, Tensor slot_row, Tensor tiles, Tensor W, T
   CHECK_I32(slot_row);
   CHECK_I32(tiles);
   TORCH_CHECK(W.dim() == 3 && W.is_contiguous() && W.size(2) == A.size(1) && W.size(0) <= 8192, "W [E, N, K]");
-  const int64_t mt = tiles.numel() / 3;
+  const int64_t mt = slot_row.numel() / std::max<int64_t>(tm, 1);
   const bool gated = act == 2 || act == 3 || act == 5;
   TORCH_CHECK(act >= 0 && act <= 5 && (!gated || W.size(1) % 2 == 0), "epilogue");
   const int64_t N = gated ? W.size(1) / 2 : W.size(1);  // gated: W holds [gate rows | up rows]
   TORCH_CHECK(tm == 64 || (tm == 128 && moe_tiled(A, W)) ||
                   (tm == 120 && moe_ring(A, W, gated) && mt * tm * 4 < (int64_t)1 << 31 && ((uintptr_t)C.data_ptr() & 15) == 0),
               "tile rows");
+  const bool by_size = tm == 128 && tiles.numel() == 1 + 4 * mt;
+  TORCH_CHECK(by_size || tiles.numel() == 1 + 3 * mt, "tiles");
   TORCH_CHECK(slot_row.numel() == mt * tm && C.is_contiguous() && C.dim() == 2 && C.size(0) == mt * tm &&
                   C.size(1) == N, "C [tiles * tm, N]");
   TORCH_CHECK(kdiv > 0 || A.size(0) == mt * tm, "A rows are the tile slots");
@@ -666,7 +671,7 @@ void moe_gemm(Tensor A, int64_t kdiv, Tensor slot_row, Tensor tiles, Tensor W, T
   }
   if (N == 0) return;
   sm_moe_gemm(A.data_ptr(), A.stride(0), kdiv, slot_row.data_ptr<int>(), tiles.data_ptr<int>(), W.data_ptr(),
-              N, W.size(2), C.data_ptr(), mt, tm, (int)act, is_f32(A), row_w ? row_w->data_ptr<float>() : nullptr,
+              N, W.size(2), C.data_ptr(), mt, tm, by_size, (int)act, is_f32(A), row_w ? row_w->data_ptr<float>() : nullptr,
               (float)limit, cur());
 }
 

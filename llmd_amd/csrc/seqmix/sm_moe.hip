@@ -374,10 +374,10 @@ template <typename T, int ACT>
 __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const T* __restrict__ A, int64_t a_stride, int kdiv,
                                                           const int* __restrict__ slot_row, const int* __restrict__ tiles,
                                                           const T* __restrict__ Wt, int N, int K, T* __restrict__ Cout,
-                                                          const float* __restrict__ row_w, float limit, int NB) {
+                                                          const float* __restrict__ row_w, float limit, int NB, const int* __restrict__ order) {
   constexpr bool GATED = gated_act_code(ACT);
   Work wk;
-  if (!find_work(tiles, NB, wk)) return;
+  if (order != nullptr ? !find_work_by_size(tiles, order, NB, wk) : !find_work(tiles, NB, wk)) return;
   const int nb = wk.nb, tile = wk.tile, e = wk.e, rows = wk.rows;
   __shared__ __attribute__((aligned(128))) char lds[4 * TBUF];
   const int tid = threadIdx.x;
@@ -536,9 +536,10 @@ void sm_moe_route_scores(const float* logits, const float* corr, int E, int k, i
 // Counters that a sort of n pairs over E experts needs as scratch.
 int64_t sm_moe_sort_scratch(int n, int E) { return moe_sort::many(n, E) ? (int64_t)moe_sort::blocks(n) * E : 0; }
 
+// order: null, or where the tiles are listed by size.
 void sm_moe_group(const int* ids, int n, int E, int tm, int* hist, int* slot_row, int* tiles, int* pair_slot,
-                  hipStream_t stream) {
-  launch_group(ids, n, E, tm, hist, slot_row, tiles, pair_slot, stream);
+                  int* order, hipStream_t stream) {
+  launch_group(ids, n, E, tm, hist, slot_row, tiles, pair_slot, order, stream);
 }
 
 // Whether the matrix-core form takes these operands: 16-byte pieces of every row, an expert (``rows`` weight rows) within
@@ -558,10 +559,11 @@ int sm_moe_ring(const void* A, int64_t a_rows, int64_t a_stride, const void* W, 
 // act: 0 none, 1 erf-GELU, 2 tanh-GELU(gate) * up, 3 SiLU(gate) * up, 4 squared ReLU, 5 clamped units. N = output
 // columns (the gated forms read a weight of 2 N rows per expert). tm: slots per tile, 128 for the matrix-core form (operands
 // that sm_moe_tiled takes), 120 for its form of many rows (sm_moe_ring), 64 for the other.
+// by_size (tiles of 128 rows): behind the tables the tiles' order (sm_moe_group), in which they are taken.
 // row_w (gated forms): fp32 weight per (token, choice) pair that scales the row's INPUT, applied to
 // both fp32 sums before the activation; nullptr = 1.
 void sm_moe_gemm(const void* A, int64_t a_stride, int kdiv, const int* slot_row, const int* tiles, const void* W,
-                 int N, int K, void* C, int max_tiles, int tm, int act, int f32, const float* row_w,
+                 int N, int K, void* C, int max_tiles, int tm, int by_size, int act, int f32, const float* row_w,
                  float limit, hipStream_t stream) {
   const bool gated = gated_act_code(act);
   if (tm == moe_ring::ROWS) {
@@ -583,10 +585,11 @@ void sm_moe_gemm(const void* A, int64_t a_stride, int kdiv, const int* slot_row,
   if (tm == TBM) {
     const int NB = (N + (gated ? 63 : 127)) / (gated ? 64 : 128);
     const int64_t items = (int64_t)max_tiles * NB;
-    const dim3 grid((unsigned)((items + 7) / 8 * 8));
+    const int* order = by_size ? tiles + 1 + 3 * (int64_t)max_tiles : nullptr;
+    const dim3 grid((unsigned)(by_size ? (int64_t)((max_tiles + 7) / 8 * 8) * NB : (items + 7) / 8 * 8));
 #define SM_MT(KERN, TYPE, GRID)                                                                                       \
   hipLaunchKernelGGL(KERN, GRID, dim3(256), 0, stream, (const TYPE*)A, a_stride, kdiv, slot_row, tiles, (const TYPE*)W, \
-                     N, K, (TYPE*)C, row_w, limit, NB)
+                     N, K, (TYPE*)C, row_w, limit, NB, order)
 #define SM_MT2(A_)                                                                  \
   if (f32) SM_MT((moe_tile_kernel<float, A_>), float, grid);                        \
   else SM_MT((moe_tile_kernel<bf16_t, A_>), bf16_t, grid)
