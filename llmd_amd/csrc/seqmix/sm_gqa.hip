@@ -175,7 +175,7 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_kernel(
   }
 }
 
-// bf16 form with 16-byte accesses: a head is dim / 8 lanes, each with eight consecutive elements (four
+// Form with 16-byte accesses (fp32: without the convolution): a head is dim / 8 lanes, each with eight consecutive elements (four
 // interleaved pairs, or one eighth of a half with its partner chunk loaded beside it). Needs
 // dim = 8 * 2^k <= 512, rotary dims a multiple of 8 (16 for the half-split pairing) and 16-byte
 // aligned rows; the launcher falls back to the element-wise kernel otherwise. TAPS > 0: with the short
@@ -208,17 +208,26 @@ __device__ __forceinline__ void st8(bf16_t* p, const float (&v)[8], float mul) {
   }
   *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
 }
+__device__ __forceinline__ void ld8(const float* p, float (&v)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = 0.f;
+  add8(p, v);
+}
+__device__ __forceinline__ void st8(float* p, const float (&v)[8], float mul) {
+  *reinterpret_cast<float4*>(p) = make_float4(v[0] * mul, v[1] * mul, v[2] * mul, v[3] * mul);
+  *reinterpret_cast<float4*>(p + 4) = make_float4(v[4] * mul, v[5] * mul, v[6] * mul, v[7] * mul);
+}
 
 // The values of tg (1 or 8) tokens, a column per thread; ``unit`` numbers the workgroups of this part.
-template <int TAPS>
-__device__ __forceinline__ void value_part(int unit, const bf16_t* __restrict__ qkv, int64_t stride,
+template <typename T, int TAPS>
+__device__ __forceinline__ void value_part(int unit, const T* __restrict__ qkv, int64_t stride,
                                            const float* __restrict__ bias, const int64_t* __restrict__ positions, int Hq,
                                            int Hkv, int dim, int vdim, float* __restrict__ v_first, int v_mode, float lam,
-                                           const int64_t* __restrict__ slots, bf16_t* __restrict__ cache, int bs,
-                                           int v_from_k, const ConvArgs<bf16_t>& cv, int tg, int T) {
+                                           const int64_t* __restrict__ slots, T* __restrict__ cache, int bs,
+                                           int v_from_k, const ConvArgs<T>& cv, int tg, int ntok) {
   const int nv = Hkv * vdim, vcol0 = v_from_k ? Hq * dim : (Hq + Hkv) * dim, nvb = (nv + NT - 1) / NT;
   const int e = (unit % nvb) * NT + threadIdx.x, t0 = unit / nvb * tg;
-  if (t0 >= T || e >= nv) return;
+  if (t0 >= ntok || e >= nv) return;
   const int col = vcol0 + e, g = e / vdim, c = e - g * vdim;
   const float vb = bias ? bias[col] : 0.f;
   const int64_t vbase = (int64_t)g * bs * (dim + vdim) + (int64_t)bs * dim + (int64_t)c * bs;  // within a page
@@ -227,14 +236,18 @@ __device__ __forceinline__ void value_part(int unit, const bf16_t* __restrict__ 
 #pragma unroll
   for (int j = 0; j < TAPS; ++j) w[j] = ld(cv.w + (int64_t)col * TAPS + j);
   const int64_t s0 = slots[t0];
-  const bool eight = tg == 8 && t0 + 8 <= T && s0 >= 0 && (s0 & 7) == 0 && (bs & 7) == 0 && slots[t0 + 7] == s0 + 7;
+  bool eight = tg == 8 && t0 + 8 <= ntok && s0 >= 0 && (s0 & 7) == 0 && (bs & 7) == 0;
+  if (eight) {
+#pragma unroll
+    for (int i = 1; i < 8; ++i) eight &= slots[t0 + i] == s0 + i;  // none that is not to be written among them
+  }
   if (eight) {  // one page, hence one sequence
     constexpr int PAST = TAPS > 1 ? TAPS - 1 : 0;
     float u[8 + PAST];
     if constexpr (PAST > 0) {
       const int s = cv.row_seq[t0], run0 = t0 - cv.seq_start[s];
       const int64_t pos0 = positions[t0];
-      const bf16_t* past = cv.state + (int64_t)cv.seq_slot[s] * PAST * cv.C;
+      const T* past = cv.state + (int64_t)cv.seq_slot[s] * PAST * cv.C;
 #pragma unroll
       for (int k = 0; k < PAST; ++k) {
         const int back = PAST - k;
@@ -260,14 +273,14 @@ __device__ __forceinline__ void value_part(int unit, const bf16_t* __restrict__ 
     st8(cache + s0 / bs * page + vbase + s0 % bs, v, 1.f);
     return;
   }
-  for (int t = t0; t < min(t0 + tg, T); ++t) {
-    const bf16_t* row = qkv + t * stride;
+  for (int t = t0; t < min(t0 + tg, ntok); ++t) {
+    const T* row = qkv + t * stride;
     float v = ld(row + col) + vb;
     if constexpr (TAPS > 0) v *= w[TAPS - 1];
     if constexpr (TAPS > 1) {
       const int s = cv.row_seq[t], run = t - cv.seq_start[s];
       const int64_t pos = positions[t];
-      bf16_t* past = cv.state + (int64_t)cv.seq_slot[s] * (TAPS - 1) * cv.C;
+      T* past = cv.state + (int64_t)cv.seq_slot[s] * (TAPS - 1) * cv.C;
 #pragma unroll
       for (int j = 0; j < TAPS - 1; ++j) {
         const int back = TAPS - 1 - j;
@@ -287,17 +300,17 @@ __device__ __forceinline__ void value_part(int unit, const bf16_t* __restrict__ 
   }
 }
 
-template <int TAPS>
+template <typename T, int TAPS>
 __global__ __launch_bounds__(NT) void qkv_rope_cache_vec_kernel(
-    const bf16_t* __restrict__ qkv, int64_t stride, const float* __restrict__ bias,
+    const T* __restrict__ qkv, int64_t stride, const float* __restrict__ bias,
     const int64_t* __restrict__ positions, const float* __restrict__ cos_sin, int Hq, int Hkv, int dim, int vdim,
     int rot_dims, int interleaved, int unit, float eps, float* __restrict__ v_first, int v_mode, float lam,
-    const int64_t* __restrict__ slots, bf16_t* __restrict__ cache, int bs, bf16_t* __restrict__ q_out,
-    const float* __restrict__ qk_w, int norm_first, int v_from_k, ConvArgs<bf16_t> cv,
-    int gh, int tg, int T, const float* __restrict__ q_scale) {
+    const int64_t* __restrict__ slots, T* __restrict__ cache, int bs, T* __restrict__ q_out,
+    const float* __restrict__ qk_w, int norm_first, int v_from_k, ConvArgs<T> cv,
+    int gh, int tg, int ntok, const float* __restrict__ q_scale) {
   if ((int)blockIdx.y >= gh) {
-    value_part<TAPS>(((int)blockIdx.y - gh) * gridDim.x + blockIdx.x, qkv, stride, bias, positions, Hq, Hkv, dim, vdim,
-                     v_first, v_mode, lam, slots, cache, bs, v_from_k, cv, tg, T);
+    value_part<T, TAPS>(((int)blockIdx.y - gh) * gridDim.x + blockIdx.x, qkv, stride, bias, positions, Hq, Hkv, dim, vdim,
+                     v_first, v_mode, lam, slots, cache, bs, v_from_k, cv, tg, ntok);
     return;
   }
   const int64_t t = blockIdx.x;
@@ -305,7 +318,7 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_vec_kernel(
   const int64_t pos = positions[t];
   int run = 0;              // place in the run
   bool single = false;      // the run is this token
-  bf16_t* past = nullptr;   // the sequence's state
+  T* past = nullptr;   // the sequence's state
   if (TAPS > 1) {
     const int s = cv.row_seq[t];
     run = (int)t - cv.seq_start[s];
@@ -313,7 +326,7 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_vec_kernel(
     past = cv.state + (int64_t)cv.seq_slot[s] * (TAPS - 1) * cv.C;
   }
   const float* cs = rot_dims ? cos_sin + positions[t] * rot_dims : nullptr;  // [cos(half) | sin(half)]
-  const bf16_t* row = qkv + t * stride;
+  const T* row = qkv + t * stride;
   const int64_t slot = slots[t];
   const int Dr = dim + vdim;
   const int64_t blk = slot >= 0 ? slot / bs : 0, off = slot >= 0 ? slot % bs : 0;
@@ -429,24 +442,25 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_vec_kernel(
   }
 }
 
+// 700 tokens of 36 heads of 128 and 4 of values, fp32: 50 us by elements (every workgroup of a token formed the sums again), here 12.
 // Norms over whole projections, 16-byte form: one workgroup holds all q and k columns of a token in registers, eight
 // per thread and pass (NP passes of 2048 columns), forms both sums at once, and takes the rotation's partner values
 // from the lane that owns them (half-split pairs; a head is dim / 8 neighbouring lanes). Sizes as for the kernel above.
-template <int NP>
+template <typename T, int NP>
 __global__ __launch_bounds__(NT) void qkv_wide_cache_vec_kernel(
-    const bf16_t* __restrict__ qkv, int64_t stride, const float* __restrict__ bias,
+    const T* __restrict__ qkv, int64_t stride, const float* __restrict__ bias,
     const int64_t* __restrict__ positions, const float* __restrict__ cos_sin, int Hq, int Hkv, int dim, int vdim,
     int rot_dims, float eps, float* __restrict__ v_first, int v_mode, float lam, const int64_t* __restrict__ slots,
-    bf16_t* __restrict__ cache, int bs, bf16_t* __restrict__ q_out, const float* __restrict__ qk_w,
-    ConvArgs<bf16_t> cv, int tg, int T, const float* __restrict__ q_scale) {
+    T* __restrict__ cache, int bs, T* __restrict__ q_out, const float* __restrict__ qk_w,
+    ConvArgs<T> cv, int tg, int ntok, const float* __restrict__ q_scale) {
   if (blockIdx.y > 0) {
-    value_part<0>(((int)blockIdx.y - 1) * gridDim.x + blockIdx.x, qkv, stride, bias, positions, Hq, Hkv, dim, vdim,
-                  v_first, v_mode, lam, slots, cache, bs, 0, cv, tg, T);
+    value_part<T, 0>(((int)blockIdx.y - 1) * gridDim.x + blockIdx.x, qkv, stride, bias, positions, Hq, Hkv, dim, vdim,
+                  v_first, v_mode, lam, slots, cache, bs, 0, cv, tg, ntok);
     return;
   }
   __shared__ float red[2][NT / 64];
   const int64_t t = blockIdx.x;
-  const bf16_t* row = qkv + t * stride;
+  const T* row = qkv + t * stride;
   const int nq = Hq * dim, nqk = (Hq + Hkv) * dim;
   float x[NP][8];
   float sq = 0.f, sk = 0.f;
@@ -1855,15 +1869,12 @@ void sm_qkv_rope_cache(const void* qkv, int64_t stride, const float* bias, const
   const int per_tok = (Hq + Hkv + NT / 64 - 1) / (NT / 64);
   const int gy = std::max(1, std::min(per_tok, 4096 / T));
   const dim3 grid(T, gy);
-  if (f32)
-    hipLaunchKernelGGL((qkv_rope_cache_kernel<float>), grid, dim3(NT), 0, stream, (const float*)qkv, stride, bias,
-                       positions, cos_sin, Hq, Hkv, dim, vdim, rot_dims, interleaved, unit, eps, v_first, v_mode, lam,
-                       slots, (float*)cache, bs, (float*)q_out, qk_w, norm_first, v_from_k, cvf, wide, q_scale);
-  else if (dim % 8 == 0 && dim <= 512 && ((dim >> 3) & ((dim >> 3) - 1)) == 0 && stride % 8 == 0 &&
-           rot_dims % (interleaved ? 8 : 16) == 0 && taps <= 8 && (taps == 0 || (C % 8 == 0 && !v_from_k)) &&
-           (((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)cache | (uintptr_t)bias | (uintptr_t)cos_sin |
-             (uintptr_t)conv_w | (uintptr_t)conv_state) & 15) == 0 &&
-           (!wide || (!interleaved && (Hq + Hkv) * dim <= 8 * NT * 8 && ((uintptr_t)qk_w & 15) == 0))) {
+  if (dim % 8 == 0 && dim <= 512 && ((dim >> 3) & ((dim >> 3) - 1)) == 0 && stride % 8 == 0 &&
+      rot_dims % (interleaved ? 8 : 16) == 0 && taps <= (f32 ? 0 : 8) && (taps == 0 || (C % 8 == 0 && !v_from_k)) &&
+      (!f32 || (int64_t)bs * vdim % 4 == 0) &&
+      (((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)cache | (uintptr_t)bias | (uintptr_t)cos_sin |
+        (uintptr_t)conv_w | (uintptr_t)conv_state) & 15) == 0 &&
+      (!wide || (!interleaved && (Hq + Hkv) * dim <= 8 * NT * 8 && ((uintptr_t)qk_w & 15) == 0))) {
     // a pass covers 256 / (dim / 8) heads: fewer workgroups per token than the element-wise form
     const int hpp = NT / (dim >> 3);
     const int per_tok_v = (Hq + Hkv + hpp - 1) / hpp;
@@ -1872,32 +1883,45 @@ void sm_qkv_rope_cache(const void* qkv, int64_t stride, const float* bias, const
     const dim3 vgrid(T, (wide ? 1 : gh) + (units + T - 1) / T);
     if (wide) {
       const int np = ((Hq + Hkv) * dim + NT * 8 - 1) / (NT * 8);
-#define SM_QWC(NP)                                                                                                    \
-  hipLaunchKernelGGL(qkv_wide_cache_vec_kernel<NP>, vgrid, dim3(NT), 0, stream, (const bf16_t*)qkv, stride, bias,     \
+#define SM_QWC(TYPE, CV, NP)                                                                                          \
+  hipLaunchKernelGGL((qkv_wide_cache_vec_kernel<TYPE, NP>), vgrid, dim3(NT), 0, stream, (const TYPE*)qkv, stride, bias, \
                      positions, cos_sin, Hq, Hkv, dim, vdim, rot_dims, eps, v_first, v_mode, lam, slots,              \
-                     (bf16_t*)cache, bs, (bf16_t*)q_out, qk_w, cvh, tg, T, q_scale)
-      if (np <= 1) SM_QWC(1);
-      else if (np <= 2) SM_QWC(2);
-      else if (np <= 4) SM_QWC(4);
-      else SM_QWC(8);
+                     (TYPE*)cache, bs, (TYPE*)q_out, qk_w, CV, tg, T, q_scale)
+#define SM_QWC2(NP)                        \
+  if (f32) SM_QWC(float, cvf, NP);         \
+  else SM_QWC(bf16_t, cvh, NP)
+      if (np <= 1) { SM_QWC2(1); }
+      else if (np <= 2) { SM_QWC2(2); }
+      else if (np <= 4) { SM_QWC2(4); }
+      else { SM_QWC2(8); }
+#undef SM_QWC2
 #undef SM_QWC
       return;
     }
-#define SM_QRC(N)                                                                                                     \
-  case N:                                                                                                             \
-    hipLaunchKernelGGL(qkv_rope_cache_vec_kernel<N>, vgrid, dim3(NT), 0, stream, (const bf16_t*)qkv, stride, bias,    \
-                       positions, cos_sin, Hq, Hkv, dim, vdim, rot_dims, interleaved, unit, eps, v_first, v_mode, lam, \
-                       slots, (bf16_t*)cache, bs, (bf16_t*)q_out, qk_w, norm_first, v_from_k, cvh, gh, tg, T,         \
-                       q_scale);                                                                                      \
-    break
-    switch (taps) {
-      SM_QRC(0); SM_QRC(1); SM_QRC(2); SM_QRC(3); SM_QRC(4); SM_QRC(5); SM_QRC(6); SM_QRC(7); SM_QRC(8);
+#define SM_QRC(TYPE, CV, N)                                                                                           \
+  hipLaunchKernelGGL((qkv_rope_cache_vec_kernel<TYPE, N>), vgrid, dim3(NT), 0, stream, (const TYPE*)qkv, stride, bias, \
+                     positions, cos_sin, Hq, Hkv, dim, vdim, rot_dims, interleaved, unit, eps, v_first, v_mode, lam,  \
+                     slots, (TYPE*)cache, bs, (TYPE*)q_out, qk_w, norm_first, v_from_k, CV, gh, tg, T, q_scale)
+#define SM_QRT(N) \
+  case N: SM_QRC(bf16_t, cvh, N); break
+    if (f32) {
+      SM_QRC(float, cvf, 0);
+      return;
     }
+    switch (taps) {
+      SM_QRT(0); SM_QRT(1); SM_QRT(2); SM_QRT(3); SM_QRT(4); SM_QRT(5); SM_QRT(6); SM_QRT(7); SM_QRT(8);
+    }
+#undef SM_QRT
 #undef SM_QRC
     // runs of one token rolled their state where they read it
     if (max_q > 1) sm_conv_state(qkv, stride, C, taps, conv_state, seq_start, seq_slot, seq_init, nseq, 1, 0, stream);
     return;
-  } else
+  }
+  if (f32)
+    hipLaunchKernelGGL((qkv_rope_cache_kernel<float>), grid, dim3(NT), 0, stream, (const float*)qkv, stride, bias,
+                       positions, cos_sin, Hq, Hkv, dim, vdim, rot_dims, interleaved, unit, eps, v_first, v_mode, lam,
+                       slots, (float*)cache, bs, (float*)q_out, qk_w, norm_first, v_from_k, cvf, wide, q_scale);
+  else
     hipLaunchKernelGGL((qkv_rope_cache_kernel<bf16_t>), grid, dim3(NT), 0, stream, (const bf16_t*)qkv, stride, bias,
                        positions, cos_sin, Hq, Hkv, dim, vdim, rot_dims, interleaved, unit, eps, v_first, v_mode, lam,
                        slots, (bf16_t*)cache, bs, (bf16_t*)q_out, qk_w, norm_first, v_from_k, cvh, wide, q_scale);

@@ -459,12 +459,35 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const T* __restrict__ 
   }
 }
 
-// bf16 rows that are 16-byte multiples: a thread sums eight columns from 16-byte loads.
-__global__ __launch_bounds__(256) void moe_combine_vec_kernel(const bf16_t* __restrict__ y,
-                                                              const int* __restrict__ pair_slot,
-                                                              const float* __restrict__ w, int k, int d,
-                                                              bf16_t* __restrict__ out, const bf16_t* __restrict__ h,
-                                                              const bf16_t* __restrict__ extra,
+// Rows of whole groups of eight: a thread sums eight columns from 16-byte loads. Bound by the rows' way from memory:
+// 700 tokens of 8 fp32 rows of 2048 (46 MB) 38 us by elements, here 13; 2048 tokens in bf16 15.7.
+__device__ __forceinline__ void fma8(float (&s)[8], float w, const bf16_t* p) {
+  const u32x4_t v = *reinterpret_cast<const u32x4_t*>(p);
+#pragma unroll
+  for (int q = 0; q < 8; ++q) s[q] += w * __uint_as_float((v[q >> 1] >> (16 * (q & 1))) << 16);
+}
+__device__ __forceinline__ void fma8(float (&s)[8], float w, const float* p) {
+  const f32x4_t v[2] = {*reinterpret_cast<const f32x4_t*>(p), *reinterpret_cast<const f32x4_t*>(p + 4)};
+#pragma unroll
+  for (int q = 0; q < 8; ++q) s[q] += w * v[q >> 2][q & 3];
+}
+__device__ __forceinline__ void put8(bf16_t* p, const float (&s)[8]) {
+  u32x4_t o;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const __bf16 a = (__bf16)s[2 * q], b = (__bf16)s[2 * q + 1];
+    o[q] = (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+  }
+  *reinterpret_cast<u32x4_t*>(p) = o;
+}
+__device__ __forceinline__ void put8(float* p, const float (&s)[8]) {
+  *reinterpret_cast<f32x4_t*>(p) = f32x4_t{s[0], s[1], s[2], s[3]};
+  *reinterpret_cast<f32x4_t*>(p + 4) = f32x4_t{s[4], s[5], s[6], s[7]};
+}
+template <typename T>
+__global__ __launch_bounds__(256) void moe_combine_vec_kernel(const T* __restrict__ y, const int* __restrict__ pair_slot,
+                                                              const float* __restrict__ w, int k, int d, T* __restrict__ out,
+                                                              const T* __restrict__ h, const T* __restrict__ extra,
                                                               const float* __restrict__ eg, int64_t eg_stride) {
   const int64_t t = blockIdx.x;
   const float ge = eg ? 1.f / (1.f + expf(-eg[t * eg_stride])) : 1.f;
@@ -472,23 +495,10 @@ __global__ __launch_bounds__(256) void moe_combine_vec_kernel(const bf16_t* __re
     float s[8] = {};
     for (int j = 0; j < k; ++j) {
       const int slot = pair_slot[t * k + j];
-      const float wj = w ? w[t * k + j] : 1.f;
-      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(slot >= 0 ? y + (int64_t)slot * d + c : h + t * d + c);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) s[q] += wj * __uint_as_float((v[q >> 1] >> (16 * (q & 1))) << 16);
+      fma8(s, w ? w[t * k + j] : 1.f, slot >= 0 ? y + (int64_t)slot * d + c : h + t * d + c);
     }
-    if (extra) {
-      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(extra + t * d + c);
-#pragma unroll
-      for (int q = 0; q < 8; ++q) s[q] += ge * __uint_as_float((v[q >> 1] >> (16 * (q & 1))) << 16);
-    }
-    u32x4_t o;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const __bf16 a = (__bf16)s[2 * q], b = (__bf16)s[2 * q + 1];
-      o[q] = (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
-    }
-    *reinterpret_cast<u32x4_t*>(out + t * d + c) = o;
+    if (extra) fma8(s, ge, extra + t * d + c);
+    put8(out + t * d + c, s);
   }
 }
 
@@ -628,9 +638,10 @@ void sm_moe_combine(const void* y, const int* pair_slot, const float* w, int k, 
 #define SM_CO(KERN, TYPE)                                                                                       \
   hipLaunchKernelGGL(KERN, dim3(T), dim3(256), 0, stream, (const TYPE*)y, pair_slot, w, k, d, (TYPE*)out,       \
                      (const TYPE*)h, (const TYPE*)extra, eg, eg_stride)
-  if (f32) SM_CO(moe_combine_kernel<float>, float);
-  else if (d % 8 == 0 && (((uintptr_t)y | (uintptr_t)out | (uintptr_t)h | (uintptr_t)extra) & 15) == 0)
-    SM_CO(moe_combine_vec_kernel, bf16_t);
+  const bool vec = d % 8 == 0 && (((uintptr_t)y | (uintptr_t)out | (uintptr_t)h | (uintptr_t)extra) & 15) == 0;
+  if (f32 && vec) SM_CO(moe_combine_vec_kernel<float>, float);
+  else if (f32) SM_CO(moe_combine_kernel<float>, float);
+  else if (vec) SM_CO(moe_combine_vec_kernel<bf16_t>, bf16_t);
   else SM_CO(moe_combine_kernel<bf16_t>, bf16_t);
 #undef SM_CO
 }
