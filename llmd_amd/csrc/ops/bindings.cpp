@@ -650,12 +650,13 @@ void mgemm_fp8(torch::Tensor y, torch::Tensor xq, torch::Tensor xs, torch::Tenso
   TORCH_CHECK(rc == 0, "mgemm_fp8 failed: ", rc);
 }
 
-extern "C" int llmd_kv_dequant_gather(const void*, const void*, int64_t, const int*, int, int, int, void*, void*,
-                                      hipStream_t);
+extern "C" int llmd_kv_dequant_gather(const void*, const void*, int64_t, const int*, int, int, int, const int*, int, int, void*,
+                                      void*, int*, hipStream_t);
 
-// fp8 paged K/V blocks of a block table -> dense bf16 copies kd / vd [entries, Hkv, bs, D] (attn_prefill.hip)
-void kv_dequant_gather(torch::Tensor k_cache, torch::Tensor v_cache, torch::Tensor block_tables, torch::Tensor kd,
-                       torch::Tensor vd) {
+// fp8 paged K/V blocks of a block table [S, maxb] -> dense bf16 copies kd / vd [entries, Hkv, bs, D] (attn_prefill.hip);
+// ctx [S]: entries well past a sequence's context are left as they are; place [entries]: the table over the copies
+void kv_dequant_gather(torch::Tensor k_cache, torch::Tensor v_cache, torch::Tensor block_tables, c10::optional<torch::Tensor> ctx,
+                       torch::Tensor kd, torch::Tensor vd, torch::Tensor place) {
   const c10::hip::OptionalHIPGuard device_guard(dev_of(k_cache));
   CHECK_CUDA(k_cache); CHECK_DT(k_cache, at::kFloat8_e4m3fn); CHECK_DT(v_cache, at::kFloat8_e4m3fn);
   CHECK_BF16(kd); CHECK_BF16(vd); CHECK_DT(block_tables, at::kInt);
@@ -666,9 +667,16 @@ void kv_dequant_gather(torch::Tensor k_cache, torch::Tensor v_cache, torch::Tens
               k_cache.stride(1) == k_cache.size(2) * k_cache.size(3), "a block's [Hkv, bs, D] contiguous");
   TORCH_CHECK(block_tables.is_contiguous() && kd.is_contiguous() && vd.is_contiguous() &&
               kd.numel() == block_tables.numel() * per && vd.numel() == kd.numel(), "kd / vd [entries, Hkv, bs, D]");
+  CHECK_DT(place, at::kInt);
+  TORCH_CHECK(block_tables.dim() == 2 && place.is_cuda() && place.is_contiguous() && place.numel() == block_tables.numel(), "place [entries]");
+  if (ctx) {
+    CHECK_DT(*ctx, at::kInt);
+    TORCH_CHECK(ctx->is_cuda() && ctx->is_contiguous() && ctx->numel() == block_tables.size(0), "ctx [S]");
+  }
   const int rc = llmd_kv_dequant_gather(k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
-                                        block_tables.data_ptr<int>(), (int)block_tables.numel(),
-                                        (int)k_cache.size(0), (int)per, kd.data_ptr(), vd.data_ptr(), cur_stream());
+                                        block_tables.data_ptr<int>(), (int)block_tables.numel(), (int)block_tables.size(1),
+                                        (int)k_cache.size(2), ctx ? ctx->data_ptr<int>() : nullptr, (int)k_cache.size(0),
+                                        (int)per, kd.data_ptr(), vd.data_ptr(), place.data_ptr<int>(), cur_stream());
   TORCH_CHECK(rc == 0, "kv_dequant_gather failed: ", rc);
 }
 

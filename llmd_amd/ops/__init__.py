@@ -391,10 +391,11 @@ def build_prefill_items(q_len: list[int], ctx_len: list[int], tpi: int) -> list[
 PREFILL_FP8_VIA_BF16 = os.environ.get("LLMD_PREFILL_FP8_VIA_BF16", "1") == "1"
 
 
-def kv_dequant_gather(k_cache, v_cache, block_tables):
+def kv_dequant_gather(k_cache, v_cache, block_tables, ctx_len=None):
     """(k, v, table): the blocks ``block_tables`` [S, maxb] names in an fp8 paged cache [blocks, Hkv,
     bs, D], widened exactly to bf16 into dense copies [S * maxb, Hkv, bs, D] and the identity table
-    over them (padding entries copy block 0, never read)."""
+    over them (padding entries copy block 0, never read). With ``ctx_len`` [S] int32 blocks 256 keys and more behind a
+    sequence's context need not be copied."""
     S, mb = block_tables.shape
     shape = (S * mb,) + tuple(k_cache.shape[1:])
     if not _gpu(k_cache):
@@ -403,8 +404,9 @@ def kv_dequant_gather(k_cache, v_cache, block_tables):
                 torch.arange(S * mb, dtype=torch.int32).view(S, mb))
     kd = torch.empty(shape, dtype=torch.bfloat16, device=k_cache.device)
     vd = torch.empty(shape, dtype=torch.bfloat16, device=k_cache.device)
-    native().kv_dequant_gather(k_cache, v_cache, block_tables.contiguous(), kd, vd)
-    return kd, vd, torch.arange(S * mb, dtype=torch.int32, device=k_cache.device).view(S, mb)
+    place = torch.empty(S, mb, dtype=torch.int32, device=k_cache.device)
+    native().kv_dequant_gather(k_cache, v_cache, block_tables.contiguous(), ctx_len, kd, vd, place)
+    return kd, vd, place
 
 
 def paged_prefill(q, k_cache, v_cache, block_tables, q_start, q_len, ctx_len, Hq, Hkv, D, scale,
@@ -420,7 +422,7 @@ def paged_prefill(q, k_cache, v_cache, block_tables, q_start, q_len, ctx_len, Hq
         out = torch.empty(q.shape[0], Hq * D, dtype=q.dtype, device=q.device)
     if (PREFILL_FP8_VIA_BF16 and k_cache.dtype == torch.float8_e4m3fn and k_cache.shape[-2] >= 16
             and D in (64, 128)):
-        k_cache, v_cache, block_tables = kv_dequant_gather(k_cache, v_cache, block_tables)
+        k_cache, v_cache, block_tables = kv_dequant_gather(k_cache, v_cache, block_tables, ctx_len)
     if items is None:
         tpi = prefill_tokens_per_item(Hq, Hkv, D, k_cache.shape[-2], k_cache.dtype == torch.float8_e4m3fn)
         it = build_prefill_items(q_len.tolist(), ctx_len.tolist(), tpi)
