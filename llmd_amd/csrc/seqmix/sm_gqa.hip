@@ -176,12 +176,14 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_kernel(
 }
 
 // Form with 16-byte accesses (fp32: without the convolution): a head is dim / 8 lanes, each with eight consecutive elements (four
-// interleaved pairs, or one eighth of a half with its partner chunk loaded beside it). Needs
+// interleaved pairs, or one eighth of a half, whose partner values come from the lane that owns them). Needs
 // dim = 8 * 2^k <= 512, rotary dims a multiple of 8 (16 for the half-split pairing) and 16-byte
-// aligned rows; the launcher falls back to the element-wise kernel otherwise. TAPS > 0: with the short
-// convolution - every lane convolves its own eight columns and the rotation's partner values come from the
-// lane that owns them, so a column of the state is read (and, for a run of one token, rolled forward) by
-// one thread only.
+// aligned rows and weights; the launcher falls back to the element-wise kernel otherwise. TAPS > 0: with the short
+// convolution - every lane convolves its own eight columns, so a column of the state is read (and, for a run of one
+// token, rolled forward) by one thread only. Bound by memory and, with bias, norm weights and angles beside the rows, by the
+// vector cache: angles are read once for all heads of a thread, weights 16 bytes at a time. 2048 tokens of 32 + 4 heads of 128
+// with bias, weights before the rotation and keys as values: 33 us with the partner's values, bias and weights read again,
+// now 17.7; without any of them 12.4.
 // blockIdx.y < gh: the heads of token blockIdx.x. The other workgroups take the values, a column per
 // thread and tg (1 or 8) tokens: the values of a page are transposed, so eight consecutive tokens of a
 // sequence whose first lands on a multiple of eight are one 16-byte store (a prompt's inner tokens).
@@ -333,14 +335,20 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_vec_kernel(
   const int lph = dim >> 3, hpp = NT / lph;  // lanes per head, heads per pass
   const int c = threadIdx.x & (lph - 1), hl = threadIdx.x / lph;
   const float q_mul = q_scale ? q_scale[pos] : 1.f;
+  const bool first = c * 8 < half;
+  float cc[8] = {}, sn[8] = {};  // half-split pairing: of this lane's columns, in every head
+  if (!interleaved && c * 8 < rot_dims) {
+    add8(cs + (first ? c * 8 : c * 8 - half), cc);
+    add8(cs + half + (first ? c * 8 : c * 8 - half), sn);
+  }
   for (int h0 = blockIdx.y * hpp; h0 < Hq + Hkv; h0 += gh * hpp) {
     const int hd = h0 + hl;
     const bool on = hd < Hq + Hkv;
     const int col = hd * dim + c * 8;  // q heads, then k heads, back to back in the projection
     float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     float ss = 0.f;
-    const float* nw = qk_w ? qk_w + (hd < Hq ? 0 : dim) : nullptr;
-    const float* nw1 = norm_first ? nw : nullptr;  // weights applied before the rotation
+    float w8[8] = {};  // the norm's weights
+    if (qk_w) add8(qk_w + (hd < Hq ? 0 : dim) + c * 8, w8);
     if (on) {
       ld8(row + col, x);
       if (bias) add8(bias + col, x);
@@ -380,14 +388,13 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_vec_kernel(
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           ss += x[i] * x[i];
-          if (nw1) x[i] *= nw1[c * 8 + i];
+          if (qk_w) x[i] *= w8[i];  // before the rotation
         }
       }
     }
-    float xp[8];  // the rotation's partner values (half-split pairing)
+    float xp[8];  // the rotation's partner values (half-split pairing), from the lane that has them (all lanes take part)
     const bool turn = on && c * 8 < rot_dims;
-    const bool first = c * 8 < half;
-    if (TAPS > 0 && rot_dims > 0 && !interleaved) {  // from the lane that convolved them (all lanes take part)
+    if (rot_dims > 0 && !interleaved) {
       const int src = turn ? (int)(threadIdx.x & 63) + (first ? half : -half) / 8 : (int)(threadIdx.x & 63);
 #pragma unroll
       for (int i = 0; i < 8; ++i) xp[i] = __shfl(x[i], src, 64);
@@ -405,19 +412,6 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_vec_kernel(
             x[2 * i + 1] = v * cc[i] + u * sn[i];
           }
         } else {
-          const int pc = first ? col + half : col - half;  // the partner chunk
-          const int f = first ? c * 8 : c * 8 - half;
-          float cc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, sn[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-          if (TAPS == 0) {
-            ld8(row + pc, xp);
-            if (bias) add8(bias + pc, xp);
-            if (nw1) {
-#pragma unroll
-              for (int i = 0; i < 8; ++i) xp[i] *= nw1[c * 8 + (first ? half : -half) + i];
-            }
-          }
-          add8(cs + f, cc);
-          add8(cs + half + f, sn);
 #pragma unroll
           for (int i = 0; i < 8; ++i) x[i] = first ? x[i] * cc[i] - xp[i] * sn[i] : x[i] * cc[i] + xp[i] * sn[i];
         }
@@ -433,9 +427,9 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_vec_kernel(
       inv *= 1.f / sqrtf(ss / (float)dim + eps);
     }
     if (!on) continue;
-    if (nw && !nw1) {
+    if (qk_w && !norm_first) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] *= nw[c * 8 + i];
+      for (int i = 0; i < 8; ++i) x[i] *= w8[i];
     }
     if (hd < Hq) st8(q_out + (t * Hq + hd) * dim + c * 8, x, inv);
     else if (slot >= 0) st8(cache + (blk * Hkv + (hd - Hq)) * bs * Dr + off * dim + c * 8, x, inv);
@@ -1872,9 +1866,9 @@ void sm_qkv_rope_cache(const void* qkv, int64_t stride, const float* bias, const
   if (dim % 8 == 0 && dim <= 512 && ((dim >> 3) & ((dim >> 3) - 1)) == 0 && stride % 8 == 0 &&
       rot_dims % (interleaved ? 8 : 16) == 0 && taps <= (f32 ? 0 : 8) && (taps == 0 || (C % 8 == 0 && !v_from_k)) &&
       (!f32 || (int64_t)bs * vdim % 4 == 0) &&
-      (((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)cache | (uintptr_t)bias | (uintptr_t)cos_sin |
+      (((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)cache | (uintptr_t)bias | (uintptr_t)cos_sin | (uintptr_t)qk_w |
         (uintptr_t)conv_w | (uintptr_t)conv_state) & 15) == 0 &&
-      (!wide || (!interleaved && (Hq + Hkv) * dim <= 8 * NT * 8 && ((uintptr_t)qk_w & 15) == 0))) {
+      (!wide || (!interleaved && (Hq + Hkv) * dim <= 8 * NT * 8))) {
     // a pass covers 256 / (dim / 8) heads: fewer workgroups per token than the element-wise form
     const int hpp = NT / (dim >> 3);
     const int per_tok_v = (Hq + Hkv + hpp - 1) / hpp;
