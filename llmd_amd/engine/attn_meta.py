@@ -10,6 +10,7 @@ from __future__ import annotations
 from dataclasses import dataclass
 from typing import Optional
 
+import numpy as np
 import torch
 
 
@@ -47,22 +48,19 @@ class SeqMeta:
         key = (tokens_per_item, balance if self.ctx_lens is not None else 0)
         it = self._items.get(key)
         if it is None:
-            rows, keys, t0 = [], [], 0
-            for s, n in enumerate(self.q_lens):
-                for a in range(0, n, tokens_per_item):
-                    c = min(tokens_per_item, n - a)
-                    rows.append((s, t0 + a, c))
-                    if key[1]:
-                        keys.append(self.ctx_lens[s] - n + a + c)
-                t0 += n
+            # numpy throughout: a stack of several attention kinds with a prompt of 2048 tokens waited for the host here
+            ql = np.asarray(self.q_lens, dtype=np.int64).reshape(-1)
+            per = -(-ql // tokens_per_item)                       # items of each run
+            seq = np.repeat(np.arange(len(ql)), per)
+            a = (np.arange(len(seq)) - np.repeat(np.cumsum(per) - per, per)) * tokens_per_item  # within the run
+            c = np.minimum(tokens_per_item, ql[seq] - a)
+            rows = np.stack([seq, (np.cumsum(ql) - ql)[seq] + a, c], 1).astype(np.int32)
             if key[1] and len(rows) > 1:
-                order = sorted(range(len(rows)), key=lambda i: -keys[i])
-                snake = []
-                for b in range(0, len(order), balance):
-                    blk = order[b:b + balance]
-                    snake.extend(blk if (b // balance) % 2 == 0 else blk[::-1])
-                rows = [rows[i] for i in snake]
-            it = torch.tensor(rows, dtype=torch.int32).view(-1, 3)
+                keys = np.asarray(self.ctx_lens, dtype=np.int64)[seq] - ql[seq] + a + c
+                order = np.argsort(-keys, kind="stable")
+                rows = rows[np.concatenate([order[b:b + balance][::-1 if b // balance % 2 else 1]
+                                            for b in range(0, len(order), balance)])]
+            it = torch.from_numpy(np.ascontiguousarray(rows))
             if self.tables.is_cuda:
                 it = it.pin_memory().to(self.tables.device, non_blocking=True)
             self._items[key] = it

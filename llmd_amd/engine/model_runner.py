@@ -26,6 +26,7 @@ import logging
 import math
 import os
 import time
+from array import array
 from typing import Optional
 
 import numpy as np
@@ -760,9 +761,10 @@ class ModelRunner:
         nd = pl["nd"]
         T = len(ids)
         swa = pl.get("swa")
-        host = torch.tensor([ids, pos, slots] + ([swa[0]] if swa is not None else []), dtype=torch.long)
-        if self.is_gpu:
-            host = host.pin_memory()
+        lists = [ids, pos, slots] + ([swa[0]] if swa is not None else [])
+        host = torch.empty(len(lists), T, dtype=torch.long, pin_memory=self.is_gpu)
+        for row, values in zip(host.numpy(), lists):  # array: a third of torch.tensor's time for a list
+            row[:] = array("q", values)
         hd = host.to(dev, non_blocking=True)
         meta = AttnMeta(num_tokens=T, positions=hd[1], slot_mapping=hd[2], num_decode=nd)
         if pl.get("seq") is not None:
@@ -819,7 +821,7 @@ class ModelRunner:
         start = np.zeros(n + 1, dtype=np.int32)
         start[1:] = np.cumsum(ql)
         row_seq = np.repeat(np.arange(n, dtype=np.int32), ql)
-        row_len = (np.asarray(pl["pos"], dtype=np.int64) + 1).astype(np.int32)
+        row_len = (np.frombuffer(array("q", pl["pos"]), dtype=np.int64) + 1).astype(np.int32)
         tables = np.concatenate([pl["d_bt"], pl["p_bt"]]) if n else np.zeros((0, self.width), np.int32)
         small = torch.from_numpy(np.concatenate([start, np.asarray(slots, np.int32), np.asarray(init, np.int32),
                                                  row_seq, row_len]))
