@@ -96,7 +96,7 @@ void llmd_rms_norm_quant(void*, int64_t, float*, const void*, int64_t, void*, in
                          hipStream_t);
 void llmd_gated_act_quant(void*, int64_t, float*, const void*, int64_t, int, int, int, float, float, hipStream_t);
 int llmd_quant_fp8_groups(const void*, int64_t, void*, int64_t, float*, int64_t, int, int, hipStream_t);
-int llmd_quant_fp8_groups_padded(const void*, int64_t, void*, int64_t, float*, int64_t, int, int, int, const int*,
+int llmd_quant_fp8_groups_padded(const void*, int64_t, void*, int64_t, float*, int64_t, int, int, int, int, const int*,
                                  hipStream_t);
 void llmd_moe_gemm_fp8(const void*, int64_t, const float*, int64_t, int, const int*, const int*, int, const void*,
                        int64_t, const float*, int, int, void*, int64_t, int, int, float, float, int, const void*,
@@ -1161,7 +1161,7 @@ void quant_fp8_groups(torch::Tensor x, torch::Tensor q, torch::Tensor scale) {
   TORCH_CHECK(rc == 0, "quant_fp8_groups failed: ", rc);
 }
 
-// x [T, d] bf16 -> q [T, kp] e4m3 (zeros past d) + per-128 scales; rows >= row_limit[0] skipped when given
+// x [T, d] bf16 -> q [T, kp] e4m3 (zeros past d) + per-128 scales (1 for the groups past d, as far as ``scale`` has them); rows >= row_limit[0] skipped when given
 void quant_fp8_groups_padded(torch::Tensor x, torch::Tensor q, torch::Tensor scale, c10::optional<torch::Tensor> row_limit) {
   const c10::hip::OptionalHIPGuard device_guard(dev_of(x));
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_INNER(x); CHECK_INNER(q); CHECK_DT(q, at::kFloat8_e4m3fn);
@@ -1178,8 +1178,8 @@ void quant_fp8_groups_padded(torch::Tensor x, torch::Tensor q, torch::Tensor sca
     lim = row_limit->data_ptr<int>();
   }
   int rc = llmd_quant_fp8_groups_padded(x.data_ptr(), x.stride(0), q.data_ptr(), q.stride(0),
-                                        scale.data_ptr<float>(), scale.stride(0), x.size(0), d, kp, lim,
-                                        cur_stream());
+                                        scale.data_ptr<float>(), scale.stride(0), x.size(0), d, kp,
+                                        (int)std::min<int64_t>(scale.size(1), (kp + 127) / 128), lim, cur_stream());
   TORCH_CHECK(rc == 0, "quant_fp8_groups_padded failed: ", rc);
 }
 

@@ -52,7 +52,8 @@ __global__ __launch_bounds__(NT) void quant_fp8_rows_kernel(const uint16_t* __re
 // 16 consecutive lanes own one group's 16 packets; the group amax is a 16-lane
 // xor-shuffle reduction. s[t][g] = amax / 448.
 // kp > d: q rows are kp bytes wide and columns [d, kp) are zero-filled (the K-padded operand of the
-// grouped GEMM); row_limit (device scalar, nullable): rows at or past it are left untouched - the
+// grouped GEMM), with scales of 1 for the groups up to ng that hold nothing else (the GEMM multiplies by them: a scale
+// left as memory had it may be a NaN); row_limit (device scalar, nullable): rows at or past it are left untouched - the
 // grouped GEMM's padded-slot rows beyond the last real expert tile, which it never reads.
 // One wave per row (4 rows per 256-thread workgroup): a row of a few thousand columns is a few
 // 8-column chunks per lane, and a 128-column group is 16 lanes, so the group amax is a 16-lane
@@ -60,7 +61,7 @@ __global__ __launch_bounds__(NT) void quant_fp8_rows_kernel(const uint16_t* __re
 __global__ __launch_bounds__(NT) void quant_fp8_groups_kernel(const uint16_t* __restrict__ x, int64_t xs,
                                                               uint8_t* __restrict__ q, int64_t qs,
                                                               float* __restrict__ scale, int64_t ss, int T,
-                                                              int d, int kp, const int* __restrict__ row_limit,
+                                                              int d, int kp, int ng, const int* __restrict__ row_limit,
                                                               float floor_) {
   const int64_t t = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -87,6 +88,7 @@ __global__ __launch_bounds__(NT) void quant_fp8_groups_kernel(const uint16_t* __
     if (ok) qr[c] = f32x8_to_fp8(f);
   }
   for (int c = nc + lane; c < kp / 8; c += 64) qr[c] = u32x2_t{0u, 0u};
+  for (int g = span / 16 + lane; g < ng; g += 64) scale[t * ss + g] = 1.f;
 }
 
 }  // namespace
@@ -96,18 +98,18 @@ extern "C" int llmd_quant_fp8_groups(const void* x, int64_t xs, void* q, int64_t
   if (T == 0) return 0;
   if (d % 8) return -1;
   hipLaunchKernelGGL(quant_fp8_groups_kernel, dim3((T + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, st,
-                     (const uint16_t*)x, xs, (uint8_t*)q, qs, scale, ss, T, d, d, (const int*)nullptr, 1e-12f);
+                     (const uint16_t*)x, xs, (uint8_t*)q, qs, scale, ss, T, d, d, 0, (const int*)nullptr, 1e-12f);
   return (int)hipGetLastError();
 }
 
-// rows of kp >= d bytes (zeros past d), rows >= *row_limit skipped (row_limit nullable)
+// rows of kp >= d bytes (zeros past d) and ng scales, rows >= *row_limit skipped (row_limit nullable)
 extern "C" int llmd_quant_fp8_groups_padded(const void* x, int64_t xs, void* q, int64_t qs, float* scale,
-                                            int64_t ss, int T, int d, int kp, const int* row_limit,
+                                            int64_t ss, int T, int d, int kp, int ng, const int* row_limit,
                                             hipStream_t st) {
   if (T == 0) return 0;
   if (d % 8 || kp % 8 || kp < d || qs < kp) return -1;
   hipLaunchKernelGGL(quant_fp8_groups_kernel, dim3((T + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, st,
-                     (const uint16_t*)x, xs, (uint8_t*)q, qs, scale, ss, T, d, kp, row_limit, 1e-12f);
+                     (const uint16_t*)x, xs, (uint8_t*)q, qs, scale, ss, T, d, kp, ng, row_limit, 1e-12f);
   return (int)hipGetLastError();
 }
 

@@ -97,6 +97,45 @@ def test_moe_gemm8_mxfp4_matches_fp32(mode, tile, stages, K, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("d,K", [(256, 512), (128, 512), (72, 512), (384, 512), (2880, 2944), (8, 1024 * 9)])
+@pytest.mark.parametrize("limit", [None, 37])
+def test_groups_past_the_row_have_finite_scales(d, K, limit):
+    """Rows padded to K by whole groups of 128 and more: the GEMM multiplies those groups' codes by their scales too, so that
+    none may be left as memory had it (-1 as an exponent is a NaN, and NaN times zero codes a NaN in every column)."""
+    torch.manual_seed(d)
+    T = 51
+    x = torch.randn(T, d, device="cuda", dtype=torch.bfloat16)
+    q = torch.full((T, K), -1, device="cuda", dtype=torch.int8).view(ops.FP8)
+    s = torch.full((T, K // 128), -1, device="cuda", dtype=torch.int32).view(torch.float32)
+    lim = None if limit is None else torch.tensor([limit], dtype=torch.int32, device="cuda")
+    ops.native().quant_fp8_groups_padded(x, q, s, lim)
+    n, real = limit or T, (d + 127) // 128
+    rq, rs = ops.quant_fp8_groups(x.cpu())
+    assert torch.equal(q[:n, :d].cpu().float(), rq[:n].float()) and torch.equal(s[:n, :real].cpu(), rs[:n])
+    assert (q[:n, d:].view(torch.uint8) == 0).all() and (s[:n, real:] == 1.0).all()
+    assert (q[n:].view(torch.int8) == -1).all() and (s[n:].view(torch.int32) == -1).all()
+
+
+@pytest.mark.gpu
+def test_moe_experts_mxfp4_narrow_rows():
+    """Experts of 256 columns, stored with 512: the same result whatever the buffers of the call held before."""
+    torch.manual_seed(3)
+    E, k, d, F, T = 8, 2, 256, 256, 90
+    x = torch.randn(T, d, device="cuda", dtype=torch.bfloat16)
+    w1q, w1s = ops.quant_mxfp4_weight(ops.pad_mxfp4_k(torch.randn(E, 2 * F, d, device="cuda") * 0.06, 512))
+    w2q, w2s = ops.quant_mxfp4_weight(ops.pad_mxfp4_k(torch.randn(E, d, F, device="cuda") * 0.06, 512))
+    w1q, w2q = ops.mxfp4_kernel_layout(w1q), ops.mxfp4_kernel_layout(w2q)
+    w1s, w2s = ops.mxfp4_scales_kernel_layout(w1s), ops.mxfp4_scales_kernel_layout(w2s)
+    ids, wts = ops.moe_topk(torch.randn(T, E, device="cuda"), k, scoring=0)
+    r = ops.moe_experts_mxfp4(x.cpu(), ids.cpu(), wts.cpu(), w1q.cpu(), w1s.cpu(), w2q.cpu(), w2s.cpu(), 2).float()
+    for fill in (0, -1):  # what the allocator hands out next
+        held = [torch.full((n,), fill, device="cuda", dtype=torch.int32) for n in (64, 360, 512, 1 << 12, 1 << 14, 1 << 20) for _ in range(8)]
+        del held
+        y = ops.moe_experts_mxfp4(x, ids, wts, w1q, w1s, w2q, w2s, 2).float().cpu()
+        assert (y - r).abs().max() < 0.06 * r.abs().max() + 1e-3, fill
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [5, 64, 700])
 def test_moe_experts_mxfp4_gpu_vs_cpu(T):
     torch.manual_seed(3)
