@@ -178,11 +178,12 @@ static inline void launch_group(const int* ids, int n, int E, int tm, int* hist,
 // same time, once from memory (tile by tile, an expert's second tile came too late for L2: 1.65 GB for 0.8 GB of weights at
 // 32768 rows). The list is cut into eight ranges, one per XCD, so that an XCD's workgroups share an expert's rows too.
 // In fp32, from 16 rows per expert on, the tiles' products differ more than their weights' streams, and the XCDs' ranges with them:
-// the tiles go to the XCDs in turn, those with the most rows first. 128 gated experts of 2048 x 768, 8 chosen, by a
-// skewed router (700 tokens: 4 to 126 rows), both products with sorting and sum, us, before / rows by 16 / and by size:
+// the tiles go to the XCDs in turn, those with the most rows first (find_work_by_size). 128 gated experts of 2048 x 768, 8 chosen,
+// by a skewed router (700 tokens: 4 to 126 rows), both products with sorting and sum, us, before / rows by 16 / and by size:
 // 700 tokens 838 / 751 / 653, 1400 1380 / 1256 / 1020, 2048 1782 / 1701 / 1394 (118 of the 152 TFLOP/s that a large product
-// reaches); by size, 200 tokens 480 / 486, 64 436 / 458. Largest and smallest in turn, so that one's products pass beside the
-// other's weights: 665, 1037, 1449. Three steps of loads ahead instead of two: equal.
+// reaches). The line: by expert / by size at 17, 19, 22, 28, 36 rows per expert, uniform router 482 / 478, 466 / 486, 485 / 494,
+// 522 / 518, 598 / 577, skewed 598 / 505, 517 / 510, 706 / 549, 778 / 577, 921 / 645; 4 rows 436 / 458. Largest and smallest in turn,
+// so that one's products pass beside the other's weights: 665, 1037, 1449. Three steps of loads ahead instead of two: equal.
 // Gated forms: the 128 weight rows are 64 gate columns and the matching up columns.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -448,13 +449,26 @@ __device__ __forceinline__ bool find_work(const int* __restrict__ tiles, int NB,
   return true;
 }
 
-// The same, the tiles with the most rows first (order: by_size above), a tile's blocks of weight rows on one XCD, the tiles to the
-// XCDs in turn.
+// The same, the tiles with the most rows first (order: by_size above). From EVEN tiles on the XCDs take tiles in turn, a tile's
+// blocks of weight rows on one of them, whose L2 then holds the tile's rows; an XCD has at most an eighth more of them than the mean.
+// With fewer tiles some XCDs would have none or one more: there they take the blocks in turn. fp32, both products with sorting and
+// sum, us, tiles by expert / tiles in turn / blocks in turn: 2 experts of 2048 x 5632 and 100 rows 491 / 720 / 491, 4 of 60 rows
+// 440 / 535 / 425, 9 of 2048 x 1408 and 60 rows 182 / 238 / 183, 24 of 85 rows 539 / 439 / 395, 64 of 66 rows (71 tiles)
+// 1005 / 778 / 763, 128 of 2048 x 768 and 44 rows (128 tiles) 638 / 630 / 638.
+constexpr int EVEN = 64;
+struct Dealt {
+  int rank, nb;  // the tile's place in ``order`` (none from ``total`` on), block of weight rows
+};
+__host__ __device__ __forceinline__ Dealt deal(int total, int NB, int block) {
+  const bool few = total < EVEN;
+  const int i = few ? block : block >> 3, j = i / NB;
+  return {few ? j : j * 8 + (block & 7), i - j * NB};
+}
 __device__ __forceinline__ bool find_work_by_size(const int* __restrict__ tiles, const int* __restrict__ order, int NB, Work& w) {
-  const int i = blockIdx.x >> 3, j = i / NB, rank = j * 8 + (blockIdx.x & 7);
-  if (rank >= tiles[0]) return false;
-  w.tile = order[rank];
-  w.nb = i - j * NB;
+  const Dealt d = deal(tiles[0], NB, blockIdx.x);
+  if (d.rank >= tiles[0]) return false;
+  w.tile = order[d.rank];
+  w.nb = d.nb;
   const int t = tiles[1 + 3 * w.tile];
   w.e = t & 0xffff;
   w.rows = t >> 16;

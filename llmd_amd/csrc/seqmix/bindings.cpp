@@ -65,6 +65,7 @@ int sm_moe_tiled(const void*, int64_t, const void*, int64_t, int64_t, int);
 void sm_moe_gemm(const void*, int64_t, int, const int*, const int*, const void*, int, int, void*, int, int, int, int, int,
                  const float*, float, hipStream_t);
 int sm_moe_ring(const void*, int64_t, int64_t, const void*, int64_t, int64_t, int, int);
+void sm_moe_deal(int, int, int, int*, int*);
 int sm_retention(const void*, int64_t, int, int, int, int, const int64_t*, const float*, int, const float*, int, float,
                  float*, const int*, const int*, const int*, void*, int, int, int, int, int, const int*, const int*,
                  float*, float*, hipStream_t);
@@ -636,6 +637,13 @@ void moe_group(Tensor ids, int64_t E, int64_t tm, Tensor slot_row, Tensor tiles,
                order ? tiles.data_ptr<int>() + 1 + 3 * mt : nullptr, cur());
 }
 
+std::pair<int, int> moe_deal(int64_t total, int64_t NB, int64_t block) {
+  TORCH_CHECK(NB >= 1 && total >= 0 && block >= 0, "tiles, blocks");
+  int rank, nb;
+  sm_moe_deal(total, NB, block, &rank, &nb);
+  return {rank, nb};
+}
+
 bool moe_tiled(Tensor A, Tensor W) {
   return sm_moe_tiled(A.data_ptr(), A.stride(0), W.data_ptr(), W.size(1), W.size(2), is_f32(A)) != 0;
 }
@@ -1038,6 +1046,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_route", &moe_route);
   m.def("moe_group", &moe_group);
   m.def("moe_tiled", &moe_tiled);
+  m.def("moe_deal", &moe_deal);
   m.def("moe_ring", &moe_ring);
   m.def("moe_gemm", &moe_gemm);
   m.def("moe_combine", &moe_combine);

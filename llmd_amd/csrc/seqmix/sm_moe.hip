@@ -552,6 +552,12 @@ void sm_moe_group(const int* ids, int n, int E, int tm, int* hist, int* slot_row
   launch_group(ids, n, E, tm, hist, slot_row, tiles, pair_slot, order, stream);
 }
 
+// Which tile (its place by size) and block of weight rows a workgroup of the form by size takes.
+void sm_moe_deal(int total, int NB, int block, int* rank, int* nb) {
+  const Dealt d = deal(total, NB, block);
+  *rank = d.rank, *nb = d.nb;
+}
+
 // Whether the matrix-core form takes these operands: 16-byte pieces of every row, an expert (``rows`` weight rows) within
 // 32-bit offsets. Its tiles have 128 slots, the other form's 64.
 int sm_moe_tiled(const void* A, int64_t a_stride, const void* W, int64_t rows, int64_t K, int f32) {

@@ -1,17 +1,17 @@
 """fp32 experts on the matrix cores (csrc/include/moe_tile.h): tiles of every number of 16-row blocks and their edges, several
-tiles of an expert, rows and columns that do not fill their last step or block, tiles taken by expert and by size."""
+tiles of an expert, rows and columns that do not fill their last step or block, tiles taken by expert and by size, how by size the
+work lies on the XCDs."""
 import pytest
 import torch
-
-pytestmark = pytest.mark.gpu
 
 FEW = [0, 1, 15, 16, 17, 20, 3, 31]
 MANY = [1, 16, 17, 33, 48, 49, 64, 65, 80, 81, 96, 97, 112, 113, 127, 128, 129, 240, 385]
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("act", ["swish_limit", "relu2"])
 @pytest.mark.parametrize("d,F", [(64, 64), (36, 20), (320, 200)])
-@pytest.mark.parametrize("counts", [FEW, MANY, [3], [40], [129] * 40])
+@pytest.mark.parametrize("counts", [FEW, MANY, [3], [40], [129] * 40, [17] * 63, [17] * 64])
 def test_experts(d, F, counts, act):
     from llmd_amd.ops import seqmix as sm
 
@@ -41,6 +41,7 @@ def test_experts(d, F, counts, act):
         assert ((got[rows].double() - z @ c.T).abs() <= bound + 1e-30).all(), e
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("spread", [1, 5, 300])
 @pytest.mark.parametrize("n", [0, 100, 4000, 9000])
 def test_tiles_by_size(n, spread):
@@ -60,3 +61,17 @@ def test_tiles_by_size(n, spread):
     assert sorted(order.tolist()) == list(range(total))
     blocks = ((tiles[1:1 + 3 * total:3] >> 16) + 15) // 16
     assert (blocks[order].diff() <= 0).all()
+
+
+@pytest.mark.parametrize("NB", [1, 3, 8, 11, 44, 88])
+def test_work_by_size_over_the_xcds(NB):
+    """Workgroups go to the eight XCDs in turn: every block of every tile is some workgroup's, no XCD has more than its share by
+    an eighth (or one block)."""
+    sm = pytest.importorskip("llmd_amd._C_seqmix")
+    for total in [*range(0, 20), 23, 24, 25, 31, 33, 62, 63, 64, 65, 71, 72, 73, 128, 129, 203]:
+        for max_tiles in (total, total + 37):
+            work = [sm.moe_deal(total, NB, b) for b in range((max_tiles + 7) // 8 * 8 * NB)]
+            at = [(b & 7, w) for b, w in enumerate(work) if w[0] < total]
+            assert sorted(w for _, w in at) == [(r, nb) for r in range(total) for nb in range(NB)]
+            most = max(sum(x == xcd for x, _ in at) for xcd in range(8))
+            assert most <= max(-(-total * NB // 8), total * NB / 8 * 1.125), (total, most)
