@@ -62,7 +62,7 @@ void sm_moe_route(const float*, int64_t, int, int, int*, float*, int, int, hipSt
 int64_t sm_moe_sort_scratch(int, int);
 void sm_moe_group(const int*, int, int, int, int*, int*, int*, int*, int*, hipStream_t);
 int sm_moe_tiled(const void*, int64_t, const void*, int64_t, int64_t, int);
-void sm_moe_gemm(const void*, int64_t, int, const int*, const int*, const void*, int, int, void*, int, int, int, int, int,
+void sm_moe_gemm(const void*, int64_t, int, const int*, const int*, const void*, int, int, void*, int, int, int, int, int, int,
                  const float*, float, hipStream_t);
 int sm_moe_ring(const void*, int64_t, int64_t, const void*, int64_t, int64_t, int, int);
 void sm_moe_deal(int, int, int, int*, int*);
@@ -665,9 +665,8 @@ void moe_gemm(Tensor A, int64_t kdiv, Tensor slot_row, Tensor tiles, Tensor W, T
   const bool gated = act == 2 || act == 3 || act == 5;
   TORCH_CHECK(act >= 0 && act <= 5 && (!gated || W.size(1) % 2 == 0), "epilogue");
   const int64_t N = gated ? W.size(1) / 2 : W.size(1);  // gated: W holds [gate rows | up rows]
-  TORCH_CHECK(tm == 64 || (tm == 128 && moe_tiled(A, W)) ||
-                  (tm == 120 && moe_ring(A, W, gated) && mt * tm * 4 < (int64_t)1 << 31 && ((uintptr_t)C.data_ptr() & 15) == 0),
-              "tile rows");
+  TORCH_CHECK(tm == 64 || ((tm == 120 || tm == 128) && moe_tiled(A, W)), "tile rows");
+  const bool ring = tm == 120 && moe_ring(A, W, gated) && mt * tm * 4 < (int64_t)1 << 31 && ((uintptr_t)C.data_ptr() & 15) == 0;
   const bool by_size = tm == 128 && tiles.numel() == 1 + 4 * mt;
   TORCH_CHECK(by_size || tiles.numel() == 1 + 3 * mt, "tiles");
   TORCH_CHECK(slot_row.numel() == mt * tm && C.is_contiguous() && C.dim() == 2 && C.size(0) == mt * tm &&
@@ -679,7 +678,7 @@ void moe_gemm(Tensor A, int64_t kdiv, Tensor slot_row, Tensor tiles, Tensor W, T
   }
   if (N == 0) return;
   sm_moe_gemm(A.data_ptr(), A.stride(0), kdiv, slot_row.data_ptr<int>(), tiles.data_ptr<int>(), W.data_ptr(),
-              N, W.size(2), C.data_ptr(), mt, tm, by_size, (int)act, is_f32(A), row_w ? row_w->data_ptr<float>() : nullptr,
+              N, W.size(2), C.data_ptr(), mt, tm, ring, by_size, (int)act, is_f32(A), row_w ? row_w->data_ptr<float>() : nullptr,
               (float)limit, cur());
 }
 

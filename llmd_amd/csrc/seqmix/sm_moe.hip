@@ -374,14 +374,14 @@ template <typename T, int ACT>
 __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const T* __restrict__ A, int64_t a_stride, int kdiv,
                                                           const int* __restrict__ slot_row, const int* __restrict__ tiles,
                                                           const T* __restrict__ Wt, int N, int K, T* __restrict__ Cout,
-                                                          const float* __restrict__ row_w, float limit, int NB, const int* __restrict__ order) {
+                                                          const float* __restrict__ row_w, float limit, int NB, int tm, const int* __restrict__ order) {
   constexpr bool GATED = gated_act_code(ACT);
   Work wk;
   if (order != nullptr ? !find_work_by_size(tiles, order, NB, wk) : !find_work(tiles, NB, wk)) return;
   const int nb = wk.nb, tile = wk.tile, e = wk.e, rows = wk.rows;
   __shared__ __attribute__((aligned(128))) char lds[4 * TBUF];
   const int tid = threadIdx.x;
-  const int64_t slot0 = (int64_t)tile * TBM;
+  const int64_t slot0 = (int64_t)tile * tm;
   const int col0 = nb * (GATED ? TBW / 2 : TBW);  // the workgroup's first output column
   MoeTile t;
   t.K = K, t.lds = lds, t.w = reinterpret_cast<const char*>(Wt + (int64_t)e * (GATED ? 2 * N : N) * K);
@@ -573,16 +573,19 @@ int sm_moe_ring(const void* A, int64_t a_rows, int64_t a_stride, const void* W, 
 }
 
 // act: 0 none, 1 erf-GELU, 2 tanh-GELU(gate) * up, 3 SiLU(gate) * up, 4 squared ReLU, 5 clamped units. N = output
-// columns (the gated forms read a weight of 2 N rows per expert). tm: slots per tile, 128 for the matrix-core form (operands
-// that sm_moe_tiled takes), 120 for its form of many rows (sm_moe_ring), 64 for the other.
+// columns (the gated forms read a weight of 2 N rows per expert). tm: slots per tile, 120 or 128 for the matrix-core form (operands
+// that sm_moe_tiled takes), 64 for the other. ring: the form of many rows (sm_moe_ring), tiles of 120. Where only one of a step's
+// two products has the sizes for it, the other takes the tiles of 120 in moe_tile_kernel: 128 experts of 2048 x 720, 8 chosen,
+// both products with sorting and sum, us, neither in it / one: 24 rows 272 / 255, 62 rows 334 / 315, 256 rows 644 / 601; of 2056 x 768,
+// 24 rows 299 / 287, 256 rows 832 / 676.
 // by_size (tiles of 128 rows): behind the tables the tiles' order (sm_moe_group), in which they are taken.
 // row_w (gated forms): fp32 weight per (token, choice) pair that scales the row's INPUT, applied to
 // both fp32 sums before the activation; nullptr = 1.
 void sm_moe_gemm(const void* A, int64_t a_stride, int kdiv, const int* slot_row, const int* tiles, const void* W,
-                 int N, int K, void* C, int max_tiles, int tm, int by_size, int act, int f32, const float* row_w,
+                 int N, int K, void* C, int max_tiles, int tm, int ring, int by_size, int act, int f32, const float* row_w,
                  float limit, hipStream_t stream) {
   const bool gated = gated_act_code(act);
-  if (tm == moe_ring::ROWS) {
+  if (ring) {
     const int cols = gated ? moe_ring::WROWS / 2 : moe_ring::WROWS;
     const int64_t items = (int64_t)max_tiles * ((N + cols - 1) / cols);
     const dim3 grid((unsigned)std::min<int64_t>((items + 7) / 8 * 8, 512));  // two workgroups per CU
@@ -598,14 +601,14 @@ void sm_moe_gemm(const void* A, int64_t a_stride, int kdiv, const int* slot_row,
 #undef SM_RING
     return;
   }
-  if (tm == TBM) {
+  if (tm != TM) {
     const int NB = (N + (gated ? 63 : 127)) / (gated ? 64 : 128);
     const int64_t items = (int64_t)max_tiles * NB;
     const int* order = by_size ? tiles + 1 + 3 * (int64_t)max_tiles : nullptr;
     const dim3 grid((unsigned)(by_size ? (int64_t)((max_tiles + 7) / 8 * 8) * NB : (items + 7) / 8 * 8));
 #define SM_MT(KERN, TYPE, GRID)                                                                                       \
   hipLaunchKernelGGL(KERN, GRID, dim3(256), 0, stream, (const TYPE*)A, a_stride, kdiv, slot_row, tiles, (const TYPE*)W, \
-                     N, K, (TYPE*)C, row_w, limit, NB, order)
+                     N, K, (TYPE*)C, row_w, limit, NB, tm, order)
 #define SM_MT2(A_)                                                                  \
   if (f32) SM_MT((moe_tile_kernel<float, A_>), float, grid);                        \
   else SM_MT((moe_tile_kernel<bf16_t, A_>), bf16_t, grid)

@@ -200,14 +200,18 @@ def moe_route(logits, k: int, sigmoid: bool = False):
 
 def _moe_tables(C, ids, E: int, h, w1, w2, gated: bool):
     """Pairs sorted by expert into tiles of rows: (slot -> pair, [number of tiles, three numbers of each, where it counts the tiles
-    by size], pair -> slot, rows per tile): 128 rows for the matrix-core GEMM, 120 for its form of many rows, 64 for sizes that only the FMA
-    form takes."""
+    by size], pair -> slot, rows per tile): 128 rows for the matrix-core GEMM, 120 where a product takes its form of many rows (the
+    other then runs over the same tiles), 64 for sizes that only the FMA form takes."""
     n = ids.numel()
     tm = 128 if C.moe_tiled(h, w1) and C.moe_tiled(w2[0], w2) else 64
-    if (n >= MOE_STREAM_FROM * E and C.moe_ring(h, w1, gated) and C.moe_ring(w2[0], w2, False)
-            and (n + E * 119) * w2.shape[2] < 1 << 30):
+
+    def count(tm):  # every expert that has rows may leave one tile partly filled
+        return max(1, (n + min(E, n) * (tm - 1)) // tm)
+
+    if tm == 128 and n >= MOE_STREAM_FROM * E and count(120) * 120 < 1 << 29 and (
+            C.moe_ring(h, w1, gated) or C.moe_ring(w2[0], w2, False) and count(120) * 120 * w2.shape[2] < 1 << 30):
         tm = 120
-    max_tiles = max(1, (n + min(E, n) * (tm - 1)) // tm)  # every expert that has rows may leave one tile partly filled
+    max_tiles = count(tm)
     slot_row = torch.empty(max_tiles * tm, dtype=torch.int32, device=h.device)
     by_size = tm == 128 and h.dtype == torch.float32 and n > 16 * E  # moe_tile.h: what it gives on both sides of the line
     tiles = torch.empty(1 + (4 if by_size else 3) * max_tiles, dtype=torch.int32, device=h.device)

@@ -1,5 +1,6 @@
 """The streamed expert GEMM (csrc/include/moe_ring.h) at the edges of its tiles: rows per expert around the pairs of 16-row
-blocks and the tile of 120, several tiles, more items than workgroups and fewer, a last block of weight rows that is half empty."""
+blocks and the tile of 120, several tiles, more items than workgroups and fewer, a last block of weight rows that is half empty,
+only one of the two products with sizes for it."""
 import pytest
 import torch
 
@@ -9,7 +10,8 @@ EDGES = [1, 15, 16, 17, 32, 33, 64, 65, 96, 97, 0, 119, 120, 121, 240, 241, 375]
 
 
 @pytest.mark.parametrize("act", ["swish_limit", "relu2"])
-@pytest.mark.parametrize("d,F,counts", [(320, 256, EDGES), (1024, 512, EDGES), (256, 256, [3]), (256, 1024, [70] * 64)])
+@pytest.mark.parametrize("d,F,counts", [(320, 256, EDGES), (1024, 512, EDGES), (256, 256, [3]), (256, 1024, [70] * 64),
+                                        (320, 200, EDGES), (264, 320, EDGES), (512, 8, [121])])
 def test_streamed_experts(d, F, counts, act, monkeypatch):
     from llmd_amd.ops import seqmix as sm
 
