@@ -25,7 +25,7 @@ constexpr int WIMG = WROWS * 128, AIMG = ROWS * 128, A0 = DW * WIMG;
 // behind the rings the next item's row numbers; a tile's last half block, which no row belongs to, is read past its image
 constexpr int IDS = A0 + DA * AIMG, LDS = IDS + 2048;
 static_assert(A0 + (DA - 1) * AIMG + MA * 4096 <= LDS && LDS <= 80 * 1024, "");  // two workgroups per CU
-constexpr uint32_t NOWHERE = 0x80000000u;
+constexpr uint32_t NOWHERE = 0x80000000u;  // past every buffer's range, whether or not the scalar offset counts in the check
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -213,7 +213,13 @@ __device__ __forceinline__ void run(const uint16_t* __restrict__ A, int64_t a_st
       ka += 128, kw += 128;
       if (kt == first && more && kdiv > 0)  // the numbers of the next item's rows
         dma<false>(ri, w * 64 + lane < nxt.rows ? (uint32_t)(nxt.tile * ROWS + w * 64 + lane) * 4 : NOWHERE, 0, l0 + IDS + w * 256);
-      if (kt == next_w) rw = rn, kw = 0;
+      if (kt == next_w) {
+        rw = rn, kw = 0;
+        if (!more) {  // nothing to read
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) vw[j] = NOWHERE;
+        }
+      }
       if (kt == next_a) {
         ka = 0;
         mi = nxt.mi;
@@ -267,8 +273,6 @@ __device__ __forceinline__ void run(const uint16_t* __restrict__ A, int64_t a_st
     if (more) {
       nxt = look(item + S);
       rn = buffer_of(nxt.w, nxt.bytes);
-    } else {
-      rn[2] = 0;  // nothing to read
     }
     switch (cur.mi) {
       case 1: run_item(Int<1>{}); break;

@@ -11,7 +11,7 @@ EDGES = [1, 15, 16, 17, 32, 33, 64, 65, 96, 97, 0, 119, 120, 121, 240, 241, 375]
 
 @pytest.mark.parametrize("act", ["swish_limit", "relu2"])
 @pytest.mark.parametrize("d,F,counts", [(320, 256, EDGES), (1024, 512, EDGES), (256, 256, [3]), (256, 1024, [70] * 64),
-                                        (320, 200, EDGES), (264, 320, EDGES), (512, 8, [121])])
+                                        (320, 200, EDGES), (264, 320, EDGES), (512, 8, [121]), (320, 320, [3])])
 def test_streamed_experts(d, F, counts, act, monkeypatch):
     from llmd_amd.ops import seqmix as sm
 
