@@ -764,6 +764,8 @@ class ModelRunner:
         lists = [ids, pos, slots] + ([swa[0]] if swa is not None else [])
         host = torch.empty(len(lists), T, dtype=torch.long, pin_memory=self.is_gpu)
         for row, values in zip(host.numpy(), lists):  # array: a third of torch.tensor's time for a list
+            if len(values) != T:  # numpy would spread a single number over the row
+                raise ValueError(f"{len(values)} positions or slots for {T} tokens")
             row[:] = array("q", values)
         hd = host.to(dev, non_blocking=True)
         meta = AttnMeta(num_tokens=T, positions=hd[1], slot_mapping=hd[2], num_decode=nd)
