@@ -1426,15 +1426,13 @@ constexpr int GATHER_PART = 8192, GATHER_SLACK = 256;
 __global__ __launch_bounds__(256) void kv_dequant_gather_kernel(const uint8_t* __restrict__ kc,
                                                                 const uint8_t* __restrict__ vc, int64_t block_stride,
                                                                 const int* __restrict__ bt, int maxb, int bs,
-                                                                const int* __restrict__ ctx, int n_blocks, int per_block,
-                                                                uint16_t* __restrict__ kd, uint16_t* __restrict__ vd,
+                                                                const int* __restrict__ ctx, int n_ctx, int n_blocks,
+                                                                int per_block, uint16_t* __restrict__ kd, uint16_t* __restrict__ vd,
                                                                 int* __restrict__ place) {
   const int e = blockIdx.x;
   if (blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) place[e] = e;
-  if (ctx != nullptr) {
-    const int s = e / maxb;
-    if ((int64_t)(e - s * maxb) * bs >= (int64_t)ctx[s] + GATHER_SLACK) return;
-  }
+  const int s = e / maxb;
+  if (s < n_ctx && (int64_t)(e - s * maxb) * bs >= (int64_t)ctx[s] + GATHER_SLACK) return;
   const int b = min(max(bt[e], 0), n_blocks - 1);  // padding entries (never read by the kernel) -> block 0
   const uint8_t* src = (blockIdx.y ? vc : kc) + (int64_t)b * block_stride;
   uint16_t* dst = (blockIdx.y ? vd : kd) + (int64_t)e * per_block;
@@ -1449,15 +1447,16 @@ __global__ __launch_bounds__(256) void kv_dequant_gather_kernel(const uint8_t* _
 }
 }  // namespace
 
-// ctx: contexts of the table's sequences (maxb entries each), or null: all entries are copied. place [entries]: 0, 1, 2 ..
+// ctx: contexts of the table's first n_ctx sequences (maxb entries each); of the others all entries are copied.
+// place [entries]: 0, 1, 2 ..
 extern "C" int llmd_kv_dequant_gather(const void* kc, const void* vc, int64_t block_stride, const int* bt,
-                                      int n_entries, int maxb, int bs, const int* ctx, int n_blocks, int per_block, void* kd,
-                                      void* vd, int* place, hipStream_t st) {
+                                      int n_entries, int maxb, int bs, const int* ctx, int n_ctx, int n_blocks, int per_block,
+                                      void* kd, void* vd, int* place, hipStream_t st) {
   if (per_block % 8 || block_stride % 8 || n_blocks <= 0) return -1;
   if (n_entries == 0) return 0;
   hipLaunchKernelGGL(kv_dequant_gather_kernel, dim3(n_entries, 2, (per_block + GATHER_PART - 1) / GATHER_PART), dim3(256), 0, st,
-                     (const uint8_t*)kc, (const uint8_t*)vc, block_stride, bt, maxb, bs, ctx, n_blocks, per_block, (uint16_t*)kd,
-                     (uint16_t*)vd, place);
+                     (const uint8_t*)kc, (const uint8_t*)vc, block_stride, bt, maxb, bs, ctx, n_ctx, n_blocks, per_block,
+                     (uint16_t*)kd, (uint16_t*)vd, place);
   return (int)hipGetLastError();
 }
 

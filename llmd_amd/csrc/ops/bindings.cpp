@@ -650,11 +650,12 @@ void mgemm_fp8(torch::Tensor y, torch::Tensor xq, torch::Tensor xs, torch::Tenso
   TORCH_CHECK(rc == 0, "mgemm_fp8 failed: ", rc);
 }
 
-extern "C" int llmd_kv_dequant_gather(const void*, const void*, int64_t, const int*, int, int, int, const int*, int, int, void*,
-                                      void*, int*, hipStream_t);
+extern "C" int llmd_kv_dequant_gather(const void*, const void*, int64_t, const int*, int, int, int, const int*, int, int, int,
+                                      void*, void*, int*, hipStream_t);
 
 // fp8 paged K/V blocks of a block table [S, maxb] -> dense bf16 copies kd / vd [entries, Hkv, bs, D] (attn_prefill.hip);
-// ctx [S]: entries well past a sequence's context are left as they are; place [entries]: the table over the copies
+// ctx (of the first sequences, all of them as a rule): entries well past a sequence's context are left as they are;
+// place [entries]: the table over the copies
 void kv_dequant_gather(torch::Tensor k_cache, torch::Tensor v_cache, torch::Tensor block_tables, c10::optional<torch::Tensor> ctx,
                        torch::Tensor kd, torch::Tensor vd, torch::Tensor place) {
   const c10::hip::OptionalHIPGuard device_guard(dev_of(k_cache));
@@ -671,12 +672,12 @@ void kv_dequant_gather(torch::Tensor k_cache, torch::Tensor v_cache, torch::Tens
   TORCH_CHECK(block_tables.dim() == 2 && place.is_cuda() && place.is_contiguous() && place.numel() == block_tables.numel(), "place [entries]");
   if (ctx) {
     CHECK_DT(*ctx, at::kInt);
-    TORCH_CHECK(ctx->is_cuda() && ctx->is_contiguous() && ctx->numel() == block_tables.size(0), "ctx [S]");
+    TORCH_CHECK(ctx->is_cuda() && ctx->is_contiguous(), "ctx [S]");
   }
   const int rc = llmd_kv_dequant_gather(k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
                                         block_tables.data_ptr<int>(), (int)block_tables.numel(), (int)block_tables.size(1),
-                                        (int)k_cache.size(2), ctx ? ctx->data_ptr<int>() : nullptr, (int)k_cache.size(0),
-                                        (int)per, kd.data_ptr(), vd.data_ptr(), place.data_ptr<int>(), cur_stream());
+                                        (int)k_cache.size(2), ctx ? ctx->data_ptr<int>() : nullptr, ctx ? (int)ctx->numel() : 0,
+                                        (int)k_cache.size(0), (int)per, kd.data_ptr(), vd.data_ptr(), place.data_ptr<int>(), cur_stream());
   TORCH_CHECK(rc == 0, "kv_dequant_gather failed: ", rc);
 }
 

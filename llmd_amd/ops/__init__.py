@@ -394,8 +394,8 @@ PREFILL_FP8_VIA_BF16 = os.environ.get("LLMD_PREFILL_FP8_VIA_BF16", "1") == "1"
 def kv_dequant_gather(k_cache, v_cache, block_tables, ctx_len=None):
     """(k, v, table): the blocks ``block_tables`` [S, maxb] names in an fp8 paged cache [blocks, Hkv,
     bs, D], widened exactly to bf16 into dense copies [S * maxb, Hkv, bs, D] and the identity table
-    over them (padding entries copy block 0, never read). With ``ctx_len`` [S] int32 blocks 256 keys and more behind a
-    sequence's context need not be copied."""
+    over them (padding entries copy block 0, never read). With ``ctx_len`` int32 blocks 256 keys and more behind a
+    sequence's context need not be copied; sequences past its end have all of theirs copied."""
     S, mb = block_tables.shape
     shape = (S * mb,) + tuple(k_cache.shape[1:])
     if not _gpu(k_cache):

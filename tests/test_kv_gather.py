@@ -25,3 +25,22 @@ def test_gather(Hkv, bs, D, known):
         m = mb if not known else min(mb, -(-(-(-int(ctx[s]) // 64) * 64) // bs))
         at = slice(s * mb, s * mb + m)
         assert torch.equal(kd[at].cpu().float(), kw[at].float()) and torch.equal(vd[at].cpu().float(), vw[at].float())
+
+
+@pytest.mark.parametrize("rows,lens", [(3, 3), (5, 3), (3, 6)])
+def test_prefill_with_other_numbers_of_contexts(rows, lens):
+    """A table may have more rows than the step has sequences, and the contexts' buffer more entries."""
+    from llmd_amd import ops
+
+    g = torch.Generator().manual_seed(rows + lens)
+    Hq, Hkv, D, bs, n, mb = 8, 2, 128, 64, 30, 6
+    k, v = (torch.randn(n, Hkv, bs, D, generator=g).to(ops.FP8).cuda() for _ in range(2))
+    bt = torch.randperm(n, generator=g)[:rows * mb].view(rows, mb).int().cuda()
+    ql, cl = [40, 1, 100], [40, 130, 380]
+    q = torch.randn(sum(ql), Hq * D, generator=g).bfloat16().cuda()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    items = i32(ops.build_prefill_items(ql, cl, ops.prefill_tokens_per_item(Hq, Hkv, D, bs, False)))
+    run = lambda bt, c: ops.paged_prefill(q, k, v, bt, i32([0, 40, 41]), i32(ql), c, Hq, Hkv, D, D ** -0.5, items=items)  # noqa: E731
+    want = run(bt[:3].contiguous(), i32(cl))
+    got = run(bt, i32(cl + [7] * (lens - 3)))
+    assert torch.isfinite(want).all() and torch.equal(got, want)
