@@ -424,9 +424,10 @@ __device__ __forceinline__ void run_tile(const MoeTile& t, int rows, WRow wrow, 
     if (rows > 96) return moe_tile_many<T, GATED, 7, 1, 2>(t, wrow, out);
     if (rows > 80) return moe_tile_many<T, GATED, 6, 1, 2>(t, wrow, out);
     if (rows > 64) return moe_tile_many<T, GATED, 5, 1, 2>(t, wrow, out);
+  } else {
+    if (rows > 64) return moe_tile_many<T, GATED, 4, 2, 2>(t, wrow, out);
   }
-  if (rows > 64) moe_tile_many<T, GATED, 4, 2, 2>(t, wrow, out);
-  else if (rows > 48) moe_tile_many<T, GATED, 4, 1, 2>(t, wrow, out);
+  if (rows > 48) moe_tile_many<T, GATED, 4, 1, 2>(t, wrow, out);
   else if (rows > 32) moe_tile_many<T, GATED, 3, 1, 2>(t, wrow, out);
   else if (rows > 16) moe_tile_few<T, GATED, 2, 3>(t, wrow, out);
   else moe_tile_few<T, GATED, 1, 3>(t, wrow, out);
