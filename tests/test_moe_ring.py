@@ -37,3 +37,37 @@ def test_streamed_experts(d, F, counts, act, monkeypatch):
         want, size = z @ w2[e].double().T, z.abs() @ w2[e].abs().double().T
         # activation, row and result are each rounded once to bf16 (2^-9): at worst that adds up over ``size``
         assert ((got[rows].double() - want).abs() <= 3 * 2.0 ** -9 * (size + want.abs()) + 2.0 ** -9).all(), e
+
+
+@pytest.mark.parametrize("kind", ["silu", "swish_limit"])
+@pytest.mark.parametrize("d,F,rows", [(320, 256, 70), (1024, 512, 130), (256, 264, 31)])
+def test_weights_on_the_input(d, F, rows, kind, monkeypatch):
+    """Several choices per token whose weights scale the expert's input (both sums, before the activation)."""
+    from llmd_amd.ops import seqmix as sm
+
+    monkeypatch.setattr(sm, "MOE_STREAM_FROM", 0)
+    g = torch.Generator(device="cuda").manual_seed(d + rows)
+    E, k = 10, 3
+    T = rows * E // k + 1
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    ids = (rand(T, E) + rand(E)).topk(k, -1).indices.int()
+    h, w1, w2 = rand(T, d).bfloat16(), (rand(E, 2 * F, d) * d ** -0.5).bfloat16(), (rand(E, d, F) * F ** -0.5).bfloat16()
+    w = torch.rand(T, k, generator=g, device="cuda") * 1.5 + 0.1
+    assert sm._moe_tables(sm.native(), ids, E, h, w1, w2, True)[3] == 120
+    got = sm.moe_gated_ffn(h, ids, w, w1, w2, kind, scale_input=True, limit=2.0)
+    want, size, rounded = (torch.zeros(T, d, dtype=torch.float64, device="cuda") for _ in range(3))
+    for e in range(E):
+        t, j = (ids == e).nonzero(as_tuple=True)
+        z = w[t, j].double()[:, None] * (h[t].double() @ w1[e].double().T)
+        a, u = z[:, :F], z[:, F:]
+        if kind == "silu":
+            z = a * torch.sigmoid(a) * u
+        else:
+            a, u = a.clamp(max=2.0), u.clamp(-2.0, 2.0)
+            z = a * torch.sigmoid(1.702 * a) * (u + 1.0)
+        y = z @ w2[e].double().T
+        want.index_add_(0, t, y)
+        size.index_add_(0, t, z.abs() @ w2[e].abs().double().T)
+        rounded.index_add_(0, t, y.abs())
+    # activation, every expert's row and the result are each rounded once to bf16 (2^-9)
+    assert ((got.double() - want).abs() <= 3 * 2.0 ** -9 * (size + rounded) + 2.0 ** -9).all()
