@@ -5,8 +5,11 @@
 // waves of row b % 2. LDS is what sets the size: 120 rows, so that the two rings and the numbers of the next item's rows are half
 // of a CU's. What bounds it: the weights' stream (137 + 71 us for 128 experts of 2048 x 768) while an expert has one tile; with
 // more of them the bytes on their way, about 60 KB per CU, against L2's latency under that load.
-// 128 experts, 8 chosen, both products with sorting and sum, us; in brackets the form before, 128 x 128 tiles through registers to
-// LDS, all rows multiplied: 200 tokens 234 (237), 400 259 (255), 1024 285 (286), 1500 304 (314), 2048 344 (354), 4096 503 (537).
+// Both products with sorting and sum, us, skewed router; in brackets the form before, 128 x 128 tiles through registers to LDS,
+// all rows multiplied. 128 experts of 2048 x 768, 8 chosen: 24 rows per expert 247 (253), 40 271 (273), 62 284 (288), 128 346 (353),
+// 256 516 (537); 8 of 2048 x 1408: 24 rows 42 (53), 256 rows 66 (79); 8 of 4096 x 8192: 24 rows 340 (336), 96 394 (411), 256 612 (649).
+// Experts of 121 to 128 rows each pay for a second tile: the last ones with 128 rows each 556 (470). A koduzen-moe prompt of 2048 takes
+// as long as before (2678), koduzen-hybrid's portions 2529 (2552).
 // Taken back: 192 and 240 rows x 256 weight rows with one workgroup per CU are faster where every expert has one tile (128 rows
 // each: 168 + 109 against 185 + 117) and lose it to a last round of few items where some have two (207 + 115, 182 + 144
 // with that round in halves); 240 x 128 rows 249 + 120.

@@ -261,9 +261,10 @@ class PagedAttention(torch.nn.Module):
         out = torch.empty(T, Hq * D, dtype=qkv.dtype, device=qkv.device)
         nd = meta.num_decode
         # Mixed steps: both on one stream. The decode rows on another one beside the prompt's, us per step of four layers (70B:
-        # two), apart / one behind the other: llama-8b, 8 rows and 300 tokens 1160 / 1080, 64 and 512 2210 / 2125, 64 and 4000
-        # 6835 / 6755, 24 and 1405 2840 / 2860, with an 8-bit cache 2800 - 3500 / 2840; 70B, 16 and 2000 5382 / 5379, 63 and 5000
-        # 13940 / 13955: the waits cost what the kernels gain beside one another.
+        # two), apart / one behind the other, of four runs: llama-8b, 8 rows and 300 tokens 1238 - 1273 / 1079 - 1083, 64 and 512
+        # 2174 - 2238 / 2131 - 2165, 64 and 4000 6832 - 8172 / 6742 - 6752, 24 and 1405 2789 - 2822 / 2805 - 2814, with an 8-bit cache
+        # 2766 - 3553 / 2801 - 2822; 70B, 16 and 2000 5403 - 5406 / 5395 - 5408, 63 and 5000 13912 - 15271 / 13918 - 13939: the waits cost
+        # what the kernels gain beside one another, and the first passes with another stream are the longest of all.
         if nd:
             ops.paged_decode(qkv[:nd], self.k_cache, self.v_cache, meta.d_block_tables,
                              meta.d_seq_lens, Hq, Hkv, D, self.scale, self.window, self.sinks,

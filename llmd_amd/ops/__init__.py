@@ -615,7 +615,7 @@ def quant_fp8_block_weight(w: torch.Tensor, block: int = 128):
 
 
 def _quant_groups_padded(x: torch.Tensor, kp: int, row_limit: Optional[torch.Tensor] = None):
-    """quant_fp8_groups into rows of ``kp`` >= d columns, zeros past d, in one kernel (GPU).
+    """quant_fp8_groups into rows of ``kp`` >= d columns, zeros past d (scales of 1 for whole groups of them), in one kernel (GPU).
     ``row_limit`` (int32 device scalar, e.g. moe_align's padded-slot total): rows at or past it
     are skipped - the grouped GEMM never reads them."""
     T, d = x.shape

@@ -220,8 +220,11 @@ def _moe_tables(C, ids, E: int, h, w1, w2, gated: bool):
     return slot_row, tiles, pair_slot, tm
 
 
-# rows per expert from which the bf16 GEMM runs as one stream per workgroup (csrc/include/moe_ring.h). 128 experts, both products
-# with sorting and sum, us, against a workgroup per tile: 12 rows 234 / 250, 25 rows 259 / 290, 44 rows 268 / 320; 4 rows 217 / 210
+# rows per expert from which the bf16 GEMM runs as one stream per workgroup (csrc/include/moe_ring.h). Both products with sorting
+# and sum, us, by a skewed router, against a workgroup per tile: 128 experts of 2048 x 768, 4 rows 218 / 220, 8 rows 229 / 231,
+# 16 rows 240 / 250, 24 rows 247 / 271, 32 rows 263 / 299; 32 of 2880 x 2880, 8 rows 286 / 305, 24 rows 301 / 339; 8 of 4096 x 8192, 8 rows
+# 322 / 314, 24 rows 333 / 318, 48 rows 340 / 361. The sides cross at 4 to 8 rows with many experts, at 24 to 64 with few wide ones,
+# whose second product has fewer items than workgroups: the line lies between.
 MOE_STREAM_FROM = int(os.environ.get("LLMD_MOE_STREAM_FROM", "24"))
 UNGATED_ACTS = {"gelu": 1, "relu2": 4}
 
