@@ -44,3 +44,29 @@ def test_prefill_with_other_numbers_of_contexts(rows, lens):
     want = run(bt[:3].contiguous(), i32(cl))
     got = run(bt, i32(cl + [7] * (lens - 3)))
     assert torch.isfinite(want).all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("D,bs,G", [(128, 64, 4), (64, 16, 1), (128, 32, 2)])
+def test_prefill_does_not_read_what_is_not_copied(D, bs, G):
+    """Long tables, short contexts, copies in memory that held NaNs."""
+    from llmd_amd import ops
+
+    g = torch.Generator().manual_seed(D + bs)
+    Hkv, n, mb = 2, 70, 64
+    Hq = Hkv * G
+    k, v = (torch.randn(n, Hkv, bs, D, generator=g).to(ops.FP8).cuda() for _ in range(2))
+    ql, cl = [1, 33, 64, 200, 5], [1, 33, 65, 257, 6 * 64 - 1]
+    S = len(ql)
+    bt = torch.randint(0, n, (S, mb), generator=g, dtype=torch.int32).cuda()
+    q = torch.randn(sum(ql), Hq * D, generator=g).bfloat16().cuda()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    start = i32([sum(ql[:i]) for i in range(S)])
+    items = i32(ops.build_prefill_items(ql, cl, ops.prefill_tokens_per_item(Hq, Hkv, D, bs, False)))
+    run = lambda k, v, bt: ops.paged_prefill(q, k, v, bt, start, i32(ql), i32(cl), Hq, Hkv, D, D ** -0.5, items=items)  # noqa: E731
+    # the same blocks, widened by torch, in the kernel that takes them as they are
+    want = run(k.bfloat16(), v.bfloat16(), bt)
+    for turn in range(2):
+        held = [torch.full((S * mb, Hkv, bs, D), -1, dtype=torch.int16, device="cuda") for _ in range(4)]
+        del held
+        got = run(k, v, bt)
+        assert torch.isfinite(got).all() and torch.equal(got, want), turn
