@@ -8,8 +8,9 @@
 // Both products with sorting and sum, us, skewed router; in brackets the form before, 128 x 128 tiles through registers to LDS,
 // all rows multiplied. 128 experts of 2048 x 768, 8 chosen: 24 rows per expert 247 (253), 40 271 (273), 62 284 (288), 128 346 (353),
 // 256 516 (537); 8 of 2048 x 1408: 24 rows 42 (53), 256 rows 66 (79); 8 of 4096 x 8192: 24 rows 340 (336), 96 394 (411), 256 612 (649).
-// Experts of 121 to 128 rows each pay for a second tile: the last ones with 128 rows each 556 (470). A koduzen-moe prompt of 2048 takes
-// as long as before (2678), koduzen-hybrid's portions 2529 (2552).
+// Over 13 sizes from 100 to 256 rows and four routings each: 32 of 2880 x 2880 7 % faster, 128 of 2048 x 768 2 %, 8 of 4096 x 8192 1 %.
+// Slower where an even router gives 112 to 136 rows, so that more experts have a second tile: there up to 14 % with the last, 8 % with
+// 128. A koduzen-moe prompt of 2048 takes as long as before (2678), koduzen-hybrid's portions 2529 (2552).
 // Taken back: 192 and 240 rows x 256 weight rows with one workgroup per CU are faster where every expert has one tile (128 rows
 // each: 168 + 109 against 185 + 117) and lose it to a last round of few items where some have two (207 + 115, 182 + 144
 // with that round in halves); 240 x 128 rows 249 + 120.
