@@ -68,6 +68,9 @@ int llmd_mgemm_silu(const void*, int64_t, const void*, int64_t, int, int, int, i
 int llmd_pgemm(const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, int, void*,
                hipStream_t);
 int64_t llmd_pgemm_ws_bytes(int, int, int, int, int);
+int llmd_tgemm_plan(int, int, int, int);
+int llmd_tgemm(const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, int, const void*, void*,
+               hipStream_t);
 int llmd_pgemm_fp8(const void*, int64_t, const float*, const void*, int64_t, const float*, void*, int64_t, int, int,
                    int, int, void*, int, hipStream_t);
 int64_t llmd_pgemm_fp8_ws_bytes(int, int, int, int);
@@ -579,6 +582,34 @@ void pgemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t epi, int64
   int rc = llmd_pgemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), y.stride(0), (int)M,
                       (int)N, (int)K, (int)epi, (int)variant, wsb > 0 ? ws.data_ptr() : nullptr, cur_stream());
   TORCH_CHECK(rc == 0, "pgemm failed: ", rc);
+}
+
+// x w^T (+ bias), or with silu silu(x wg^T) * (x wu^T) of w = [gate; up], on the tile that llmd_tgemm_plan has for these
+// sizes (csrc/ops/tgemm.hip), or on `tile`; nothing where it has none or the operands are not what the kernel reads
+std::optional<torch::Tensor> tgemm(const torch::Tensor& x, const torch::Tensor& w, const std::optional<torch::Tensor>& bias,
+                                   bool silu, int64_t tile) {
+  if (!x.is_cuda() || x.device() != w.device() || x.dim() != 2 || w.dim() != 2 || x.scalar_type() != at::kBFloat16 ||
+      w.scalar_type() != at::kBFloat16)
+    return std::nullopt;
+  const int64_t M = x.size(0), K = x.size(1), rows = w.size(0), N = silu ? rows / 2 : rows;
+  const auto off = [](const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0; };
+  if (w.size(1) != K || rows % (silu ? 16 : 8) || M > (1 << 30) || rows > (1 << 30) || K > (1 << 30) || x.stride(1) != 1 ||
+      w.stride(1) != 1 || x.stride(0) < K || w.stride(0) < K || x.stride(0) % 8 || w.stride(0) % 8 || off(x) || off(w) ||
+      ((M - 1) * x.stride(0) + K) * 2 > 0x7fffffffLL || ((rows - 1) * w.stride(0) + K) * 2 > 0x7fffffffLL)
+    return std::nullopt;
+  if (bias && (silu || bias->scalar_type() != at::kBFloat16 || bias->device() != x.device() || bias->dim() != 1 ||
+               bias->size(0) != N || (N > 1 && bias->stride(0) != 1) || off(*bias)))
+    return std::nullopt;
+  const int code = tile ? (int)tile : llmd_tgemm_plan((int)M, (int)rows, (int)K, silu ? 1 : 0);
+  if (code == 0) return std::nullopt;
+  const c10::hip::OptionalHIPGuard device_guard(dev_of(x));
+  torch::Tensor y = torch::empty({M, N}, x.options()), ws;
+  if (code % 10 > 1) ws = torch::empty({code % 10, M, N}, x.options().dtype(torch::kFloat));
+  const int rc = llmd_tgemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N, (int)M, (int)N,
+                            (int)K, silu ? 1 : 0, code, bias ? bias->data_ptr() : nullptr,
+                            ws.defined() ? ws.data_ptr() : nullptr, cur_stream());
+  TORCH_CHECK(rc == 0, "tgemm failed: ", rc);
+  return y;
 }
 
 // y = (xs . xq) (ws . wq)^T for prefill-sized M on the fp8 256 x 256 LDS-DMA GEMM (csrc/ops/pgemm8.hip,
@@ -1355,6 +1386,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_debug (llmd_amd/build.p
   m.def("mgemm_add_rmsnorm", &mgemm_add_rmsnorm, "decode o / down projection with residual-add + RMSNorm in its split-K reduce");
   m.def("pgemm_fp8", &pgemm_fp8, "prefill fp8 W8A8 GEMM (256x256 LDS-DMA tiles on 16x16x128 f8f6f4 MFMA), "
         "per-token x per-channel scales, optional fused SiLU-and-mul");
+  m.def("tgemm", &tgemm, "bf16 GEMM of prompt-sized steps on the tile that fits, or None", py::arg("x"), py::arg("w"),
+        py::arg("bias") = std::nullopt, py::arg("silu") = false, py::arg("tile") = 0);
+  m.def("tgemm_plan", &llmd_tgemm_plan, "tile of tgemm for (M, N, K, silu): mi * 100 + ni * 10 + ranges of K, or 0");
   m.def("pgemm", &pgemm, "prefill bf16 GEMM (256x256 LDS-DMA MFMA tiles), optional fused SiLU-and-mul",
         py::arg("y"), py::arg("x"), py::arg("w"), py::arg("epi"), py::arg("variant"), py::arg("split_k") = true);
   m.def("mgemm_fp8", &mgemm_fp8);

@@ -21,7 +21,6 @@ ONE all-reduce per layer sums both.
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 
 from llmd_amd import ops
 from llmd_amd.engine.attn_meta import AttnMeta
@@ -139,7 +138,7 @@ class DeepseekMoE(torch.nn.Module):
 
     def forward(self, x):
         cfg = self.cfg
-        logits = F.linear(x, self.gate).float()
+        logits = ops.router_linear(x, self.gate).float()
         ids, w = ops.moe_topk(logits, self.k, scoring=1 if cfg.scoring_func == "sigmoid" else 0, bias=self.bias,
                               n_group=cfg.n_group, topk_group=cfg.topk_group, renorm=cfg.norm_topk_prob,
                               routed_scale=cfg.routed_scaling_factor)

@@ -20,7 +20,6 @@ DP attention (wide-EP) tokens are exchanged with ``parallel/ep.py``
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 
 from llmd_amd import ops
 from llmd_amd.engine.config import ModelConfig
@@ -65,7 +64,7 @@ class GptOssMoE(torch.nn.Module):
 
     def forward(self, x):
         T = x.shape[0]
-        logits = F.linear(x, self.router_w, self.router_b).float()
+        logits = ops.router_linear(x, self.router_w, self.router_b).float()
         ids, w = ops.moe_topk(logits, self.k, scoring=2)
         if not self.ep:
             return run_experts(self, x, ids, w, ops.ACT_SWIGLU_OAI, self.alpha, self.limit, b1=self.b1, b2=self.b2)

@@ -13,7 +13,6 @@ token exchange, EPLB). HF expert tensors (``mlp.experts.{e}.gate_proj`` /
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 
 from llmd_amd import ops
 from llmd_amd.engine.config import ModelConfig
@@ -54,7 +53,7 @@ class SparseMoE(torch.nn.Module):
                                                   0.02), requires_grad=False)
 
     def forward(self, x):
-        logits = F.linear(x, self.gate)
+        logits = ops.router_linear(x, self.gate)
         ids, w = ops.moe_topk(logits, self.k, scoring=0, renorm=self.renorm)
         fn = lambda xx, ii, ww: run_experts(self, xx, ii, ww, ops.ACT_SILU)  # noqa: E731
         if self.dp_ep:

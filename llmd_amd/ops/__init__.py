@@ -1366,6 +1366,29 @@ def pgemm_silu(x: torch.Tensor, w: torch.Tensor, variant: int = 3, out: Optional
     return pgemm(x, w, epi=3, out=out, variant=variant, split_k=False)
 
 
+def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """A call that nobody differentiates, batches, traces or watches: one whose library product a kernel may stand in for."""
+    return (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter)
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.maybe_current_level() is None
+            and torch._C._get_tracing_state() is None and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._len_torch_function_stack() == 0)
+
+
+def tgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, silu: bool = False):
+    """x w^T (+ bias), or silu(x wg^T) * (x wu^T) for w = [gate; up], on the GEMM whose tile fits the sizes
+    (csrc/ops/tgemm.hip, which holds the rule), or None where it is not taken."""
+    if PGEMM_AUTO == "0" or not _gpu(x) or not _plain(x, w):
+        return None
+    return native().tgemm(x, w, bias, silu)
+
+
+def router_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """A router's logits: prompts on ``tgemm`` (2048 x (128, 2048) hipBLASLt 12.4 us, here 7), the rest on the library."""
+    y = tgemm(x, w, bias) if x.dim() == 2 and x.shape[0] > 64 else None
+    return torch.nn.functional.linear(x, w, bias) if y is None else y
+
+
 def pgemm_pack_gate_up(w: torch.Tensor) -> torch.Tensor:
     """[2F, K] (gate rows, then up rows) -> the fused-SiLU pgemm layout: per
     256-row tile, 128 gate rows then the matching 128 up rows (F % 128 == 0)."""
@@ -1515,7 +1538,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     stream kernel (csrc/ops/skinny_gemm.hip, M <= 64, ops/dgemm_table.py), unlisted
     shapes by ``decode_rule`` (without a bias, which hipBLASLt adds for nothing) -
     prefill-sized M on the prefill GEMM where the shipped table (ops/pgemm_table.py)
-    has it ahead of hipBLASLt - everything else on hipBLASLt."""
+    has it ahead of hipBLASLt, other M above 64 on the GEMM with a tile for the size
+    (``tgemm``) - everything else on hipBLASLt."""
     if PGEMM_AUTO != "0" and x.dim() == 2 and x.shape[0] >= PGEMM_MIN_M and pgemm_ok(x, w):
         plan = pgemm_wins(x, w)
         if plan is not None:
@@ -1538,6 +1562,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
             rule = decode_rule(M, w.shape[0], w.shape[1])
             if rule is not None:
                 return rule[0](x, w, rule[1])
+    if x.dim() == 2 and x.shape[0] > 64:
+        y = tgemm(x, w, bias)
+        if y is not None:
+            return y
     return torch.nn.functional.linear(x, w, bias)
 
 

@@ -1,0 +1,89 @@
+"""Prompt-sized bf16 GEMM with a tile for every size (csrc/ops/tgemm.hip) against the fp32 product of the same operands."""
+import pytest
+import torch
+
+from llmd_amd import ops
+
+TILES = [(2, 2), (3, 2), (3, 3), (3, 4), (4, 3), (4, 4), (4, 6), (4, 8), (5, 4), (5, 6), (5, 8), (6, 4), (6, 6), (6, 8),
+         (8, 5), (8, 6), (8, 7)]
+
+
+def _operands(M, N, K, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed + M * 31 + N * 7 + K)
+    return (torch.randn(M, K, generator=g, device="cuda").bfloat16(),
+            (torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).bfloat16())
+
+
+def _close(y, ref):
+    # one rounding to bf16 (2^-9 of the value), and fp32 sums of K products of order 1 / sqrt(K)
+    assert (y.float() - ref).abs().le(ref.abs() * 2.0 ** -8 + 1e-5).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mi,ni", TILES)
+def test_tiles_edges(mi, ni):
+    """One row and column group, a tile less one row, whole tiles and the first row of the next one; one K-step up to
+    more than the stages hold; rows further apart than K."""
+    for M, N, K in ((1, 8, 64), (32 * mi - 1, 32 * ni - 8, 128), (32 * mi, 32 * ni, 320), (64 * mi + 1, 96 * ni + 8, 448)):
+        x, w = _operands(M, N, K)
+        wide = torch.zeros(M, K + 8, device="cuda", dtype=torch.bfloat16)
+        wide[:, :K] = x
+        bias = torch.linspace(-2, 2, N, device="cuda").bfloat16()
+        ref = x.float() @ w.float().t()
+        y = ops.native().tgemm(x, w, None, False, mi * 100 + ni * 10 + 1)
+        _close(y, ref)
+        assert torch.equal(ops.native().tgemm(wide[:, :K], w, None, False, mi * 100 + ni * 10 + 1), y)
+        _close(ops.native().tgemm(x, w, bias, False, mi * 100 + ni * 10 + 1), ref + bias.float())
+        w2 = torch.cat([w, w.flip(0)])
+        _close(ops.native().tgemm(x, w2, None, True, mi * 100 + ni * 10 + 1),
+               torch.nn.functional.silu(ref) * ref.flip(1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mi,ni,ranges", [(2, 2, 8), (4, 4, 2), (4, 8, 4), (6, 8, 3), (8, 8, 2), (8, 8, 3)])
+def test_ranges_of_k(mi, ni, ranges):
+    """The ranges' sums are added in order and rounded once; the last range may be the shorter one."""
+    for M, N, K in ((1, 8, 64 * 22), (32 * mi + 1, 64 * ni + 8, 64 * 23)):
+        x, w = _operands(M, N, K)
+        bias = torch.linspace(-2, 2, N, device="cuda").bfloat16()
+        ref = x.float() @ w.float().t()
+        code = mi * 100 + ni * 10 + ranges
+        _close(ops.native().tgemm(x, w, None, False, code), ref)
+        _close(ops.native().tgemm(x, w, bias, False, code), ref + bias.float())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(65, 2048, 2048), (300, 5120, 2048), (700, 2176, 1536), (1429, 4096, 4096)])
+def test_linear_takes_it(M, N, K):
+    """ops.linear on an unlisted shape: the same bits as the tile's own call, in a row's result whatever M."""
+    code = ops.native().tgemm_plan(M, N, K, 0)
+    assert code and code % 10 == 1
+    x, w = _operands(M, N, K)
+    y = ops.linear(x, w)
+    _close(y, x.float() @ w.float().t())
+    assert torch.equal(y, ops.native().tgemm(x, w, None, False, code))
+    assert torch.equal(y[:65], ops.native().tgemm(x[:65], w, None, False, 221))
+
+
+@pytest.mark.gpu
+def test_refused_or_left():
+    """Operands that the kernel does not read stay with the library; one of its tiles for another shape raises."""
+    x, w = _operands(130, 256, 128)
+    nat = ops.native()
+    for a, b in ((x.float(), w.float()), (x[None], w), (x, w[:255]), (x[:, ::2], w[:, ::2]), (x[:64], w),
+                 (torch.cat([x, x], 1)[:, 4:132], w)):
+        assert nat.tgemm(a, b) is None
+    assert ops.tgemm(x.clone().requires_grad_(), w) is None
+    g = ops.linear(x.clone().requires_grad_(), w)
+    assert g.requires_grad
+    assert nat.tgemm(x[:, :120].contiguous(), w[:, :120].contiguous()) is None  # K of no whole step
+    with pytest.raises(RuntimeError):
+        nat.tgemm(x, w, None, False, 991)
+    with pytest.raises(RuntimeError):
+        nat.tgemm(x, w, None, False, 443)  # two steps of K in three ranges
+
+
+def test_cpu_tensors_stay_with_the_library():
+    x, w = torch.randn(130, 64).bfloat16(), torch.randn(16, 64).bfloat16()
+    assert ops.tgemm(x, w) is None
+    assert torch.equal(ops.linear(x, w), torch.nn.functional.linear(x, w))
