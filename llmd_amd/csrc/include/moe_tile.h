@@ -159,7 +159,8 @@ static inline void launch_group(const int* ids, int n, int E, int tm, int* hist,
 }
 
 // On the matrix cores, both types: a workgroup owns one tile (up to 128 rows of one expert) and 128 weight rows.
-// bf16: v_mfma_f32_16x16x32_bf16; fp32: v_mfma_f32_16x16x4_f32 on the same 16-byte pieces (element j of a lane's piece belongs
+// bf16: v_mfma_f32_16x16x32_bf16; fp32: the same on three parts of every number (moe_tile_split below), and for rows with infinities
+// and NaNs v_mfma_f32_16x16x4_f32 on the same 16-byte pieces (element j of a lane's piece belongs
 // to product j, in both operands alike). Weights are the products' A operand: a lane ends up with four neighbouring columns of
 // one row. fp32 accumulation in a fixed order of K: a row's sums do not depend on its tile. Loads run PD steps of 128 bytes
 // per row ahead of the products, in registers; LDS has two buffers and one barrier per step.
@@ -169,17 +170,17 @@ static inline void launch_group(const int* ids, int n, int E, int tm, int* hist,
 //                   several tiles.)
 //   more rows     : weights pass LDS too, read from memory a whole 128-byte line per eight lanes. Up to 64 rows the waves
 //                   split the weight rows, beyond that two by two in bf16, where the reads of LDS count. In fp32 the products
-//                   do (256 FLOP per clock and CU): there the waves split the weight rows up to the end, and a tile costs
+//                   and the splitting do: there the waves split the weight rows up to the end, and a tile costs
 //                   its blocks of 16 rows, not 128.
 // 128 gated experts of 2048 x 768, first + second product, us. bf16, 512 rows: 64 x 128 tiles through one LDS buffer 147 + 82,
-// this 138 + 73 (5.7 and 5.4 TB/s of weights). fp32, 5600 rows: FMA form 1707 + 905, this 412 + 210; 128 rows: 213 + 99.
+// this 138 + 73 (5.7 and 5.4 TB/s of weights). fp32, 5600 rows by a skewed router: FMA form 1707 + 905, fp32 instructions 412 + 210, this 365 + 185.
 //
 // Work items are (expert, block of weight rows, tile), the tiles of one block side by side: they read the same weights at the
 // same time, once from memory (tile by tile, an expert's second tile came too late for L2: 1.65 GB for 0.8 GB of weights at
 // 32768 rows). The list is cut into eight ranges, one per XCD, so that an XCD's workgroups share an expert's rows too.
 // In fp32, from 16 rows per expert on, the tiles' products differ more than their weights' streams, and the XCDs' ranges with them:
 // the tiles go to the XCDs in turn, those with the most rows first (find_work_by_size). 128 gated experts of 2048 x 768, 8 chosen,
-// by a skewed router (700 tokens: 4 to 126 rows), both products with sorting and sum, us, before / rows by 16 / and by size:
+// by a skewed router (700 tokens: 4 to 126 rows), both products with sorting and sum, us, fp32 instructions, before / rows by 16 / and by size:
 // 700 tokens 838 / 751 / 653, 1400 1380 / 1256 / 1020, 2048 1782 / 1701 / 1394 (118 of the 152 TFLOP/s that a large product
 // reaches). The line: by expert / by size at 17, 19, 22, 28, 36 rows per expert, uniform router 482 / 478, 466 / 486, 485 / 494,
 // 522 / 518, 598 / 577, skewed 598 / 505, 517 / 510, 706 / 549, 778 / 577, 921 / 645; 4 rows 436 / 458. Largest and smallest in turn,
@@ -416,21 +417,221 @@ __device__ __forceinline__ void moe_tile_many(const MoeTile& t, WRow wrow, Out o
       out((wm * MI + i) * 16 + r16, (GATED ? wn * 8 * NC : wn * 16 * NC) + c * 16 + kq * 4, acc[c][i], acc[(c + NC / 2) % NC][i]);
 }
 
+// fp32 on the bf16 units: a number is the sum of three bf16 parts (8 bits of its 24 each, rounded to nearest: exact), and the six
+// products of parts that reach 2^-26 of a product are formed, in fp32 sums. Six 16 x 16 x 32 instructions of 16 cycles for what takes
+// eight of 32 cycles in 16 x 16 x 4 fp32, beside 5.5 vector instructions per number split. Both products with sorting and sum of 128
+// gated experts of 2048 x 768 with as many rows each, us, fp32 instructions / parts: 1 row 427 / 434, 16 453 / 449, 32 514 / 493, 44
+// 590 / 524, 64 705 / 580, 80 835 / 660, 120 1240 / 940 (up to 64 rows the weights' stream counts, 414 us at its best); by a
+// skewed router, 700 tokens 631 / 556, 1400 1002 / 805, 2048 1364 / 1072. Off 64 bits, relative: (2048, 768) 1.20e-6 / 1.03e-6, (4096, 2048)
+// 1.75e-6 / 1.53e-6, (1000, 500) 8.7e-7 / 7.4e-7 (fewer roundings of the sums). Elements below 2^-109 lose parts to the units' flush
+// of bf16 denormals.
+struct Parts {
+  u32x4_t p[3];  // 8 elements: largest part first
+};
+// part i of four elements to (lo, hi); x: what is left of them
+__device__ __forceinline__ void take_part(f32x4_t& x, uint32_t& lo, uint32_t& hi) {
+  // (as casts, hipcc rounds every element twice: once for its pair, once to subtract it)
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(lo) : "v"(x[0]), "v"(x[1]));
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(hi) : "v"(x[2]), "v"(x[3]));
+  x[0] -= __uint_as_float(lo << 16), x[1] -= __uint_as_float(lo & 0xffff0000u);
+  x[2] -= __uint_as_float(hi << 16), x[3] -= __uint_as_float(hi & 0xffff0000u);
+}
+__device__ __forceinline__ Parts split8(const u32x4_t& first, const u32x4_t& second) {
+  f32x4_t x = __builtin_bit_cast(f32x4_t, first), y = __builtin_bit_cast(f32x4_t, second);
+  Parts r;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    uint32_t a, b, c, d;
+    take_part(x, a, b);
+    take_part(y, c, d);
+    r.p[i] = u32x4_t{a, b, c, d};
+  }
+  return r;
+}
+
+// fp32: rows as parts in LDS (split once), weights as they are, each wave splits its own. Up to 32 rows (DIRECT) the weights go straight to
+// registers as in moe_tile_few, else through LDS. A lane's 8 of a step's 32 elements are pieces kq and kq + 4 of a row, in
+// both operands. Every tile size sums in the same order: a row's bits do not depend on its tile.
+// LDS: two buffers of 128 weight rows of 128 bytes, two of 3 parts x 128 rows x 64 bytes; piece q of 16 bytes of row r of a part at
+// place q ^ F(r / 4 mod 4), F = 0 2 3 1. Parts of an infinite or NaN element, or of one that rounds to infinity, make NaNs of the
+// sums that it belongs to: rows with a sum that is not finite are not put out; true if there are any (bit i of rows_left: row 16 i + this
+// lane's).
+constexpr int SROW = 64, SPART = TBM * SROW, SBUF = 3 * SPART;
+constexpr int SLDS = 2 * TBUF + 2 * SBUF;  // 80 KB: two workgroups per CU
+template <bool GATED, int MI, int PD, bool DIRECT, typename WRow, typename Out>
+__device__ __forceinline__ bool moe_tile_split(const MoeTile& t, WRow wrow, Out out, uint32_t& rows_left) {
+  constexpr int NA = (MI + 1) / 2;  // a thread's pieces of the rows in a step
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, kq = lane >> 4;
+  const int kb = t.K * 4, nk = kb >> 7;
+  const auto place = [](int row, int q) { return row * SROW + ((q ^ (0x1E >> (2 * (row >> 2 & 3)) & 3)) * 16); };
+  const int wr = lds_wr(tid), sa = 2 * TBUF + place(tid >> 3, tid & 3) + (tid & 4) * 2, ra = 2 * TBUF + place(r16, kq);
+  // the wave's weight rows: gated 16 gate rows and their up rows, else 32 neighbours
+  const auto own = [&](int c) { return GATED ? c * 64 + wave * 16 : wave * 32 + c * 16; };
+  uint32_t wp[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    wp[i] = DIRECT ? wrow(own(i >> 1) + r16) + kq * 16 + (i & 1) * 64 : wrow((tid >> 3) + 32 * i) + (tid & 7) * 16;
+  f32x4_t acc[2][MI];
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) acc[c][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  u32x4_t wb[PD][4], ab[PD][NA];
+  auto load_a = [&](int s, int kt) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i) ab[s][i] = *reinterpret_cast<const u32x4_t*>(t.ap[i] + kt * 128);
+  };
+  auto load_w = [&](int s, int kt) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) wb[s][i] = *reinterpret_cast<const u32x4_t*>(t.w + kt * 128 + wp[i]);
+  };
+  auto store = [&](int s, int buf) {
+    if constexpr (!DIRECT) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4_t*>(t.lds + buf * TBUF + wr + i * 32 * TLS) = wb[s][i];
+    }
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      f32x4_t x = __builtin_bit_cast(f32x4_t, ab[s][i]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        uint32_t lo, hi;
+        take_part(x, lo, hi);
+        *reinterpret_cast<uint64_t*>(t.lds + buf * SBUF + p * SPART + sa + i * 32 * SROW) = lo | (uint64_t)hi << 32;
+      }
+    }
+  };
+  auto products = [&](int s, int buf) {
+    Parts w[2];
+    constexpr int AHEAD = MI < 6 ? 1 : 0;  // blocks whose parts are read beforehand: registers
+    u32x4_t a[1 + AHEAD][3];
+    auto read_a = [&](int i) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) a[i & AHEAD][p] = *reinterpret_cast<const u32x4_t*>(t.lds + buf * SBUF + p * SPART + ra + i * 16 * SROW);
+    };
+    if constexpr (AHEAD) read_a(0);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      if constexpr (DIRECT) {
+        w[c] = split8(wb[s][2 * c], wb[s][2 * c + 1]);
+      } else {
+        const char* at = t.lds + buf * TBUF;
+        const int rw = own(c) * TLS + lds_rd(r16, kq);
+        w[c] = split8(*reinterpret_cast<const u32x4_t*>(at + rw), *reinterpret_cast<const u32x4_t*>(at + (rw ^ 64)));
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (i + AHEAD < MI) read_a(i + AHEAD);
+#pragma unroll
+      for (int k = 5; k >= 0; --k) {  // the smallest products first
+        constexpr int PW[6] = {0, 0, 1, 1, 0, 2}, PA[6] = {0, 1, 0, 1, 2, 0};
+#pragma unroll
+        for (int c = 0; c < 2; ++c) mma16<uint16_t>(acc[c][i], w[c].p[PW[k]], a[i & AHEAD][PA[k]]);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  k_steps<PD>(
+      nk,
+      [&](int s) {
+        load_a(s, s);
+        load_w(s, s);
+      },
+      [&](auto more) {
+        store(0, 0);
+        if constexpr (more) {
+          load_a(0, PD);
+          if constexpr (!DIRECT) load_w(0, PD);
+        }
+      },
+      [&](auto s, int kt, auto next, auto more_a, auto more_w) {
+        meet();  // buffer kt & 1 is written, the other one read
+        if constexpr (next) {
+          store((s + 1) % PD, (kt + 1) & 1);
+          if constexpr (more_a) {
+            load_a((s + 1) % PD, kt + 1 + PD);
+            if constexpr (!DIRECT) load_w((s + 1) % PD, kt + 1 + PD);
+          }
+        }
+        products(s, kt & 1);
+        if constexpr (DIRECT && more_w) load_w(s, kt + PD);
+      });
+  if (kb & 127) {  // the rest of K, a multiple of 16 bytes: pieces past the end are zeros
+    const int left = kb & 127;
+    const u32x4_t zero = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < NA; ++i) ab[0][i] = (tid & 7) * 16 < left ? *reinterpret_cast<const u32x4_t*>(t.ap[i] + nk * 128) : zero;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      wb[0][i] = (DIRECT ? kq * 16 + (i & 1) * 64 : (tid & 7) * 16) < left ? *reinterpret_cast<const u32x4_t*>(t.w + nk * 128 + wp[i]) : zero;
+    meet();
+    store(0, 0);
+    meet();
+    products(0, 0);
+  }
+  // a bit per row of the tile, of all waves together (they hold the rows' other columns)
+  if constexpr (!DIRECT) meet();  // (with DIRECT nothing else lies there)
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    bool finite = true;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) finite &= fabsf(acc[c][i][q]) < INFINITY;
+    uint64_t m = __ballot(!finite);
+    m |= m >> 32;
+    m |= m >> 16;
+    if (lane == 0) reinterpret_cast<uint16_t*>(t.lds)[wave * 8 + i] = (uint16_t)m;
+  }
+  meet();
+  uint32_t any = 0, mine = 0;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int o = 0; o < 4; ++o) m |= reinterpret_cast<const uint16_t*>(t.lds)[o * 8 + i];
+    any |= m;
+    mine |= (m >> r16 & 1) << i;
+  }
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int c = 0; c < (GATED ? 1 : 2); ++c)
+      if ((mine >> i & 1) == 0) out(i * 16 + r16, own(c) + kq * 4, acc[c][i], acc[1][i]);
+  rows_left = mine;
+  return any != 0;
+}
+
 // One tile of ``rows`` rows: the body for its size.
 template <typename T, bool GATED, typename WRow, typename Out>
 __device__ __forceinline__ void run_tile(const MoeTile& t, int rows, WRow wrow, Out out) {
   if constexpr (sizeof(T) == 4) {
-    if (rows > 112) return moe_tile_many<T, GATED, 8, 1, 2>(t, wrow, out);
-    if (rows > 96) return moe_tile_many<T, GATED, 7, 1, 2>(t, wrow, out);
-    if (rows > 80) return moe_tile_many<T, GATED, 6, 1, 2>(t, wrow, out);
-    if (rows > 64) return moe_tile_many<T, GATED, 5, 1, 2>(t, wrow, out);
+    bool left;
+    uint32_t which;
+    if (rows > 112) left = moe_tile_split<GATED, 8, 2, false>(t, wrow, out, which);
+    else if (rows > 96) left = moe_tile_split<GATED, 7, 2, false>(t, wrow, out, which);
+    else if (rows > 80) left = moe_tile_split<GATED, 6, 2, false>(t, wrow, out, which);
+    else if (rows > 64) left = moe_tile_split<GATED, 5, 2, false>(t, wrow, out, which);
+    else if (rows > 48) left = moe_tile_split<GATED, 4, 2, false>(t, wrow, out, which);
+    else if (rows > 32) left = moe_tile_split<GATED, 3, 2, false>(t, wrow, out, which);
+    else if (rows > 16) left = moe_tile_split<GATED, 2, 3, true>(t, wrow, out, which);
+    else left = moe_tile_split<GATED, 1, 3, true>(t, wrow, out, which);
+    if (left) {  // rows with infinities and NaNs: as fp32 has them (in the same lanes)
+      meet();
+      moe_tile_many<T, GATED, 8, 1, 2>(t, wrow, [&](int r, int c, const f32x4_t& g, const f32x4_t& u) {
+        if (which >> (r >> 4) & 1) out(r, c, g, u);
+      });
+    }
+    return;
   } else {
     if (rows > 64) return moe_tile_many<T, GATED, 4, 2, 2>(t, wrow, out);
+    if (rows > 48) return moe_tile_many<T, GATED, 4, 1, 2>(t, wrow, out);
+    if (rows > 32) return moe_tile_many<T, GATED, 3, 1, 2>(t, wrow, out);
+    if (rows > 16) return moe_tile_few<T, GATED, 2, 3>(t, wrow, out);
+    moe_tile_few<T, GATED, 1, 3>(t, wrow, out);
   }
-  if (rows > 48) moe_tile_many<T, GATED, 4, 1, 2>(t, wrow, out);
-  else if (rows > 32) moe_tile_many<T, GATED, 3, 1, 2>(t, wrow, out);
-  else if (rows > 16) moe_tile_few<T, GATED, 2, 3>(t, wrow, out);
-  else moe_tile_few<T, GATED, 1, 3>(t, wrow, out);
 }
 
 // The work item of a workgroup: expert, tile, block of weight rows; false: none left.

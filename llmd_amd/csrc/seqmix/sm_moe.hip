@@ -379,7 +379,7 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const T* __restrict__ 
   Work wk;
   if (order != nullptr ? !find_work_by_size(tiles, order, NB, wk) : !find_work(tiles, NB, wk)) return;
   const int nb = wk.nb, tile = wk.tile, e = wk.e, rows = wk.rows;
-  __shared__ __attribute__((aligned(128))) char lds[4 * TBUF];
+  __shared__ __attribute__((aligned(128))) char lds[sizeof(T) == 4 ? SLDS : 4 * TBUF];
   const int tid = threadIdx.x;
   const int64_t slot0 = (int64_t)tile * tm;
   const int col0 = nb * (GATED ? TBW / 2 : TBW);  // the workgroup's first output column

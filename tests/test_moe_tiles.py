@@ -101,3 +101,48 @@ def test_interleaved_experts_few_rows(d, F):
         want, size = a @ w2[e].double().T * w[rows], a.abs() @ w2[e].abs().double().T * w[rows]
         # the activation, the expert's row and the result are each rounded to bf16 once
         assert ((got[rows] - want).abs() <= 3 * 2.0 ** -9 * (size + want.abs()) + 2.0 ** -9).all()
+
+
+@pytest.mark.parametrize("d,F", [(256, 96), (100, 72)])
+def test_float32_rows_alone_and_together(d, F):
+    """fp32 experts form their products from three bf16 parts of every number: within the bound of fp32 sums for every tile
+    height, a row's bits whatever its tile, and rows with infinities, NaNs or numbers that a part cannot hold as fp32 has them
+    without a trace in the others."""
+    from llmd_amd.ops import seqmix as sm
+
+    g = torch.Generator().manual_seed(d)
+    E = 8
+    ids = _counts_to_ids([9, 30, 40, 60, 75, 90, 110, 128], 0)
+    T = ids.shape[0]
+    h = torch.randn(T, d, generator=g) * torch.exp(2 * torch.randn(T, d, generator=g))
+    w1 = torch.randn(E, F, d, generator=g) / d ** 0.5
+    w2 = torch.randn(E, d, F, generator=g) / F ** 0.5
+
+    def run(h, ids):
+        n = len(h)
+        return sm.moe_ffn(h.cuda(), ids.cuda(), torch.ones(n, 1, device="cuda"), w1.cuda(), w2.cuda(), "relu2").cpu()
+
+    got = run(h, ids)
+    x, e = h.double(), ids[:, 0].long()
+    a = torch.einsum("td,tfd->tf", x, w1.double()[e])
+    ea = torch.einsum("td,tfd->tf", x.abs(), w1.double()[e].abs()) * (d + 8) * 2.0 ** -24  # of the first sums
+    a, ea = a.clamp(min=0) ** 2, 2 * (a.abs() + ea) * ea + a * a * 2.0 ** -23
+    want = torch.einsum("tf,tdf->td", a, w2.double()[e])
+    bound = torch.einsum("tf,tdf->td", ea + a * (F + 8) * 2.0 ** -24, w2.double()[e].abs())
+    assert ((got - want).abs() <= bound).all()
+    few = torch.arange(0, T, 7)
+    assert torch.equal(run(h[few], ids[few]), got[few])
+    bad = h.clone()
+    rows = [int((e == i).nonzero()[3]) for i in range(E)]
+    values = [float("inf"), -float("inf"), float("nan"), 3.4e38] * 2
+    for r, v in zip(rows, values):
+        bad[r, 5] = v
+    out = run(bad, ids)
+    rest = torch.ones(T, dtype=torch.bool)
+    rest[rows] = False
+    assert torch.equal(out[rest], got[rest])
+    for r, v in zip(rows, values):
+        z = w1[e[r]].double() @ bad[r].double()  # +-inf, NaN or large: squares that overflow
+        full = torch.where(z.isnan(), 0.0, z.clamp(min=0) ** 2).float()
+        want = torch.where(full[None] * w2[e[r]] == 0, torch.zeros(()), full[None] * w2[e[r]])
+        assert torch.equal(out[r].isfinite(), torch.isfinite(want.sum(1)))
