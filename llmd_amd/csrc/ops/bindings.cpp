@@ -71,6 +71,8 @@ int64_t llmd_pgemm_ws_bytes(int, int, int, int, int);
 int llmd_tgemm_plan(int, int, int, int);
 int llmd_tgemm(const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, int, const void*, void*,
                hipStream_t);
+int llmd_fgemm_plan(int, int, int);
+int llmd_fgemm(const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, const void*, void*, hipStream_t);
 int llmd_pgemm_fp8(const void*, int64_t, const float*, const void*, int64_t, const float*, void*, int64_t, int, int,
                    int, int, void*, int, hipStream_t);
 int64_t llmd_pgemm_fp8_ws_bytes(int, int, int, int);
@@ -609,6 +611,32 @@ std::optional<torch::Tensor> tgemm(const torch::Tensor& x, const torch::Tensor& 
                             (int)K, silu ? 1 : 0, code, bias ? bias->data_ptr() : nullptr,
                             ws.defined() ? ws.data_ptr() : nullptr, cur_stream());
   TORCH_CHECK(rc == 0, "tgemm failed: ", rc);
+  return y;
+}
+
+// x w^T (+ bias) in fp32 on the tile that llmd_fgemm_plan has for these sizes (csrc/ops/fgemm.hip), or on `tile`; nothing where it
+// has none or the operands are not what the kernel reads
+std::optional<torch::Tensor> fgemm(const torch::Tensor& x, const torch::Tensor& w, const std::optional<torch::Tensor>& bias,
+                                   int64_t tile) {
+  if (!x.is_cuda() || x.device() != w.device() || x.dim() != 2 || w.dim() != 2 || x.scalar_type() != at::kFloat ||
+      w.scalar_type() != at::kFloat)
+    return std::nullopt;
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0), most = 1 << 30;
+  const auto off = [](const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0; };
+  if (w.size(1) != K || M > most || N > most || K > most || x.stride(1) != 1 || w.stride(1) != 1 || x.stride(0) < K ||
+      w.stride(0) < K || x.stride(0) % 4 || w.stride(0) % 4 || w.stride(0) > most / 128 || off(x) || off(w))
+    return std::nullopt;
+  if (bias && (bias->scalar_type() != at::kFloat || bias->device() != x.device() || bias->dim() != 1 || bias->size(0) != N ||
+               (N > 1 && bias->stride(0) != 1)))
+    return std::nullopt;
+  const int code = tile ? (int)tile : llmd_fgemm_plan((int)M, (int)N, (int)K);
+  if (code == 0) return std::nullopt;
+  const c10::hip::OptionalHIPGuard device_guard(dev_of(x));
+  torch::Tensor y = torch::empty({M, N}, x.options()), ws;
+  if (code % 10 > 1) ws = torch::empty({code % 10, M, N}, x.options());
+  const int rc = llmd_fgemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N, (int)M, (int)N, (int)K,
+                            code, bias ? bias->data_ptr() : nullptr, ws.defined() ? ws.data_ptr() : nullptr, cur_stream());
+  TORCH_CHECK(rc == 0, "fgemm failed: ", rc);
   return y;
 }
 
@@ -1389,6 +1417,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_debug (llmd_amd/build.p
   m.def("tgemm", &tgemm, "bf16 GEMM of prompt-sized steps on the tile that fits, or None", py::arg("x"), py::arg("w"),
         py::arg("bias") = std::nullopt, py::arg("silu") = false, py::arg("tile") = 0);
   m.def("tgemm_plan", &llmd_tgemm_plan, "tile of tgemm for (M, N, K, silu): mi * 100 + ni * 10 + ranges of K, or 0");
+  m.def("fgemm", &fgemm, "fp32 GEMM of prompt-sized steps on the bf16 matrix units, or None", py::arg("x"), py::arg("w"),
+        py::arg("bias") = std::nullopt, py::arg("tile") = 0);
+  m.def("fgemm_plan", &llmd_fgemm_plan, "tile of fgemm for (M, N, K): mi * 100 + ni * 10 + ranges of K, or 0");
   m.def("pgemm", &pgemm, "prefill bf16 GEMM (256x256 LDS-DMA MFMA tiles), optional fused SiLU-and-mul",
         py::arg("y"), py::arg("x"), py::arg("w"), py::arg("epi"), py::arg("variant"), py::arg("split_k") = true);
   m.def("mgemm_fp8", &mgemm_fp8);

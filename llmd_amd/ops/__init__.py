@@ -1383,6 +1383,14 @@ def tgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     return native().tgemm(x, w, bias, silu)
 
 
+def fgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None):
+    """fp32 x w^T (+ bias) on the bf16 matrix units, three parts of every number (csrc/ops/fgemm.hip, which holds the rule), or
+    None where it is not taken. No further from 64 bits than the library's fp32 product."""
+    if not _gpu(x) or not _plain(x, w):
+        return None
+    return native().fgemm(x, w, bias)
+
+
 def router_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """A router's logits: prompts on ``tgemm`` (2048 x (128, 2048) hipBLASLt 12.4 us, here 7), the rest on the library."""
     y = tgemm(x, w, bias) if x.dim() == 2 and x.shape[0] > 64 else None
@@ -1539,7 +1547,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
     shapes by ``decode_rule`` (without a bias, which hipBLASLt adds for nothing) -
     prefill-sized M on the prefill GEMM where the shipped table (ops/pgemm_table.py)
     has it ahead of hipBLASLt, other M above 64 on the GEMM with a tile for the size
-    (``tgemm``) - everything else on hipBLASLt."""
+    (``tgemm``; in fp32 ``fgemm``) - everything else on hipBLASLt."""
     if PGEMM_AUTO != "0" and x.dim() == 2 and x.shape[0] >= PGEMM_MIN_M and pgemm_ok(x, w):
         plan = pgemm_wins(x, w)
         if plan is not None:
@@ -1563,7 +1571,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
             if rule is not None:
                 return rule[0](x, w, rule[1])
     if x.dim() == 2 and x.shape[0] > 64:
-        y = tgemm(x, w, bias)
+        y = fgemm(x, w, bias) if x.dtype == torch.float32 else tgemm(x, w, bias)
         if y is not None:
             return y
     return torch.nn.functional.linear(x, w, bias)
