@@ -58,7 +58,7 @@ __global__ __launch_bounds__(NT, 1) void tgemm_kernel(const uint16_t* __restrict
                                                       const uint16_t* __restrict__ W, int64_t ldw,
                                                       uint16_t* __restrict__ C, int64_t ldc, int M, int N, int K,
                                                       const uint16_t* __restrict__ bias, int nsplit,
-                                                      float* __restrict__ ws) {
+                                                      int rounded, float* __restrict__ ws) {
   constexpr int ST = stages(MI, NI), D = MI + NI, R = MI + NI, T = MI * NI;
   constexpr int STG = 4096 * (MI + NI), OPW = 4096 * MI;
   constexpr int BM = 32 * MI, BN = 32 * NI;
@@ -243,7 +243,8 @@ __global__ __launch_bounds__(NT, 1) void tgemm_kernel(const uint16_t* __restrict
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[e]), __float_as_uint(y[e]), false, false);
-        const float g = __uint_as_float(s[0]), u = __uint_as_float(s[1]);
+        float g = __uint_as_float(s[0]), u = __uint_as_float(s[1]);
+        if (rounded) g = __uint_as_float((uint32_t)f2bf(g) << 16), u = __uint_as_float((uint32_t)f2bf(u) << 16);
         o[e] = g / (1.f + __expf(-g)) * u;
       }
       u32x2_t p;
@@ -323,8 +324,9 @@ double tgemm_us(int M, int N, int K, int mi, int ni, int ns) {
 //  * Below 65 rows the decode kernels.
 //  * Whole products with 256 x 256 tiles and, up to K 2048, those of 256 x 224: pgemm.hip or hipBLASLt as before (2551 x (5632, 2048): hipBLASLt
 //    47.5, here 50.6; 2048 x (8192, 8192) 180 both). Elsewhere at most 8 % slower than hipBLASLt, on average 22 % faster.
-//  * SiLU: where the 256 x 256 tiles of pgemm.hip take more than 3 % longer (1429 x (28672, 4096) 300 / 252, 2048: 359
-//    / 352; 2300: 399 / 399, not taken), above mgemm.hip's 256 rows (100 x (28672, 4096): 51, here 53).
+//  * silu 1: in place of the 256 x 256 tiles of pgemm.hip where these take more than 3 % longer (1429 x (28672, 4096) 300 / 252,
+//    2048: 359 / 352; 2300: 399 / 399, not taken). silu 2: in place of a product and the activation's own pass, where no
+//    more than 5 % slower than 256 x 256 tiles. Both above mgemm.hip's 256 rows (100 x (28672, 4096): 51, here 53).
 //  * More than one range of K only for what the chip takes at once, ranges of at least 8 steps, and where it gains 10 %: 512 x (4096,
 //    14336) 98 with one, 65 with four. Sums of at most 256 MB.
 extern "C" int llmd_tgemm_plan(int M, int N, int K, int silu) {
@@ -347,28 +349,29 @@ extern "C" int llmd_tgemm_plan(int M, int N, int K, int silu) {
     }
   }
   if (code % 10 == 1 && (area >= 64 || (K <= 2048 && area >= 56 && !silu))) return 0;
-  if (silu && best > 0.97 * tgemm_us(M, N, K, 8, 8, 1)) return 0;
+  if (silu && best > (silu == 1 ? 0.97 : 1.05) * tgemm_us(M, N, K, 8, 8, 1)) return 0;
   return code;
 }
 
-// A tile of llmd_tgemm_plan. N: columns of C; W [N, K], with epi 1 [2 N, K] (gate rows, then up rows). bias: [N] or null (epi 0).
-// ranges > 1 (epi 0): sums in ws [ranges, M, N]. -1: not taken.
+// A tile of llmd_tgemm_plan. N: columns of C; W [N, K], with silu [2 N, K] (gate rows, then up rows); 1: of the fp32 sums, 2: of the
+// sums rounded to bf16, as a pass of its own would find them. bias: [N] or null (no silu).
+// ranges > 1 (no silu): sums in ws [ranges, M, N]. -1: not taken.
 extern "C" int llmd_tgemm(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N,
-                          int K, int epi, int code, const void* bias, void* ws, hipStream_t st) {
+                          int K, int silu, int code, const void* bias, void* ws, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
   const int mi = code / 100, ni = code / 10 % 10, nsplit = code % 10;
-  if (N % 8 || K % BK || K <= 0 || lda % 8 || ldw % 8 || ldc % 8 || (epi != EPI_NONE && epi != EPI_SILU)) return -1;
+  if (N % 8 || K % BK || K <= 0 || lda % 8 || ldw % 8 || ldc % 8 || silu < 0 || silu > 2) return -1;
   const int nk = K / BK;
   if (nsplit < 1 || nsplit > nk || (nsplit - 1) * ((nk + nsplit - 1) / nsplit) >= nk) return -1;
-  if ((nsplit > 1 && (epi != EPI_NONE || ws == nullptr)) || (bias != nullptr && epi != EPI_NONE)) return -1;
+  if ((nsplit > 1 && (silu || ws == nullptr)) || (bias != nullptr && silu)) return -1;
   // buffer offsets are 31-bit byte offsets
-  const int64_t wrows = epi == EPI_SILU ? 2 * (int64_t)N : N;
+  const int64_t wrows = silu ? 2 * (int64_t)N : N;
   if (((int64_t)(M - 1) * lda + K) * 2 > 0x7fffffffLL || ((wrows - 1) * ldw + K) * 2 > 0x7fffffffLL) return -2;
-  const int tc = epi == EPI_SILU ? 16 * ni : 32 * ni;
+  const int tc = silu ? 16 * ni : 32 * ni;
   const auto launch = [&](auto kernel) {
     const int64_t grid = (int64_t)((M + 32 * mi - 1) / (32 * mi)) * ((N + tc - 1) / tc) * nsplit;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NT), 0, st, (const uint16_t*)A, lda, (const uint16_t*)W, ldw,
-                       (uint16_t*)C, ldc, M, N, K, (const uint16_t*)bias, nsplit, (float*)ws);
+                       (uint16_t*)C, ldc, M, N, K, (const uint16_t*)bias, nsplit, silu == 2, (float*)ws);
     if (nsplit > 1)
       hipLaunchKernelGGL(tgemm_reduce_kernel, dim3((unsigned)(((int64_t)M * (N / 8) + 255) / 256)), dim3(256), 0, st,
                          (const float*)ws, nsplit, M, N, (const uint16_t*)bias, (uint16_t*)C, ldc);
@@ -376,9 +379,9 @@ extern "C" int llmd_tgemm(const void* A, int64_t lda, const void* W, int64_t ldw
   };
 #define T_CASE(MI, NI)                                                              \
   if (mi == MI && ni == NI)                                                         \
-    return epi == EPI_SILU ? launch(tgemm_kernel<MI, NI, EPI_SILU>)                 \
-           : nsplit > 1    ? launch(tgemm_kernel<MI, NI, EPI_F32>)                  \
-                           : launch(tgemm_kernel<MI, NI, EPI_NONE>);
+    return silu         ? launch(tgemm_kernel<MI, NI, EPI_SILU>)                    \
+           : nsplit > 1 ? launch(tgemm_kernel<MI, NI, EPI_F32>)                     \
+                        : launch(tgemm_kernel<MI, NI, EPI_NONE>);
   TGEMM_TILES(T_CASE)
 #undef T_CASE
   if (mi == 8 && ni == 8 && nsplit > 1) return launch(tgemm_kernel<8, 8, EPI_F32>);

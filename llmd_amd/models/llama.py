@@ -41,10 +41,10 @@ class LlamaMLP(torch.nn.Module):
             # prefill: gate/up GEMM with the SiLU-and-mul in its epilogue: on tiles that fill whole rounds of the
             # chip (csrc/ops/tgemm.hip) where these take less time than the 256 x 256 ones, which run (csrc/ops/pgemm.hip
             # EPI_SILU_STD) where the shipped table has it ahead of hipBLASLt + the act kernel
-            y = ops.tgemm(x, gu.weight, silu=True) if x.shape[0] > 256 else None
+            v = ops.pgemm_silu_plan(x, gu.weight)
+            y = ops.tgemm(x, gu.weight, silu=1 if v == 6 else 2) if x.shape[0] > 256 else None
             if y is not None:
                 return y
-            v = ops.pgemm_silu_plan(x, gu.weight)
             if v is not None:
                 return ops.pgemm_silu(x, gu.weight, variant=v)
             # decode: the same fusion in the medium-M GEMM (csrc/ops/mgemm.hip ACT form)

@@ -1375,8 +1375,9 @@ def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
             and torch._C._len_torch_function_stack() == 0)
 
 
-def tgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, silu: bool = False):
-    """x w^T (+ bias), or silu(x wg^T) * (x wu^T) for w = [gate; up], on the GEMM whose tile fits the sizes
+def tgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, silu: int = 0):
+    """x w^T (+ bias), or silu(x wg^T) * (x wu^T) for w = [gate; up] (1: of the fp32 sums as ``pgemm_silu`` variant 6, 2: of the
+    sums in bf16, the bits of ``linear`` + ``gated_act``), on the GEMM whose tile fits the sizes
     (csrc/ops/tgemm.hip, which holds the rule), or None where it is not taken."""
     if PGEMM_AUTO == "0" or not _gpu(x) or not _plain(x, w):
         return None

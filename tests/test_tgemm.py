@@ -30,13 +30,14 @@ def test_tiles_edges(mi, ni):
         wide[:, :K] = x
         bias = torch.linspace(-2, 2, N, device="cuda").bfloat16()
         ref = x.float() @ w.float().t()
-        y = ops.native().tgemm(x, w, None, False, mi * 100 + ni * 10 + 1)
+        y = ops.native().tgemm(x, w, None, 0, mi * 100 + ni * 10 + 1)
         _close(y, ref)
-        assert torch.equal(ops.native().tgemm(wide[:, :K], w, None, False, mi * 100 + ni * 10 + 1), y)
+        assert torch.equal(ops.native().tgemm(wide[:, :K], w, None, 0, mi * 100 + ni * 10 + 1), y)
         _close(ops.native().tgemm(x, w, bias, False, mi * 100 + ni * 10 + 1), ref + bias.float())
         w2 = torch.cat([w, w.flip(0)])
-        _close(ops.native().tgemm(x, w2, None, True, mi * 100 + ni * 10 + 1),
-               torch.nn.functional.silu(ref) * ref.flip(1))
+        _close(ops.native().tgemm(x, w2, None, 1, mi * 100 + ni * 10 + 1), torch.nn.functional.silu(ref) * ref.flip(1))
+        z = ops.native().tgemm(x, w2, None, 0, mi * 100 + ni * 10 + 1)
+        assert torch.equal(ops.native().tgemm(x, w2, None, 2, mi * 100 + ni * 10 + 1), ops.gated_act(z, ops.ACT_SILU))
 
 
 @pytest.mark.gpu
@@ -48,7 +49,7 @@ def test_ranges_of_k(mi, ni, ranges):
         bias = torch.linspace(-2, 2, N, device="cuda").bfloat16()
         ref = x.float() @ w.float().t()
         code = mi * 100 + ni * 10 + ranges
-        _close(ops.native().tgemm(x, w, None, False, code), ref)
+        _close(ops.native().tgemm(x, w, None, 0, code), ref)
         _close(ops.native().tgemm(x, w, bias, False, code), ref + bias.float())
 
 
@@ -61,8 +62,8 @@ def test_linear_takes_it(M, N, K):
     x, w = _operands(M, N, K)
     y = ops.linear(x, w)
     _close(y, x.float() @ w.float().t())
-    assert torch.equal(y, ops.native().tgemm(x, w, None, False, code))
-    assert torch.equal(y[:65], ops.native().tgemm(x[:65], w, None, False, 221))
+    assert torch.equal(y, ops.native().tgemm(x, w, None, 0, code))
+    assert torch.equal(y[:65], ops.native().tgemm(x[:65], w, None, 0, 221))
 
 
 @pytest.mark.gpu
@@ -78,9 +79,9 @@ def test_refused_or_left():
     assert g.requires_grad
     assert nat.tgemm(x[:, :120].contiguous(), w[:, :120].contiguous()) is None  # K of no whole step
     with pytest.raises(RuntimeError):
-        nat.tgemm(x, w, None, False, 991)
+        nat.tgemm(x, w, None, 0, 991)
     with pytest.raises(RuntimeError):
-        nat.tgemm(x, w, None, False, 443)  # two steps of K in three ranges
+        nat.tgemm(x, w, None, 0, 443)  # two steps of K in three ranges
 
 
 def test_cpu_tensors_stay_with_the_library():
