@@ -58,6 +58,21 @@ __device__ __forceinline__ u32x4_t pack8(const float* f) {
   return v;
 }
 
+// max(0, .)^2 of a number in bf16, in bf16
+__device__ __forceinline__ float relu2_bf(float f) {
+  const float a = fmaxf(__uint_as_float((uint32_t)f2bf(f) << 16), 0.f);
+  return a * a;
+}
+// four sums as bf16, squared ReLU of them where it is asked for
+__device__ __forceinline__ uint2 pack4(const f32x4_t v, int relu2) {
+  f32x4_t o = v;
+  if (relu2) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = relu2_bf(v[e]);
+  }
+  return make_uint2((uint32_t)f2bf(o[0]) | ((uint32_t)f2bf(o[1]) << 16), (uint32_t)f2bf(o[2]) | ((uint32_t)f2bf(o[3]) << 16));
+}
+
 // ---- FP8 (OCP e4m3fn on gfx950). KV-cache / activation storage
 // format; math stays bf16/f32. Scales are applied outside (folded into the
 // softmax scale / output), so conversions here are unscaled.

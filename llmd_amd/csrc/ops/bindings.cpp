@@ -54,10 +54,10 @@ int llmd_mla_rope_cache(const void*, int64_t, void*, int64_t, const void*, int64
 int llmd_lora_bgmv(const void*, int64_t, const void*, const void*, int, int, int, int, const int*, float*, void*,
                    int64_t, hipStream_t);
 int llmd_skinny_gemm(const void*, int64_t, const void*, int64_t, int, int, int, int, int, int, void*, int64_t,
-                     float*, hipStream_t);
+                     float*, int, hipStream_t);
 int llmd_dgemm_supported(int, int, int);
 int llmd_mgemm(const void*, int64_t, const void*, int64_t, int, int, int, int, int, int, void*, int64_t, float*,
-               int*, hipStream_t);
+               int*, int, hipStream_t);
 int llmd_mgemm_lds(int, int, int);
 int llmd_mgemm_partials(const void*, int64_t, const void*, int64_t, int, int, int, int, int, int, float*, hipStream_t);
 int llmd_reduce_rope_cache(const float*, int, int, void*, int64_t, const int64_t*, const float*, int, int, int, int,
@@ -469,7 +469,7 @@ void lora_bgmv(torch::Tensor y, torch::Tensor x, torch::Tensor A, torch::Tensor 
 // y [M, N] = x [M, K] . w [N, K]^T for M <= 64 (decode GEMMs): rb row blocks of
 // 16 per workgroup, nsplit-way split-K, occ workgroups per CU (ops.skinny_plan)
 void skinny_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t rb, int64_t nsplit, int64_t occ,
-                 torch::Tensor part) {
+                 torch::Tensor part, bool relu2) {
   const c10::hip::OptionalHIPGuard device_guard(dev_of(y));
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_BF16(y); CHECK_INNER(x); CHECK_INNER(w); CHECK_INNER(y);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && y.dim() == 2, "skinny_gemm: 2-D operands");
@@ -485,7 +485,7 @@ void skinny_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t rb, 
   }
   int rc = llmd_skinny_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), M, N, K, (int)rb, (int)nsplit,
                             (int)occ, y.data_ptr(), y.stride(0), nsplit > 1 ? part.data_ptr<float>() : nullptr,
-                            cur_stream());
+                            relu2, cur_stream());
   TORCH_CHECK(rc == 0, "skinny_gemm failed: ", rc);
 }
 
@@ -523,7 +523,7 @@ int* mgemm_counters(const torch::Device& d, int64_t tiles) {
 }
 
 void mgemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t wrb, int64_t nsplit, int64_t stages,
-           torch::Tensor part) {
+           torch::Tensor part, bool relu2) {
   const c10::hip::OptionalHIPGuard device_guard(dev_of(y));
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_BF16(y); CHECK_INNER(x); CHECK_INNER(w); CHECK_INNER(y);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && y.dim() == 2, "mgemm: 2-D operands");
@@ -539,7 +539,7 @@ void mgemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t wrb, int64
   int rc = llmd_mgemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), M, N, K, (int)wrb, (int)nsplit,
                       (int)stages, y.data_ptr(), y.stride(0), nsplit > 1 ? part.data_ptr<float>() : nullptr,
                       nsplit > 1 ? mgemm_counters(y.device(), (N + 64 * wrb - 1) / (64 * wrb)) : nullptr,
-                      cur_stream());
+                      relu2, cur_stream());
   TORCH_CHECK(rc == 0, "mgemm failed: ", rc);
 }
 
@@ -586,10 +586,12 @@ void pgemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t epi, int64
   TORCH_CHECK(rc == 0, "pgemm failed: ", rc);
 }
 
-// x w^T (+ bias), or with silu silu(x wg^T) * (x wu^T) of w = [gate; up] (1: of the fp32 sums, 2: of the sums in bf16), on the tile that llmd_tgemm_plan has for these
+// x w^T (+ bias); with act silu(x wg^T) * (x wu^T) of w = [gate; up] (1: of the fp32 sums, 2: of the sums in bf16) or max(0, x w^T)^2
+// (3: of the sums in bf16), on the tile that llmd_tgemm_plan has for these
 // sizes (csrc/ops/tgemm.hip), or on `tile`; nothing where it has none or the operands are not what the kernel reads
 std::optional<torch::Tensor> tgemm(const torch::Tensor& x, const torch::Tensor& w, const std::optional<torch::Tensor>& bias,
-                                   int64_t silu, int64_t tile) {
+                                   int64_t act, int64_t tile) {
+  const bool silu = act == 1 || act == 2;
   if (!x.is_cuda() || x.device() != w.device() || x.dim() != 2 || w.dim() != 2 || x.scalar_type() != at::kBFloat16 ||
       w.scalar_type() != at::kBFloat16)
     return std::nullopt;
@@ -602,13 +604,13 @@ std::optional<torch::Tensor> tgemm(const torch::Tensor& x, const torch::Tensor& 
   if (bias && (silu || bias->scalar_type() != at::kBFloat16 || bias->device() != x.device() || bias->dim() != 1 ||
                bias->size(0) != N || (N > 1 && bias->stride(0) != 1) || off(*bias)))
     return std::nullopt;
-  const int code = tile ? (int)tile : llmd_tgemm_plan((int)M, (int)rows, (int)K, (int)silu);
+  const int code = tile ? (int)tile : llmd_tgemm_plan((int)M, (int)rows, (int)K, silu ? (int)act : 0);
   if (code == 0) return std::nullopt;
   const c10::hip::OptionalHIPGuard device_guard(dev_of(x));
   torch::Tensor y = torch::empty({M, N}, x.options()), ws;
   if (code % 10 > 1) ws = torch::empty({code % 10, M, N}, x.options().dtype(torch::kFloat));
   const int rc = llmd_tgemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N, (int)M, (int)N,
-                            (int)K, (int)silu, code, bias ? bias->data_ptr() : nullptr,
+                            (int)K, (int)act, code, bias ? bias->data_ptr() : nullptr,
                             ws.defined() ? ws.data_ptr() : nullptr, cur_stream());
   TORCH_CHECK(rc == 0, "tgemm failed: ", rc);
   return y;
@@ -1406,16 +1408,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_debug (llmd_amd/build.p
   m.def("kvx_ipc_close", &kvx_ipc_close);
   m.def("mla_attention", &mla_attention);
   m.def("mla_v2_shape", &mla_v2_shape, "H=128 MLA kernel shape: 10 * waves + head blocks per wave");
-  m.def("skinny_gemm", &skinny_gemm);
+  m.def("skinny_gemm", &skinny_gemm, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("rb"), py::arg("nsplit"), py::arg("occ"),
+        py::arg("part"), py::arg("relu2") = false);
   m.def("skinny_supported", &skinny_supported);
-  m.def("mgemm", &mgemm);
+  m.def("mgemm", &mgemm, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("wrb"), py::arg("nsplit"), py::arg("stages"),
+        py::arg("part"), py::arg("relu2") = false);
   m.def("mgemm_partials", &mgemm_partials, "split-K partials of the medium-M GEMM (no reduce); returns nsplit");
   m.def("reduce_rope_cache", &reduce_rope_cache, "QKV split-K reduce + RoPE + paged cache write");
   m.def("mgemm_add_rmsnorm", &mgemm_add_rmsnorm, "decode o / down projection with residual-add + RMSNorm in its split-K reduce");
   m.def("pgemm_fp8", &pgemm_fp8, "prefill fp8 W8A8 GEMM (256x256 LDS-DMA tiles on 16x16x128 f8f6f4 MFMA), "
         "per-token x per-channel scales, optional fused SiLU-and-mul");
   m.def("tgemm", &tgemm, "bf16 GEMM of prompt-sized steps on the tile that fits, or None", py::arg("x"), py::arg("w"),
-        py::arg("bias") = std::nullopt, py::arg("silu") = 0, py::arg("tile") = 0);
+        py::arg("bias") = std::nullopt, py::arg("act") = 0, py::arg("tile") = 0);
   m.def("tgemm_plan", &llmd_tgemm_plan, "tile of tgemm for (M, N, K, silu): mi * 100 + ni * 10 + ranges of K, or 0");
   m.def("fgemm", &fgemm, "fp32 GEMM of prompt-sized steps on the bf16 matrix units, or None", py::arg("x"), py::arg("w"),
         py::arg("bias") = std::nullopt, py::arg("tile") = 0);

@@ -65,7 +65,7 @@ __global__ __launch_bounds__(NT, 1) void mgemm_kernel(const void* __restrict__ x
                                                       int N, int K, int steps_per_split, uint16_t* __restrict__ y,
                                                       int64_t y_stride, float* __restrict__ part,
                                                       const float* __restrict__ xs, const float* __restrict__ wsc,
-                                                      int* __restrict__ cnt) {
+                                                      int* __restrict__ cnt, int relu2) {
   using G = Geo<MB, WRB, S>;
   using E = typename std::conditional<F8, uint8_t, uint16_t>::type;
   constexpr int CE = 16 / sizeof(E);  // elements per 16-B chunk
@@ -294,9 +294,7 @@ __global__ __launch_bounds__(NT, 1) void mgemm_kernel(const void* __restrict__ x
         acc[rb][mb] = v;
       }
       if (whole) {
-        const uint32_t lo = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
-        const uint32_t hi = (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-        *reinterpret_cast<uint2*>(y + (int64_t)m * y_stride + n) = make_uint2(lo, hi);
+        *reinterpret_cast<uint2*>(y + (int64_t)m * y_stride + n) = pack4(v, relu2);
       } else {
         *reinterpret_cast<f32x4_t*>(part + ((int64_t)sp * M + m) * N + n) = v;
       }
@@ -341,16 +339,14 @@ __global__ __launch_bounds__(NT, 1) void mgemm_kernel(const void* __restrict__ x
 }
 
 __global__ __launch_bounds__(256) void mgemm_reduce_kernel(const float* __restrict__ part, int nsplit, int M, int N,
-                                                           uint16_t* __restrict__ y, int64_t y_stride) {
+                                                           uint16_t* __restrict__ y, int64_t y_stride, int relu2) {
   const int64_t i4 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   const int64_t total = (int64_t)M * N;
   if (i4 >= total) return;
   const int m = (int)(i4 / N), n = (int)(i4 % N);
   f32x4_t s = *reinterpret_cast<const f32x4_t*>(part + i4);
   for (int k = 1; k < nsplit; ++k) s += *reinterpret_cast<const f32x4_t*>(part + (int64_t)k * total + i4);
-  const uint32_t lo = (uint32_t)f2bf(s[0]) | ((uint32_t)f2bf(s[1]) << 16);
-  const uint32_t hi = (uint32_t)f2bf(s[2]) | ((uint32_t)f2bf(s[3]) << 16);
-  *reinterpret_cast<uint2*>(y + (int64_t)m * y_stride + n) = make_uint2(lo, hi);
+  *reinterpret_cast<uint2*>(y + (int64_t)m * y_stride + n) = pack4(s, relu2);
 }
 
 // The o / down projection's split-K partials -> y = bf16(sum); residual += y (rounded to bf16);
@@ -427,7 +423,7 @@ __global__ __launch_bounds__(256 * VPT) void mgemm_reduce_norm_kernel(const floa
 }
 
 typedef void (*mkern_t)(const void*, int64_t, const void*, int64_t, int, int, int, int, uint16_t*, int64_t,
-                        float*, const float*, const float*, int*);
+                        float*, const float*, const float*, int*, int);
 
 // X row blocks (16 rows) of the tile for M rows: 64 / 96 / 128 rows as before, and 192 / 256 (the
 // 129-256-row decode batches: 256 in flight, SURVEY K08 "M <= 256"; only 1- and 2-row-block W
@@ -520,10 +516,10 @@ extern "C" int llmd_mgemm_lds(int M, int wrb, int stages) {
 // Y = X W^T, M <= 128, K % 64 == 0, N % 4 == 0; wrb: 64-row W tiles per workgroup
 // (1, 2 or 4), nsplit K splits (part: nsplit * M * N fp32 when > 1), stages 3 or 4.
 // cnt: nullptr = split-K partials summed by mgemm_reduce_kernel; else a zeroed int slab of >= N / (64 wrb)
-// counters for the in-kernel fixup (left zeroed again)
+// counters for the in-kernel fixup (left zeroed again). relu2: max(0, .)^2 of the numbers in bf16
 extern "C" int llmd_mgemm(const void* x, int64_t x_stride, const void* w, int64_t w_stride, int M, int N, int K,
                           int wrb, int nsplit, int stages, void* y, int64_t y_stride, float* part, int* cnt,
-                          hipStream_t st) {
+                          int relu2, hipStream_t st) {
   if (M < 1 || M > 256 || K % 64 != 0 || N % 4 != 0 || nsplit < 1 || x_stride % 8 || w_stride % 8) return -1;
   if (llmd_mgemm_lds(M, wrb, stages) == 0) return -1;
   const int mb = mgemm_mb(M);
@@ -534,13 +530,13 @@ extern "C" int llmd_mgemm(const void* x, int64_t x_stride, const void* w, int64_
   nsplit = (nk + per - 1) / per;  // no empty splits
   const int bn = 64 * wrb;
   dim3 grid((N + bn - 1) / bn, nsplit);
-  if (grid.x % 8) cnt = nullptr;  // the fixup needs every split of a tile on one XCD
+  if (grid.x % 8 || relu2) cnt = nullptr;  // the fixup needs every split of a tile on one XCD
   hipLaunchKernelGGL(k, grid, dim3(NT), 0, st, x, x_stride, w, w_stride, M, N, K, per, (uint16_t*)y, y_stride, part,
-                     (const float*)nullptr, (const float*)nullptr, nsplit > 1 ? cnt : nullptr);
+                     (const float*)nullptr, (const float*)nullptr, nsplit > 1 ? cnt : nullptr, relu2);
   if (nsplit > 1 && cnt == nullptr) {
     const int64_t total4 = (int64_t)M * N / 4;
     hipLaunchKernelGGL(mgemm_reduce_kernel, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, st, part, nsplit,
-                       M, N, (uint16_t*)y, y_stride);
+                       M, N, (uint16_t*)y, y_stride, relu2);
   }
   return (int)hipGetLastError();
 }
@@ -562,7 +558,7 @@ extern "C" int llmd_mgemm_partials(const void* x, int64_t x_stride, const void* 
   const int bn = 64 * wrb;
   dim3 grid((N + bn - 1) / bn, nsplit);
   hipLaunchKernelGGL(k, grid, dim3(NT), 0, st, x, x_stride, w, w_stride, M, N, K, per, (uint16_t*)nullptr,
-                     (int64_t)0, part, (const float*)nullptr, (const float*)nullptr, (int*)nullptr);
+                     (int64_t)0, part, (const float*)nullptr, (const float*)nullptr, (int*)nullptr, 0);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? nsplit : -(int)e - 100;
 }
@@ -588,7 +584,7 @@ extern "C" int llmd_mgemm_add_rmsnorm(const void* x, int64_t x_stride, const voi
   const int bn = 64 * wrb;
   dim3 grid((N + bn - 1) / bn, nsplit);
   hipLaunchKernelGGL(k, grid, dim3(NT), 0, st, x, x_stride, w, w_stride, M, N, K, per, (uint16_t*)out, out_stride,
-                     part, (const float*)nullptr, (const float*)nullptr, (int*)nullptr);
+                     part, (const float*)nullptr, (const float*)nullptr, (int*)nullptr, 0);
   const int vpt = (N / 8 + 255) / 256;  // the unfused norm's chunks per thread (its launch rounds to 1, 2, 4)
 #define RN(V)                                                                                                   \
   hipLaunchKernelGGL((mgemm_reduce_norm_kernel<V>), dim3(M), dim3(256 * V), 0, st, (const float*)part, nsplit, M, \
@@ -617,11 +613,11 @@ extern "C" int llmd_mgemm_fp8(const void* x, int64_t x_stride, const float* xs, 
   dim3 grid((N + bn - 1) / bn, nsplit);
   if (grid.x % 8) cnt = nullptr;
   hipLaunchKernelGGL(k, grid, dim3(NT), 0, st, x, x_stride, w, w_stride, M, N, K, per, (uint16_t*)y, y_stride, part,
-                     xs, ws, nsplit > 1 ? cnt : nullptr);
+                     xs, ws, nsplit > 1 ? cnt : nullptr, 0);
   if (nsplit > 1 && cnt == nullptr) {
     const int64_t total4 = (int64_t)M * N / 4;
     hipLaunchKernelGGL(mgemm_reduce_kernel, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, st, part, nsplit,
-                       M, N, (uint16_t*)y, y_stride);
+                       M, N, (uint16_t*)y, y_stride, 0);
   }
   return (int)hipGetLastError();
 }
@@ -640,6 +636,6 @@ extern "C" int llmd_mgemm_silu(const void* x, int64_t x_stride, const void* w, i
   const int bn = 64 * wrb;
   dim3 grid((N + bn - 1) / bn, 1);
   hipLaunchKernelGGL(k, grid, dim3(NT), 0, st, x, x_stride, w, w_stride, M, N, K, K / 64, (uint16_t*)y, y_stride,
-                     (float*)nullptr, (const float*)nullptr, (const float*)nullptr, (int*)nullptr);
+                     (float*)nullptr, (const float*)nullptr, (const float*)nullptr, (int*)nullptr, 0);
   return (int)hipGetLastError();
 }

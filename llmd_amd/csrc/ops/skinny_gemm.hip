@@ -15,7 +15,7 @@
 // again in 4 and are summed through LDS at the end (a 2-level tree), so every
 // wave streams whole 32-k steps of all RB row blocks. Loads run one chunk of U
 // k-steps ahead in two statically indexed register sets.
-// Epilogue: bf16 rows when the K range is whole (gridDim.y == 1), else fp32
+// Epilogue (relu2: the rows' max(0, .)^2, of the numbers in bf16): bf16 rows when the K range is whole (gridDim.y == 1), else fp32
 // partials [split][M][N] summed and rounded by dgemm_reduce_kernel.
 #include "llmd_common.h"
 
@@ -30,7 +30,7 @@ __global__ __launch_bounds__(NT, OCC) void dgemm_kernel(const uint16_t* __restri
                                                         const uint16_t* __restrict__ wt, int64_t w_stride,
                                                         int M, int N, int K, int nquad_split,
                                                         uint16_t* __restrict__ y, int64_t y_stride,
-                                                        float* __restrict__ part) {
+                                                        float* __restrict__ part, int relu2) {
   __shared__ __attribute__((aligned(16))) f32x4_t red[2][RB][MB][64];
   const int tile = blockIdx.x, sp = blockIdx.y, nsplit = gridDim.y;
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
@@ -165,9 +165,7 @@ __global__ __launch_bounds__(NT, OCC) void dgemm_kernel(const uint16_t* __restri
       const int n = row0 + 16 * rb + 4 * g;
       if (n >= N) continue;  // N % 4 == 0 (host check): all 4 in or all out
       if (nsplit == 1) {
-        const uint32_t lo = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
-        const uint32_t hi = (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-        *reinterpret_cast<uint2*>(y + (int64_t)m * y_stride + n) = make_uint2(lo, hi);
+        *reinterpret_cast<uint2*>(y + (int64_t)m * y_stride + n) = pack4(v, relu2);
       } else {
         *reinterpret_cast<f32x4_t*>(part + ((int64_t)sp * M + m) * N + n) = v;
       }
@@ -176,16 +174,14 @@ __global__ __launch_bounds__(NT, OCC) void dgemm_kernel(const uint16_t* __restri
 }
 
 __global__ __launch_bounds__(256) void dgemm_reduce_kernel(const float* __restrict__ part, int nsplit, int M, int N,
-                                                           uint16_t* __restrict__ y, int64_t y_stride) {
+                                                           uint16_t* __restrict__ y, int64_t y_stride, int relu2) {
   const int64_t i4 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   const int64_t total = (int64_t)M * N;
   if (i4 >= total) return;
   const int m = (int)(i4 / N), n = (int)(i4 % N);  // N % 4 == 0: the 4 stay in one row
   f32x4_t s = *reinterpret_cast<const f32x4_t*>(part + i4);
   for (int k = 1; k < nsplit; ++k) s += *reinterpret_cast<const f32x4_t*>(part + (int64_t)k * total + i4);
-  const uint32_t lo = (uint32_t)f2bf(s[0]) | ((uint32_t)f2bf(s[1]) << 16);
-  const uint32_t hi = (uint32_t)f2bf(s[2]) | ((uint32_t)f2bf(s[3]) << 16);
-  *reinterpret_cast<uint2*>(y + (int64_t)m * y_stride + n) = make_uint2(lo, hi);
+  *reinterpret_cast<uint2*>(y + (int64_t)m * y_stride + n) = pack4(s, relu2);
 }
 
 // register budget per lane: the two chunk sets (2 U steps x 2 loads x (RB + MB)
@@ -198,7 +194,7 @@ constexpr bool fits(int rb, int mb, int u, int occ) {
 constexpr int pick_u(int rb, int mb, int occ) { return fits(rb, mb, 2, occ) ? 2 : (fits(rb, mb, 1, occ) ? 1 : 0); }
 
 typedef void (*kern_t)(const uint16_t*, int64_t, const uint16_t*, int64_t, int, int, int, int, uint16_t*, int64_t,
-                       float*);
+                       float*, int);
 
 template <int RB, int MB>
 kern_t pick(int occ) {
@@ -245,7 +241,7 @@ extern "C" int llmd_dgemm_supported(int M, int rb, int occ) {
 // K splits, occ workgroups per CU. part: nsplit * M * N fp32 when nsplit > 1.
 extern "C" int llmd_skinny_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_stride, int M, int N,
                                 int K, int rb, int nsplit, int occ, void* y, int64_t y_stride, float* part,
-                                hipStream_t st) {
+                                int relu2, hipStream_t st) {
   if (M < 1 || M > 64 || K % 256 != 0 || N % 4 != 0 || nsplit < 1 || !llmd_dgemm_supported(M, rb, occ)) return -1;
   const int nq = K / 256;
   const int per = (nq + nsplit - 1) / nsplit;
@@ -255,11 +251,11 @@ extern "C" int llmd_skinny_gemm(const void* x, int64_t x_stride, const void* w, 
   if (k == nullptr) return -2;
   dim3 grid((N + 16 * rb - 1) / (16 * rb), nsplit);
   hipLaunchKernelGGL(k, grid, dim3(NT), 0, st, (const uint16_t*)x, x_stride, (const uint16_t*)w, w_stride, M, N, K,
-                     per, (uint16_t*)y, y_stride, part);
+                     per, (uint16_t*)y, y_stride, part, relu2);
   if (nsplit > 1) {
     const int64_t total4 = (int64_t)M * N / 4;
     hipLaunchKernelGGL(dgemm_reduce_kernel, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, st, part, nsplit,
-                       M, N, (uint16_t*)y, y_stride);
+                       M, N, (uint16_t*)y, y_stride, relu2);
   }
   return (int)hipGetLastError();
 }

@@ -1,5 +1,5 @@
 // Dense bf16 GEMM of prompt-sized steps with a tile for every size: C[M, N] = A[M, K] . W[N, K]^T (+ bias), or
-// silu(gate) * up of W = [gate; up]. pgemm.hip's 256 x 256 tiles leave CUs idle wherever their number is not a little
+// silu(gate) * up of W = [gate; up], or max(0, C)^2. pgemm.hip's 256 x 256 tiles leave CUs idle wherever their number is not a little
 // below a multiple of 256; here a tile is 32 MI x 32 NI (64 x 64 .. 256 x 256), chosen so that the tiles fill whole
 // rounds of the chip (tgemm_plan below).
 //
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(NT, 1) void tgemm_kernel(const uint16_t* __restrict
                                                       const uint16_t* __restrict__ W, int64_t ldw,
                                                       uint16_t* __restrict__ C, int64_t ldc, int M, int N, int K,
                                                       const uint16_t* __restrict__ bias, int nsplit,
-                                                      int rounded, float* __restrict__ ws) {
+                                                      int form, float* __restrict__ ws) {
   constexpr int ST = stages(MI, NI), D = MI + NI, R = MI + NI, T = MI * NI;
   constexpr int STG = 4096 * (MI + NI), OPW = 4096 * MI;
   constexpr int BM = 32 * MI, BN = 32 * NI;
@@ -229,10 +229,7 @@ __global__ __launch_bounds__(NT, 1) void tgemm_kernel(const uint16_t* __restrict
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] += __uint_as_float(e & 1 ? q[e >> 1] & 0xffff0000u : q[e >> 1] << 16);
         }
-        u32x2_t p;
-        p[0] = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
-        p[1] = (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-        *reinterpret_cast<u32x2_t*>(img + (16 * i + fr) * PITCH + 32 * j + 8 * fq) = p;
+        *reinterpret_cast<uint2*>(img + (16 * i + fr) * PITCH + 32 * j + 8 * fq) = pack4(v, form);
       }
   } else {
 #pragma unroll
@@ -244,7 +241,7 @@ __global__ __launch_bounds__(NT, 1) void tgemm_kernel(const uint16_t* __restrict
       for (int e = 0; e < 4; ++e) {
         const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[e]), __float_as_uint(y[e]), false, false);
         float g = __uint_as_float(s[0]), u = __uint_as_float(s[1]);
-        if (rounded) g = __uint_as_float((uint32_t)f2bf(g) << 16), u = __uint_as_float((uint32_t)f2bf(u) << 16);
+        if (form) g = __uint_as_float((uint32_t)f2bf(g) << 16), u = __uint_as_float((uint32_t)f2bf(u) << 16);
         o[e] = g / (1.f + __expf(-g)) * u;
       }
       u32x2_t p;
@@ -269,7 +266,7 @@ __global__ __launch_bounds__(NT, 1) void tgemm_kernel(const uint16_t* __restrict
 // C = the ranges' sums in their order; a thread per 8 columns of a row
 __global__ __launch_bounds__(256) void tgemm_reduce_kernel(const float* __restrict__ ws, int nsplit, int M, int N,
                                                            const uint16_t* __restrict__ bias,
-                                                           uint16_t* __restrict__ C, int64_t ldc) {
+                                                           uint16_t* __restrict__ C, int64_t ldc, int relu2) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x, cols = N / 8;
   if (t >= M * cols) return;
   const int m = (int)(t / cols), n = (int)(t % cols) * 8;
@@ -288,6 +285,10 @@ __global__ __launch_bounds__(256) void tgemm_reduce_kernel(const float* __restri
     unpack8(*reinterpret_cast<const u32x4_t*>(bias + n), g);
 #pragma unroll
     for (int e = 0; e < 8; ++e) f[e] += g[e];
+  }
+  if (relu2) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = relu2_bf(f[e]);
   }
   *reinterpret_cast<u32x4_t*>(C + m * ldc + n) = pack8(f);
 }
@@ -353,14 +354,16 @@ extern "C" int llmd_tgemm_plan(int M, int N, int K, int silu) {
   return code;
 }
 
-// A tile of llmd_tgemm_plan. N: columns of C; W [N, K], with silu [2 N, K] (gate rows, then up rows); 1: of the fp32 sums, 2: of the
-// sums rounded to bf16, as a pass of its own would find them. bias: [N] or null (no silu).
-// ranges > 1 (no silu): sums in ws [ranges, M, N]. -1: not taken.
+// A tile of llmd_tgemm_plan. N: columns of C; W [N, K], with act 1 and 2 [2 N, K]. act 0: none, 1: silu of gate (the first N rows of W)
+// times up (the others), 2: the same of the sums rounded to bf16, as a pass of its own would find them, 3: max(0, .)^2 of the sums rounded
+// to bf16. bias: [N] or null (no silu).
+// Ranges > 1 (no silu): sums in ws [ranges, M, N]. -1: not taken.
 extern "C" int llmd_tgemm(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N,
-                          int K, int silu, int code, const void* bias, void* ws, hipStream_t st) {
+                          int K, int act, int code, const void* bias, void* ws, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
   const int mi = code / 100, ni = code / 10 % 10, nsplit = code % 10;
-  if (N % 8 || K % BK || K <= 0 || lda % 8 || ldw % 8 || ldc % 8 || silu < 0 || silu > 2) return -1;
+  if (N % 8 || K % BK || K <= 0 || lda % 8 || ldw % 8 || ldc % 8 || act < 0 || act > 3) return -1;
+  const bool silu = act == 1 || act == 2;
   const int nk = K / BK;
   if (nsplit < 1 || nsplit > nk || (nsplit - 1) * ((nk + nsplit - 1) / nsplit) >= nk) return -1;
   if ((nsplit > 1 && (silu || ws == nullptr)) || (bias != nullptr && silu)) return -1;
@@ -371,10 +374,10 @@ extern "C" int llmd_tgemm(const void* A, int64_t lda, const void* W, int64_t ldw
   const auto launch = [&](auto kernel) {
     const int64_t grid = (int64_t)((M + 32 * mi - 1) / (32 * mi)) * ((N + tc - 1) / tc) * nsplit;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NT), 0, st, (const uint16_t*)A, lda, (const uint16_t*)W, ldw,
-                       (uint16_t*)C, ldc, M, N, K, (const uint16_t*)bias, nsplit, silu == 2, (float*)ws);
+                       (uint16_t*)C, ldc, M, N, K, (const uint16_t*)bias, nsplit, act >= 2, (float*)ws);
     if (nsplit > 1)
       hipLaunchKernelGGL(tgemm_reduce_kernel, dim3((unsigned)(((int64_t)M * (N / 8) + 255) / 256)), dim3(256), 0, st,
-                         (const float*)ws, nsplit, M, N, (const uint16_t*)bias, (uint16_t*)C, ldc);
+                         (const float*)ws, nsplit, M, N, (const uint16_t*)bias, (uint16_t*)C, ldc, act == 3);
     return (int)hipGetLastError();
   };
 #define T_CASE(MI, NI)                                                              \

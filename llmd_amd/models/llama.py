@@ -42,7 +42,7 @@ class LlamaMLP(torch.nn.Module):
             # chip (csrc/ops/tgemm.hip) where these take less time than the 256 x 256 ones, which run (csrc/ops/pgemm.hip
             # EPI_SILU_STD) where the shipped table has it ahead of hipBLASLt + the act kernel
             v = ops.pgemm_silu_plan(x, gu.weight)
-            y = ops.tgemm(x, gu.weight, silu=1 if v == 6 else 2) if x.shape[0] > 256 else None
+            y = ops.tgemm(x, gu.weight, act=1 if v == 6 else 2) if x.shape[0] > 256 else None
             if y is not None:
                 return y
             if v is not None:

@@ -52,6 +52,7 @@ import math
 import torch
 import torch.nn.functional as F
 
+from llmd_amd import ops
 from llmd_amd.engine.attn_meta import AttnMeta
 from llmd_amd.ops import seqmix as sm
 
@@ -712,7 +713,9 @@ class SquaredReluMLP(torch.nn.Module):
         self.down = ColumnLinear(ff, d_model, shard=False, device=device, dtype=dtype)
 
     def forward(self, h):
-        return self.down(sm.relu2(self.up(h)))
+        up = self.up
+        z = ops.linear_relu2(h, up.weight) if up.weight.dtype == torch.bfloat16 and up.lora is None and up.bias is None else None
+        return self.down(sm.relu2(up(h)) if z is None else z)
 
 
 class ShortConv(torch.nn.Module):

@@ -1184,13 +1184,14 @@ def skinny_plan(M: int, N: int, K: int, num_cus: int = _NUM_CUS) -> tuple[int, i
 SKINNY_TUNED: dict[tuple[int, int, int], tuple[int, int, int]] = {}
 
 
-def skinny_gemm(x: torch.Tensor, w: torch.Tensor, plan: Optional[tuple[int, int, int]] = None) -> torch.Tensor:
+def skinny_gemm(x: torch.Tensor, w: torch.Tensor, plan: Optional[tuple[int, int, int]] = None,
+                relu2: bool = False) -> torch.Tensor:
     M, K = x.shape
     N = w.shape[0]
     rb, ns, occ = plan or skinny_plan(M, N, K)
     y = torch.empty(M, N, dtype=x.dtype, device=x.device)
     part = torch.empty(ns * M * N if ns > 1 else 0, dtype=torch.float32, device=x.device)
-    native().skinny_gemm(y, x, w, rb, ns, occ, part)
+    native().skinny_gemm(y, x, w, rb, ns, occ, part, relu2)
     return y
 
 
@@ -1217,16 +1218,16 @@ def dgemm_choice(M: int, N: int, K: int) -> Optional[tuple[int, int, int]]:
     return None
 
 
-def mgemm(x: torch.Tensor, w: torch.Tensor, plan: tuple[int, int, int]) -> torch.Tensor:
+def mgemm(x: torch.Tensor, w: torch.Tensor, plan: tuple[int, int, int], relu2: bool = False) -> torch.Tensor:
     """Y = X W^T for up to 256 rows on the LDS-DMA medium-M decode GEMM
     (csrc/ops/mgemm.hip, made for 33 and more: fewer fill a block of 32); plan = (wrb: 64-row W tiles per workgroup, nsplit,
-    stages)."""
+    stages). relu2: max(0, .)^2 of the numbers in bf16."""
     M, K = x.shape
     N = w.shape[0]
     wrb, ns, stages = plan
     y = torch.empty(M, N, dtype=x.dtype, device=x.device)
     part = torch.empty(ns * M * N if ns > 1 else 0, dtype=torch.float32, device=x.device)
-    native().mgemm(y, x, w, wrb, ns, stages, part)
+    native().mgemm(y, x, w, wrb, ns, stages, part, relu2)
     return y
 
 
@@ -1375,13 +1376,13 @@ def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
             and torch._C._len_torch_function_stack() == 0)
 
 
-def tgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, silu: int = 0):
-    """x w^T (+ bias), or silu(x wg^T) * (x wu^T) for w = [gate; up] (1: of the fp32 sums as ``pgemm_silu`` variant 6, 2: of the
-    sums in bf16, the bits of ``linear`` + ``gated_act``), on the GEMM whose tile fits the sizes
-    (csrc/ops/tgemm.hip, which holds the rule), or None where it is not taken."""
+def tgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act: int = 0):
+    """x w^T (+ bias) on the GEMM whose tile fits the sizes (csrc/ops/tgemm.hip, which holds the rule), or None where it is not taken.
+    act: silu(x wg^T) * (x wu^T) for w = [gate; up], 1: of the fp32 sums as ``pgemm_silu`` variant 6, 2: of the sums in bf16, the bits
+    of ``linear`` + ``gated_act``; 3: max(0, x w^T)^2 of the sums in bf16."""
     if PGEMM_AUTO == "0" or not _gpu(x) or not _plain(x, w):
         return None
-    return native().tgemm(x, w, bias, silu)
+    return native().tgemm(x, w, bias, act)
 
 
 def fgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None):
@@ -1540,6 +1541,29 @@ def _listed(M: int, N: int, K: int) -> bool:
     return (m, N, K) in DGEMM_TABLE or (M >= 33 and (64, N, K) in MGEMM_TABLE)
 
 
+def _unlisted_rule(x: torch.Tensor, w: torch.Tensor):
+    M = x.shape[0] if x.dim() == 2 else 0
+    if (1 <= M <= 64 and mgemm_ok(x, w) and not _listed(M, w.shape[0], w.shape[1]) and x.data_ptr() % 16 == 0
+            and w.data_ptr() % 16 == 0):
+        return decode_rule(M, w.shape[0], w.shape[1])
+    return None
+
+
+def linear_relu2(x: torch.Tensor, w: torch.Tensor):
+    """max(0, x w^T)^2 in the product's epilogue, the bits of ``linear`` and a pass of its own (relu2: 2048 x 5632 8 us, 9 rows 4.8),
+    or None where ``linear`` takes a kernel without it."""
+    if x.dim() != 2 or not _gpu(x) or not _SKINNY:
+        return None
+    if x.shape[0] <= 64:
+        rule = _unlisted_rule(x, w)
+        return None if rule is None else rule[0](x, w, rule[1], True)
+    M, (N, K) = x.shape[0], w.shape
+    if (PGEMM_AUTO == "measure" or (M <= 256 and mgemm_choice(M, N, K) is not None)
+            or (M >= PGEMM_MIN_M and pgemm_plan(M, N, K) is not None)):
+        return None
+    return tgemm(x, w, None, 3)
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Dense projection: decode-sized M on our decode GEMM kernels where their
     measured dispatch tables have them ahead of hipBLASLt - the medium-M LDS-DMA
@@ -1566,11 +1590,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
             if plan is not None:
                 y = skinny_gemm(x, w, plan)
                 return y if bias is None else y.add_(bias)
-        if bias is None and 1 <= M <= 64 and mgemm_ok(x, w) and not _listed(M, w.shape[0], w.shape[1]) and \
-                x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
-            rule = decode_rule(M, w.shape[0], w.shape[1])
-            if rule is not None:
-                return rule[0](x, w, rule[1])
+        rule = _unlisted_rule(x, w) if bias is None else None
+        if rule is not None:
+            return rule[0](x, w, rule[1])
     if x.dim() == 2 and x.shape[0] > 64:
         y = fgemm(x, w, bias) if x.dtype == torch.float32 else tgemm(x, w, bias)
         if y is not None:

@@ -88,3 +88,15 @@ def test_cpu_tensors_stay_with_the_library():
     x, w = torch.randn(130, 64).bfloat16(), torch.randn(16, 64).bfloat16()
     assert ops.tgemm(x, w) is None
     assert torch.equal(ops.linear(x, w), torch.nn.functional.linear(x, w))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 5632, 2048), (9, 2048, 1024), (16, 1024, 8192), (17, 5632, 2048), (64, 768, 4096), (65, 5632, 2048),
+                                   (700, 2048, 5632), (256, 1024, 16384)])
+def test_squared_relu_in_the_epilogue(M, N, K):
+    """Every kernel that ops.linear takes for these sizes, with one range of K and several: the bits of the two passes."""
+    from llmd_amd.ops import seqmix as sm
+
+    x, w = _operands(M, N, K)
+    y = ops.linear_relu2(x, w)
+    assert y is not None and torch.equal(y, sm.relu2(ops.linear(x, w)))
