@@ -22,8 +22,8 @@ void llmd_layer_norm(void*, int64_t, void*, int64_t, void*, int64_t, const void*
 void llmd_fused_add_rms_norm(void*, int64_t, void*, int64_t, const void*, int, int, float,
                              hipStream_t);
 int llmd_qk_rms_norm(void*, int64_t, const void*, const void*, int, int, int, int, float, hipStream_t);
-void llmd_rope_cache(void*, int64_t, const int64_t*, const float*, int, int, int, int,
-                     const int64_t*, void*, void*, int64_t, int, int, int, int, float, float, hipStream_t);
+int llmd_rope_cache(void*, int64_t, const int64_t*, const float*, int, int, int, int, const int64_t*, void*, void*, int64_t,
+                    int, int, int, int, float, float, const void*, const void*, float, hipStream_t);
 void llmd_gated_act(void*, int64_t, const void*, int64_t, int, int, int, float, float, hipStream_t);
 int llmd_paged_decode(const void*, int64_t, const void*, const void*, int64_t, int, const int*, int,
                       const int*, int, int, int, int, float, int, const float*, int, int, void*,
@@ -61,7 +61,8 @@ int llmd_mgemm(const void*, int64_t, const void*, int64_t, int, int, int, int, i
 int llmd_mgemm_lds(int, int, int);
 int llmd_mgemm_partials(const void*, int64_t, const void*, int64_t, int, int, int, int, int, int, float*, hipStream_t);
 int llmd_reduce_rope_cache(const float*, int, int, void*, int64_t, const int64_t*, const float*, int, int, int, int,
-                           const int64_t*, void*, void*, int64_t, int, int, int, int, float, float, hipStream_t);
+                           const int64_t*, void*, void*, int64_t, int, int, int, int, float, float, const void*, const void*,
+                           float, hipStream_t);
 int llmd_mgemm_add_rmsnorm(const void*, int64_t, const void*, int64_t, int, int, int, int, int, int, float*, void*,
                            int64_t, const void*, float, void*, int64_t, hipStream_t);
 int llmd_mgemm_silu(const void*, int64_t, const void*, int64_t, int, int, int, int, int, void*, int64_t, hipStream_t);
@@ -225,11 +226,25 @@ bool is_fp8_cache(const torch::Tensor& c) {
   return t == at::kFloat8_e4m3fn;
 }
 
+// Norm weights of the heads of q and k, [D], both or neither
+std::pair<const void*, const void*> qk_weights(const c10::optional<torch::Tensor>& qw, const c10::optional<torch::Tensor>& kw,
+                                               int64_t D, int rot, bool neox) {
+  TORCH_CHECK(qw.has_value() == kw.has_value(), "q and k norm weights: both or neither");
+  if (!qw.has_value()) return {nullptr, nullptr};
+  CHECK_CUDA(*qw); CHECK_BF16(*qw); CHECK_CUDA(*kw); CHECK_BF16(*kw);
+  TORCH_CHECK(qw->numel() == D && kw->numel() == D && qw->is_contiguous() && kw->is_contiguous() &&
+                  (uintptr_t)qw->data_ptr() % 16 == 0 && (uintptr_t)kw->data_ptr() % 16 == 0 && neox && rot == D &&
+                  (D == 64 || D == 128 || D == 256),
+              "q and k norm weights: [D], on 16 bytes, heads of 64, 128 or 256 that are rotated whole and in halves");
+  return {qw->data_ptr(), kw->data_ptr()};
+}
+
 // qkv [T, (Hq+2Hkv)*D]; k_cache/v_cache: per-layer strided views
 // [num_blocks, Hkv, bs, D] (block stride arbitrary, inner [Hkv,bs,D] contiguous)
 void rope_cache(torch::Tensor qkv, torch::Tensor positions, torch::Tensor cos_sin, int64_t Hq,
                 int64_t Hkv, int64_t D, torch::Tensor slots, torch::Tensor k_cache,
-                torch::Tensor v_cache, bool neox, double k_scale, double v_scale) {
+                torch::Tensor v_cache, bool neox, double k_scale, double v_scale, c10::optional<torch::Tensor> qw,
+                c10::optional<torch::Tensor> kw, double eps) {
   const c10::hip::OptionalHIPGuard device_guard(dev_of(qkv));
   CHECK_CUDA(qkv); CHECK_BF16(qkv); CHECK_INNER(qkv);
   CHECK_DT(positions, at::kLong); CHECK_DT(slots, at::kLong); CHECK_DT(cos_sin, at::kFloat);
@@ -248,17 +263,21 @@ void rope_cache(torch::Tensor qkv, torch::Tensor positions, torch::Tensor cos_si
               "k_cache inner layout");
   TORCH_CHECK(v_cache.sizes() == k_cache.sizes() && v_cache.strides() == k_cache.strides(),
               "v_cache layout");
-  llmd_rope_cache(qkv.data_ptr(), qkv.stride(0), positions.data_ptr<int64_t>(),
-                  cos_sin.data_ptr<float>(), rot, Hq, Hkv, D, slots.data_ptr<int64_t>(),
-                  k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0), k_cache.size(2), T,
-                  neox ? 1 : 0, f8 ? 1 : 0, (float)(1.0 / k_scale), (float)(1.0 / v_scale), cur_stream());
+  const auto nw = qk_weights(qw, kw, D, rot, neox);
+  const int rc = llmd_rope_cache(qkv.data_ptr(), qkv.stride(0), positions.data_ptr<int64_t>(),
+                                 cos_sin.data_ptr<float>(), rot, Hq, Hkv, D, slots.data_ptr<int64_t>(),
+                                 k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0), k_cache.size(2), T,
+                                 neox ? 1 : 0, f8 ? 1 : 0, (float)(1.0 / k_scale), (float)(1.0 / v_scale), nw.first,
+                                 nw.second, (float)eps, cur_stream());
+  TORCH_CHECK(rc == 0, "rope_cache failed: ", rc);
 }
 
 // The decode QKV projection's split-K partials (mgemm_partials) reduced, rotated and written to the paged
 // cache in one kernel: qkv [T, W] receives the projection (Q rotated), K / V go to the cache.
 void reduce_rope_cache(torch::Tensor part, int64_t nsplit, torch::Tensor qkv, torch::Tensor positions,
                        torch::Tensor cos_sin, int64_t Hq, int64_t Hkv, int64_t D, torch::Tensor slots,
-                       torch::Tensor k_cache, torch::Tensor v_cache, bool neox, double k_scale, double v_scale) {
+                       torch::Tensor k_cache, torch::Tensor v_cache, bool neox, double k_scale, double v_scale,
+                       c10::optional<torch::Tensor> qw, c10::optional<torch::Tensor> kw, double eps) {
   const c10::hip::OptionalHIPGuard device_guard(dev_of(qkv));
   CHECK_CUDA(qkv); CHECK_BF16(qkv); CHECK_INNER(qkv); CHECK_DT(part, at::kFloat);
   CHECK_DT(positions, at::kLong); CHECK_DT(slots, at::kLong); CHECK_DT(cos_sin, at::kFloat);
@@ -274,11 +293,12 @@ void reduce_rope_cache(torch::Tensor part, int64_t nsplit, torch::Tensor qkv, to
   TORCH_CHECK(k_cache.dim() == 4 && k_cache.size(1) == Hkv && k_cache.size(3) == D &&
               k_cache.stride(3) == 1 && k_cache.stride(2) == D && k_cache.stride(1) == k_cache.size(2) * D &&
               v_cache.sizes() == k_cache.sizes() && v_cache.strides() == k_cache.strides(), "k/v cache layout");
+  const auto nw = qk_weights(qw, kw, D, rot, neox);
   int rc = llmd_reduce_rope_cache(part.data_ptr<float>(), (int)nsplit, W, qkv.data_ptr(), qkv.stride(0),
                                   positions.data_ptr<int64_t>(), cos_sin.data_ptr<float>(), rot, Hq, Hkv, D,
                                   slots.data_ptr<int64_t>(), k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
                                   k_cache.size(2), T, neox ? 1 : 0, f8 ? 1 : 0, (float)(1.0 / k_scale),
-                                  (float)(1.0 / v_scale), cur_stream());
+                                  (float)(1.0 / v_scale), nw.first, nw.second, (float)eps, cur_stream());
   TORCH_CHECK(rc == 0, "reduce_rope_cache failed: ", rc);
 }
 
@@ -1390,7 +1410,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_debug (llmd_amd/build.p
   m.def("fused_add_rms_norm", &fused_add_rms_norm);
   m.def("qk_rms_norm", &qk_rms_norm, "Qwen3 per-head q/k RMSNorm in place in the fused QKV output");
   m.def("layer_norm", &layer_norm);
-  m.def("rope_cache", &rope_cache);
+  m.def("rope_cache", &rope_cache, py::arg("qkv"), py::arg("positions"), py::arg("cos_sin"), py::arg("Hq"), py::arg("Hkv"), py::arg("D"), py::arg("slots"),
+        py::arg("k_cache"), py::arg("v_cache"), py::arg("neox"), py::arg("k_scale"), py::arg("v_scale"), py::arg("qw") = py::none(),
+        py::arg("kw") = py::none(), py::arg("eps") = 0.0);
   m.def("gated_act", &gated_act);
   m.def("paged_decode", &paged_decode);
   m.def("paged_prefill", &paged_prefill);
@@ -1414,7 +1436,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_debug (llmd_amd/build.p
   m.def("mgemm", &mgemm, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("wrb"), py::arg("nsplit"), py::arg("stages"),
         py::arg("part"), py::arg("relu2") = false);
   m.def("mgemm_partials", &mgemm_partials, "split-K partials of the medium-M GEMM (no reduce); returns nsplit");
-  m.def("reduce_rope_cache", &reduce_rope_cache, "QKV split-K reduce + RoPE + paged cache write");
+  m.def("reduce_rope_cache", &reduce_rope_cache, "QKV split-K reduce + RoPE + paged cache write", py::arg("part"), py::arg("nsplit"),
+        py::arg("qkv"), py::arg("positions"), py::arg("cos_sin"), py::arg("Hq"), py::arg("Hkv"), py::arg("D"), py::arg("slots"),
+        py::arg("k_cache"), py::arg("v_cache"), py::arg("neox"), py::arg("k_scale"), py::arg("v_scale"), py::arg("qw") = py::none(),
+        py::arg("kw") = py::none(), py::arg("eps") = 0.0);
   m.def("mgemm_add_rmsnorm", &mgemm_add_rmsnorm, "decode o / down projection with residual-add + RMSNorm in its split-K reduce");
   m.def("pgemm_fp8", &pgemm_fp8, "prefill fp8 W8A8 GEMM (256x256 LDS-DMA tiles on 16x16x128 f8f6f4 MFMA), "
         "per-token x per-channel scales, optional fused SiLU-and-mul");

@@ -68,21 +68,18 @@ class LlamaMLP(torch.nn.Module):
 def qkv_fused_plan(lin, x):
     """Medium-M GEMM plan of the QKV projection when its split-K reduce can be fused with RoPE + the
     cache write (ops.reduce_rope_cache), or None: bf16 weights without bias or LoRA, decode-sized M,
-    a shipped plan that splits K."""
+    a plan that splits K."""
     if (not isinstance(x, torch.Tensor) or lin.bias is not None or lin.lora is not None
             or lin.weight.dtype != torch.bfloat16 or not (ops.MGEMM_NORM and ops._SKINNY)
             or lin.weight.shape[0] > 24576):
         return None
-    if not (x.dim() == 2 and 33 <= x.shape[0] <= 128 and ops.mgemm_ok(x, lin.weight)):
-        return None
-    plan = ops.mgemm_choice(x.shape[0], lin.weight.shape[0], lin.weight.shape[1])
-    return plan if plan is not None and plan[1] >= 2 and lin.weight.shape[1] // 64 >= 2 else None
+    return ops.split_plan(x, lin.weight)
 
 
 def norm_fused_plan(lin, x):
     """Medium-M GEMM plan for ``lin(x)`` with the following residual-add + RMSNorm fused into its
     split-K reduce (ops.mgemm_add_rmsnorm), or None: bf16 TP1 row-parallel linears without bias or
-    LoRA at decode-sized M (33..128) whose shipped plan splits K."""
+    LoRA at decode-sized M (up to 128) whose plan splits K."""
     if (not isinstance(x, torch.Tensor) or lin.bias is not None or lin.lora is not None
             or lin.weight.dtype != torch.bfloat16 or (lin.reduce and get_state().tp_size > 1)):
         return None
@@ -111,10 +108,6 @@ class LlamaDecoderLayer(torch.nn.Module):
     def _make_mlp(self, cfg, idx, device):
         return LlamaMLP(cfg, device)
 
-    def _apply_qk_norm(self, qkv):
-        a = self.attn
-        ops.qk_rms_norm(qkv, self.q_norm.weight, self.k_norm.weight, a.Hq, a.Hkv, self.q_norm.eps)
-
     def forward(self, x, residual, meta: AttnMeta):
         x, residual, _ = self.run(x, residual, meta)
         return x, residual
@@ -136,16 +129,16 @@ class LlamaDecoderLayer(torch.nn.Module):
             x = self.input_layernorm(x, quant=q_in)
         else:
             x, residual = self.input_layernorm(x, residual, quant=q_in)
-        p = None if (self.qk_norm or q_in) else qkv_fused_plan(self.qkv, x)
+        norm = (self.q_norm.weight, self.k_norm.weight, self.q_norm.eps) if self.qk_norm else None
+        p = None if q_in else qkv_fused_plan(self.qkv, x)
+        if p is not None and norm is not None and not ops.rope_norms(norm, self.attn.D, self.attn.cos_sin, self.attn.neox):
+            p = None
         if p is not None:  # decode: the QKV split-K reduce fused with RoPE + the cache write
             parts = ops.mgemm_partials(x, self.qkv.weight, p)
             a = self.attn(torch.empty(x.shape[0], self.qkv.weight.shape[0], dtype=x.dtype, device=x.device), meta,
-                          parts=parts)
+                          parts=parts, qk_norm=norm)
         else:
-            qkv = self.qkv(x)
-            if self.qk_norm:
-                self._apply_qk_norm(qkv)
-            a = self.attn(qkv, meta)
+            a = self.attn(self.qkv(x), meta, qk_norm=norm)
         q_mlp = isinstance(self.mlp, LlamaMLP) and wants_fp8_input(self.mlp.gate_up)
         p = None if q_mlp else norm_fused_plan(self.o_proj, a)
         if p is not None:

@@ -103,9 +103,20 @@ def fused_add_layer_norm(x: torch.Tensor, residual: torch.Tensor, w: torch.Tenso
 
 
 # ---------------------------------------------------------------- rope + cache
+def rope_norms(qk_norm, D: int, cos_sin: torch.Tensor, neox: bool) -> bool:
+    """Whether the rotation's kernels norm these heads themselves."""
+    return neox and cos_sin.shape[1] == D and D in (64, 128, 256) and all(w.data_ptr() % 16 == 0 for w in qk_norm[:2])
+
+
 def rope_cache(qkv, positions, cos_sin, Hq, Hkv, D, slots, k_cache, v_cache, neox=True, k_scale=1.0,
-               v_scale=1.0):
-    """RoPE + paged KV write; bf16 or fp8 e4m3fn caches (fp8 stores x / scale)."""
+               v_scale=1.0, qk_norm=None):
+    """RoPE + paged KV write; bf16 or fp8 e4m3fn caches (fp8 stores x / scale). ``qk_norm`` = (q weights, k weights, eps): ``qk_rms_norm``
+    first, in the same pass where neox rotates whole heads of 64, 128 or 256 (the K columns of qkv then stay as they were)."""
+    if qk_norm is not None:
+        if _gpu(qkv) and rope_norms(qk_norm, D, cos_sin, neox):
+            native().rope_cache(qkv, positions, cos_sin, Hq, Hkv, D, slots, k_cache, v_cache, neox, k_scale, v_scale, *qk_norm)
+            return
+        qk_rms_norm(qkv, qk_norm[0], qk_norm[1], Hq, Hkv, qk_norm[2])
     if not _gpu(qkv):
         ref.rope_cache(qkv, positions, cos_sin, Hq, Hkv, D, slots, k_cache, v_cache, neox, k_scale, v_scale)
         return
@@ -1237,15 +1248,23 @@ MGEMM_NORM = os.environ.get("LLMD_MGEMM_NORM", "1") == "1"
 
 
 def mgemm_norm_plan(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, int, int]]:
-    """The shipped medium-M plan of this projection when it is split over K (so its partials can be
+    """The medium-M plan of this projection when it is split over K (so its partials can be
     reduced together with the residual-add + RMSNorm), else None."""
-    if not (MGEMM_NORM and _SKINNY and x.dim() == 2 and 33 <= x.shape[0] <= 128 and mgemm_ok(x, w)
-            and w.shape[0] % 8 == 0 and w.shape[0] <= 8192 and w.shape[1] >= 128):
+    if not (MGEMM_NORM and w.shape[0] <= 8192):
         return None
-    plan = mgemm_choice(x.shape[0], w.shape[0], w.shape[1])
-    if plan is None or plan[1] < 2:
+    return split_plan(x, w)
+
+
+def split_plan(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, int, int]]:
+    """The plan with which ``linear(x, w)`` runs on the medium-M GEMM with several ranges of K (``mgemm_partials`` of up to 128 rows), of
+    the measured table or the rule on sizes, or None."""
+    if not (_SKINNY and x.dim() == 2 and 1 <= x.shape[0] <= 128 and mgemm_ok(x, w) and w.shape[0] % 8 == 0 and w.shape[1] >= 128):
         return None
-    return plan
+    plan = mgemm_choice(x.shape[0], w.shape[0], w.shape[1]) if x.shape[0] >= 33 else None
+    if plan is None:
+        rule = _unlisted_rule(x, w)
+        plan = rule[1] if rule is not None and rule[0] is mgemm else None
+    return plan if plan is not None and plan[1] >= 2 else None
 
 
 def mgemm_partials(x: torch.Tensor, w: torch.Tensor, plan: tuple[int, int, int]):
@@ -1258,12 +1277,12 @@ def mgemm_partials(x: torch.Tensor, w: torch.Tensor, plan: tuple[int, int, int])
 
 
 def reduce_rope_cache(part: torch.Tensor, nsplit: int, qkv: torch.Tensor, positions, cos_sin, Hq, Hkv, D, slots,
-                      k_cache, v_cache, neox=True, k_scale=1.0, v_scale=1.0):
-    """The QKV projection's split-K reduce + RoPE + paged KV write in one kernel (rope_cache.hip):
-    ``qkv`` [T, W] (allocated, unwritten) receives the projection with Q rotated - bit-identical to
+                      k_cache, v_cache, neox=True, k_scale=1.0, v_scale=1.0, qk_norm=None):
+    """The QKV projection's split-K reduce + RoPE (after the heads' norm, ``rope_norms``) + paged KV write in one kernel
+    (rope_cache.hip): ``qkv`` [T, W] (allocated, unwritten) receives the projection with Q rotated - bit-identical to
     mgemm + rope_cache."""
     native().reduce_rope_cache(part, nsplit, qkv, positions, cos_sin, Hq, Hkv, D, slots, k_cache, v_cache, neox,
-                               k_scale, v_scale)
+                               k_scale, v_scale, *(qk_norm or ()))
 
 
 def mgemm_add_rmsnorm(x: torch.Tensor, w: torch.Tensor, plan: tuple[int, int, int], residual: torch.Tensor,

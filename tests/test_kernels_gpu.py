@@ -59,6 +59,56 @@ def _cache(nblk, Hkv, bs, D, L=1):
     return kv[:, 0, 0], kv[:, 0, 1]
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D", [(1, 32, 4, 128), (64, 32, 4, 128), (37, 9, 3, 128), (9, 16, 2, 64), (3, 5, 1, 64), (5, 8, 8, 256)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_rope_cache_norms_the_heads(T, Hq, Hkv, D, fp8):
+    """The norm inside the rotation's pass, alone and behind the sums over ranges of K: Q and the caches have the bits of qk_rms_norm and
+    a pass of its own; rows without a slot leave the caches alone."""
+    torch.manual_seed(0)
+    K, W = 1024, (Hq + 2 * Hkv) * D
+    x, w = (torch.randn(n, K, device=DEV, dtype=torch.bfloat16) for n in (T, W))
+    part, ns = ops.mgemm_partials(x, w, (1, 2, 4))
+    qkv = ops.mgemm(x, w, (1, 2, 4))
+    norm = (torch.randn(D, device=DEV, dtype=torch.bfloat16), torch.randn(D, device=DEV, dtype=torch.bfloat16), 1e-6)
+    pos, slots = torch.randint(0, 512, (T,), device=DEV), torch.randperm(8 * 16, device=DEV)[:T]
+    slots[T // 2] = -1
+    cs = ops.rope_cos_sin(D, 512, 1e4, device=DEV)
+    got = []
+    for form in range(3):
+        kc, vc = (c.to(torch.float8_e4m3fn if fp8 else torch.bfloat16) for c in _cache(8, Hkv, 16, D))
+        y = torch.empty_like(qkv) if form == 2 else qkv.clone()
+        tail = (pos, cs, Hq, Hkv, D, slots, kc, vc, True, 0.5, 0.25)
+        if form == 0:
+            ops.qk_rms_norm(y, norm[0], norm[1], Hq, Hkv, norm[2])
+            ops.rope_cache(y, *tail)
+        elif form == 1:
+            assert ops.rope_norms(norm, D, cs, True)
+            ops.rope_cache(y, *tail, qk_norm=norm)
+        else:
+            ops.reduce_rope_cache(part, ns, y, *tail, qk_norm=norm)
+        got.append((y[:, : Hq * D], kc.float(), vc.float()))
+    for form in (1, 2):
+        for a, b in zip(got[0], got[form]):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,N,K", [(1, 9216, 4096), (17, 2048, 4096), (64, 2048, 4096), (33, 1024, 8192)])
+def test_norm_behind_the_ranges_of_unlisted_sizes(T, N, K):
+    """A projection that the rule on sizes splits over K, with the residual's norm in the pass over its sums."""
+    torch.manual_seed(0)
+    x, w = torch.randn(T, K, device=DEV, dtype=torch.bfloat16), torch.randn(N, K, device=DEV, dtype=torch.bfloat16) * K ** -0.5
+    r, g = torch.randn(T, N, device=DEV, dtype=torch.bfloat16), torch.randn(N, device=DEV, dtype=torch.bfloat16)
+    y, r1 = ops.linear(x, w), r.clone()
+    ops.fused_add_rms_norm(y, r1, g, 1e-6)
+    plan = ops.split_plan(x, w)
+    assert plan is not None
+    assert (ops.mgemm_norm_plan(x, w) is None) == (N > 8192)
+    if N <= 8192:
+        out = ops.mgemm_add_rmsnorm(x, w, plan, r, g, 1e-6)
+        assert torch.equal(out, y) and torch.equal(r, r1)
+
+
+
 @pytest.mark.parametrize("neox", [True, False])
 @pytest.mark.parametrize("Hq,Hkv,D,rot,bs", [(32, 8, 128, 128, 16), (64, 8, 64, 64, 64), (8, 2, 128, 64, 32)])
 def test_rope_cache(neox, Hq, Hkv, D, rot, bs):
