@@ -58,6 +58,8 @@ int llmd_skinny_gemm(const void*, int64_t, const void*, int64_t, int, int, int, 
 int llmd_dgemm_supported(int, int, int);
 int llmd_mgemm(const void*, int64_t, const void*, int64_t, int, int, int, int, int, int, void*, int64_t, float*,
                int*, int, hipStream_t);
+int llmd_skinny_norm(const void*, int64_t, const void*, int64_t, const void*, float, void*, int64_t, const void*, int64_t, int, int,
+                     int, int, int, void*, int64_t, int, hipStream_t);
 int llmd_mgemm_lds(int, int, int);
 int llmd_mgemm_partials(const void*, int64_t, const void*, int64_t, int, int, int, int, int, int, float*, hipStream_t);
 int llmd_reduce_rope_cache(const float*, int, int, void*, int64_t, const int64_t*, const float*, int, int, int, int,
@@ -489,11 +491,12 @@ void lora_bgmv(torch::Tensor y, torch::Tensor x, torch::Tensor A, torch::Tensor 
 // y [M, N] = x [M, K] . w [N, K]^T for M <= 64 (decode GEMMs): rb row blocks of
 // 16 per workgroup, nsplit-way split-K, occ workgroups per CU (ops.skinny_plan)
 void skinny_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t rb, int64_t nsplit, int64_t occ,
-                 torch::Tensor part, bool relu2) {
+                 torch::Tensor part, int64_t act) {
   const c10::hip::OptionalHIPGuard device_guard(dev_of(y));
   CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_BF16(y); CHECK_INNER(x); CHECK_INNER(w); CHECK_INNER(y);
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && y.dim() == 2, "skinny_gemm: 2-D operands");
-  const int M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(act != 2 || w.size(0) % 2 == 0, "skinny_gemm: [gate; up]");
+  const int M = x.size(0), K = x.size(1), N = act == 2 ? w.size(0) / 2 : w.size(0);
   TORCH_CHECK(M >= 1 && M <= 64 && w.size(1) == K && K % 256 == 0, "skinny_gemm: M <= 64, K % 256 == 0");
   TORCH_CHECK(N % 4 == 0, "skinny_gemm: N % 4 == 0");
   TORCH_CHECK(y.size(0) == M && y.size(1) == N, "skinny_gemm: output shape");
@@ -505,8 +508,27 @@ void skinny_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t rb, 
   }
   int rc = llmd_skinny_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), M, N, K, (int)rb, (int)nsplit,
                             (int)occ, y.data_ptr(), y.stride(0), nsplit > 1 ? part.data_ptr<float>() : nullptr,
-                            relu2, cur_stream());
+                            (int)act, cur_stream());
   TORCH_CHECK(rc == 0, "skinny_gemm failed: ", rc);
+}
+
+// y = rmsnorm(x + residual) * gamma times w^T (silu: SiLU of its first half times the other), residual_out = x + residual
+void skinny_norm(torch::Tensor y, torch::Tensor x, torch::Tensor residual, torch::Tensor gamma, double eps,
+                 torch::Tensor residual_out, torch::Tensor w, int64_t rb, int64_t occ, bool silu) {
+  const c10::hip::OptionalHIPGuard device_guard(dev_of(y));
+  for (const auto& t : {x, residual, gamma, residual_out, w, y}) {
+    CHECK_CUDA(t); CHECK_BF16(t); CHECK_INNER(t);
+    TORCH_CHECK((uintptr_t)t.data_ptr() % 16 == 0, "skinny_norm: 16-byte addresses");
+  }
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && y.dim() == 2, "skinny_norm: 2-D operands");
+  const int M = x.size(0), K = x.size(1), N = silu ? w.size(0) / 2 : w.size(0);
+  TORCH_CHECK(M >= 1 && w.size(1) == K && residual.sizes() == x.sizes() && residual_out.sizes() == x.sizes() &&
+                  gamma.numel() == K && y.size(0) == M && y.size(1) == N && (!silu || w.size(0) % 2 == 0), "skinny_norm: shapes");
+  TORCH_CHECK(w.stride(0) % 8 == 0 && y.stride(0) % 4 == 0, "skinny_norm: row alignment");
+  const int rc = llmd_skinny_norm(x.data_ptr(), x.stride(0), residual.data_ptr(), residual.stride(0), gamma.data_ptr(),
+                                  (float)eps, residual_out.data_ptr(), residual_out.stride(0), w.data_ptr(), w.stride(0), M, N,
+                                  K, (int)rb, (int)occ, y.data_ptr(), y.stride(0), silu ? 2 : 0, cur_stream());
+  TORCH_CHECK(rc == 0, "skinny_norm failed: ", rc);
 }
 
 extern "C" int llmd_mla_v2_shape(int R, int fp8);
@@ -1431,7 +1453,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_debug (llmd_amd/build.p
   m.def("mla_attention", &mla_attention);
   m.def("mla_v2_shape", &mla_v2_shape, "H=128 MLA kernel shape: 10 * waves + head blocks per wave");
   m.def("skinny_gemm", &skinny_gemm, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("rb"), py::arg("nsplit"), py::arg("occ"),
-        py::arg("part"), py::arg("relu2") = false);
+        py::arg("part"), py::arg("act") = 0);
+  m.def("skinny_norm", &skinny_norm);
   m.def("skinny_supported", &skinny_supported);
   m.def("mgemm", &mgemm, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("wrb"), py::arg("nsplit"), py::arg("stages"),
         py::arg("part"), py::arg("relu2") = false);

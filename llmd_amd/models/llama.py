@@ -51,6 +51,10 @@ class LlamaMLP(torch.nn.Module):
             p = ops.mgemm_silu_plan(x, gu.weight)
             if p is not None:
                 return ops.mgemm_silu(x, gu.weight, p)
+            # a few rows: the same in the stream kernel (csrc/ops/skinny_gemm.hip act 2)
+            p = ops.skinny_whole(x, gu.weight) if gu.weight.shape[0] % 16 == 0 else None
+            if p is not None:
+                return ops.skinny_gemm(x, gu.weight, p, 2)
         x0 = x[0] if isinstance(x, tuple) else x
         if (wants_fp8_input(self.down) and wants_fp8_input(gu) and gu.bias is None and x0.dim() == 2
                 and ops._gpu(x0) and ops.pgemm8_silu_planned(x0.shape[0], gu.weight.shape[0], gu.weight.shape[1])):
@@ -84,6 +88,15 @@ def norm_fused_plan(lin, x):
             or lin.weight.dtype != torch.bfloat16 or (lin.reduce and get_state().tp_size > 1)):
         return None
     return ops.mgemm_norm_plan(x, lin.weight)
+
+
+def normed_product(norm, lin, x, residual, silu=False):
+    """(``lin`` of ``norm(x, residual)``, the new residual) from one launch (ops.norm_linear), or None: bf16 weights without bias or
+    LoRA and a row or a few."""
+    if (residual is None or not isinstance(x, torch.Tensor) or lin.bias is not None or lin.lora is not None
+            or lin.weight.dtype != torch.bfloat16 or not ops._gpu(x)):
+        return None
+    return ops.norm_linear(x, residual, norm.weight, norm.eps, lin.weight, silu)
 
 
 class LlamaDecoderLayer(torch.nn.Module):
@@ -122,7 +135,8 @@ class LlamaDecoderLayer(torch.nn.Module):
         bit-identical to GEMM + reduce + fused_add_rms_norm, two launches fewer)."""
         # W8A8: the norms emit fp8 + per-row scales straight into the fp8 GEMMs
         q_in = wants_fp8_input(self.qkv)
-        if normed:
+        fused = None if normed else normed_product(self.input_layernorm, self.qkv, x, residual)
+        if normed or fused is not None:
             pass
         elif residual is None:
             residual = x.clone()
@@ -130,7 +144,7 @@ class LlamaDecoderLayer(torch.nn.Module):
         else:
             x, residual = self.input_layernorm(x, residual, quant=q_in)
         norm = (self.q_norm.weight, self.k_norm.weight, self.q_norm.eps) if self.qk_norm else None
-        p = None if q_in else qkv_fused_plan(self.qkv, x)
+        p = None if q_in or fused is not None else qkv_fused_plan(self.qkv, x)
         if p is not None and norm is not None and not ops.rope_norms(norm, self.attn.D, self.attn.cos_sin, self.attn.neox):
             p = None
         if p is not None:  # decode: the QKV split-K reduce fused with RoPE + the cache write
@@ -138,7 +152,11 @@ class LlamaDecoderLayer(torch.nn.Module):
             a = self.attn(torch.empty(x.shape[0], self.qkv.weight.shape[0], dtype=x.dtype, device=x.device), meta,
                           parts=parts, qk_norm=norm)
         else:
-            a = self.attn(self.qkv(x), meta, qk_norm=norm)
+            if fused is not None:
+                qkv, residual = fused
+            else:
+                qkv = self.qkv(x)
+            a = self.attn(qkv, meta, qk_norm=norm)
         q_mlp = isinstance(self.mlp, LlamaMLP) and wants_fp8_input(self.mlp.gate_up)
         p = None if q_mlp else norm_fused_plan(self.o_proj, a)
         if p is not None:
@@ -146,6 +164,10 @@ class LlamaDecoderLayer(torch.nn.Module):
             x = ops.mgemm_add_rmsnorm(a, self.o_proj.weight, p, residual, pn.weight, pn.eps)
         else:
             x = self.o_proj(a)
+            if type(self.mlp) is LlamaMLP and not wants_fp8_input(self.mlp.down):
+                fused = normed_product(self.post_attention_layernorm, self.mlp.gate_up, x, residual, silu=True)
+                if fused is not None:
+                    return self.mlp.down(fused[0]), fused[1], False
             x, residual = self.post_attention_layernorm(x, residual, quant=q_mlp)
         if next_norm is not None and type(self.mlp) is LlamaMLP:
             h = self.mlp.hidden(x)

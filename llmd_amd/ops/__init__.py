@@ -1196,14 +1196,47 @@ SKINNY_TUNED: dict[tuple[int, int, int], tuple[int, int, int]] = {}
 
 
 def skinny_gemm(x: torch.Tensor, w: torch.Tensor, plan: Optional[tuple[int, int, int]] = None,
-                relu2: bool = False) -> torch.Tensor:
+                act: int = 0) -> torch.Tensor:
+    """act 1: max(0, .)^2 of the numbers in bf16; 2: silu(x wg^T) * (x wu^T) of them for w = [gate; up] and one range of K."""
     M, K = x.shape
-    N = w.shape[0]
-    rb, ns, occ = plan or skinny_plan(M, N, K)
+    N = w.shape[0] // 2 if act == 2 else w.shape[0]
+    rb, ns, occ = plan or skinny_plan(M, w.shape[0], K)
     y = torch.empty(M, N, dtype=x.dtype, device=x.device)
     part = torch.empty(ns * M * N if ns > 1 else 0, dtype=torch.float32, device=x.device)
-    native().skinny_gemm(y, x, w, rb, ns, occ, part, relu2)
+    native().skinny_gemm(y, x, w, rb, ns, occ, part, int(act))
     return y
+
+
+def skinny_whole(x: torch.Tensor, w: torch.Tensor) -> Optional[tuple[int, int, int]]:
+    """The plan with which ``linear(x, w)`` runs on the stream kernel with one range of K, or None."""
+    if not (_SKINNY and skinny_ok(x, w)) or x.data_ptr() % 16 or w.data_ptr() % 16 or (
+            x.shape[0] >= 33 and mgemm_choice(x.shape[0], *w.shape) is not None):
+        return None
+    plan = dgemm_choice(x.shape[0], *w.shape)
+    if plan is None:
+        rule = _unlisted_rule(x, w)
+        plan = rule[1] if rule is not None and rule[0] is skinny_gemm else None
+    return plan if plan is not None and plan[1] == 1 else None
+
+
+NORM_ROWS = 2  # rows up to which each workgroup of the stream kernel norms them itself (measured there)
+
+
+def norm_linear(x: torch.Tensor, residual: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch.Tensor, silu: bool = False):
+    """(``linear`` of rmsnorm(x + residual) * gamma, x + residual) in one launch where the stream kernel takes the product of a few
+    rows, else None; silu: silu(. wg^T) * (. wu^T) for w = [gate; up]. The bits of ``fused_add_rms_norm``, ``linear`` and ``gated_act``,
+    but residual itself is left alone."""
+    if (x.dim() != 2 or x.shape[0] > NORM_ROWS or x.shape[1] > 8192 or residual.shape != x.shape or residual.dtype != x.dtype
+            or gamma.dtype != x.dtype or (silu and w.shape[0] % 16) or residual.stride(1) != 1 or residual.stride(0) % 8
+            or residual.data_ptr() % 16 or gamma.data_ptr() % 16):
+        return None
+    plan = skinny_whole(x, w)
+    if plan is None:
+        return None
+    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    y = torch.empty(x.shape[0], w.shape[0] // 2 if silu else w.shape[0], dtype=x.dtype, device=x.device)
+    native().skinny_norm(y, x, residual, gamma, eps, out, w, plan[0], plan[2], silu)
+    return y, out
 
 
 def skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -1238,7 +1271,7 @@ def mgemm(x: torch.Tensor, w: torch.Tensor, plan: tuple[int, int, int], relu2: b
     wrb, ns, stages = plan
     y = torch.empty(M, N, dtype=x.dtype, device=x.device)
     part = torch.empty(ns * M * N if ns > 1 else 0, dtype=torch.float32, device=x.device)
-    native().mgemm(y, x, w, wrb, ns, stages, part, relu2)
+    native().mgemm(y, x, w, wrb, ns, stages, part, bool(relu2))
     return y
 
 
@@ -1575,7 +1608,7 @@ def linear_relu2(x: torch.Tensor, w: torch.Tensor):
         return None
     if x.shape[0] <= 64:
         rule = _unlisted_rule(x, w)
-        return None if rule is None else rule[0](x, w, rule[1], True)
+        return None if rule is None else rule[0](x, w, rule[1], 1)
     M, (N, K) = x.shape[0], w.shape
     if (PGEMM_AUTO == "measure" or (M <= 256 and mgemm_choice(M, N, K) is not None)
             or (M >= PGEMM_MIN_M and pgemm_plan(M, N, K) is not None)):

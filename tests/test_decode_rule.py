@@ -53,3 +53,43 @@ def test_rule_against_float32_wide(M, N, K):
     want = (x.double() @ w.double().T).float()
     # bf16 rounding of the result, fp32 rounding of K products of order 1 (partial sums up to about 4 sqrt(K))
     assert ((got - want).abs() <= 2 ** -8 * want.abs() + 2 ** -22 * 4 * K).all()
+
+
+def _same_silu(got, want):
+    """Tiles of gate and up rows begin their sweeps of K elsewhere than tiles of either: sums in another order, a few of which fall on
+    the next number in bf16, 2^-7 away at most. |g| < 6 here, so silu(g) u moves by up to (1 + |g|) + 1 times that, and its own
+    rounding. Sums near zero: a wave adds up to 64 times, each time off by 2^-24 of at most sum |x w| < 64, and |u| < 4."""
+    assert ((got - want).abs() <= 2 ** -7 * 9 * want.abs() + 1e-3).all() and (got != want).float().mean() < 0.02
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 6144, 4096), (1, 28672, 4096), (1, 2048, 2048), (1, 528, 1024), (1, 4096, 768), (2, 6144, 4096),
+                                   (3, 1040, 2048), (4, 1024, 8192)])
+def test_norm_and_silu_in_the_stream_kernel(M, N, K, monkeypatch):
+    """The bits of fused_add_rms_norm and linear, or skinny_gemm's SiLU, and a residual that stays."""
+    monkeypatch.setattr(ops, "NORM_ROWS", 4)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, r = (torch.randn(M, K, device="cuda", dtype=torch.bfloat16, generator=g) for _ in range(2))
+    w = torch.randn(N, K, device="cuda", dtype=torch.bfloat16, generator=g) * K ** -0.5
+    gamma = torch.randn(K, device="cuda", dtype=torch.bfloat16, generator=g)
+    if (plan := ops.skinny_whole(x, w)) is None:
+        pytest.skip("another kernel takes this product")
+    x1, r1, r0 = x.clone(), r.clone(), r.clone()
+    ops.fused_add_rms_norm(x1, r1, gamma, 1e-5)
+    y = ops.linear(x1, w)
+    act = ops.skinny_gemm(x1, w, plan, 2)
+    _same_silu(act, ops.gated_act(y, ops.ACT_SILU))
+    for silu, want in ((False, y), (True, act)):
+        out, res = ops.norm_linear(x, r, gamma, 1e-5, w, silu)
+        assert torch.equal(out, want) and torch.equal(res, r1) and torch.equal(r, r0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [7, 16, 17, 33, 64])
+def test_silu_in_the_stream_kernel_of_more_rows(M):
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, 1024, device="cuda", dtype=torch.bfloat16, generator=g)
+    w = torch.randn(1040, 1024, device="cuda", dtype=torch.bfloat16, generator=g) / 32
+    for rb in (1, 2, 3):
+        want = ops.gated_act(ops.skinny_gemm(x, w, (rb, 1, 1)), ops.ACT_SILU)
+        _same_silu(ops.skinny_gemm(x, w, (rb, 1, 1), 2), want)
