@@ -509,7 +509,21 @@ void skinny_gemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t rb, 
   int rc = llmd_skinny_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), M, N, K, (int)rb, (int)nsplit,
                             (int)occ, y.data_ptr(), y.stride(0), nsplit > 1 ? part.data_ptr<float>() : nullptr,
                             (int)act, cur_stream());
-  TORCH_CHECK(rc == 0, "skinny_gemm failed: ", rc);
+  TORCH_CHECK(rc > 0, "skinny_gemm failed: ", rc);
+}
+
+// The sums over several ranges of K of x w^T, [ranges, M, N], for a consumer that adds them up; returns the ranges
+int64_t skinny_partials(torch::Tensor x, torch::Tensor w, int64_t rb, int64_t nsplit, int64_t occ, torch::Tensor part) {
+  const c10::hip::OptionalHIPGuard device_guard(dev_of(x));
+  CHECK_CUDA(x); CHECK_BF16(x); CHECK_BF16(w); CHECK_INNER(x); CHECK_INNER(w); CHECK_CUDA(part); CHECK_DT(part, at::kFloat);
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1) && part.is_contiguous(), "skinny_partials: shapes");
+  const int M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0, "skinny_partials: row alignment");
+  TORCH_CHECK(part.numel() >= nsplit * (int64_t)M * N, "skinny_partials: workspace");
+  const int rc = llmd_skinny_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), M, N, K, (int)rb, (int)nsplit,
+                                  (int)occ, nullptr, 0, part.data_ptr<float>(), 0, cur_stream());
+  TORCH_CHECK(rc >= 2, "skinny_partials failed: ", rc);
+  return rc;
 }
 
 // y = rmsnorm(x + residual) * gamma times w^T (silu: SiLU of its first half times the other), residual_out = x + residual
@@ -1455,6 +1469,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_debug (llmd_amd/build.p
   m.def("skinny_gemm", &skinny_gemm, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("rb"), py::arg("nsplit"), py::arg("occ"),
         py::arg("part"), py::arg("act") = 0);
   m.def("skinny_norm", &skinny_norm);
+  m.def("skinny_partials", &skinny_partials);
   m.def("skinny_supported", &skinny_supported);
   m.def("mgemm", &mgemm, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("wrb"), py::arg("nsplit"), py::arg("stages"),
         py::arg("part"), py::arg("relu2") = false);

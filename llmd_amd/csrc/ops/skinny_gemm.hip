@@ -354,15 +354,17 @@ extern "C" int llmd_dgemm_supported(int M, int rb, int occ) {
 
 // Y = X W^T with a planned decomposition: rb row blocks per workgroup, nsplit
 // K splits, occ workgroups per CU. part: nsplit * M * N fp32 when nsplit > 1.
-// act: 0 none, 1 squared ReLU, 2 SiLU of the first N rows of W times the other N (nsplit 1)
+// act: 0 none, 1 squared ReLU, 2 SiLU of the first N rows of W times the other N (nsplit 1). y null: the ranges' sums only, [ranges][M][N]
+// in part. Returns the number of ranges, or an error < 0
 extern "C" int llmd_skinny_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_stride, int M, int N,
                                 int K, int rb, int nsplit, int occ, void* y, int64_t y_stride, float* part,
                                 int act, hipStream_t st) {
-  if (act < 0 || act > 2 || (act == 2 && (nsplit != 1 || N % 8))) return -1;
+  if (act < 0 || act > 2 || (act == 2 && (nsplit != 1 || N % 8)) || (y == nullptr && nsplit < 2)) return -1;
   if (M < 1 || M > 64 || K % 256 != 0 || N % 4 != 0 || nsplit < 1 || !llmd_dgemm_supported(M, rb, occ)) return -1;
   const int nq = K / 256;
   const int per = (nq + nsplit - 1) / nsplit;
   nsplit = (nq + per - 1) / per;  // no empty splits
+  if (y == nullptr && nsplit < 2) return -3;
   const int MB = (M + 15) / 16;
   kern_t k = pick_all(MB, rb, occ);
   if (k == nullptr) return -2;
@@ -370,12 +372,13 @@ extern "C" int llmd_skinny_gemm(const void* x, int64_t x_stride, const void* w, 
   dim3 grid((N + cols - 1) / cols, nsplit);
   hipLaunchKernelGGL(k, grid, dim3(NT), 0, st, (const uint16_t*)x, x_stride, (const uint16_t*)w, w_stride, M, N, K,
                      per, (uint16_t*)y, y_stride, part, act);
-  if (nsplit > 1) {
+  if (nsplit > 1 && y != nullptr) {
     const int64_t total4 = (int64_t)M * N / 4;
     hipLaunchKernelGGL(dgemm_reduce_kernel, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, st, part, nsplit,
                        M, N, (uint16_t*)y, y_stride, act);
   }
-  return (int)hipGetLastError();
+  const hipError_t err = hipGetLastError();
+  return err == hipSuccess ? nsplit : -(int)err;
 }
 
 // Y = rmsnorm(x + res, gamma) W^T (act 0) or its SiLU (act 2), res_out = x + res in bf16: the plan's rb and occ, whole K ranges

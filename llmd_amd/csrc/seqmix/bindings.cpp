@@ -44,8 +44,8 @@ int sm_gdelta_scan(const void*, int64_t, const void*, const void*, const void*, 
                    const int*, const int*, const int*, void*, int, int, hipStream_t);
 void sm_hyper_embed(const int64_t*, const void*, int64_t, float*, int, int, int, int, hipStream_t);
 void sm_hyper_norm(const float*, const float*, const void*, float, void*, int, int, int, int, int, hipStream_t);
-void sm_hyper_update_norm(float*, const void*, int64_t, const float*, const float*, const float*, const void*, float,
-                          void*, int, int, int, int, int, hipStream_t);
+int sm_hyper_update_norm(float*, const void*, int64_t, const float*, int, const float*, const float*, const float*, const void*,
+                         float, void*, int, int, int, int, int, hipStream_t);
 void sm_gated_act(const void*, int64_t, int, int, void*, int, int, float, hipStream_t);
 void sm_qkv_rope_cache(const void*, int64_t, const float*, const int64_t*, const float*, int, int, int, int, int, int,
                        int, float, float*, int, float, const int64_t*, void*, int, void*, const float*, int, int, int,
@@ -73,8 +73,9 @@ int sm_retention_chunk();
 int sm_retention_cols();
 void sm_bigram_embed(const int64_t*, const void*, float, int64_t, const void*, int64_t, int64_t, int64_t, int*,
                      const int*, const int*, const int*, const int*, int*, float*, void*, int, int, int, hipStream_t);
-void sm_post_norm_add(const void*, int64_t, const void*, int64_t, float, float, const float*, const void*, float*, float,
-                      const void*, void*, int, int, int, hipStream_t);
+int sm_post_norm_add(const void*, int64_t, const float*, int, const void*, int64_t, float, float, const float*, const void*, float*,
+                     float, const void*, void*, const void*, int, void*, const int*, const int*, const int*, int, int, int,
+                     hipStream_t);
 int sm_gated_delta_rows(int);
 int sm_gated_delta_scan(const void*, int64_t, int, int, int, int, const void*, int64_t, const void*, int64_t, int,
                         const float*, const float*, const void*, int64_t, int, const void*, float, float*, const int*,
@@ -394,6 +395,18 @@ void hyper_norm(Tensor X, Tensor w_in, Tensor norm_w, double eps, Tensor out, bo
                 rms ? 1 : 0, is_f32(norm_w), cur());
 }
 
+// A projection's fp32 sums over ranges of K, [ranges, T, d], in place of its output
+bool is_parts(const Tensor& y, int64_t T, int64_t d) {
+  return y.dim() == 3 && y.is_cuda() && y.scalar_type() == at::kFloat && y.is_contiguous() && y.size(0) >= 1 && y.size(1) == T &&
+         y.size(2) == d;
+}
+// and added up, for operands that the kernels do not read so
+Tensor sum_parts(const Tensor& y, const Tensor& like) {
+  Tensor s = y[0];
+  for (int64_t k = 1; k < y.size(0); ++k) s = s + y[k];
+  return s.to(like.scalar_type());
+}
+
 void hyper_update_norm(Tensor X, Tensor y, Tensor mix, Tensor w_out, std::optional<Tensor> next_in,
                        std::optional<Tensor> next_w, double eps, std::optional<Tensor> out, bool rms) {
   const c10::hip::OptionalHIPGuard g(dev_of(X));
@@ -401,7 +414,10 @@ void hyper_update_norm(Tensor X, Tensor y, Tensor mix, Tensor w_out, std::option
   CHECK_F32(mix);
   CHECK_F32(w_out);
   const int S = X.size(0), T = X.size(1), d = X.size(2);
-  TORCH_CHECK(y.is_cuda() && act_ok(y) && y.dim() == 2 && y.size(0) == T && y.size(1) == d && y.stride(1) == 1, "y [T, d]");
+  const bool parts = is_parts(y, T, d);
+  if (parts) TORCH_CHECK(out, "sums over ranges come with a bfloat16 output");
+  const Tensor like = parts ? *out : y;
+  TORCH_CHECK(parts || (y.is_cuda() && act_ok(y) && y.dim() == 2 && y.size(0) == T && y.size(1) == d && y.stride(1) == 1), "y [T, d]");
   TORCH_CHECK(mix.numel() == (int64_t)S * S && w_out.numel() == S, "mix [S, S], out [S]");
   const float* nin = nullptr;
   const void* nw = nullptr;
@@ -409,16 +425,19 @@ void hyper_update_norm(Tensor X, Tensor y, Tensor mix, Tensor w_out, std::option
   if (next_w) {
     TORCH_CHECK(next_in && out, "next_in and out come with next_w");
     CHECK_F32(*next_in);
-    CHECK_ACT(*next_w, y);
-    CHECK_ACT(*out, y);
+    CHECK_ACT(*next_w, like);
+    CHECK_ACT(*out, like);
     TORCH_CHECK(next_in->numel() == S && next_w->is_contiguous() && next_w->numel() == d && out->is_contiguous() &&
                     out->dim() == 2 && out->size(0) == T && out->size(1) == d, "next norm shapes");
     nin = next_in->data_ptr<float>();
     nw = next_w->data_ptr();
     o = out->data_ptr();
   }
-  sm_hyper_update_norm(X.data_ptr<float>(), y.data_ptr(), y.stride(0), mix.data_ptr<float>(), w_out.data_ptr<float>(),
-                       nin, nw, (float)eps, o, S, T, d, rms ? 1 : 0, is_f32(y), cur());
+  const int rc = sm_hyper_update_norm(X.data_ptr<float>(), parts ? nullptr : y.data_ptr(), parts ? 0 : y.stride(0),
+                                      parts ? y.data_ptr<float>() : nullptr, parts ? (int)y.size(0) : 0,
+                                      mix.data_ptr<float>(), w_out.data_ptr<float>(), nin, nw, (float)eps, o, S, T, d,
+                                      rms ? 1 : 0, is_f32(like), cur());
+  if (rc != 0) hyper_update_norm(X, sum_parts(y, like), mix, w_out, next_in, next_w, eps, out, rms);
 }
 
 void gated_act(Tensor gu, int64_t F, int64_t kind, Tensor out, double limit) {
@@ -744,18 +763,26 @@ void bigram_embed(Tensor ids, Tensor table, double scale, std::optional<Tensor> 
                   out.data_ptr(), T, d, is_f32(table), cur());
 }
 
+void input_conv(Tensor h, Tensor w, Tensor state, Tensor row_seq, Tensor seq_start, Tensor seq_slot, Tensor seq_init,
+                int64_t max_q, Tensor out, std::optional<Tensor> w2, std::optional<Tensor> out2);
+
 void post_norm_add(Tensor y, std::optional<Tensor> y2, double a, double b, std::optional<Tensor> bias, Tensor w_post,
-                   Tensor x, double eps, std::optional<Tensor> next_w, Tensor out) {
+                   Tensor x, double eps, std::optional<Tensor> next_w, Tensor out, std::optional<Tensor> conv_w,
+                   std::optional<Tensor> conv_state, std::optional<Tensor> row_seq, std::optional<Tensor> seq_slot,
+                   std::optional<Tensor> seq_init) {
   const c10::hip::OptionalHIPGuard g(dev_of(y));
-  TORCH_CHECK(y.is_cuda() && act_ok(y) && y.dim() == 2 && y.stride(1) == 1, "y");
-  const int T = y.size(0), d = y.size(1);
   CHECK_F32(x);
-  CHECK_ACT(w_post, y);
-  CHECK_ACT(out, y);
+  TORCH_CHECK(x.dim() == 2, "x [T, d]");
+  const int T = x.size(0), d = x.size(1);
+  const bool parts = is_parts(y, T, d);
+  const Tensor like = parts ? out : y;
+  TORCH_CHECK(parts || (y.is_cuda() && act_ok(y) && y.dim() == 2 && y.size(0) == T && y.size(1) == d && y.stride(1) == 1), "y [T, d]");
+  CHECK_ACT(w_post, like);
+  CHECK_ACT(out, like);
   TORCH_CHECK(x.dim() == 2 && x.size(0) == T && x.size(1) == d && d <= 65536 && w_post.is_contiguous() &&
                   w_post.numel() == d && out.is_contiguous() && out.sizes() == x.sizes(), "x, out [T, d]; w [d]");
   if (y2) {
-    CHECK_ACT(*y2, y);
+    CHECK_ACT(*y2, like);
     TORCH_CHECK(y2->dim() == 2 && y2->stride(1) == 1 && y2->size(0) == T && y2->size(1) == d, "y2 [T, d]");
   }
   if (bias) {
@@ -763,12 +790,33 @@ void post_norm_add(Tensor y, std::optional<Tensor> y2, double a, double b, std::
     TORCH_CHECK(bias->numel() == d, "bias [d]");
   }
   if (next_w) {
-    CHECK_ACT(*next_w, y);
+    CHECK_ACT(*next_w, like);
     TORCH_CHECK(next_w->is_contiguous() && next_w->numel() == d, "next_w [d]");
   }
-  sm_post_norm_add(y.data_ptr(), y.stride(0), y2 ? y2->data_ptr() : nullptr, y2 ? y2->stride(0) : 0, (float)a,
-                   (float)b, bias ? bias->data_ptr<float>() : nullptr, w_post.data_ptr(), x.data_ptr<float>(),
-                   (float)eps, next_w ? next_w->data_ptr() : nullptr, out.data_ptr(), T, d, is_f32(y), cur());
+  if (conv_w) {
+    TORCH_CHECK(conv_state && row_seq && seq_slot && seq_init, "a convolution comes with its state and sequences");
+    CHECK_ACT(*conv_w, like);
+    CHECK_ACT(*conv_state, like);
+    CHECK_I32(*row_seq); CHECK_I32(*seq_slot); CHECK_I32(*seq_init);
+    TORCH_CHECK(conv_w->dim() == 2 && conv_w->is_contiguous() && conv_w->size(0) == d && conv_w->size(1) >= 2 && conv_w->size(1) <= 4,
+                "conv weights [d, 2 to 4 taps]");
+    TORCH_CHECK(conv_state->dim() == 3 && conv_state->is_contiguous() && conv_state->size(2) == d &&
+                    conv_state->size(1) == conv_w->size(1) - 1, "conv state [slots, taps-1, d]");
+    TORCH_CHECK(row_seq->numel() == T && seq_slot->numel() == T && seq_init->numel() == T, "one token of every sequence");
+  }
+  const int rc = sm_post_norm_add(
+      parts ? nullptr : y.data_ptr(), parts ? 0 : y.stride(0), parts ? y.data_ptr<float>() : nullptr, parts ? (int)y.size(0) : 0,
+      y2 ? y2->data_ptr() : nullptr, y2 ? y2->stride(0) : 0, (float)a, (float)b, bias ? bias->data_ptr<float>() : nullptr,
+      w_post.data_ptr(), x.data_ptr<float>(), (float)eps, next_w ? next_w->data_ptr() : nullptr, out.data_ptr(),
+      conv_w ? conv_w->data_ptr() : nullptr, conv_w ? (int)conv_w->size(1) : 0, conv_w ? conv_state->data_ptr() : nullptr,
+      conv_w ? row_seq->data_ptr<int>() : nullptr, conv_w ? seq_slot->data_ptr<int>() : nullptr,
+      conv_w ? seq_init->data_ptr<int>() : nullptr, T, d, is_f32(like), cur());
+  if (rc != 0) {  // (float32, other widths, operands off 16 bytes: one pass after the other)
+    const Tensor h = conv_w ? at::empty_like(out) : out;
+    post_norm_add(parts ? sum_parts(y, like) : y, y2, a, b, bias, w_post, x, eps, next_w, h, {}, {}, {}, {}, {});
+    if (conv_w)
+      input_conv(h, *conv_w, *conv_state, *row_seq, at::arange(T + 1, row_seq->options()), *seq_slot, *seq_init, 1, out, {}, {});
+  }
 }
 
 void gated_delta_scan(Tensor xc, int64_t G, int64_t dk, int64_t H, int64_t dv, Tensor beta_raw, Tensor decay_raw,

@@ -196,8 +196,19 @@ __global__ __launch_bounds__(NT) void post_norm_add_kernel(const T* __restrict__
 // The same for bf16 rows of d = 8 n <= 8 * NT * NCH elements with 16-byte accesses: a thread keeps its
 // NCH chunks of eight elements in registers from the first pass to the last, so y is read once, x read
 // and written once and out written once; a small step's rows are a few loads deep instead of d / NT.
-template <int NCH>
-__global__ __launch_bounds__(NT) void post_norm_add_vec_kernel(const bf16_t* __restrict__ y, int64_t y_stride,
+// parts.p: y as its product's sums over ranges of K. TAPS: of a step of single tokens, the next reader's short convolution
+// (sm_scan.hip's input_conv: out + conv(out), over the bf16 numbers, the sequence's state read and rolled) comes from the same pass.
+// Both spare a launch of 4.7 us where a row has a microsecond of work.
+struct RowConv {
+  const bf16_t* w;  // [d][TAPS]
+  bf16_t* state;    // [slots][TAPS - 1][d]
+  const int* row_seq;
+  const int* seq_slot;
+  const int* seq_init;
+};
+template <int NCH, int TAPS>
+__global__ __launch_bounds__(NT) void post_norm_add_vec_kernel(const bf16_t* __restrict__ y, int64_t y_stride, Parts parts,
+                                                              RowConv conv,
                                                               const bf16_t* __restrict__ y2, int64_t y2_stride,
                                                               float a, float b, const float* __restrict__ bias,
                                                               const bf16_t* __restrict__ wp, float* __restrict__ x,
@@ -226,7 +237,8 @@ __global__ __launch_bounds__(NT) void post_norm_add_vec_kernel(const bf16_t* __r
   for (int k = 0; k < NCH; ++k) {
     const int c = (k * NT + threadIdx.x) * 8;
     if (c < d) {
-      ld8(y + row * y_stride + c, v[k]);
+      if (parts.p) add_parts(parts, row * d + c, v[k]);
+      else ld8(y + row * y_stride + c, v[k]);
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[k][i] *= a;
       if (y2) {
@@ -281,6 +293,38 @@ __global__ __launch_bounds__(NT) void post_norm_add_vec_kernel(const bf16_t* __r
       o.y = pack(v[k][2] * inv2 * w[2], v[k][3] * inv2 * w[3]);
       o.z = pack(v[k][4] * inv2 * w[4], v[k][5] * inv2 * w[5]);
       o.w = pack(v[k][6] * inv2 * w[6], v[k][7] * inv2 * w[7]);
+      if constexpr (TAPS > 0) {
+        const int s = conv.row_seq[row];
+        const bool init = conv.seq_init[s] != 0;
+        bf16_t* st_ = conv.state + (int64_t)conv.seq_slot[s] * (TAPS - 1) * d + c;
+        float wr[8 * TAPS], xv[8], r[8];  // channel i, tap j at i * TAPS + j
+#pragma unroll
+        for (int i = 0; i < TAPS; ++i) ld8(conv.w + (int64_t)c * TAPS + 8 * i, wr + 8 * i);
+        uint4 old[TAPS - 1];
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j)
+          old[j] = init ? *reinterpret_cast<const uint4*>(st_ + (int64_t)j * d) : make_uint4(0, 0, 0, 0);
+        const auto wide = [](const uint4& q, float* f) {
+          f[0] = __uint_as_float(q.x << 16); f[1] = __uint_as_float(q.x & 0xffff0000u);
+          f[2] = __uint_as_float(q.y << 16); f[3] = __uint_as_float(q.y & 0xffff0000u);
+          f[4] = __uint_as_float(q.z << 16); f[5] = __uint_as_float(q.z & 0xffff0000u);
+          f[6] = __uint_as_float(q.w << 16); f[7] = __uint_as_float(q.w & 0xffff0000u);
+        };
+        wide(o, xv);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r[i] = xv[i] + wr[i * TAPS + TAPS - 1] * xv[i];
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j) {
+          float f[8];
+          wide(old[j], f);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) r[i] += wr[i * TAPS + j] * f[i];
+        }
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j)
+          *reinterpret_cast<uint4*>(st_ + (int64_t)j * d) = j + 1 < TAPS - 1 ? old[j + 1 < TAPS - 1 ? j + 1 : j] : o;
+        o = make_uint4(pack(r[0], r[1]), pack(r[2], r[3]), pack(r[4], r[5]), pack(r[6], r[7]));
+      }
       *reinterpret_cast<uint4*>(out + row * d + c) = o;
     }
   }
@@ -653,25 +697,42 @@ void sm_bigram_embed(const int64_t* ids, const void* table, float scale, int64_t
                        (const bf16_t*)bigram, rows, prev_state, row_seq, seq_start, seq_slot, x, (bf16_t*)out, d);
 }
 
-void sm_post_norm_add(const void* y, int64_t y_stride, const void* y2, int64_t y2_stride, float a, float b,
-                      const float* bias, const void* wp, float* x, float eps, const void* wn, void* out, int T, int d,
-                      int f32, hipStream_t stream) {
-  if (T == 0) return;
+// Whether rows of d take the 16-byte form: the only one that reads parts or convolves
+int sm_post_norm_vec(int d) { return d % 8 == 0 && d <= 8 * NT * 4; }
+
+// parts: fp32 [nparts][T][d] in place of y, or null. cw: the next reader's filters (2 to 4 taps), or null. -1: not on these operands
+int sm_post_norm_add(const void* y, int64_t y_stride, const float* parts, int nparts, const void* y2, int64_t y2_stride,
+                     float a, float b, const float* bias, const void* wp, float* x, float eps, const void* wn, void* out,
+                     const void* cw, int taps, void* state, const int* row_seq, const int* seq_slot, const int* seq_init,
+                     int T, int d, int f32, hipStream_t stream) {
+  if (T == 0) return 0;
   const int nch = (d / 8 + NT - 1) / NT;
-  const bool aligned = (((uintptr_t)y | (uintptr_t)y2 | (uintptr_t)bias | (uintptr_t)wp | (uintptr_t)x | (uintptr_t)wn |
-                         (uintptr_t)out) & 15) == 0 && y_stride % 8 == 0 && y2_stride % 8 == 0;
-  if (!f32 && d % 8 == 0 && nch <= 4 && aligned) {
-#define SM_PNA(N)                                                                                                     \
-  hipLaunchKernelGGL(post_norm_add_vec_kernel<N>, dim3(T), dim3(NT), 0, stream, (const bf16_t*)y, y_stride,           \
+  const bool aligned = (((uintptr_t)y | (uintptr_t)parts | (uintptr_t)y2 | (uintptr_t)bias | (uintptr_t)wp | (uintptr_t)x |
+                         (uintptr_t)wn | (uintptr_t)out | (uintptr_t)cw | (uintptr_t)state) & 15) == 0 &&
+                       y_stride % 8 == 0 && y2_stride % 8 == 0;
+  if (!f32 && sm_post_norm_vec(d) && aligned && (!cw || (taps >= 2 && taps <= 4))) {
+    const Parts pt{parts, nparts, (int64_t)T * d};
+    const RowConv cv{(const bf16_t*)cw, (bf16_t*)state, row_seq, seq_slot, seq_init};
+#define SM_PNA2(N, TP)                                                                                                \
+  hipLaunchKernelGGL((post_norm_add_vec_kernel<N, TP>), dim3(T), dim3(NT), 0, stream, (const bf16_t*)y, y_stride, pt, cv, \
                      (const bf16_t*)y2, y2_stride, a, b, bias, (const bf16_t*)wp, x, eps, (const bf16_t*)wn,          \
                      (bf16_t*)out, d)
+#define SM_PNA(N)                    \
+  do {                               \
+    if (!cw) SM_PNA2(N, 0);          \
+    else if (taps == 2) SM_PNA2(N, 2); \
+    else if (taps == 3) SM_PNA2(N, 3); \
+    else SM_PNA2(N, 4);              \
+  } while (0)
     if (nch <= 1) SM_PNA(1);
     else if (nch == 2) SM_PNA(2);
     else if (nch == 3) SM_PNA(3);
     else SM_PNA(4);
+#undef SM_PNA2
 #undef SM_PNA
-    return;
+    return 0;
   }
+  if (parts || cw) return -1;
   if (f32)
     hipLaunchKernelGGL((post_norm_add_kernel<float>), dim3(T), dim3(NT), 0, stream, (const float*)y, y_stride,
                        (const float*)y2, y2_stride, a, b, bias, (const float*)wp, x, eps, (const float*)wn,
@@ -680,6 +741,7 @@ void sm_post_norm_add(const void* y, int64_t y_stride, const void* y2, int64_t y
     hipLaunchKernelGGL((post_norm_add_kernel<bf16_t>), dim3(T), dim3(NT), 0, stream, (const bf16_t*)y, y_stride,
                        (const bf16_t*)y2, y2_stride, a, b, bias, (const bf16_t*)wp, x, eps, (const bf16_t*)wn,
                        (bf16_t*)out, d);
+  return 0;
 }
 
 void sm_embed_scale(const int64_t* ids, const void* table, float scale, float* o0, float* o1, int T, int d,

@@ -31,7 +31,7 @@ from llmd_amd.ops import seqmix as sm
 from llmd_amd.parallel.state import get_state
 
 from .layers import LMHead, VocabEmbedding
-from .mixers import GroupedAttention, Hgrn2Mixer, InputConv, LatentAttention, SquaredReluMLP, _param
+from .mixers import GroupedAttention, Hgrn2Mixer, InputConv, LatentAttention, SquaredReluMLP, _param, reads_parts
 
 
 def make_mixer(spec: dict, d: int, eps: float, max_pos: int, device, dtype, earlier: list):
@@ -73,6 +73,7 @@ class KakalornLayer(torch.nn.Module):
         self.canon1 = InputConv(d, cfg.conv_taps, device, dtype)
         self.mix = make_mixer(spec, d, eps, max_pos, device, dtype, earlier)
         self.mlp = make_mlp(spec.get("mlp"), d, device, dtype)
+        reads_parts(self.mix, self.mlp)
         for n in ("norm1", "norm1b") + (("norm2", "norm2b") if self.mlp is not None else ()):
             setattr(self, n, _param((d,), device, dtype, fill=1.0))
 
@@ -126,14 +127,17 @@ class KakalornForCausalLM(torch.nn.Module):
         d, eps, dt = self.cfg.hidden_size, self.cfg.rms_norm_eps, self.dtype
         x = torch.empty(T, d, dtype=torch.float32, device=input_ids.device)
         h = sm.embed_norm(input_ids, self.embed.weight, self.layers[0].norm1 if L else self.norm, eps, x, dt)
+        conv = None  # the convolution that h has been through
         for i, l in enumerate(self.layers):
             nxt = self.layers[i + 1].norm1 if i + 1 < L else self.norm   # the last pass norms for the head
-            y = l.mix(l.canon1(h, meta), meta)
+            y = l.mix(h if conv is not None else l.canon1(h, meta), meta)
+            c = self.layers[i + 1].canon1 if i + 1 < L else None
+            conv = (c.weight, c.state, meta.seq) if c is not None and sm.row_conv(x, c.weight, meta.seq, dt) else None
             if l.mlp is None:
-                h = sm.post_norm_add(y, l.norm1b, x, eps, dt, nxt)
+                h = sm.post_norm_add(y, l.norm1b, x, eps, dt, nxt, conv=conv)
             else:
                 h = sm.post_norm_add(y, l.norm1b, x, eps, dt, l.norm2)
-                h = sm.post_norm_add(l.mlp(h), l.norm2b, x, eps, dt, nxt)
+                h = sm.post_norm_add(l.mlp(h), l.norm2b, x, eps, dt, nxt, conv=conv)
             if layer_out is not None:
                 layer_out.append(x.clone())
         return h

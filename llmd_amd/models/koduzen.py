@@ -27,7 +27,7 @@ from llmd_amd.parallel.state import get_state
 
 from .hyper import HyperConnection, stream_stack
 from .layers import LMHead, VocabEmbedding
-from .mixers import GatedMLP, GroupedAttention, RetentionMixer, ScoreMoE, _param
+from .mixers import GatedMLP, GroupedAttention, RetentionMixer, ScoreMoE, _param, reads_parts
 
 ACT = "swish_limit"
 
@@ -72,6 +72,7 @@ class KoduzenLayer(torch.nn.Module):
         S, learned = max(1, cfg.hyper_streams), cfg.hyper_streams > 0
         self.mix = make_mixer(spec, d, eps, max_pos, device, dtype, earlier)
         self.mlp = make_mlp(spec.get("mlp"), d, device, dtype)
+        reads_parts(self.mix, self.mlp)
         self.norm1 = _param((d,), device, dtype, fill=1.0)
         self.hc1 = HyperConnection(S, learned, device, dtype)
         if self.mlp is not None:

@@ -120,8 +120,13 @@ class ColumnLinear(torch.nn.Module):
                                        requires_grad=False) if bias else None
 
     lora = None  # engine/lora.py LoRATarget when multi-LoRA is enabled
+    parts = False  # its reader takes sums over ranges of K (ops.linear_parts) in place of the output
 
     def forward(self, x):
+        if self.parts and self.bias is None and self.lora is None and self.weight.dtype == torch.bfloat16:
+            y = ops.linear_parts(x, self.weight)
+            if y is not None:
+                return y
         y = _linear(self, x, self.bias)
         if self.lora is not None:
             self.lora.apply(y, x)

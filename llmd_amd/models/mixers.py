@@ -468,6 +468,14 @@ class GroupedAttention(torch.nn.Module):
         return self.o(o)
 
 
+def reads_parts(*modules):
+    """The residual's pass behind these sublayers (post_norm_add, hyper_update_norm) adds up their last projection's ranges of K."""
+    for m in modules:
+        last = m.down if isinstance(m, (GatedMLP, SquaredReluMLP)) else getattr(m, "o", None)
+        if isinstance(last, ColumnLinear):
+            last.parts = True
+
+
 class GatedMLP(torch.nn.Module):
     """W_down (act(W_gate h) * (W_up h)), gate and up as one projection; act "gelu_tanh" or "silu". act
     "swish_limit": g sigmoid(1.702 g) (u + 1) with g = min(W_gate h, limit), u = clamp(W_up h, -limit, limit)."""

@@ -31,7 +31,7 @@ from llmd_amd.parallel.state import get_state
 
 from .hyper import HyperConnection, stream_stack
 from .layers import LMHead, VocabEmbedding
-from .mixers import GatedMLP, GroupedAttention, ScoreMoE, _param
+from .mixers import GatedMLP, GroupedAttention, ScoreMoE, _param, reads_parts
 
 
 def make_mixer(spec: dict, d: int, eps: float, max_pos: int, device, dtype):
@@ -62,6 +62,7 @@ class NegunexLayer(torch.nn.Module):
         S, learned = max(1, cfg.hyper_streams), cfg.hyper_streams > 0
         self.mix = make_mixer(spec, d, self.eps, max_pos, device, dtype)
         self.mlp = make_mlp(spec.get("mlp"), d, device, dtype)
+        reads_parts(self.mix, self.mlp)
         self.norm1 = _param((d,), device, dtype, fill=1.0)
         self.hc1 = HyperConnection(S, learned, device, dtype)
         if self.mlp is not None:

@@ -1309,6 +1309,29 @@ def mgemm_partials(x: torch.Tensor, w: torch.Tensor, plan: tuple[int, int, int])
     return part, int(ns)
 
 
+def linear_parts(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """x w^T as fp32 sums over ranges of K, [ranges, T, N], for a reader that adds them up and rounds to bf16, or None. Up to 16 rows
+    and outputs of half of the CUs' blocks of 16: the stream kernel with as many ranges as fill the CUs; else where ``linear`` has
+    ranges of K anyway. us with the norm that reads it, ``linear`` / here: (2048, 2048) 8.6 / 7.9 at one row, 9.5 / 8.5 at 9, 12.5 / 10.5
+    at 64; (2048, 5632) 13.9 / 11.0, 14.1 / 11.9, 15.9 / 14.0; (4096, 4096) at 9 has 256 blocks: 14.0, and 14.1 with two ranges."""
+    if x.dim() != 2 or not _SKINNY or w.shape[0] % 8 or not mgemm_ok(x, w):
+        return None
+    M, (N, K) = x.shape[0], w.shape
+    tiles = -(-N // 16)
+    if M <= 16 and tiles <= 128 and K % 256 == 0 and 1024 <= K <= 8192 and not _listed(M, N, K):
+        if x.data_ptr() % 16 or w.data_ptr() % 16:
+            return None
+        ns = min(256 // tiles, K // 512)
+        part = torch.empty(ns * M * N, dtype=torch.float32, device=x.device)
+        ns = native().skinny_partials(x, w, 1, ns, 2, part)
+    else:
+        plan = split_plan(x, w)
+        if plan is None:
+            return None
+        part, ns = mgemm_partials(x, w, plan)
+    return part[:ns * M * N].view(ns, M, N)
+
+
 def reduce_rope_cache(part: torch.Tensor, nsplit: int, qkv: torch.Tensor, positions, cos_sin, Hq, Hkv, D, slots,
                       k_cache, v_cache, neox=True, k_scale=1.0, v_scale=1.0, qk_norm=None):
     """The QKV projection's split-K reduce + RoPE (after the heads' norm, ``rope_norms``) + paged KV write in one kernel

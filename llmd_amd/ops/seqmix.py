@@ -272,7 +272,8 @@ def hyper_update_norm(X, y, mix, w_out, next_in=None, next_w=None, eps: float = 
                       rms: bool = False):
     """X[t] <- sum_s mix[s, t] X[s] + w_out[t] y for all streams at once, in place (fp32); with
     ``next_w`` also returns the layer norm (``rms``: the RMS norm) of sum_s next_in[s] X[s], the next sublayer's input (or
-    the model's final norm over the plain sum), from the same pass."""
+    the model's final norm over the plain sum), from the same pass. ``y`` may be the sums over ranges of K of its projection, fp32
+    [ranges, T, d] (``ops.linear_parts``)."""
     if not X.is_cuda:
         return ref.hyper_update_norm(X, y, mix, w_out, next_in, next_w, eps, out_dtype, rms)
     out = torch.empty(X.shape[1:], dtype=out_dtype, device=X.device) if next_w is not None else None
@@ -482,15 +483,23 @@ def bigram_embed(ids, table, scale: float, bigram, buckets: int, mul_prev: int, 
 
 
 def post_norm_add(y, w_post, x, eps: float, out_dtype, next_w=None, y2=None, a: float = 1.0, b: float = 1.0,
-                  bias=None):
+                  bias=None, conv=None):
     """x += rms_norm(a y + b y2 + bias) * w_post on the fp32 residual, in place (plain weights, eps
     inside the root; ``y2`` and ``bias`` optional). Returns the next reader's input from the same
-    pass: x in the activation type, or rms_norm(x) * next_w when ``next_w`` is given."""
+    pass: x in the activation type, or rms_norm(x) * next_w when ``next_w`` is given. ``y`` may be the sums over ranges of K of its
+    projection, fp32 [ranges, T, d] (``ops.linear_parts``). ``conv`` = (w, state, seq): ``input_conv`` of that, where ``row_conv``."""
     if not x.is_cuda:
         return ref.post_norm_add(y, w_post, x, eps, out_dtype, next_w, y2, a, b, bias)
     out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    native().post_norm_add(y, y2, float(a), float(b), bias, w_post, x, float(eps), next_w, out)
+    cv = (conv[0], conv[1], conv[2].row_seq, conv[2].seq_slot, conv[2].seq_init) if conv is not None else (None,) * 5
+    native().post_norm_add(y, y2, float(a), float(b), bias, w_post, x, float(eps), next_w, out, *cv)
     return out
+
+
+def row_conv(x, w, seq, dtype) -> bool:
+    """Whether ``post_norm_add`` over the residual x runs the convolution ``w`` [C, taps] that follows it: a step of single tokens."""
+    return (x.is_cuda and dtype == torch.bfloat16 and seq.max_q == 1 and seq.seq_slot.numel() == x.shape[0]
+            and 2 <= w.shape[1] <= 4 and x.shape[1] % 8 == 0 and x.shape[1] <= 8192)
 
 
 def gated_delta_scan(xc, G: int, dk: int, H: int, dv: int, beta_raw, decay_raw, A, dt_bias, gate_raw,

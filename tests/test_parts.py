@@ -1,0 +1,74 @@
+"""Projections handed on as sums over ranges of K, and the residual's passes that read them (csrc/seqmix/sm_elementwise.hip, sm_hyper.hip)."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from llmd_amd import ops
+from llmd_amd.ops import seqmix as sm
+
+pytestmark = pytest.mark.gpu
+
+
+def _rand(*shape, dtype=torch.bfloat16, seed=0, scale=1.0):
+    g = torch.Generator(device="cuda").manual_seed(seed + sum(shape))
+    return (torch.randn(*shape, device="cuda", generator=g) * scale).to(dtype)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 2048, 2048), (9, 2048, 5632), (16, 1024, 8192), (5, 520, 1280), (16, 2048, 1024), (17, 2048, 2048),
+                                   (64, 2048, 5632), (33, 1000, 1024), (9, 4096, 4096)])
+def test_parts_are_the_product(M, N, K):
+    x, w = _rand(M, K), _rand(N, K, seed=1, scale=K ** -0.5)
+    p = ops.linear_parts(x, w)
+    if p is None:
+        assert (M, N) == (9, 4096)
+        return
+    assert p.shape[1:] == (M, N) and p.shape[0] >= 2
+    want = x.double() @ w.double().t()
+    assert (p.double().sum(0) - want).abs().max() < 2e-5  # K / ranges products of about 1 / sqrt(K) each, summed in fp32
+    if M > 16:
+        assert torch.equal(p[0] if p.shape[0] == 1 else _added(p), ops.linear(x, w))
+
+
+def _added(p):
+    s = p[0]
+    for k in range(1, p.shape[0]):
+        s = s + p[k]
+    return s.bfloat16()
+
+
+@pytest.mark.parametrize("T,d,n", [(1, 2048, 2), (9, 2048, 8), (64, 1000, 3), (3, 8192, 2), (5, 8200, 2), (4, 2052, 2)])
+@pytest.mark.parametrize("S", [1, 2, 4, 5])
+def test_readers_of_parts(T, d, n, S):
+    """The bits of the pass over the sums and the reader behind it; rows off the 16-byte forms are added up first."""
+    p, w, wn = _rand(n, T, d, dtype=torch.float32), _rand(d, seed=1), _rand(d, seed=2)
+    y = _added(p)
+    if S == 1:
+        x0, x1 = (_rand(T, d, dtype=torch.float32, seed=3) for _ in range(2))
+        for nxt in (wn, None):
+            a, b = (sm.post_norm_add(v, w, x, 1e-5, torch.bfloat16, nxt) for v, x in ((y, x0), (p, x1)))
+            assert torch.equal(a, b) and torch.equal(x0, x1)
+    X0, X1 = (_rand(S, T, d, dtype=torch.float32, seed=4) for _ in range(2))
+    mix, out, nin = _rand(S, S, dtype=torch.float32), _rand(S, dtype=torch.float32), _rand(S, dtype=torch.float32, seed=5)
+    a, b = (sm.hyper_update_norm(X, v, mix, out, nin, wn, 1e-5, torch.bfloat16, True) for v, X in ((y, X0), (p, X1)))
+    assert torch.equal(a, b) and torch.equal(X0, X1)
+
+
+@pytest.mark.parametrize("T,d,taps", [(1, 2048, 4), (9, 2048, 4), (64, 1000, 3), (3, 8192, 2), (2, 4104, 4)])
+def test_convolution_in_the_norm(T, d, taps):
+    """post_norm_add with the next reader's convolution: the bits of the two passes, states rolled and only those of the step."""
+    y, w, wn, cw = _rand(T, d), _rand(d, seed=1), _rand(d, seed=2), _rand(d, taps, seed=3, scale=0.2)
+    x0, x1 = (_rand(T, d, dtype=torch.float32, seed=4) for _ in range(2))
+    s0, s1 = (_rand(T + 3, taps - 1, d, seed=5) for _ in range(2))
+    i32 = dict(dtype=torch.int32, device="cuda")
+    seq = SimpleNamespace(row_seq=torch.arange(T, **i32), seq_start=torch.arange(T + 1, **i32), seq_slot=torch.randperm(T + 3)[:T].to(**i32),
+                          seq_init=(torch.arange(T, **i32) % 3 != 1).int(), max_q=1)
+    assert sm.row_conv(x0, cw, seq, torch.bfloat16)
+    for _ in range(2):
+        a = sm.input_conv(sm.post_norm_add(y, w, x0, 1e-5, torch.bfloat16, wn), cw, s0, seq)
+        b = sm.post_norm_add(y, w, x1, 1e-5, torch.bfloat16, wn, conv=(cw, s1, seq))
+        assert torch.equal(a, b) and torch.equal(x0, x1) and torch.equal(s0, s1)
+    odd = torch.empty(T * d + 8, device="cuda", dtype=torch.bfloat16)[1:T * d + 1].view(T, d).copy_(y)  # off 16 bytes: one pass after the other
+    b = sm.post_norm_add(odd, w, x1, 1e-5, torch.bfloat16, wn, conv=(cw, s1, seq))
+    a = sm.input_conv(sm.post_norm_add(odd, w, x0, 1e-5, torch.bfloat16, wn), cw, s0, seq)
+    assert torch.equal(a, b) and torch.equal(s0, s1)
