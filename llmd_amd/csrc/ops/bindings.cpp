@@ -72,7 +72,7 @@ int llmd_pgemm(const void*, int64_t, const void*, int64_t, void*, int64_t, int, 
                hipStream_t);
 int64_t llmd_pgemm_ws_bytes(int, int, int, int, int);
 int llmd_tgemm_plan(int, int, int, int);
-int llmd_tgemm(const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, int, const void*, void*,
+int llmd_tgemm(const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, float, int, const void*, void*,
                hipStream_t);
 int llmd_fgemm_plan(int, int, int);
 int llmd_fgemm(const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, const void*, void*, hipStream_t);
@@ -643,11 +643,11 @@ void pgemm(torch::Tensor y, torch::Tensor x, torch::Tensor w, int64_t epi, int64
 }
 
 // x w^T (+ bias); with act silu(x wg^T) * (x wu^T) of w = [gate; up] (1: of the fp32 sums, 2: of the sums in bf16) or max(0, x w^T)^2
-// (3: of the sums in bf16), on the tile that llmd_tgemm_plan has for these
+// (3: of the sums in bf16) or the clamped units (4) of the sums in bf16, on the tile that llmd_tgemm_plan has for these
 // sizes (csrc/ops/tgemm.hip), or on `tile`; nothing where it has none or the operands are not what the kernel reads
 std::optional<torch::Tensor> tgemm(const torch::Tensor& x, const torch::Tensor& w, const std::optional<torch::Tensor>& bias,
-                                   int64_t act, int64_t tile) {
-  const bool silu = act == 1 || act == 2;
+                                   int64_t act, int64_t tile, double limit) {
+  const bool silu = act == 1 || act == 2 || act == 4;
   if (!x.is_cuda() || x.device() != w.device() || x.dim() != 2 || w.dim() != 2 || x.scalar_type() != at::kBFloat16 ||
       w.scalar_type() != at::kBFloat16)
     return std::nullopt;
@@ -660,13 +660,13 @@ std::optional<torch::Tensor> tgemm(const torch::Tensor& x, const torch::Tensor& 
   if (bias && (silu || bias->scalar_type() != at::kBFloat16 || bias->device() != x.device() || bias->dim() != 1 ||
                bias->size(0) != N || (N > 1 && bias->stride(0) != 1) || off(*bias)))
     return std::nullopt;
-  const int code = tile ? (int)tile : llmd_tgemm_plan((int)M, (int)rows, (int)K, silu ? (int)act : 0);
+  const int code = tile ? (int)tile : llmd_tgemm_plan((int)M, (int)rows, (int)K, silu ? std::min((int)act, 2) : 0);
   if (code == 0) return std::nullopt;
   const c10::hip::OptionalHIPGuard device_guard(dev_of(x));
   torch::Tensor y = torch::empty({M, N}, x.options()), ws;
   if (code % 10 > 1) ws = torch::empty({code % 10, M, N}, x.options().dtype(torch::kFloat));
   const int rc = llmd_tgemm(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), N, (int)M, (int)N,
-                            (int)K, (int)act, code, bias ? bias->data_ptr() : nullptr,
+                            (int)K, (int)act, (float)limit, code, bias ? bias->data_ptr() : nullptr,
                             ws.defined() ? ws.data_ptr() : nullptr, cur_stream());
   TORCH_CHECK(rc == 0, "tgemm failed: ", rc);
   return y;
@@ -1482,7 +1482,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_debug (llmd_amd/build.p
   m.def("pgemm_fp8", &pgemm_fp8, "prefill fp8 W8A8 GEMM (256x256 LDS-DMA tiles on 16x16x128 f8f6f4 MFMA), "
         "per-token x per-channel scales, optional fused SiLU-and-mul");
   m.def("tgemm", &tgemm, "bf16 GEMM of prompt-sized steps on the tile that fits, or None", py::arg("x"), py::arg("w"),
-        py::arg("bias") = std::nullopt, py::arg("act") = 0, py::arg("tile") = 0);
+        py::arg("bias") = std::nullopt, py::arg("act") = 0, py::arg("tile") = 0, py::arg("limit") = 0.0);
   m.def("tgemm_plan", &llmd_tgemm_plan, "tile of tgemm for (M, N, K, silu): mi * 100 + ni * 10 + ranges of K, or 0");
   m.def("fgemm", &fgemm, "fp32 GEMM of prompt-sized steps on the bf16 matrix units, or None", py::arg("x"), py::arg("w"),
         py::arg("bias") = std::nullopt, py::arg("tile") = 0);

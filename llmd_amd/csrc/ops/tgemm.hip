@@ -58,7 +58,7 @@ __global__ __launch_bounds__(NT, 1) void tgemm_kernel(const uint16_t* __restrict
                                                       const uint16_t* __restrict__ W, int64_t ldw,
                                                       uint16_t* __restrict__ C, int64_t ldc, int M, int N, int K,
                                                       const uint16_t* __restrict__ bias, int nsplit,
-                                                      int form, float* __restrict__ ws) {
+                                                      int form, float limit, float* __restrict__ ws) {
   constexpr int ST = stages(MI, NI), D = MI + NI, R = MI + NI, T = MI * NI;
   constexpr int STG = 4096 * (MI + NI), OPW = 4096 * MI;
   constexpr int BM = 32 * MI, BN = 32 * NI;
@@ -242,7 +242,13 @@ __global__ __launch_bounds__(NT, 1) void tgemm_kernel(const uint16_t* __restrict
         const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[e]), __float_as_uint(y[e]), false, false);
         float g = __uint_as_float(s[0]), u = __uint_as_float(s[1]);
         if (form) g = __uint_as_float((uint32_t)f2bf(g) << 16), u = __uint_as_float((uint32_t)f2bf(u) << 16);
-        o[e] = g / (1.f + __expf(-g)) * u;
+        if (form == 2) {  // the bits of sm_hyper.hip's clamped units
+          g = fminf(g, limit);
+          u = fminf(fmaxf(u, -limit), limit);
+          o[e] = g * __builtin_amdgcn_rcpf(1.f + __expf(-(1.702f * g))) * (u + 1.f);
+        } else {
+          o[e] = g / (1.f + __expf(-g)) * u;
+        }
       }
       u32x2_t p;
       p[0] = (uint32_t)f2bf(o[0]) | ((uint32_t)f2bf(o[1]) << 16);
@@ -354,16 +360,16 @@ extern "C" int llmd_tgemm_plan(int M, int N, int K, int silu) {
   return code;
 }
 
-// A tile of llmd_tgemm_plan. N: columns of C; W [N, K], with act 1 and 2 [2 N, K]. act 0: none, 1: silu of gate (the first N rows of W)
+// A tile of llmd_tgemm_plan. N: columns of C; W [N, K], with act 1, 2 and 4 [2 N, K]. act 0: none, 1: silu of gate (the first N rows of W)
 // times up (the others), 2: the same of the sums rounded to bf16, as a pass of its own would find them, 3: max(0, .)^2 of the sums rounded
-// to bf16. bias: [N] or null (no silu).
+// to bf16, 4: the clamped units g sigmoid(1.702 g) (u + 1), g <= limit and |u| <= limit, of these. bias: [N] or null (no silu).
 // Ranges > 1 (no silu): sums in ws [ranges, M, N]. -1: not taken.
 extern "C" int llmd_tgemm(const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N,
-                          int K, int act, int code, const void* bias, void* ws, hipStream_t st) {
+                          int K, int act, float limit, int code, const void* bias, void* ws, hipStream_t st) {
   if (M <= 0 || N <= 0) return 0;
   const int mi = code / 100, ni = code / 10 % 10, nsplit = code % 10;
-  if (N % 8 || K % BK || K <= 0 || lda % 8 || ldw % 8 || ldc % 8 || act < 0 || act > 3) return -1;
-  const bool silu = act == 1 || act == 2;
+  if (N % 8 || K % BK || K <= 0 || lda % 8 || ldw % 8 || ldc % 8 || act < 0 || act > 4) return -1;
+  const bool silu = act == 1 || act == 2 || act == 4;
   const int nk = K / BK;
   if (nsplit < 1 || nsplit > nk || (nsplit - 1) * ((nk + nsplit - 1) / nsplit) >= nk) return -1;
   if ((nsplit > 1 && (silu || ws == nullptr)) || (bias != nullptr && silu)) return -1;
@@ -374,7 +380,7 @@ extern "C" int llmd_tgemm(const void* A, int64_t lda, const void* W, int64_t ldw
   const auto launch = [&](auto kernel) {
     const int64_t grid = (int64_t)((M + 32 * mi - 1) / (32 * mi)) * ((N + tc - 1) / tc) * nsplit;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(NT), 0, st, (const uint16_t*)A, lda, (const uint16_t*)W, ldw,
-                       (uint16_t*)C, ldc, M, N, K, (const uint16_t*)bias, nsplit, act >= 2, (float*)ws);
+                       (uint16_t*)C, ldc, M, N, K, (const uint16_t*)bias, nsplit, act == 4 ? 2 : act >= 2, limit, (float*)ws);
     if (nsplit > 1)
       hipLaunchKernelGGL(tgemm_reduce_kernel, dim3((unsigned)(((int64_t)M * (N / 8) + 255) / 256)), dim3(256), 0, st,
                          (const float*)ws, nsplit, M, N, (const uint16_t*)bias, (uint16_t*)C, ldc, act == 3);

@@ -46,7 +46,7 @@ void sm_hyper_embed(const int64_t*, const void*, int64_t, float*, int, int, int,
 void sm_hyper_norm(const float*, const float*, const void*, float, void*, int, int, int, int, int, hipStream_t);
 int sm_hyper_update_norm(float*, const void*, int64_t, const float*, int, const float*, const float*, const float*, const void*,
                          float, void*, int, int, int, int, int, hipStream_t);
-void sm_gated_act(const void*, int64_t, int, int, void*, int, int, float, hipStream_t);
+int sm_gated_act(const void*, const float*, int, int64_t, int, int, void*, int, int, float, hipStream_t);
 void sm_qkv_rope_cache(const void*, int64_t, const float*, const int64_t*, const float*, int, int, int, int, int, int,
                        int, float, float*, int, float, const int64_t*, void*, int, void*, const float*, int, int, int,
                        int, const void*, void*, int, const int*, const int*, const int*, const int*, int, int, int,
@@ -442,11 +442,15 @@ void hyper_update_norm(Tensor X, Tensor y, Tensor mix, Tensor w_out, std::option
 
 void gated_act(Tensor gu, int64_t F, int64_t kind, Tensor out, double limit) {
   const c10::hip::OptionalHIPGuard g(dev_of(gu));
-  TORCH_CHECK(gu.is_cuda() && act_ok(gu) && gu.dim() == 2 && gu.stride(1) == 1 && gu.size(1) >= 2 * F && F >= 1, "gu");
-  CHECK_ACT(out, gu);
-  TORCH_CHECK(out.is_contiguous() && out.dim() == 2 && out.size(0) == gu.size(0) && out.size(1) == F &&
-                  kind >= 0 && kind <= 2, "out [T, F]");
-  sm_gated_act(gu.data_ptr(), gu.stride(0), F, kind, out.data_ptr(), gu.size(0), is_f32(gu), (float)limit, cur());
+  const int64_t T = out.size(0), W = gu.size(-1);
+  const bool parts = is_parts(gu, T, W);
+  const Tensor like = parts ? out : gu;
+  TORCH_CHECK(F >= 1 && W >= 2 * F && (parts || (gu.is_cuda() && act_ok(gu) && gu.dim() == 2 && gu.stride(1) == 1)), "gu");
+  CHECK_ACT(out, like);
+  TORCH_CHECK(out.is_contiguous() && out.dim() == 2 && gu.size(-2) == T && out.size(1) == F && kind >= 0 && kind <= 2, "out [T, F]");
+  const int rc = sm_gated_act(parts ? nullptr : gu.data_ptr(), parts ? gu.data_ptr<float>() : nullptr, parts ? (int)gu.size(0) : 0,
+                              parts ? W : gu.stride(0), F, kind, out.data_ptr(), T, is_f32(like), (float)limit, cur());
+  if (rc != 0) gated_act(sum_parts(gu, like), F, kind, out, limit);
 }
 
 void qkv_rope_cache(Tensor qkv, std::optional<Tensor> bias, Tensor positions, std::optional<Tensor> cos_sin, int64_t Hq,

@@ -219,9 +219,10 @@ __global__ __launch_bounds__(NT) void gated_act_kernel(const T* __restrict__ gu,
   st(out + i, gate1<T, KIND>(ld(gu + t * stride + j), ld(gu + t * stride + F + j), limit));
 }
 
-// bf16, F % 8 == 0, 16-byte aligned rows: eight columns per thread from 16-byte loads.
+// bf16, F % 8 == 0, 16-byte aligned rows: eight columns per thread from 16-byte loads. parts.p: gu as its product's sums over ranges of
+// K, rows of stride (64 x 2 x 1536: 4.9 + 4.6 us, here 4.5).
 template <int KIND>
-__global__ __launch_bounds__(NT) void gated_act_vec_kernel(const bf16_t* __restrict__ gu, int64_t stride, int F,
+__global__ __launch_bounds__(NT) void gated_act_vec_kernel(const bf16_t* __restrict__ gu, Parts parts, int64_t stride, int F,
                                                            bf16_t* __restrict__ out, int64_t n8, float limit) {
   const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
   if (i >= n8) return;
@@ -229,10 +230,15 @@ __global__ __launch_bounds__(NT) void gated_act_vec_kernel(const bf16_t* __restr
   const int64_t t = i / f8;
   const int j = (int)(i - t * f8) * 8;
   float g[8], v[8], o[8];
-  ld4(gu + t * stride + j, *reinterpret_cast<float(*)[4]>(&g[0]));
-  ld4(gu + t * stride + j + 4, *reinterpret_cast<float(*)[4]>(&g[4]));
-  ld4(gu + t * stride + F + j, *reinterpret_cast<float(*)[4]>(&v[0]));
-  ld4(gu + t * stride + F + j + 4, *reinterpret_cast<float(*)[4]>(&v[4]));
+  if (parts.p) {
+    add_parts(parts, t * stride + j, g);
+    add_parts(parts, t * stride + F + j, v);
+  } else {
+    ld4(gu + t * stride + j, *reinterpret_cast<float(*)[4]>(&g[0]));
+    ld4(gu + t * stride + j + 4, *reinterpret_cast<float(*)[4]>(&g[4]));
+    ld4(gu + t * stride + F + j, *reinterpret_cast<float(*)[4]>(&v[0]));
+    ld4(gu + t * stride + F + j + 4, *reinterpret_cast<float(*)[4]>(&v[4]));
+  }
 #pragma unroll
   for (int q = 0; q < 8; ++q) o[q] = gate1<bf16_t, KIND>(g[q], v[q], limit);
   st4(out + t * F + j, *reinterpret_cast<float(*)[4]>(&o[0]));
@@ -302,21 +308,24 @@ int sm_hyper_update_norm(float* X, const void* y, int64_t y_stride, const float*
   return 0;
 }
 
-void sm_gated_act(const void* gu, int64_t stride, int F, int kind, void* out, int T, int f32, float limit,
+// parts: fp32 [nparts][T][stride] in place of gu, or null. -1: not on these operands
+int sm_gated_act(const void* gu, const float* parts, int nparts, int64_t stride, int F, int kind, void* out, int T, int f32, float limit,
                   hipStream_t stream) {
   const int64_t n = (int64_t)T * F;
-  if (n == 0) return;
-  if (!f32 && F % 8 == 0 && stride % 8 == 0 && (((uintptr_t)gu | (uintptr_t)out) & 15) == 0) {
+  if (n == 0) return 0;
+  if (!f32 && F % 8 == 0 && stride % 8 == 0 && (((uintptr_t)gu | (uintptr_t)parts | (uintptr_t)out) & 15) == 0) {
     const int64_t n8 = n / 8;
     const dim3 g8((unsigned)((n8 + NT - 1) / NT));
+    const Parts pt{parts, nparts, T * stride};
 #define SM_GV(K) \
-  hipLaunchKernelGGL((gated_act_vec_kernel<K>), g8, dim3(NT), 0, stream, (const bf16_t*)gu, stride, F, (bf16_t*)out, n8, limit)
+  hipLaunchKernelGGL((gated_act_vec_kernel<K>), g8, dim3(NT), 0, stream, (const bf16_t*)gu, pt, stride, F, (bf16_t*)out, n8, limit)
     if (kind == 0) SM_GV(0);
     else if (kind == 1) SM_GV(1);
     else SM_GV(2);
 #undef SM_GV
-    return;
+    return 0;
   }
+  if (parts) return -1;
   const dim3 grid((unsigned)((n + NT - 1) / NT));
 #define SM_GO(TYPE, K) \
   hipLaunchKernelGGL((gated_act_kernel<TYPE, K>), grid, dim3(NT), 0, stream, (const TYPE*)gu, stride, F, (TYPE*)out, n, limit)
@@ -330,6 +339,7 @@ void sm_gated_act(const void* gu, int64_t stride, int F, int kind, void* out, in
     else SM_GO(bf16_t, 2);
   }
 #undef SM_GO
+  return 0;
 }
 
 }  // extern "C"

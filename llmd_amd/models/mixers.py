@@ -484,10 +484,15 @@ class GatedMLP(torch.nn.Module):
         super().__init__()
         self.ff, self.act, self.limit = ff, act, float(limit)
         self.gate_up = ColumnLinear(d_model, 2 * ff, shard=False, device=device, dtype=dtype)
+        self.gate_up.parts = True
         self.down = ColumnLinear(ff, d_model, shard=False, device=device, dtype=dtype)
 
     def forward(self, h):
-        return self.down(sm.gated_act(self.gate_up(h), self.ff, self.act, self.limit))
+        gu = self.gate_up
+        z = None
+        if self.act == "swish_limit" and gu.weight.dtype == torch.bfloat16 and gu.lora is None and gu.bias is None:
+            z = ops.linear_clamped(h, gu.weight, self.limit)
+        return self.down(sm.gated_act(gu(h), self.ff, self.act, self.limit) if z is None else z)
 
 
 class ScoreMoE(torch.nn.Module):

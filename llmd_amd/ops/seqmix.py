@@ -404,10 +404,12 @@ ACT_KINDS = {"gelu_tanh": 0, "silu": 1, "swish_limit": 2}
 
 def gated_act(gu, Fh: int, kind: str, limit: float = 0.0):
     """act(gu[:, :Fh]) * gu[:, Fh:], act the tanh form of GELU or SiLU, fp32 arithmetic. "swish_limit":
-    g sigmoid(1.702 g) (u + 1) with g = min(gu[:, :Fh], limit) and u = clamp(gu[:, Fh:], -limit, limit)."""
+    g sigmoid(1.702 g) (u + 1) with g = min(gu[:, :Fh], limit) and u = clamp(gu[:, Fh:], -limit, limit). ``gu`` [ranges, T, 2 Fh]: the
+    sums of its product (``ops.linear_parts``), result in bfloat16."""
     if not gu.is_cuda:
         return ref.gated_act(gu, Fh, kind, limit)
-    out = torch.empty(gu.shape[0], Fh, dtype=gu.dtype, device=gu.device)
+    parts = gu.dim() == 3
+    out = torch.empty(gu.shape[-2], Fh, dtype=torch.bfloat16 if parts else gu.dtype, device=gu.device)
     native().gated_act(gu, int(Fh), ACT_KINDS[kind], out, float(limit))
     return out
 

@@ -72,3 +72,21 @@ def test_convolution_in_the_norm(T, d, taps):
     b = sm.post_norm_add(odd, w, x1, 1e-5, torch.bfloat16, wn, conv=(cw, s1, seq))
     a = sm.input_conv(sm.post_norm_add(odd, w, x0, 1e-5, torch.bfloat16, wn), cw, s0, seq)
     assert torch.equal(a, b) and torch.equal(s0, s1)
+
+
+@pytest.mark.parametrize("T,F,n", [(1, 2560, 2), (64, 512, 8), (9, 1004, 3), (5, 36, 2)])
+@pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "swish_limit"])
+def test_gated_units_of_parts(T, F, n, kind):
+    p = _rand(n, T, 2 * F, dtype=torch.float32, scale=3.0)
+    assert torch.equal(sm.gated_act(p, F, kind, 7.0), sm.gated_act(_added(p), F, kind, 7.0))
+
+
+@pytest.mark.parametrize("M,F,K", [(257, 512, 2048), (901, 2560, 2048), (300, 264, 1024), (2722, 1024, 2048)])
+def test_clamped_units_in_the_epilogue(M, F, K):
+    """The bits of the product and the units' pass, infinities and numbers beyond the limit among the sums."""
+    x, w = _rand(M, K), _rand(2 * F, K, seed=1, scale=3 * K ** -0.5)
+    w[3], w[F + 5] = float("inf"), float("-inf")
+    y = ops.linear_clamped(x, w, 2.5)
+    assert y is not None
+    want = sm.gated_act(ops.linear(x, w), F, "swish_limit", 2.5)
+    assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.nan_to_num(), want.nan_to_num())
