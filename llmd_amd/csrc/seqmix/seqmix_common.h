@@ -103,16 +103,17 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 // Keys per range of a step whose attention rows are cut into ``nsplit`` key ranges. A captured step has as many ranges as the
 // longest context it may be replayed with; how many keys they take follows the longest context of the replay (``longest``, on
 // the device). ``split_keys`` is the size the ranges were planned with and never exceeded.
-__device__ __forceinline__ int range_keys(const int* longest, int nsplit, int split_keys) {
+// ``least``: keys that a range has at least.
+__device__ __forceinline__ int range_keys(const int* longest, int nsplit, int split_keys, int least = 128) {
   if (longest == nullptr) return split_keys;
   const int span = min(*longest, nsplit * split_keys), part = nsplit * 64;
-  return min(split_keys, max(128, (span + part - 1) / part * 64));
+  return min(split_keys, max(least, (span + part - 1) / part * 64));
 }
 // How many of the ranges can hold keys then: those behind neither run nor are merged. One sequence of 2000 tokens, 16 latent
 // heads, ranges planned for 131072: 49.1 us when they did, 20.3 (25.2 planned for 2000).
-__device__ __forceinline__ int ranges_used(const int* longest, int nsplit, int split_keys) {
+__device__ __forceinline__ int ranges_used(const int* longest, int nsplit, int split_keys, int least = 128) {
   if (longest == nullptr) return nsplit;
-  const int keys = range_keys(longest, nsplit, split_keys);
+  const int keys = range_keys(longest, nsplit, split_keys, least);
   return max(1, (min(*longest, nsplit * split_keys) + keys - 1) / keys);
 }
 

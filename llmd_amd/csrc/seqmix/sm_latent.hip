@@ -231,6 +231,11 @@ __device__ __forceinline__ void split_weights(const float* p, bf16x8_t& hi, bf16
   lo = __builtin_bit_cast(bf16x8_t, lw);
 }
 
+// Keys of a range: one tile while that makes up to 32 ranges (the merge is longer with more), else two. A tile takes a decode
+// workgroup 4.5 us, most of it waiting for its keys: 9 rows of 577 to 1777 keys, 16 heads, with the merge 27.4 us in ranges of 192,
+// 23.3 of 64; one of 300 25.5 / 17.0; 16 of up to 300 25.2 / 16.6; four of 8000 keep theirs of 128, 27.1 (30.8 of 64).
+__device__ __forceinline__ int least_keys(const int* longest) { return longest != nullptr && *longest <= 32 * 64 ? 64 : 128; }
+
 // One tile's rows of the paged cache, in 16-byte chunks with the lanes along a row: KEYS keys from k0 on, zeros from
 // kend on and past Dk. All chunks are requested before any is used. one_page: the tile lies inside one
 // page (page sizes that are multiples of KEYS), so its block-table entry is read once.
@@ -479,8 +484,8 @@ __global__ __launch_bounds__(NT, 2) void latent_attention_mfma_kernel(
   // decode steps split a row's keys over blockIdx.y: this workgroup takes [kbeg, kend)
   const int nsplit = gridDim.y;
   if (nsplit > 1) {
-    if ((int)blockIdx.y >= ranges_used(longest, nsplit, split_keys)) return;
-    split_keys = range_keys(longest, nsplit, split_keys);
+    if ((int)blockIdx.y >= ranges_used(longest, nsplit, split_keys, least_keys(longest))) return;
+    split_keys = range_keys(longest, nsplit, split_keys, least_keys(longest));
   }
   const int kbeg = nsplit > 1 ? kbase + blockIdx.y * split_keys : kbase;
   const int kend = nsplit > 1 ? min(maxlen, kbeg + split_keys) : maxlen;
@@ -629,8 +634,8 @@ __global__ __launch_bounds__(NT, 2) void latent_decode_mfma_kernel(
   const int kbase = window > 0 ? (max(0, row_len[tok0] - window) / DKT) * DKT : 0;
   const int nsplit = gridDim.y;
   if (nsplit > 1) {
-    if ((int)blockIdx.y >= ranges_used(longest, nsplit, split_keys)) return;
-    split_keys = range_keys(longest, nsplit, split_keys);
+    if ((int)blockIdx.y >= ranges_used(longest, nsplit, split_keys, least_keys(longest))) return;
+    split_keys = range_keys(longest, nsplit, split_keys, least_keys(longest));
   }
   const int kbeg = nsplit > 1 ? kbase + blockIdx.y * split_keys : kbase;
   const int kend = nsplit > 1 ? min(maxlen, kbeg + split_keys) : maxlen;
@@ -775,7 +780,7 @@ __global__ __launch_bounds__(NT) void latent_attention_merge_kernel(const int* _
   const int64_t p0 = (int64_t)item * nsplit * 64 + row;
   const int64_t tok = tok0 + row / H, h = row % H;
   const float w = gate ? 1.f / (1.f + expf(-ld(gate + tok * gate_stride + h))) : 1.f;
-  merge_ranges<NT>(part_ml + p0 * 2, 128, part_o + p0 * R, (int64_t)64 * R, ranges_used(longest, nsplit, split_keys), R,
+  merge_ranges<NT>(part_ml + p0 * 2, 128, part_o + p0 * R, (int64_t)64 * R, ranges_used(longest, nsplit, split_keys, least_keys(longest)), R,
                    [](float x) { return exp2f(x); }, [&](int c, float v) { st(out + (tok * H + h) * R + c, v * w); });
 }
 

@@ -50,3 +50,30 @@ def test_rows_do_not_depend_on_the_cut(R, dr, bs, window):
             rows.append(sm.latent_attention(q[a:b], cache, whole.tables, m.row_seq, m.row_len, 0.05, R, 4, seq=m, window=window))
         out.append(torch.cat(rows))
     assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("longest", [1, 63, 64, 65, 130, 2047, 2048, 2049, 3000])
+def test_decode_ranges_follow_the_longest_context(longest):
+    """Ranges planned for 4096 keys, of one tile up to 2048 and two behind: every key is met once, whatever the replay's lengths."""
+    from llmd_amd.ops import seqmix as sm
+
+    H, R, dr, bs, n = 16, 512, 64, 64, 3
+    g = torch.Generator(device="cuda").manual_seed(longest)
+    lens = [longest, max(1, longest - 64), max(1, longest // 2)]
+    W = 64
+    cache = torch.randn(n * W, bs, R + dr, device="cuda", generator=g).bfloat16()
+    q = torch.randn(n, H, R + dr, device="cuda", generator=g).bfloat16()
+    i32 = dict(dtype=torch.int32, device="cuda")
+    tables = torch.randperm(n * W, device="cuda", generator=g).to(torch.int32).view(n, W)
+    items = torch.tensor([[i, i, 1] for i in range(n)], **i32)
+    rows = torch.tensor(lens, **i32)
+    for ns, split in ((32, 128), (16, 256), (64, 64)):
+        out = torch.empty(n, H, R, dtype=torch.bfloat16, device="cuda")
+        po, pm = torch.full((n * ns * 64 * R,), float("nan"), device="cuda"), torch.full((n * ns * 128,), float("nan"), device="cuda")
+        assert sm.native().latent_attention_mfma(q, cache, tables, items, rows, 0.05, R, out, ns, split, po, pm, None, 0, H,
+                                                 torch.tensor([longest], **i32))
+        for i, L in enumerate(lens):
+            kv = cache[tables[i].long()].view(-1, R + dr)[:L].double()
+            want = torch.softmax(q[i].double() @ kv.t() * 0.05, -1) @ kv[:, :R]
+            assert (out[i].double() - want).norm() / want.norm() < 4e-3  # bf16 results, 2^-9 each
