@@ -18,6 +18,7 @@ void sm_xielu(const void*, float, float, void*, int64_t, int, hipStream_t);
 void sm_softcap(float*, float, int64_t, hipStream_t);
 void sm_latent_rope_cache(const void*, int64_t, const void*, int64_t, const void*, float, const int64_t*, const float*,
                           int, int, int, int, int, const int64_t*, void*, void*, int, int, int, hipStream_t);
+int sm_head_product(const void*, int64_t, int64_t, const void*, int, int, int, int, void*, int64_t, int64_t, hipStream_t);
 int sm_latent_attention(const void*, const void*, const int*, int, int, const int*, const int*, float, int, int, int,
                         int, int, void*, int, const void*, int64_t, int, hipStream_t);
 int sm_latent_attention_mfma(const void*, const void*, const int*, int, int, const int*, int, const int*, float, int,
@@ -393,6 +394,20 @@ void hyper_norm(Tensor X, Tensor w_in, Tensor norm_w, double eps, Tensor out, bo
   TORCH_CHECK(out.is_contiguous() && out.dim() == 2 && out.size(0) == T && out.size(1) == d, "out [T, d]");
   sm_hyper_norm(X.data_ptr<float>(), w_in.data_ptr<float>(), norm_w.data_ptr(), (float)eps, out.data_ptr(), S, T, d,
                 rms ? 1 : 0, is_f32(norm_w), cur());
+}
+
+// out[t][h] = x[t][h] w[h]^T: x [T, H, K] and out [T, H, N] with neighbouring last elements, w [H, N, K]; false: not these operands
+bool head_product(Tensor x, Tensor w, Tensor out) {
+  const c10::hip::OptionalHIPGuard g(dev_of(x));
+  const auto ok = [&](const Tensor& t) {
+    return t.is_cuda() && t.device() == x.device() && t.scalar_type() == at::kBFloat16 && t.dim() == 3;
+  };
+  TORCH_CHECK(ok(x) && ok(w) && ok(out), "head_product: bfloat16, three dimensions");
+  const int64_t T = x.size(0), H = x.size(1), K = x.size(2), N = w.size(1);
+  TORCH_CHECK(w.size(0) == H && w.size(2) == K && out.size(0) == T && out.size(1) == H && out.size(2) == N, "head_product: shapes");
+  if ((K > 1 && x.stride(2) != 1) || (N > 1 && out.stride(2) != 1) || !w.is_contiguous() || T > 64) return false;
+  return sm_head_product(x.data_ptr(), x.stride(0), x.stride(1), w.data_ptr(), H, K, N, T, out.data_ptr(), out.stride(0),
+                         out.stride(1), cur()) == 0;
 }
 
 // A projection's fp32 sums over ranges of K, [ranges, T, d], in place of its output
@@ -1103,6 +1118,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_combine", &moe_combine);
   m.def("bigram_embed", &bigram_embed);
   m.def("post_norm_add", &post_norm_add);
+  m.def("head_product", &head_product);
   m.def("gated_delta_scan", &gated_delta_scan);
   m.def("embed_norm", &embed_norm);
   m.def("rms_norm", &rms_norm);

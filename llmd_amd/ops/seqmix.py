@@ -97,6 +97,12 @@ def latent_rope_cache(q, kv, norm_w, eps, positions, cos_sin, H, dn, dr, rot_dim
                                q_abs, bool(interleaved))
 
 
+def head_product(x, w, out):
+    """out[t, h] = x[t, h] w[h]^T for x [T, H, K], w [H, N, K], out [T, H, N] (neighbouring last elements), up to 64 rows in bfloat16
+    (csrc/seqmix/sm_latent.hip head_product_kernel), or False."""
+    return x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= 64 and native().head_product(x, w, out)
+
+
 LATENT_DECODE_WGS = int(os.environ.get("LLMD_LATENT_DECODE_WGS", "512"))  # workgroups a decode-only step aims for
 MFMA_ATTENTION = os.environ.get("LLMD_LATENT_MFMA", "1") == "1"
 

@@ -90,3 +90,22 @@ def test_clamped_units_in_the_epilogue(M, F, K):
     assert y is not None
     want = sm.gated_act(ops.linear(x, w), F, "swish_limit", 2.5)
     assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.nan_to_num(), want.nan_to_num())
+
+
+@pytest.mark.parametrize("T,H,K,N", [(1, 16, 512, 128), (9, 16, 128, 512), (17, 3, 256, 16), (33, 5, 128, 48), (64, 32, 512, 128), (16, 128, 128, 64)])
+def test_head_product(T, H, K, N):
+    x, w = _rand(T, H, K + 64)[:, :, :K], _rand(H, N, K, seed=1, scale=K ** -0.5)
+    buf = torch.full((T, H, N + 64), 7.0, device="cuda", dtype=torch.bfloat16)
+    assert sm.head_product(x, w, buf[:, :, :N])
+    want = torch.einsum("thk,hnk->thn", x.double().cpu(), w.double().cpu())
+    assert (buf[:, :, :N].double().cpu() - want).abs().max() <= 2 ** -8 * want.abs().max()  # rounded once to bf16
+    assert (buf[:, :, N:] == 7).all()
+
+
+def test_head_product_leaves_the_rest():
+    x, w = _rand(4, 8, 128), _rand(8, 64, 128)
+    out = torch.empty(4, 8, 64, device="cuda", dtype=torch.bfloat16)
+    assert not sm.head_product(x[:, :, :64], w[:, :, :64].contiguous(), out)                          # k in quarters of 32
+    assert not sm.head_product(_rand(65, 8, 128), w, torch.empty(65, 8, 64, device="cuda", dtype=torch.bfloat16))
+    assert not sm.head_product(_rand(33, 64, 128), _rand(64, 64, 128), torch.empty(33, 64, 64, device="cuda", dtype=torch.bfloat16))
+    assert not sm.head_product(_rand(4, 8, 129)[:, :, 1:], w, out)                                    # off 16 bytes
