@@ -266,7 +266,8 @@ constexpr Tile TILES[] = {{4, 4, 1, 1.06, 1.16}, {3, 3, 1, 0.75, 0.80}, {4, 2, 1
 }  // namespace
 
 // The tile for a product of these sizes, as mi * 100 + ni * 10 + ranges of K, or 0: not here. Taken where it is 7 % faster than what the
-// vendor's kernels reach (115 TFLOP/s below 2048 rows): 350 x (5120, 2048) 65 / 60, not taken; 350 x (11264, 2048) 150 / 111; 350 x (2048,
+// vendor's kernels reach (115 TFLOP/s below 2048 rows; 90, seen 65 to 102, where 64 x 64 tiles leave more than a quarter of their second or
+// a later round empty: 700 x (2048, 1536) 58 / 42, 700 x (2048, 768) 34 / 25): 350 x (5120, 2048) 65 / 60, not taken; 350 x (11264, 2048) 150 / 111; 350 x (2048,
 // 4096) 52 / 64, not taken; from some 500 rows on all of them but narrow ones (700 x (132, 2048) 19 / 33). Ranges of K where
 // the tiles leave CUs idle, of at least 16 steps, sums of at most 256 MB: 700 x (2048, 4096) 98 with one, 78 with two.
 extern "C" int llmd_fgemm_plan(int M, int N, int K) {
@@ -289,7 +290,9 @@ extern "C" int llmd_fgemm_plan(int M, int N, int K) {
         code = t.mi * 100 + t.ni * 10 + r;
       }
     }
-  return best < 0.93 * 2.0 * M * N * K / 115e6 + 2.0 ? code : 0;
+  const int64_t blocks = (int64_t)((M + 63) / 64) * ((N + 63) / 64), rounds = (blocks + 255) / 256;
+  const double rate = rounds > 1 && 4 * blocks < 3 * 256 * rounds ? 90e6 : 115e6;
+  return best < 0.93 * 2.0 * M * N * K / rate + 2.0 ? code : 0;
 }
 
 // code: of llmd_fgemm_plan. ws: [ranges, M, N] with more than one range. -1: not taken.
