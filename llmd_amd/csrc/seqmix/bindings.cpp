@@ -58,6 +58,7 @@ int sm_grouped_attention(const void*, const void*, const int*, int, int, const i
 int sm_grouped_attention_mfma(const void*, const void*, const int*, int, int, const int*, int, const int*, float, int,
                               int, int, int, const void*, int64_t, void*, int, int, float*, float*, int, const float*,
                               int, const float*, int, int, int, const int*, int, hipStream_t);
+int sm_router(const void*, int64_t, const void*, int, int, int, float*, hipStream_t);
 void sm_moe_route_scores(const float*, const float*, int, int, int*, float*, int, int, int, float, hipStream_t);
 void sm_moe_route(const float*, int64_t, int, int, int*, float*, int, int, hipStream_t);
 int64_t sm_moe_sort_scratch(int, int);
@@ -628,6 +629,19 @@ bool grouped_attention_mfma(Tensor q, Tensor cache, int64_t dim, int64_t vdim, T
   return rc == 0;
 }
 
+// x [M, K] w [N, K]^T in fp32 of bfloat16 operands, or nothing where the kernel does not take them
+std::optional<Tensor> router_logits(Tensor x, Tensor w) {
+  if (!x.is_cuda() || x.device() != w.device() || x.dim() != 2 || w.dim() != 2 || x.scalar_type() != at::kBFloat16 ||
+      w.scalar_type() != at::kBFloat16 || x.size(1) != w.size(1) || x.stride(1) != 1 || !w.is_contiguous() || x.size(0) > 8192 || w.size(0) > 8192)
+    return std::nullopt;
+  const c10::hip::OptionalHIPGuard g(dev_of(x));
+  if ((x.size(0) + 15) / 16 * ((w.size(0) + 15) / 16) >= 512) return std::nullopt;
+  Tensor y = torch::empty({x.size(0), w.size(0)}, x.options().dtype(torch::kFloat32));
+  if (sm_router(x.data_ptr(), x.stride(0), w.data_ptr(), x.size(0), w.size(0), x.size(1), y.data_ptr<float>(), cur()) != 0)
+    return std::nullopt;
+  return y;
+}
+
 void moe_route_scores(Tensor logits, Tensor correction, int64_t k, Tensor ids, Tensor w, int64_t groups, int64_t keep,
                       double scale) {
   const c10::hip::OptionalHIPGuard g(dev_of(logits));
@@ -1118,6 +1132,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_combine", &moe_combine);
   m.def("bigram_embed", &bigram_embed);
   m.def("post_norm_add", &post_norm_add);
+  m.def("router_logits", &router_logits);
   m.def("head_product", &head_product);
   m.def("gated_delta_scan", &gated_delta_scan);
   m.def("embed_norm", &embed_norm);

@@ -502,6 +502,79 @@ __global__ __launch_bounds__(256) void moe_combine_vec_kernel(const T* __restric
   }
 }
 
+// Router logits: y = x W^T in fp32 from bf16 rows and weights. Their products are exact in fp32, so the fp32 matrix instructions on
+// widened operands give what a product of float copies gave, without the copies: a lane's four neighbouring k of a step of 16 are
+// the operands of four instructions, which is also the order in which the float product that stood here added (the same bits
+// at 1 .. 800 x (132, 2048)).
+// Bound by the instructions' chain (one waits 75 cycles for the one before): four waves per 16 x 16 numbers, which take 32 k of every 128
+// each and are added up in order. Chunks of 128 k come to LDS two ahead, in 16-byte pieces whose place in a row is turned by the row's
+// number: the eight bytes that a lane takes then lie in banks of their own.
+// us, copy and float product / here: 1 x (132, 2048) 11.2 / 9.2, 64 12.3 / 9.2, 700 16.1 / 11.3, 800 x (64, 1024) 13.1 / 6.3; up to 511 such blocks
+// and K 2048: 64 x (128, 4096) 14.3 / 15.0; 2048 x (132, 2048) in the order of its float product, one chain of all k, 34.1 / 28.9,
+// but 1500 24.1 / 28.2 and 2722 33.7 / 37.3.
+constexpr int RCH = 128, RROW = RCH * 2, RBLK = 16 * RROW, RSTAGE = 2 * RBLK;  // k of a chunk, bytes of a row, of 16 rows, of both operands
+template <int N>
+__device__ __forceinline__ void router_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+__global__ __launch_bounds__(256) void router_kernel(const bf16_t* __restrict__ x, int64_t xs, const bf16_t* __restrict__ w, int M,
+                                                     int N, int K, int nb, float* __restrict__ y) {
+  __shared__ __attribute__((aligned(16))) char ring[3 * RSTAGE];  // 16 rows of x, then 16 of w
+  __shared__ __attribute__((aligned(16))) f32x4_t red[3][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, r16 = lane & 15;
+  const int m0 = blockIdx.x / nb * 16, n0 = blockIdx.x % nb * 16;
+  const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring + wave * 1024;
+  // a wave's copy of 1 KB is four rows: lane l's 16 bytes are piece (l % 16) ^ row of row 4 wave + l / 16
+  const int row = 4 * wave + (lane >> 4), piece = ((lane & 15) ^ row) * 16;
+  const uint32_t xo = (uint32_t)((min(m0 + row, M - 1) - m0) * xs * 2) + piece;
+  const uint32_t wo = (uint32_t)((min(n0 + row, N - 1) - n0) * (int64_t)K * 2) + piece;
+  const char* xb = (const char*)(x + m0 * xs);
+  const char* wb = (const char*)(w + (int64_t)n0 * K);
+  const auto fetch = [&](int c) {
+    const uint32_t at = lds + c % 3 * RSTAGE;
+    copy_1k(xb + (int64_t)c * RROW, xo, at);
+    copy_1k(wb + (int64_t)c * RROW, wo, at + RBLK);
+  };
+  int at[2];  // of the wave's two steps of 16 k in a chunk
+#pragma unroll
+  for (int b = 0; b < 2; ++b) at[b] = r16 * RROW + ((4 * wave + 2 * b + (g >> 1)) ^ r16) * 16 + 8 * (g & 1);
+  const int chunks = K / RCH;
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  fetch(0);
+  if (chunks > 1) fetch(1);
+  for (int c = 0; c < chunks; ++c) {
+    if (c + 1 == chunks) router_wait<0>();
+    else router_wait<2>();
+    __builtin_amdgcn_s_barrier();  // chunk c is there, chunk c - 1 no longer read
+    asm volatile("" ::: "memory");
+    if (c + 2 < chunks) fetch(c + 2);
+    const char* t = ring + c % 3 * RSTAGE;
+    uint2 a[2], q[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      a[b] = *reinterpret_cast<const uint2*>(t + at[b]);
+      q[b] = *reinterpret_cast<const uint2*>(t + RBLK + at[b]);
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const uint32_t av[4] = {a[b].x << 16, a[b].x & 0xffff0000u, a[b].y << 16, a[b].y & 0xffff0000u};
+      const uint32_t qv[4] = {q[b].x << 16, q[b].x & 0xffff0000u, q[b].y << 16, q[b].y & 0xffff0000u};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(qv[j]), __uint_as_float(av[j]), acc, 0, 0, 0);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads of the chunk are done
+  }
+  if (wave > 0) red[wave - 1][lane] = acc;
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) acc += red[i][lane];
+  // acc[r] = y[m0 + r16][n0 + 4 g + r]
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (m0 + r16 < M && n0 + 4 * g + r < N) y[(int64_t)(m0 + r16) * N + n0 + 4 * g + r] = acc[r];
+}
+
 }  // namespace
 
 extern "C" {
@@ -523,6 +596,17 @@ void sm_moe_route(const float* logits, int64_t stride, int E, int k, int* ids, f
   }
   hipLaunchKernelGGL(moe_route_kernel, dim3((T + 255) / 256), dim3(256), 0, stream, logits, stride, E, k, ids, w, T,
                      sigmoid);
+}
+
+// x [M, K] bf16 rows xs apart, w [N, K], y [M, N] fp32. -1: not these operands
+int sm_router(const void* x, int64_t xs, const void* w, int M, int N, int K, float* y, hipStream_t stream) {
+  if (M == 0 || N == 0) return 0;
+  if (K < RCH || K % RCH || K > 2048 || xs % 8 || xs < 0 || xs > (1 << 24) || (((uintptr_t)x | (uintptr_t)w) & 15) || M > 8192 || N > 8192)
+    return -1;
+  const int nb = (N + 15) / 16, blocks = (M + 15) / 16 * nb;
+  if (blocks >= 512) return -1;
+  hipLaunchKernelGGL(router_kernel, dim3(blocks), dim3(256), 0, stream, (const bf16_t*)x, xs, (const bf16_t*)w, M, N, K, nb, y);
+  return 0;
 }
 
 void sm_moe_route_scores(const float* logits, const float* corr, int E, int k, int* ids, float* w, int T, int groups,

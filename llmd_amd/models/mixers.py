@@ -529,7 +529,9 @@ class ScoreMoE(torch.nn.Module):
         self.router32, self.correction32 = self.router.data.float(), self.correction.data.float()
 
     def forward(self, h):
-        logits = F.linear(h.float(), self.router32)
+        logits = sm.router_logits(h, self.router.data)
+        if logits is None:
+            logits = F.linear(h.float(), self.router32)
         ids, w = sm.moe_route_scores(logits, self.correction32, self.k, self.groups, self.keep, self.scale)
         return sm.moe_gated_ffn(h, ids, w, self.w1, self.w2, self.act, limit=self.limit,
                                 extra=self.shared(h) if self.shared is not None else None)
@@ -649,7 +651,9 @@ class SigmoidMoE(torch.nn.Module):
         self.router32 = self.router.data.float()
 
     def forward(self, h):
-        logits = F.linear(h.float(), self.router32)
+        logits = sm.router_logits(h, self.router.data)
+        if logits is None:
+            logits = F.linear(h.float(), self.router32)
         ids, w = sm.moe_route(logits, self.k, sigmoid=True)
         return sm.moe_gated_ffn(h, ids, w, self.w1, self.w2, self.act, scale_input=True)
 

@@ -420,6 +420,11 @@ def gated_act(gu, Fh: int, kind: str, limit: float = 0.0):
     return out
 
 
+def router_logits(x, w):
+    """x w^T in fp32 for bfloat16 x [T, d] and w [N, d] (csrc/seqmix/sm_moe.hip router_kernel), or None."""
+    return native().router_logits(x, w) if x.is_cuda and x.dtype == torch.bfloat16 else None
+
+
 def moe_route_scores(logits, correction, k: int, groups: int = 1, keep: int = 1, scale: float = 1.0):
     """Scores = softmax over ALL router outputs (fp32); the k largest of score + correction are
     chosen (ties: lower index); weights = the chosen scores / (their sum + 1e-20) * scale. ``groups`` > 1: the

@@ -109,3 +109,16 @@ def test_head_product_leaves_the_rest():
     assert not sm.head_product(_rand(65, 8, 128), w, torch.empty(65, 8, 64, device="cuda", dtype=torch.bfloat16))
     assert not sm.head_product(_rand(33, 64, 128), _rand(64, 64, 128), torch.empty(33, 64, 64, device="cuda", dtype=torch.bfloat16))
     assert not sm.head_product(_rand(4, 8, 129)[:, :, 1:], w, out)                                    # off 16 bytes
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 132, 2048), (16, 16, 128), (17, 15, 256), (64, 132, 2048), (300, 8, 384), (800, 132, 2048), (33, 256, 1024)])
+def test_router_logits(M, N, K):
+    """fp32 sums of exact products: each of the four partial sums adds up to 512 times, off by 2^-24 of sum |x w| each."""
+    x, w = _rand(M, K + 64)[:, :K], _rand(N, K, seed=1)
+    y = sm.router_logits(x, w)
+    want = x.double() @ w.double().t()
+    bound = x.double().abs() @ w.double().abs().t() * (min(K // 4, 512) + 3) * 2 ** -24
+    assert y.dtype == torch.float32 and ((y.double() - want).abs() <= bound).all()
+    if (N, K) == (132, 2048):  # the order of the float product in its place
+        assert torch.equal(y, torch.nn.functional.linear(x.float(), w.float()))
+    assert sm.router_logits(x[:, :96], w[:, :96].contiguous()) is None and sm.router_logits(_rand(8192, K), w) is None or N < 16
