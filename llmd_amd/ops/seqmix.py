@@ -129,8 +129,9 @@ def latent_attention(q_abs, cache, tables, row_seq, row_len, scale: float, R: in
         nsplit, split, po, pm = 1, 0, None, None
         rows = H if seq.max_q == 1 else 0   # decode-only step: one token per item, its rows shared by the waves
         span = min(seq.max_len, window + 64) if window else seq.max_len   # keys a row's tiles hold at most
-        if rows and span > 128:
-            # cut the keys into ranges so that items x row blocks x ranges fill the chip: of one tile up to 32 of them, else of two
+        if rows and span > 64:
+            # cut the keys into ranges so that items x row blocks x ranges fill the chip: of one tile up to 32 of them (as a captured
+            # step does, whatever it was captured for: the same bits), else of two
             n = items.shape[0] * -(-H // 16)
             nsplit = max(1, min(-(-LATENT_DECODE_WGS // n), max(span // 128, min(-(-span // 64), 32))))
             split = -(-span // (nsplit * 64)) * 64
