@@ -29,8 +29,7 @@ def _init_weight(t: torch.Tensor, std: float, gen: Optional[torch.Generator] = N
 
 
 def _linear(mod, x, bias):
-    """bf16 weights -> hipBLASLt GEMM, or the decode GEMM kernel for the decode
-    shapes where it measured faster (ops.linear); fp8 weights (quantize_fp8) ->
+    """bf16 and fp32 weights -> the GEMM that ``ops.linear`` has for the sizes; fp8 weights (quantize_fp8) ->
     W8A8 GEMM with dynamic per-token activation scales."""
     w = mod.weight
     if w.dtype == torch.float8_e4m3fn:

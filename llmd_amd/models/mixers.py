@@ -42,7 +42,7 @@ constant is an argument, so another stack can reuse them.
 Recurrent state lives in the engine's state pool (engine/state_cache.py): a mixer with
 ``state_shapes()`` gets its per-slot tensors through ``bind_state``; the step's
 ``AttnMeta.seq`` says which slot each run of tokens continues. Matrix products go to the
-vendor GEMM through ``ops.linear``; everything between them runs in the kernels of
+GEMM through ``ops.linear``; everything between them runs in the kernels of
 ``ops.seqmix`` (fp32 where the recurrences, norms and scores need it).
 """
 from __future__ import annotations
