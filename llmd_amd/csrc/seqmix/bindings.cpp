@@ -45,6 +45,8 @@ int sm_gdelta_scan(const void*, int64_t, const void*, const void*, const void*, 
                    const int*, const int*, const int*, void*, int, int, hipStream_t);
 void sm_hyper_embed(const int64_t*, const void*, int64_t, float*, int, int, int, int, hipStream_t);
 void sm_hyper_norm(const float*, const float*, const void*, float, void*, int, int, int, int, int, hipStream_t);
+int sm_hyper_embed_norm(const int64_t*, const void*, int64_t, float*, const float*, const void*, float, void*, int, int, int, int,
+                        int, hipStream_t);
 int sm_hyper_update_norm(float*, const void*, int64_t, const float*, int, const float*, const float*, const float*, const void*,
                          float, void*, int, int, int, int, int, hipStream_t);
 int sm_gated_act(const void*, const float*, int, int64_t, int, int, void*, int, int, float, hipStream_t);
@@ -395,6 +397,26 @@ void hyper_norm(Tensor X, Tensor w_in, Tensor norm_w, double eps, Tensor out, bo
   TORCH_CHECK(out.is_contiguous() && out.dim() == 2 && out.size(0) == T && out.size(1) == d, "out [T, d]");
   sm_hyper_norm(X.data_ptr<float>(), w_in.data_ptr<float>(), norm_w.data_ptr(), (float)eps, out.data_ptr(), S, T, d,
                 rms ? 1 : 0, is_f32(norm_w), cur());
+}
+
+// hyper_embed, then hyper_norm of its streams
+void hyper_embed_norm(Tensor ids, Tensor table, Tensor X, Tensor w_in, Tensor norm_w, double eps, Tensor out, bool rms) {
+  const c10::hip::OptionalHIPGuard g(dev_of(ids));
+  TORCH_CHECK(ids.is_cuda() && ids.scalar_type() == torch::kInt64 && ids.is_contiguous(), "ids: int64");
+  TORCH_CHECK(table.is_cuda() && act_ok(table) && table.dim() == 2 && table.is_contiguous(), "table");
+  check_streams(X);
+  CHECK_F32(w_in);
+  CHECK_ACT(norm_w, table);
+  CHECK_ACT(out, table);
+  const int S = X.size(0), T = ids.numel(), d = table.size(1);
+  TORCH_CHECK(X.size(1) == T && X.size(2) == d, "X [S, T, d]");
+  TORCH_CHECK(w_in.numel() == S && norm_w.is_contiguous() && norm_w.numel() == d && out.is_contiguous() && out.dim() == 2 &&
+                  out.size(0) == T && out.size(1) == d, "weights, out [T, d]");
+  if (sm_hyper_embed_norm(ids.data_ptr<int64_t>(), table.data_ptr(), table.size(0), X.data_ptr<float>(), w_in.data_ptr<float>(),
+                          norm_w.data_ptr(), (float)eps, out.data_ptr(), S, T, d, rms ? 1 : 0, is_f32(table), cur()) != 0) {
+    hyper_embed(ids, table, X);
+    hyper_norm(X, w_in, norm_w, eps, out, rms);
+  }
 }
 
 // out[t][h] = x[t][h] w[h]^T: x [T, H, K] and out [T, H, N] with neighbouring last elements, w [H, N, K]; false: not these operands
@@ -1132,6 +1154,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("moe_combine", &moe_combine);
   m.def("bigram_embed", &bigram_embed);
   m.def("post_norm_add", &post_norm_add);
+  m.def("hyper_embed_norm", &hyper_embed_norm);
   m.def("router_logits", &router_logits);
   m.def("head_product", &head_product);
   m.def("gated_delta_scan", &gated_delta_scan);

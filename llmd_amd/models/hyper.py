@@ -41,9 +41,8 @@ def stream_stack(ids, table, ones, subs, final_norm, eps: float, dtype, rms: boo
     sublayer in order; ``ones`` [S] fp32 reads the plain sum for the final norm. Returns that norm's
     output; ``layer_out``: optional list that receives the sum of the streams after every layer."""
     X = torch.empty(ones.numel(), ids.shape[0], table.shape[1], dtype=torch.float32, device=ids.device)
-    sm.hyper_embed(ids, table, X)
     first_in, first_w = (subs[0][0].in32, subs[0][1]) if subs else (ones, final_norm)
-    h = sm.hyper_norm(X, first_in, first_w, eps, dtype, rms)
+    h = sm.hyper_embed_norm(ids, table, X, first_in, first_w, eps, dtype, rms)
     for i, (hc, _, fn, ends_layer) in enumerate(subs):
         nxt_in, nxt_w = (subs[i + 1][0].in32, subs[i + 1][1]) if i + 1 < len(subs) else (ones, final_norm)
         h = sm.hyper_update_norm(X, fn(h), hc.mix32, hc.out32, nxt_in, nxt_w, eps, dtype, rms)

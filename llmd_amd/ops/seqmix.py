@@ -275,6 +275,16 @@ def hyper_norm(X, w_in, norm_w, eps: float, out_dtype, rms: bool = False):
     return out
 
 
+def hyper_embed_norm(ids, table, X, w_in, norm_w, eps: float, out_dtype, rms: bool = False):
+    """``hyper_embed`` and the ``hyper_norm`` of its streams, in one pass."""
+    if not ids.is_cuda or table.dtype != out_dtype or norm_w.dtype != out_dtype:
+        hyper_embed(ids, table, X)
+        return hyper_norm(X, w_in, norm_w, eps, out_dtype, rms)
+    out = torch.empty(X.shape[1:], dtype=out_dtype, device=X.device)
+    native().hyper_embed_norm(ids, table, X, w_in, norm_w, float(eps), out, bool(rms))
+    return out
+
+
 def hyper_update_norm(X, y, mix, w_out, next_in=None, next_w=None, eps: float = 0.0, out_dtype=None,
                       rms: bool = False):
     """X[t] <- sum_s mix[s, t] X[s] + w_out[t] y for all streams at once, in place (fp32); with

@@ -122,3 +122,18 @@ def test_router_logits(M, N, K):
     if (N, K) == (132, 2048):  # the order of the float product in its place
         assert torch.equal(y, torch.nn.functional.linear(x.float(), w.float()))
     assert sm.router_logits(x[:, :96], w[:, :96].contiguous()) is None and sm.router_logits(_rand(8192, K), w) is None or N < 16
+
+
+@pytest.mark.parametrize("T,d,S", [(1, 2048, 2), (64, 2048, 1), (5, 1000, 3), (3, 4096, 4), (2, 4104, 2), (7, 17, 16)])
+@pytest.mark.parametrize("rms", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_embedding_and_first_norm(T, d, S, rms, dtype):
+    """The bits of the two passes; ids outside the table give zeros."""
+    table, w, w_in = _rand(50, d, dtype=dtype), _rand(d, seed=1, dtype=dtype), _rand(S, dtype=torch.float32)
+    ids = torch.arange(T, device="cuda") * 7 % 50
+    ids[-1] = 50 if T > 1 else 3
+    X0, X1 = (torch.full((S, T, d), float("nan"), device="cuda") for _ in range(2))
+    sm.hyper_embed(ids, table, X0)
+    a = sm.hyper_norm(X0, w_in, w, 1e-5, dtype, rms)
+    b = sm.hyper_embed_norm(ids, table, X1, w_in, w, 1e-5, dtype, rms)
+    assert torch.equal(X0, X1) and torch.equal(a, b)
