@@ -418,16 +418,20 @@ __device__ __forceinline__ void moe_tile_many(const MoeTile& t, WRow wrow, Out o
 }
 
 // fp32 on the bf16 units: a number is the sum of three bf16 parts (8 bits of its 24 each, rounded to nearest: exact), and the six
-// products of parts that reach 2^-26 of a product are formed, in fp32 sums. Six 16 x 16 x 32 instructions of 16 cycles for what takes
-// eight of 32 cycles in 16 x 16 x 4 fp32, beside 5.5 vector instructions per number split. Both products with sorting and sum of 128
+// largest products of parts are formed, in fp32 sums: a second part is at most 2^-8 of its number and a third 2^-17, so that each of the
+// two largest products left out is at most 2^-25 of the whole. Numbers are taken times 2^24 and sums times 2^-48: the last bit of the
+// smallest fp32 number, 2^-149, is then a normal bf16 number too (as they are, numbers of 2^-116
+// give sums 2e-6 off and numbers of 2^-132 0.14). Numbers from 2^104 and sums from 2^80 on overflow so and are done again like infinities.
+// Six 16 x 16 x 32 instructions of 16 cycles for what takes eight of 32 cycles in 16 x 16 x 4 fp32, beside 6.5 vector instructions per number split. Both products with sorting and sum of 128
 // gated experts of 2048 x 768 with as many rows each, us, fp32 instructions / parts: 1 row 427 / 434, 16 453 / 449, 32 514 / 493, 44
 // 590 / 524, 64 705 / 580, 80 835 / 660, 120 1240 / 940 (up to 64 rows the weights' stream counts, 414 us at its best); by a
 // skewed router, 700 tokens 631 / 556, 1400 1002 / 805, 2048 1364 / 1072. Off 64 bits, relative: (2048, 768) 1.20e-6 / 1.03e-6, (4096, 2048)
-// 1.75e-6 / 1.53e-6, (1000, 500) 8.7e-7 / 7.4e-7 (fewer roundings of the sums). Elements below 2^-109 lose parts to the units' flush
-// of bf16 denormals.
+// 1.75e-6 / 1.53e-6, (1000, 500) 8.7e-7 / 7.4e-7 (fewer roundings of the sums).
+// The scaling is in none of these times: 128 rows of 8 chosen 327 / 330 us, 700 tokens 576 / 581, 2048 1118 / 1148.
 struct Parts {
   u32x4_t p[3];  // 8 elements: largest part first
 };
+constexpr float SPLIT_UP = 0x1p24f, SPLIT_DOWN = 0x1p-48f;
 // part i of four elements to (lo, hi); x: what is left of them
 __device__ __forceinline__ void take_part(f32x4_t& x, uint32_t& lo, uint32_t& hi) {
   // (as casts, hipcc rounds every element twice: once for its pair, once to subtract it)
@@ -437,7 +441,7 @@ __device__ __forceinline__ void take_part(f32x4_t& x, uint32_t& lo, uint32_t& hi
   x[2] -= __uint_as_float(hi << 16), x[3] -= __uint_as_float(hi & 0xffff0000u);
 }
 __device__ __forceinline__ Parts split8(const u32x4_t& first, const u32x4_t& second) {
-  f32x4_t x = __builtin_bit_cast(f32x4_t, first), y = __builtin_bit_cast(f32x4_t, second);
+  f32x4_t x = __builtin_bit_cast(f32x4_t, first) * SPLIT_UP, y = __builtin_bit_cast(f32x4_t, second) * SPLIT_UP;
   Parts r;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
@@ -492,7 +496,7 @@ __device__ __forceinline__ bool moe_tile_split(const MoeTile& t, WRow wrow, Out 
     }
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
-      f32x4_t x = __builtin_bit_cast(f32x4_t, ab[s][i]);
+      f32x4_t x = __builtin_bit_cast(f32x4_t, ab[s][i]) * SPLIT_UP;
 #pragma unroll
       for (int p = 0; p < 3; ++p) {
         uint32_t lo, hi;
@@ -579,7 +583,7 @@ __device__ __forceinline__ bool moe_tile_split(const MoeTile& t, WRow wrow, Out 
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) finite &= fabsf(acc[c][i][q]) < INFINITY;
+      for (int q = 0; q < 4; ++q) finite &= fabsf(acc[c][i][q]) < INFINITY, acc[c][i][q] *= SPLIT_DOWN;
     uint64_t m = __ballot(!finite);
     m |= m >> 32;
     m |= m >> 16;

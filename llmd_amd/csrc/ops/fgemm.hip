@@ -1,9 +1,11 @@
-// fp32 products y[M, N] = x[M, K] . w[N, K]^T (+ bias) of prompt-sized steps on the bf16 matrix units: every number is the exact
-// sum of three bf16 parts, and the six products of parts that reach 2^-26 of a product are formed in fp32 sums, the largest ones in
-// sums of their own, so that a sum is rounded once per 32 products (moe_tile.h has the same for experts).
+// fp32 products y[M, N] = x[M, K] . w[N, K]^T (+ bias) of prompt-sized steps on the bf16 matrix units: every number, times 2^24, is the
+// exact sum of three bf16 parts, and the six largest of the nine products of parts are formed in fp32 sums (what is left out is at most
+// 2^-24 of a product: moe_tile.h, which has the same for experts), the largest ones in sums of their own, so that a sum is rounded once
+// per 32 products.
 //
-// What bounds it: 96 products of parts (16 cycles each) and some 200 vector instructions to split the next numbers, of which a SIMD
-// takes two beside a product without losing time, per 128 x 128 x 32: 1536 cycles at least, 2300 measured. Each number is
+// What bounds it: 96 products of parts (16 cycles each) and some 230 vector instructions to scale and split the next numbers, of which a
+// SIMD takes two beside a product without losing time, per 128 x 128 x 32: 1536 cycles at least, 2300 measured without the scaling,
+// which costs 2 to 3 % (700 x (3072, 2048) 59.8 / 61.6 us, 2048 x (5120, 2048) 240 / 246). Each number is
 // split once per workgroup, on its way from registers to LDS; the splitting, LDS reads and loads lie between the products in
 // the order they are written here. Three buffers of LDS: a step's first operands are read beside the step before it.
 //
@@ -83,7 +85,8 @@ __global__ __launch_bounds__(256, 1) void fgemm_kernel(const float* __restrict__
   uint32_t v[3][4];
   auto load = [&](int s, int p, int h, int kt) { g[s][p][h] = reinterpret_cast<const f32x4_t*>(src[p] + min(kt, nk - 1) * BK)[h]; };
   auto part = [&](int s, int p, int pair, int o) {
-    const float* x = reinterpret_cast<const float*>(&g[s][p][pair >> 1]) + 2 * (pair & 1);
+    float* x = reinterpret_cast<float*>(&g[s][p][pair >> 1]) + 2 * (pair & 1);
+    if (o == 0) x[0] *= SPLIT_UP, x[1] *= SPLIT_UP;
     asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(v[o][pair]) : "v"(x[0]), "v"(x[1]));
   };
   auto rest = [&](int s, int p, int pair, int o, int h) {
@@ -93,15 +96,15 @@ __global__ __launch_bounds__(256, 1) void fgemm_kernel(const float* __restrict__
   auto put = [&](char* buf, int p, int o) {
     *reinterpret_cast<u32x4_t*>(buf + o * PL + st + p * 4096) = u32x4_t{v[o][0], v[o][1], v[o][2], v[o][3]};
   };
-  constexpr int PER = 33, U = PER * NP, S = 6 * MI * NI;  // side works of a pass and of a step; products of a step
+  constexpr int PER = 33, PI = 57, U = PER * NP, S = 6 * MI * NI;  // side works and instructions of a pass; works, products of a step
   // instructions before side work u
   constexpr auto before = [](int u) {
-    const int q = u % PER, r = q % 13;
-    return u / PER * 49 + (q >= 26 ? 42 + q - 26 : q / 13 * 21 + (r < 4 ? r : 2 * r - 4));
+    const int q = u % PER, r = q % 13, first = q < 13 ? 3 : 1;  // (a pair's first part: two products and the rounding)
+    return u / PER * PI + (q >= 26 ? 50 + q - 26 : q / 13 * 29 + (r < 4 ? first * r : 4 * first + 2 * (r - 4)));
   };
   constexpr auto first_at = [before](int n) {  // the first side work from product n on
     int u = 0;
-    while (u < U && before(u) * S < n * (NP * 49)) ++u;
+    while (u < U && before(u) * S < n * (NP * PI)) ++u;
     return u;
   };
   // side work u: the pass's 4 pairs split part by part, each part's 16 bytes to LDS, the pass's next loads
@@ -203,7 +206,7 @@ __global__ __launch_bounds__(256, 1) void fgemm_kernel(const float* __restrict__
     for (int j = 0; j < NI; ++j) {
       big[i][j] = big[i][j] + small[i][j];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) finite &= fabsf(big[i][j][q]) < INFINITY;
+      for (int q = 0; q < 4; ++q) finite &= fabsf(big[i][j][q]) < INFINITY, big[i][j][q] *= SPLIT_DOWN;
     }
     if (!finite) marks[wr * 16 * MI + 16 * i + r16] = 1;
   }
@@ -261,7 +264,7 @@ struct Tile {
   int mi, ni, per_cu;
   double one, full;
 };
-constexpr Tile TILES[] = {{4, 4, 1, 1.06, 1.16}, {3, 3, 1, 0.75, 0.80}, {4, 2, 1, 0.73, 0.78}, {2, 2, 2, 0.50, 0.79}};
+constexpr Tile TILES[] = {{4, 4, 1, 1.09, 1.19}, {3, 3, 1, 0.77, 0.82}, {4, 2, 1, 0.75, 0.80}, {2, 2, 2, 0.51, 0.81}};
 
 }  // namespace
 

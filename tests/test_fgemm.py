@@ -13,14 +13,14 @@ def _operands(M, N, K):
     return x * torch.exp(2 * torch.randn(M, K, generator=g, device="cuda")), torch.randn(N, K, generator=g, device="cuda")
 
 
-def _close(y, x, w, bias=None):
+def _close(y, x, w, bias=None, least=0.0):
     ref, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
     if bias is not None:
         ref, size = ref + bias.double(), size + bias.double().abs()
     # per 32 products a rounding of the sum to the nearest (the six kinds of products of parts apart: a sixteenth of that), the parts
-    # left out 2^-25 of a product, and the roundings of ranges and bias
+    # left out at most 2^-24 of a product, and the roundings of ranges and bias
     K = x.shape[1]
-    assert ((y.double() - ref).abs() <= size * (K / 32 * 1.1 + 8) * 2.0 ** -24).all()
+    assert ((y.double() - ref).abs() <= size * (K / 32 * 1.1 + 8) * 2.0 ** -24 + least).all()
 
 
 @pytest.mark.parametrize("mi,ni", [(4, 4), (3, 3), (4, 2), (2, 2)])
@@ -45,6 +45,18 @@ def test_ranges_of_k(M, N, K, code):
     bias = torch.linspace(-2, 2, N, device="cuda")
     _close(ops.native().fgemm(x, w, None, code), x, w)
     _close(ops.native().fgemm(x, w, bias, code), x, w, bias)
+
+
+@pytest.mark.parametrize("code", [441, 332, 421, 221])
+@pytest.mark.parametrize("ex,ew", [(-104, 0), (-112, 0), (0, -116), (-124, 100), (60, -132), (-140, 120), (-60, -56), (90, -100), (50, 40)])
+def test_small_and_large_numbers(ex, ew, code):
+    """Numbers all of whose parts or some of them are below bf16's normal range, among them fp32's own denormals; numbers and sums that
+    overflow when scaled. The same relative bound, but for the last bit of a denormal sum."""
+    x, w = _operands(140, 100, 32 * 9 + 4)
+    x, w = (x.double() * 2.0 ** ex).float(), (w.double() * 2.0 ** ew).float()
+    y = ops.native().fgemm(x, w, None, code)
+    assert y.abs().max() > 0
+    _close(y, x, w, least=2.0 ** -149)
 
 
 @pytest.mark.parametrize("code", [441, 331, 421, 221, 222])

@@ -146,3 +146,26 @@ def test_float32_rows_alone_and_together(d, F):
         full = torch.where(z.isnan(), 0.0, z.clamp(min=0) ** 2).float()
         want = torch.where(full[None] * w2[e[r]] == 0, torch.zeros(()), full[None] * w2[e[r]])
         assert torch.equal(out[r].isfinite(), torch.isfinite(want.sum(1)))
+
+
+@pytest.mark.parametrize("ex,ew", [(-112, 0), (-124, 60), (0, -116), (60, -132), (-135, 70)])
+def test_float32_small_numbers(ex, ew):
+    """Rows and weights whose bf16 parts reach below bf16's normal range, fp32's own denormals among them: within the relative bound of
+    ordinary numbers, through both products. The clamped units of sums z this small are z / 2, and the second weights pick them."""
+    from llmd_amd.ops import seqmix as sm
+
+    g = torch.Generator().manual_seed(7)
+    d, F, E = 100, 72, 4
+    ids = _counts_to_ids([9, 30, 60, 110], 0)
+    T = ids.shape[0]
+    up = lambda t, e: (t.double() * 2.0 ** e).float()  # noqa: E731
+    h, w1 = up(torch.randn(T, d, generator=g), ex), up(torch.randn(E, F, d, generator=g) / d ** 0.5, ew)
+    w2 = torch.eye(d, F).expand(E, d, F).contiguous()
+    got = sm.moe_gated_ffn(h.cuda(), ids.cuda(), torch.ones(T, 1, device="cuda"), torch.cat([w1, w1], 1).cuda(), w2.cuda(),
+                           "swish_limit", limit=1e30).cpu().double()
+    e = ids[:, 0].long()
+    z = torch.einsum("td,tfd->tf", h.double(), w1.double()[e])
+    size = torch.einsum("td,tfd->tf", h.double().abs(), w1.double()[e].abs())
+    # d fp32 additions at worst, the units' reciprocal and products, the last bit of denormal results
+    bound = size / 2 * (d + 8) * 2.0 ** -24 + z.abs() * 2.0 ** -20 + 2.0 ** -148
+    assert ((got[:, :F] - z / 2).abs() <= bound).all() and got[:, :F].abs().max() > 0 and (got[:, F:] == 0).all()
