@@ -173,8 +173,14 @@ class WeightSync:
         return True
 
     def _finish(self, n: int, t0: float, src: str, weights_id: str) -> dict:
-        if self.runner.is_gpu:
-            torch.cuda.synchronize(self.runner.device)
+        r = self.runner
+        if r.is_gpu:
+            torch.cuda.synchronize(r.device)
+        if hasattr(r.model, "finalize"):  # constants derived from the weights, and the steps captured with them
+            r.model.finalize()
+            if r.graphs:
+                r.graphs.clear()
+                r.capture_graphs()
         self.version += 1
         self.weights_id = weights_id
         self.weights_pending = False

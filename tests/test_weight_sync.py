@@ -78,6 +78,32 @@ def test_update_from_disk_matches_fresh_engine(tmp_path, model, quant):
     assert _run(eng) == ref
 
 
+STACKS = ["tiny-kakalorn", "tiny-koduzen", "tiny-kokatar", "tiny-negunex", "tiny-zumizen"]
+
+
+def _update_of_a_stack(tmp_path, model, device):
+    a, b = _ckpts(tmp_path, model=model)
+    ref = _run(LLMEngine(_cfg(a, device=device, model=model)))
+    eng = LLMEngine(_cfg(b, device=device, model=model))
+    assert [t for t, _ in _run(eng)] != [t for t, _ in ref]
+    eng.weight_sync_cmd({"op": "update_from_disk", "path": a})
+    assert _run(eng) == ref
+    return eng.runner
+
+
+@pytest.mark.parametrize("model", STACKS)
+def test_update_of_weights_with_derived_constants(tmp_path, model):
+    """Stacks that keep constants made from their weights (transposed latent matrices, fp32 routers, decays): made again."""
+    _update_of_a_stack(tmp_path, model, "cpu")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", STACKS)
+def test_update_of_weights_with_derived_constants_gpu(tmp_path, model):
+    r = _update_of_a_stack(tmp_path, model, "cuda")
+    assert r.graphs and r._graph_constants == r._seq_constants  # captured again with them
+
+
 def _tp_worker(rank, world, port, ws_port, a, b, out):
     """rank 0: trainer (WeightSender); ranks 1, 2: TP=2 engine (driver, follower)."""
     from safetensors.torch import load_file
