@@ -73,7 +73,7 @@ class KakalornLayer(torch.nn.Module):
         self.canon1 = InputConv(d, cfg.conv_taps, device, dtype)
         self.mix = make_mixer(spec, d, eps, max_pos, device, dtype, earlier)
         self.mlp = make_mlp(spec.get("mlp"), d, device, dtype)
-        reads_parts(self.mix, self.mlp)
+        reads_parts(sm.norm_reads_parts(d), self.mix, self.mlp)
         for n in ("norm1", "norm1b") + (("norm2", "norm2b") if self.mlp is not None else ()):
             setattr(self, n, _param((d,), device, dtype, fill=1.0))
 

@@ -472,12 +472,13 @@ class GroupedAttention(torch.nn.Module):
         return self.o(o)
 
 
-def reads_parts(*modules):
-    """The residual's pass behind these sublayers (post_norm_add, hyper_update_norm) adds up their last projection's ranges of K."""
+def reads_parts(reads: bool, *modules):
+    """The residual's pass behind these sublayers (post_norm_add, hyper_update_norm) adds up their last projection's ranges of K where it
+    ``reads`` them; where not, the projection adds them up itself."""
     for m in modules:
         last = m.down if isinstance(m, (GatedMLP, SquaredReluMLP)) else getattr(m, "o", None)
         if isinstance(last, ColumnLinear):
-            last.parts = True
+            last.parts = reads
 
 
 class GatedMLP(torch.nn.Module):
@@ -488,7 +489,7 @@ class GatedMLP(torch.nn.Module):
         super().__init__()
         self.ff, self.act, self.limit = ff, act, float(limit)
         self.gate_up = ColumnLinear(d_model, 2 * ff, shard=False, device=device, dtype=dtype)
-        self.gate_up.parts = True
+        self.gate_up.parts = sm.units_read_parts(ff)
         self.down = ColumnLinear(ff, d_model, shard=False, device=device, dtype=dtype)
 
     def forward(self, h):

@@ -27,6 +27,7 @@ import torch
 from llmd_amd import ops
 from llmd_amd.engine.attn_meta import AttnMeta
 from llmd_amd.engine.config import ModelConfig
+from llmd_amd.ops import seqmix as sm
 from llmd_amd.parallel.state import get_state
 
 from .hyper import HyperConnection, stream_stack
@@ -62,7 +63,7 @@ class NegunexLayer(torch.nn.Module):
         S, learned = max(1, cfg.hyper_streams), cfg.hyper_streams > 0
         self.mix = make_mixer(spec, d, self.eps, max_pos, device, dtype)
         self.mlp = make_mlp(spec.get("mlp"), d, device, dtype)
-        reads_parts(self.mix, self.mlp)
+        reads_parts(sm.streams_read_parts(S, d), self.mix, self.mlp)
         self.norm1 = _param((d,), device, dtype, fill=1.0)
         self.hc1 = HyperConnection(S, learned, device, dtype)
         if self.mlp is not None:

@@ -416,6 +416,22 @@ def grouped_attention(q, cache, dim, vdim, scale: float, seq, gate=None, slopes=
     return out
 
 
+def norm_reads_parts(d: int) -> bool:
+    """Whether ``post_norm_add`` reads sums over ranges of K itself: rows that its 16-byte form holds in registers. (Others are added up a
+    launch per range, where the product's own pass is one.)"""
+    return d % 8 == 0 and d <= 8192
+
+
+def streams_read_parts(S: int, d: int) -> bool:
+    """The same of ``hyper_update_norm``: its float4 form, of up to four streams."""
+    return S <= 4 and d % 4 == 0
+
+
+def units_read_parts(F: int) -> bool:
+    """The same of ``gated_act``: its 16-byte form."""
+    return F % 8 == 0
+
+
 ACT_KINDS = {"gelu_tanh": 0, "silu": 1, "swish_limit": 2}
 
 
@@ -523,7 +539,7 @@ def post_norm_add(y, w_post, x, eps: float, out_dtype, next_w=None, y2=None, a: 
 def row_conv(x, w, seq, dtype) -> bool:
     """Whether ``post_norm_add`` over the residual x runs the convolution ``w`` [C, taps] that follows it: a step of single tokens."""
     return (x.is_cuda and dtype == torch.bfloat16 and seq.max_q == 1 and seq.seq_slot.numel() == x.shape[0]
-            and 2 <= w.shape[1] <= 4 and x.shape[1] % 8 == 0 and x.shape[1] <= 8192)
+            and 2 <= w.shape[1] <= 4 and norm_reads_parts(x.shape[1]))
 
 
 def gated_delta_scan(xc, G: int, dk: int, H: int, dv: int, beta_raw, decay_raw, A, dt_bias, gate_raw,

@@ -25,6 +25,36 @@ def test_rule_by_rounds_of_tiles():
     assert ops.decode_rule(17, 10884, 3072) == one and ops.decode_rule(17, 8192, 3072) == (ops.mgemm, (1, 2, 4))
 
 
+@pytest.mark.parametrize("model,streams,reads", [("tiny-koduzen", 4, True), ("tiny-koduzen", 5, False), ("tiny-negunex", 2, True),
+                                                 ("tiny-negunex", 16, False)])
+def test_sums_over_ranges_only_for_streams_that_read_them(model, streams, reads):
+    """hyper_update_norm reads them for up to four streams; the products before more of them add up their ranges themselves."""
+    import dataclasses
+
+    from llmd_amd.engine.config import EngineConfig
+    from llmd_amd.models import build_model
+    from llmd_amd.models.layers import ColumnLinear
+
+    mc = dataclasses.replace(EngineConfig.create(model).model_config, hyper_streams=streams)
+    last = [getattr(m, "o", None) or getattr(m, "down", None) for l in build_model(mc, device="cpu", max_pos=64).layers
+            for m in (l.mix, l.mlp)]
+    last = [m for m in last if isinstance(m, ColumnLinear)]
+    assert last and all(m.parts == reads for m in last)
+
+
+def test_sums_over_ranges_only_for_rows_that_read_them():
+    from llmd_amd.models.mixers import GatedMLP, SquaredReluMLP, reads_parts
+    from llmd_amd.ops import seqmix as sm
+
+    mlp = lambda ff: GatedMLP(64, ff, "silu", "cpu", torch.bfloat16)  # noqa: E731
+    assert mlp(96).gate_up.parts and not mlp(100).gate_up.parts
+    for d, reads in ((8192, True), (8200, False), (2052, False)):
+        m = SquaredReluMLP(8, 8, "cpu", torch.bfloat16)
+        reads_parts(sm.norm_reads_parts(d), m)
+        assert m.down.parts == reads
+    assert sm.streams_read_parts(4, 2052) and not sm.streams_read_parts(4, 2050)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
 @pytest.mark.parametrize("N,K", [(4, 768), (132, 2048), (2128, 2048), (4100, 768), (16380, 1024), (1024, 8192), (2048, 4096),
