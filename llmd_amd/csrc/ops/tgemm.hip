@@ -333,11 +333,13 @@ double tgemm_us(int M, int N, int K, int mi, int ni, int ns) {
 //    47.5, here 50.6; 2048 x (8192, 8192) 180 both). Elsewhere at most 8 % slower than hipBLASLt, on average 22 % faster.
 //  * silu 1: in place of the 256 x 256 tiles of pgemm.hip where these take more than 3 % longer (1429 x (28672, 4096) 300 / 252,
 //    2048: 359 / 352; 2300: 399 / 399, not taken). silu 2: in place of a product and the activation's own pass, where no
-//    more than 5 % slower than 256 x 256 tiles. Both above mgemm.hip's 256 rows (100 x (28672, 4096): 51, here 53).
+//    more than 5 % slower than 256 x 256 tiles, and only where that product itself has one range of K: 512 x (512, 8192) in two ranges with the
+//    activation behind it 18 us, here 26; 300 x (1024, 8192) 23 / 28; of 3500 such sizes the two were 24 % faster on average. Both above mgemm.hip's 256 rows (100 x (28672, 4096): 51, here 53).
 //  * More than one range of K only for what the chip takes at once, ranges of at least 8 steps, and where it gains 10 %: 512 x (4096,
 //    14336) 98 with one, 65 with four. Sums of at most 256 MB.
 extern "C" int llmd_tgemm_plan(int M, int N, int K, int silu) {
   if (M < (silu ? 257 : 65) || N < 8 || K < BK || K % BK) return 0;
+  if (silu == 2 && llmd_tgemm_plan(M, N, K, 0) % 10 > 1) return 0;
   double best = 1e30;
   int code = 0, area = 0;
   const int nk = K / BK;

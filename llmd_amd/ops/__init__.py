@@ -1454,8 +1454,8 @@ def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
 def tgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, act: int = 0, limit: float = 0.0):
     """x w^T (+ bias) on the GEMM whose tile fits the sizes (csrc/ops/tgemm.hip, which holds the rule), or None where it is not taken.
     act: silu(x wg^T) * (x wu^T) for w = [gate; up], 1: of the fp32 sums as ``pgemm_silu`` variant 6, 2: of the sums in bf16, the bits
-    of ``linear`` + ``gated_act``; 3: max(0, x w^T)^2 of the sums in bf16; 4: the clamped units of act 2's operands, the bits of
-    ``linear`` + ``seqmix.gated_act``."""
+    of the product (one range of K) + ``gated_act``; 3: max(0, x w^T)^2 of the sums in bf16; 4: the clamped units of act 2's operands,
+    the bits of the product + ``seqmix.gated_act``."""
     if PGEMM_AUTO == "0" or not _gpu(x) or not _plain(x, w):
         return None
     return native().tgemm(x, w, bias, act, 0, limit)

@@ -66,6 +66,16 @@ def test_linear_takes_it(M, N, K):
     assert torch.equal(y[:65], ops.native().tgemm(x[:65], w, None, 0, 221))
 
 
+def test_gated_forms_where_the_product_is_whole():
+    """In place of a product and the activation's pass only where that product has one range of K: its bits, and no slower."""
+    plan = ops.native().tgemm_plan
+    assert plan(1429, 11264, 2048, 2) and plan(300, 1024, 8192, 0) % 10 > 1
+    for M in (257, 300, 385, 512, 1000, 2048, 4500):
+        for N in (256, 512, 1024, 2048, 11264):
+            for K in (512, 2048, 4096, 8192, 16384):
+                assert plan(M, N, K, 0) % 10 <= 1 or plan(M, N, K, 2) == 0, (M, N, K)
+
+
 @pytest.mark.gpu
 def test_refused_or_left():
     """Operands that the kernel does not read stay with the library; one of its tiles for another shape raises."""
