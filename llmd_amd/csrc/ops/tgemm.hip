@@ -324,13 +324,30 @@ double tgemm_us(int M, int N, int K, int mi, int ni, int ns) {
   return t;
 }
 
+// Whole products on which hipBLASLt is the faster one more often than not, from 21 us on (below it is on 0.3 % of them by more than 3 %):
+//  * tiles for two thirds of the CUs: a product of few rows that waits for its weights, 128 x (15360, 8448) 63 / 87;
+//  * columns in whole tiles of 256, and 256 x 256 tiles whose rounds the outputs fill by more than 0.6: the library overlaps a round's
+//    fixed part with the next one, 3456 x (14848, 576) 74 / 88, 6272 x (3840, 3008) 116 / 126. Below 51 us only at K 512
+//    and less and fuller rounds (2560 x (5120, 2560), 0.78 full, 62.6 / 61.0), from 190 us on only up to K 1024, elsewhere the two are the same.
+// 57500 random sizes (M 65 .. 8192, N 64 .. 32768, K 256 .. 16384, half of each on whole tiles; weights from memory), the library's time over
+// the one here: 1.79 on average, below 0.95 in 3.3 % of them, below 0.90 in 1.0 %. On these 2.2 % of the sizes it is 0.975 on average,
+// and without them the others' shares are 2.3 % and 0.4 %, the lowest 0.77 (640 x (19200, 768)).
+bool left_to_library(int M, int N, int K, int mi, int ni, double us) {
+  if (us <= 21) return false;
+  const int64_t tiles = (int64_t)((M + 32 * mi - 1) / (32 * mi)) * ((N + 32 * ni - 1) / (32 * ni));
+  if (3 * tiles <= 2 * NUM_CUS) return true;
+  const int64_t big = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
+  const double full = (double)M * N / ((double)((big + 255) / 256) * 256 * 65536);
+  return N % 256 == 0 && (us > 51 ? full > 0.6 && (us <= 190 || K <= 1024) : K <= 512 && full > 0.75);
+}
+
 }  // namespace
 
 // The tile for a product of these sizes, as mi * 100 + ni * 10 + ranges of K, or 0: not here. N: rows of W (with silu
 // those of gate and up).
 //  * Below 65 rows the decode kernels.
 //  * Whole products with 256 x 256 tiles and, up to K 2048, those of 256 x 224: pgemm.hip or hipBLASLt as before (2551 x (5632, 2048): hipBLASLt
-//    47.5, here 50.6; 2048 x (8192, 8192) 180 both). Elsewhere at most 8 % slower than hipBLASLt, on average 22 % faster.
+//    47.5, here 50.6; 2048 x (8192, 8192) 180 both), and those that left_to_library has.
 //  * silu 1: in place of the 256 x 256 tiles of pgemm.hip where these take more than 3 % longer (1429 x (28672, 4096) 300 / 252,
 //    2048: 359 / 352; 2300: 399 / 399, not taken). silu 2: in place of a product and the activation's own pass, where no
 //    more than 5 % slower than 256 x 256 tiles, and only where that product itself has one range of K: 512 x (512, 8192) in two ranges with the
@@ -357,7 +374,8 @@ extern "C" int llmd_tgemm_plan(int M, int N, int K, int silu) {
       }
     }
   }
-  if (code % 10 == 1 && (area >= 64 || (K <= 2048 && area >= 56 && !silu))) return 0;
+  if (code % 10 == 1 && (area >= 64 || (!silu && ((K <= 2048 && area >= 56) || left_to_library(M, N, K, code / 100, code / 10 % 10, best)))))
+    return 0;
   if (silu && best > (silu == 1 ? 0.97 : 1.05) * tgemm_us(M, N, K, 8, 8, 1)) return 0;
   return code;
 }
