@@ -17,13 +17,14 @@
 // k-steps ahead in two statically indexed register sets.
 // Epilogue (act 1: the rows' max(0, .)^2, of the numbers in bf16): bf16 rows when the K range is whole (gridDim.y == 1), else fp32
 // partials [split][M][N] summed and rounded by dgemm_reduce_kernel. act 2, whole ranges only: W = [gate; up] of N rows each, a block
-// of 16 rows is 8 of gate and the same 8 of up, and silu(gate) * up of the numbers in bf16 is stored, the bits of a pass of its own.
+// of 16 rows is 8 of gate and the same 8 of up, and silu(gate) * up of the numbers in bf16 is stored. A pass of its own gives the same but where
+// the sums, whose order begins elsewhere in K (rot below), fall on the next number in bf16.
 //
 // NORM: X is rmsnorm(x + res) * gamma, made by every workgroup for itself (the bits of rmsnorm.hip's fused add: the same chunks per
 // thread, the same sums) and kept in LDS while its first weights are on their way; the first workgroup stores x + res to res_out, another
 // buffer than res, which later workgroups still read. Bound by the weights as without it: what it saves is the norm's launch.
 // us of norm, product and (28672) SiLU in a row, apart / here: one row (6144, 4096) 15.9 / 14.7, (28672, 4096) 50.5 / 46.0, (2048, 2048)
-// 7.4 / 6.2, two rows 16.2 / 16.1, 52.4 / 50.9, 7.5 / 7.3; four rows lose (16.7 / 19.1): their norms are longer than the launch.
+// 7.4 / 6.2, two rows 16.2 / 16.1, 52.4 / 50.9, 7.5 / 7.3; four rows lost (16.7 / 19.1): their norms are longer than the launch.
 #include "llmd_common.h"
 
 using namespace llmd;
@@ -44,7 +45,7 @@ struct Norm {
 };
 
 constexpr int NORM_K = 8192;      // row width of the NORM form
-constexpr int NORM_ROWS = 4;      // and its rows
+constexpr int NORM_ROWS = 2;      // and its rows
 
 template <int RB, int MB, int U, int OCC, bool NORM>
 __device__ __forceinline__ void dgemm(const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ wt,

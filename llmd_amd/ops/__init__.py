@@ -1197,7 +1197,8 @@ SKINNY_TUNED: dict[tuple[int, int, int], tuple[int, int, int]] = {}
 
 def skinny_gemm(x: torch.Tensor, w: torch.Tensor, plan: Optional[tuple[int, int, int]] = None,
                 act: int = 0) -> torch.Tensor:
-    """act 1: max(0, .)^2 of the numbers in bf16; 2: silu(x wg^T) * (x wu^T) of them for w = [gate; up] and one range of K."""
+    """act 1: max(0, .)^2 of the numbers in bf16; 2: silu(x wg^T) * (x wu^T) of them for w = [gate; up] and one range of K (sums in another
+    order than act 0's, where tiles of gate and up rows begin elsewhere in K)."""
     M, K = x.shape
     N = w.shape[0] // 2 if act == 2 else w.shape[0]
     rb, ns, occ = plan or skinny_plan(M, w.shape[0], K)
@@ -1224,8 +1225,8 @@ NORM_ROWS = 2  # rows up to which each workgroup of the stream kernel norms them
 
 def norm_linear(x: torch.Tensor, residual: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch.Tensor, silu: bool = False):
     """(``linear`` of rmsnorm(x + residual) * gamma, x + residual) in one launch where the stream kernel takes the product of a few
-    rows, else None; silu: silu(. wg^T) * (. wu^T) for w = [gate; up]. The bits of ``fused_add_rms_norm``, ``linear`` and ``gated_act``,
-    but residual itself is left alone."""
+    rows, else None; silu: silu(. wg^T) * (. wu^T) for w = [gate; up]. The bits of ``fused_add_rms_norm`` and ``linear`` (silu: of
+    ``skinny_gemm``'s act 2), but residual itself is left alone."""
     if (x.dim() != 2 or x.shape[0] > NORM_ROWS or x.shape[1] > 8192 or residual.shape != x.shape or residual.dtype != x.dtype
             or gamma.dtype != x.dtype or (silu and w.shape[0] % 16) or residual.stride(1) != 1 or residual.stride(0) % 8
             or residual.data_ptr() % 16 or gamma.data_ptr() % 16):
@@ -1645,7 +1646,7 @@ def _other_kernel(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def linear_clamped(x: torch.Tensor, w: torch.Tensor, limit: float):
     """g sigmoid(1.702 g) (u + 1) with g = min(x wg^T, limit), u = clamp(x wu^T, -limit, limit), w = [gate; up], in the product's
-    epilogue: the bits of ``linear`` and ``seqmix.gated_act``, or None where not there. 2048 x (3072, 2048) 32.8 + 5.8 us, here
+    epilogue: the bits of the whole product and ``seqmix.gated_act``, or None where not there. 2048 x (3072, 2048) 32.8 + 5.8 us, here
     32.7; 2722 x (11264, 2048) 111.6 + 16.4, here 120.4."""
     if x.dim() != 2 or not _gpu(x) or x.shape[0] <= 256 or _other_kernel(x, w):
         return None

@@ -92,26 +92,52 @@ def _same_silu(got, want):
     assert ((got - want).abs() <= 2 ** -7 * 9 * want.abs() + 1e-3).all() and (got != want).float().mean() < 0.02
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(1, 6144, 4096), (1, 28672, 4096), (1, 2048, 2048), (1, 528, 1024), (1, 4096, 768), (2, 6144, 4096),
-                                   (3, 1040, 2048), (4, 1024, 8192)])
-def test_norm_and_silu_in_the_stream_kernel(M, N, K, monkeypatch):
-    """The bits of fused_add_rms_norm and linear, or skinny_gemm's SiLU, and a residual that stays."""
-    monkeypatch.setattr(ops, "NORM_ROWS", 4)
+def _normed(M, N, K):
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     x, r = (torch.randn(M, K, device="cuda", dtype=torch.bfloat16, generator=g) for _ in range(2))
     w = torch.randn(N, K, device="cuda", dtype=torch.bfloat16, generator=g) * K ** -0.5
     gamma = torch.randn(K, device="cuda", dtype=torch.bfloat16, generator=g)
-    if (plan := ops.skinny_whole(x, w)) is None:
-        pytest.skip("another kernel takes this product")
-    x1, r1, r0 = x.clone(), r.clone(), r.clone()
+    x1, r1 = x.clone(), r.clone()
     ops.fused_add_rms_norm(x1, r1, gamma, 1e-5)
+    return x, r, w, gamma, x1, r1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 6144, 4096), (1, 28672, 4096), (1, 2048, 2048), (1, 528, 1024), (1, 4096, 768), (2, 6144, 4096),
+                                   (1, 10240, 8192), (1, 8192, 8192)])
+def test_norm_and_silu_in_the_stream_kernel(M, N, K):
+    """The bits of fused_add_rms_norm and linear, or skinny_gemm's SiLU, and a residual that stays."""
+    x, r, w, gamma, x1, r1 = _normed(M, N, K)
+    r0, plan = r.clone(), ops.skinny_whole(x, w)
+    assert plan is not None
     y = ops.linear(x1, w)
     act = ops.skinny_gemm(x1, w, plan, 2)
     _same_silu(act, ops.gated_act(y, ops.ACT_SILU))
     for silu, want in ((False, y), (True, act)):
         out, res = ops.norm_linear(x, r, gamma, 1e-5, w, silu)
         assert torch.equal(out, want) and torch.equal(res, r1) and torch.equal(r, r0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("rb,occ", [(1, 2), (3, 2), (8, 1)])
+@pytest.mark.parametrize("N,K", [(144, 256), (1040, 2048), (400, 4352), (272, 8192)])
+def test_norm_in_the_stream_kernel_of_any_plan(M, rb, occ, N, K):
+    """Rows of one 16-byte piece per thread up to four, with and without a rest; row blocks that N does not fill."""
+    x, r, w, gamma, x1, r1 = _normed(M, N, K)
+    res = torch.empty_like(r)
+    for silu in (False, True):
+        y = torch.empty(M, N // 2 if silu else N, device="cuda", dtype=torch.bfloat16)
+        ops.native().skinny_norm(y, x, r, gamma, 1e-5, res, w, rb, occ, silu)
+        assert torch.equal(y, ops.skinny_gemm(x1, w, (rb, 1, occ), 2 if silu else 0)) and torch.equal(res, r1)
+
+
+@pytest.mark.gpu
+def test_norm_in_the_stream_kernel_of_two_rows_at_most():
+    x, r, w, gamma, _, _ = _normed(3, 1040, 2048)
+    assert ops.norm_linear(x, r, gamma, 1e-5, w) is None
+    with pytest.raises(RuntimeError):
+        ops.native().skinny_norm(torch.empty(3, 1040, device="cuda", dtype=torch.bfloat16), x, r, gamma, 1e-5, torch.empty_like(r), w, 1, 2, False)
 
 
 @pytest.mark.gpu
