@@ -121,7 +121,14 @@ def test_router_logits(M, N, K):
     assert y.dtype == torch.float32 and ((y.double() - want).abs() <= bound).all()
     if (N, K) == (132, 2048):  # the order of the float product in its place
         assert torch.equal(y, torch.nn.functional.linear(x.float(), w.float()))
-    assert sm.router_logits(x[:, :96], w[:, :96].contiguous()) is None and sm.router_logits(_rand(8192, K), w) is None or N < 16
+    assert sm.router_logits(x[:, :96], w[:, :96].contiguous()) is None
+    if N >= 16:  # 512 blocks of 16 x 16 and more
+        assert sm.router_logits(_rand(8192, K), w) is None
+
+
+def test_router_logits_of_longer_rows_stay_with_the_library():
+    """Beyond K 2048 the order of the sums is not the float product's."""
+    assert sm.router_logits(_rand(9, 2048), _rand(132, 2048)) is not None and sm.router_logits(_rand(9, 2176), _rand(132, 2176)) is None
 
 
 @pytest.mark.parametrize("T,d,S", [(1, 2048, 2), (64, 2048, 1), (5, 1000, 3), (3, 4096, 4), (2, 4104, 2), (7, 17, 16)])
