@@ -324,21 +324,20 @@ double tgemm_us(int M, int N, int K, int mi, int ni, int ns) {
   return t;
 }
 
-// Whole products on which hipBLASLt is the faster one more often than not, from 21 us on (below it is on 0.3 % of them by more than 3 %):
-//  * tiles for two thirds of the CUs: a product of few rows that waits for its weights, 128 x (15360, 8448) 63 / 87;
-//  * columns in whole tiles of 256, and 256 x 256 tiles whose rounds the outputs fill by more than 0.6: the library overlaps a round's
-//    fixed part with the next one, 3456 x (14848, 576) 74 / 88, 6272 x (3840, 3008) 116 / 126. Below 51 us only at K 512
-//    and less and fuller rounds (2560 x (5120, 2560), 0.78 full, 62.6 / 61.0), from 190 us on only up to K 1024, elsewhere the two are the same.
-// 57500 random sizes (M 65 .. 8192, N 64 .. 32768, K 256 .. 16384, half of each on whole tiles; weights from memory), the library's time over
-// the one here: 1.79 on average, below 0.95 in 3.3 % of them, below 0.90 in 1.0 %. On these 2.2 % of the sizes it is 0.975 on average,
-// and without them the others' shares are 2.3 % and 0.4 %, the lowest 0.77 (640 x (19200, 768)).
+// Whole products on which hipBLASLt is the faster one:
+//  * 113 to 128 rows on tiles for two thirds of the CUs, products that wait for their weights: its own 128 rows are split over K, 128 x (15168,
+//    6400) 50.3 / 64.7 (105 x (14144, 4288) 43.2 / 39.5, 172 x (19200, 2048) 31.5 / 31.3);
+//  * columns in whole tiles of 256, K up to 1024, and 256 x 256 tiles whose rounds the outputs fill by more than 0.8: it overlaps a round's
+//    fixed part with the next one, 1920 x (28928, 576) 75.6 / 94.2 (K 1024 to 3072 as full: 1.05 times its time on average).
+// 1975 random sizes of 21 us and more (M 65 .. 8192, N 64 .. 32768, K 256 .. 16384, half of each on whole tiles; weights from memory, 50 ms of
+// each product at a time: after a pause the clock tells more than the kernel), the library's time over the one here: 1.23 on average, below
+// 0.95 in 3.8 % of them, below 0.90 in 1.1 %. On these 2 % it is 0.94; of the others 2.9 % are below 0.95 and 0.3 % below 0.90, the lowest 0.88.
+// Below 21 us 0.3 % of 40000 sizes are more than 3 % slower here.
 bool left_to_library(int M, int N, int K, int mi, int ni, double us) {
-  if (us <= 21) return false;
   const int64_t tiles = (int64_t)((M + 32 * mi - 1) / (32 * mi)) * ((N + 32 * ni - 1) / (32 * ni));
-  if (3 * tiles <= 2 * NUM_CUS) return true;
+  if (us > 21 && M > 112 && M <= 128 && 3 * tiles <= 2 * NUM_CUS) return true;
   const int64_t big = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-  const double full = (double)M * N / ((double)((big + 255) / 256) * 256 * 65536);
-  return N % 256 == 0 && (us > 51 ? full > 0.6 && (us <= 190 || K <= 1024) : K <= 512 && full > 0.75);
+  return us > 21 && N % 256 == 0 && K <= 1024 && (double)M * N > 0.8 * (double)((big + 255) / 256 * 256 * 65536);
 }
 
 }  // namespace

@@ -76,11 +76,12 @@ def test_gated_forms_where_the_product_is_whole():
                 assert plan(M, N, K, 0) % 10 <= 1 or plan(M, N, K, 2) == 0, (M, N, K)
 
 
-@pytest.mark.parametrize("M,N,K,left", [(128, 15360, 8448, True), (128, 15360, 2048, False), (3456, 14848, 576, True), (3456, 14800, 576, False),
-                                        (6272, 3840, 3008, True), (5248, 5632, 256, True), (1429, 4096, 4096, False), (2600, 3072, 2048, False)])
+@pytest.mark.parametrize("M,N,K,left", [(128, 15168, 6400, True), (113, 15168, 6400, True), (112, 15168, 6400, False), (128, 15168, 2048, False),
+                                        (128, 18944, 6400, False), (1920, 28928, 576, True), (1920, 28944, 576, False), (1920, 28928, 1088, False),
+                                        (1429, 4096, 4096, False), (2600, 3072, 2048, False)])
 def test_sizes_left_to_the_library(M, N, K, left):
-    """Products for two thirds of the CUs that wait for their weights; columns in whole tiles of 256 that fill the rounds of 256 x 256 tiles;
-    and sizes on the other side of each line."""
+    """128 rows on tiles for two thirds of the CUs that wait for their weights; columns in whole tiles of 256, short K, that fill the rounds
+    of 256 x 256 tiles; and sizes on the other side of each line."""
     assert (ops.native().tgemm_plan(M, N, K, 0) == 0) == left
 
 
