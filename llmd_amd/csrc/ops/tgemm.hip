@@ -307,10 +307,10 @@ __global__ __launch_bounds__(256) void tgemm_reduce_kernel(const float* __restri
 constexpr int TILES[][2] = {TGEMM_TILES(T_TILE){8, 8}};  // (the last one only with several ranges of K)
 #undef T_TILE
 
-// Time of a product in us, fitted to 6000 timings (20 sizes of W, M 65 .. 4500, 36 tiles, one and more ranges of K; off by
-// 6 %; the tile it picks is 0.7 % slower than the best one on average): a round is its tiles' fixed part and its
-// K-steps, each bound by the CU (b: LDS and load path) together with the chip (pw: power, e: L2); the weights' bytes
-// from HBM beside it.
+// Time of a product in us, fitted to 4305 timings (21 sizes of W, M 65 .. 4500, 18 tiles, one and more ranges of K; off by 6 %; the tile it
+// picks is 0.9 % slower than the best one on average; of 2484 random sizes of 21 us and more nine in ten take 3 % less to 21 % more):
+// a round is its tiles' fixed part and its K-steps, each bound by the CU (cu: LDS and load path) together with the chip (chip: power and
+// L2); the weights' bytes from HBM beside it.
 double tgemm_us(int M, int N, int K, int mi, int ni, int ns) {
   const int64_t nt = (int64_t)((M + 32 * mi - 1) / (32 * mi)) * ((N + 32 * ni - 1) / (32 * ni)) * ns;
   const int steps = (K / BK + ns - 1) / ns;
@@ -329,9 +329,9 @@ double tgemm_us(int M, int N, int K, int mi, int ni, int ns) {
 //    6400) 50.3 / 64.7 (105 x (14144, 4288) 43.2 / 39.5, 172 x (19200, 2048) 31.5 / 31.3);
 //  * columns in whole tiles of 256, K up to 1024, and 256 x 256 tiles whose rounds the outputs fill by more than 0.8: it overlaps a round's
 //    fixed part with the next one, 1920 x (28928, 576) 75.6 / 94.2 (K 1024 to 3072 as full: 1.05 times its time on average).
-// 1975 random sizes of 21 us and more (M 65 .. 8192, N 64 .. 32768, K 256 .. 16384, half of each on whole tiles; weights from memory, 50 ms of
-// each product at a time: after a pause the clock tells more than the kernel), the library's time over the one here: 1.23 on average, below
-// 0.95 in 3.8 % of them, below 0.90 in 1.1 %. On these 2 % it is 0.94; of the others 2.9 % are below 0.95 and 0.3 % below 0.90, the lowest 0.88.
+// 2484 random sizes of 21 us and more (M 65 .. 8192, N 64 .. 32768, K 256 .. 16384, half of each on whole tiles; weights from memory, 25 ms of
+// each product at a time: after a pause the clock tells more than the kernel), the library's time over the one here: 1.22 on average, below
+// 0.95 in 4.2 % of them, below 0.90 in 1.3 %. On these 2 % it is 0.94; of the others 3.3 % are below 0.95 and 0.5 % below 0.90, the lowest 0.87.
 // Below 21 us 0.3 % of 40000 sizes are more than 3 % slower here.
 bool left_to_library(int M, int N, int K, int mi, int ni, double us) {
   const int64_t tiles = (int64_t)((M + 32 * mi - 1) / (32 * mi)) * ((N + 32 * ni - 1) / (32 * ni));
