@@ -679,6 +679,110 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int MKT = 32;  // keys per tile
 
+// Online softmax of 16 rows over tiles of 32 keys, shared by the forms for prompts (a row has the same bits in each). A lane holds one
+// row's scores of eight neighbouring keys, 8 kq .. 8 kq + 7 of the tile, which four lanes share.
+// The weights are exp2(score - ref), and a row's ref moves only when one of its own scores passes it by 2^RISE: after a row's
+// first tiles a step has neither a maximum across lanes nor products with the accumulators. Every row decides for itself (one that
+// stays is multiplied by 1), so its bits do not depend on the rows beside it. The sums stay with the lanes until the end.
+constexpr float RISE = 8.f;
+
+// (fmaxf takes an instruction more for each operand)
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float d;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+  return d;
+}
+
+struct RowSoftmax {
+  float ref;   // what the weights are relative to; 0 before the first key
+  float rise;  // ref moves when a score passes it by more: -infinity before the first key
+  float l;     // this lane's part of the sum of weights
+  // a sink is a score that is already counted
+  __device__ __forceinline__ void start(const float* sinks, int head, int kq) {
+    ref = sinks ? sinks[head] * 1.44269504088896341f : 0.f;
+    rise = sinks ? RISE : -INFINITY;
+    l = sinks && kq == 0 ? 1.f : 0.f;
+  }
+  __device__ __forceinline__ float top() const { return rise < 0.f ? -INFINITY : ref; }
+};
+
+// a: the products of this lane's row with keys key0 .. key0 + 7 of a tile (i = 4 kb + r in a[kb][r]); x: what the weights are exp2 of
+__device__ __forceinline__ void row_scores(const f32x4_t (&a)[2], float scale2, float slope, bool sloped, int dist, float ref, float (&x)[8]) {
+  if (sloped) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf(a[i >> 2][i & 3], scale2, __builtin_fmaf(-slope, (float)dist - (float)i, -ref));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf(a[i >> 2][i & 3], scale2, -ref);
+  }
+}
+__device__ __forceinline__ float top8(const float (&x)[8]) {
+  return max3(max3(x[0], x[1], x[2]), max3(x[3], x[4], x[5]), max3(x[6], x[7], x[7]));
+}
+// the weights in two bf16 parts: hi = a weight's upper 16 bits (truncated), lo = the upper 16 bits of the exact rest; hi + lo
+// differs from the fp32 weight by less than 2^-16 of it, with no rounding arithmetic
+__device__ __forceinline__ void row_weights(const float (&x)[8], RowSoftmax& s, bf16x8_t& pah, bf16x8_t& pal) {
+  float p[8];
+  u32x4_t hw, lw;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) p[i] = __builtin_amdgcn_exp2f(x[i]);
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    const uint32_t u0 = __float_as_uint(p[i]), u1 = __float_as_uint(p[i + 1]);
+    const uint32_t r0 = __float_as_uint(p[i] - __uint_as_float(u0 & 0xffff0000u));
+    const uint32_t r1 = __float_as_uint(p[i + 1] - __uint_as_float(u1 & 0xffff0000u));
+    hw[i >> 1] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // the upper halves of both
+    lw[i >> 1] = __builtin_amdgcn_perm(r1, r0, 0x07060302u);
+  }
+  pah = __builtin_bit_cast(bf16x8_t, hw);
+  pal = __builtin_bit_cast(bf16x8_t, lw);
+  s.l += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+}
+// A tile for one block of rows. From mylen on, outside of its chunk (from mylo) and its window (from mywlo, and below keep) a row
+// sees nothing; plain: every row sees the whole tile.
+template <int NCB, bool CALM>
+__device__ __forceinline__ void weigh(const f32x4_t (&a)[2], float scale2, float slope, bool sloped, bool plain, int key0, int mylen,
+                                      int mylo, int mywlo, int keep, RowSoftmax& s, f32x4_t (&o)[NCB], bf16x8_t& pah, bf16x8_t& pal) {
+  float x[8];
+  if (CALM && plain && !sloped) {  // most tiles: no mask, and no row's reference moves
+    row_scores(a, scale2, 0.f, false, 0, s.ref, x);
+    if (!__any(top8(x) > s.rise)) {
+      row_weights(x, s, pah, pal);
+      return;
+    }
+  }
+  auto scores = [&](float ref) {
+    row_scores(a, scale2, slope, sloped, mylen - 1 - key0, ref, x);
+    if (!plain) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int key = key0 + i;
+        const bool in = (key < mylen) & (key >= mylo) & ((key >= mywlo) | (key < keep));
+        x[i] = in ? x[i] : -INFINITY;
+      }
+    }
+  };
+  scores(s.ref);
+  float mx = top8(x);
+  if (__any(mx > s.rise)) {
+    mx = row_max(mx);
+    const bool up = mx > s.rise;
+    const float ref = up ? s.ref + mx : s.ref;
+    const float corr = s.rise < 0.f ? 1.f : __builtin_amdgcn_exp2f(s.ref - ref);  // (nothing summed yet: nothing to correct)
+#pragma unroll
+    for (int n = 0; n < NCB; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[n][r] *= corr;
+    s.l *= corr;
+    s.ref = ref;
+    if (up) s.rise = RISE;
+    scores(ref);
+  }
+  row_weights(x, s, pah, pal);
+}
+// the tile's key that row r of the score product's block kb is: lanes come to hold neighbours
+__device__ __forceinline__ int dealt_key(int r, int kb) { return 8 * (r >> 2) + 4 * kb + (r & 3); }
+
 // DkP = 32 NKS >= dim and VP = 16 NCB >= vdim are the padded sizes (zeros in LDS and in the
 // query fragments). items [n, 3] = (sequence, first token row, tokens), tokens * G <= 64 RB: a wave
 // owns RB blocks of 16 rows (block rb of wave w = item rows 16 (4 rb + w) ..), so a key tile's
@@ -763,16 +867,12 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
       }
       qf[rb][ks] = __builtin_bit_cast(bf16x8_t, v);
     }
-  // o[rb][n][r] = this lane's row, column 16 n + 4 kq + r; m, l: the row's maximum (base 2) and sum of weights so far, the same
-  // in its four lanes
+  // o[rb][n][r] = this lane's row, column 16 n + 4 kq + r
   f32x4_t o[RB][NCB];
-  float m[RB], l[RB];
+  RowSoftmax sm[RB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
-    // a sink is a score that is already counted (by the first key range only)
-    const bool sk = sinks != nullptr && blockIdx.z == 0;
-    m[rb] = sk ? sinks[myhead[rb]] * 1.44269504088896341f : -INFINITY;
-    l[rb] = sk ? 1.f : 0.f;
+    sm[rb].start(blockIdx.z == 0 ? sinks : nullptr, myhead[rb], kq);  // (a sink in the first key range only)
 #pragma unroll
     for (int n = 0; n < NCB; ++n) o[rb][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
@@ -855,19 +955,15 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
     for (int i = 0; i < NCK; ++i) {
       const int e = threadIdx.x + i * NT;
       const int j = e / CK, c = e - j * CK;
-      if (e < MKT * CK && c * 8 < dim) *reinterpret_cast<u32x4_t*>(&kb_[j * KS + c * 8]) = pk[i];
+      // key rows in the order that the lanes read them
+      const int row = (j >> 2 & 1) * 16 + (j >> 3) * 4 + (j & 3);
+      if (e < MKT * CK && c * 8 < dim) *reinterpret_cast<u32x4_t*>(&kb_[row * KS + c * 8]) = pk[i];
     }
 #pragma unroll
     for (int i = 0; i < NCV; ++i) {
       const int e = threadIdx.x + i * NT;
       const int d = e / CV, j8 = e - d * CV;
-      // a value column's keys are stored in the order the weights arrive in: position 8 q + i holds
-      // key 4 q + i (i < 4) or key 16 + 4 q + i - 4, so one 16-byte read gives a lane its eight keys
-      if (d < vdim) {
-        const int base = d * VS + (j8 & 1) * 16 + (j8 >> 1) * 4;
-        *reinterpret_cast<uint2*>(&vb_[base]) = make_uint2(pv[i][0], pv[i][1]);
-        *reinterpret_cast<uint2*>(&vb_[base + 8]) = make_uint2(pv[i][2], pv[i][3]);
-      }
+      if (d < vdim) *reinterpret_cast<u32x4_t*>(&vb_[d * VS + j8 * 8]) = pv[i];
     }
   };
   if (kbeg < kend) fetch(kbeg);
@@ -890,8 +986,10 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
     const bf16_t* const tK = sK + cur * MKT * KS;
     const bf16_t* const tV = sVt + cur * VP * VS;
     const bool plain = k0 >= full_lo && k0 + MKT <= full_hi;  // every key visible to every row: no masks
-    // scores of this lane's rows against keys k0 + 16 kb + 4 kq + r
-    float sc[RB][2][4];
+    // The weights never pass through LDS. After S^T = K Q^T this lane holds, for its query row r16, eight neighbouring keys (the
+    // key rows are dealt so), which is exactly one B operand of the second product O^T += V^T P^T. Its result comes out in the
+    // lanes that own the row, so neither the reference nor the sums ever change lanes.
+    bf16x8_t pah[RB], pal[RB];
     {
       f32x4_t a[RB][2];
 #pragma unroll
@@ -906,71 +1004,8 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
         }
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) sc[rb][i >> 2][i & 3] = a[rb][i >> 2][i & 3] * scale2;
-    }
-    if (!plain) {
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int key = k0 + (i >> 2) * 16 + kq * 4 + (i & 3);
-          const bool in = (key < mylen[rb]) & (key >= mylo[rb]) & ((key >= mywlo[rb]) | (key < keep));
-          float& v = sc[rb][i >> 2][i & 3];
-          v = in ? v - myslope[rb] * (float)(mylen[rb] - 1 - key) : -INFINITY;
-        }
-    } else if (slopes != nullptr) {
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const float dist = (float)(mylen[rb] - 1 - k0 - kq * 4);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) sc[rb][i >> 2][i & 3] -= myslope[rb] * (dist - (float)((i >> 2) * 16 + (i & 3)));
-      }
-    }
-    // The weights never pass through LDS. After S^T = K Q^T this lane holds, for its query row r16, the keys
-    // 4 kq .. 4 kq + 3 of both 16-key halves of the tile - eight keys, which is exactly one B operand of the second product
-    // O^T += V^T P^T if the contraction index is ordered that way; the value operand below is read in the same order (the
-    // order of a contraction is free as long as both operands agree). Its result comes out in the lanes that own the row, so
-    // neither the running maximum nor the sums ever change lanes.
-    bf16x8_t pah[RB], pal[RB];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      float mx = -INFINITY;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[rb][kb][r]);
-      mx = row_max(mx);
-      const float mn = fmaxf(m[rb], mx), mref = mn == -INFINITY ? 0.f : mn;  // a row with no key yet
-      const float corr = __builtin_amdgcn_exp2f(m[rb] - mref);
-      if (__any(corr != 1.f)) {  // some row's maximum moved; a row whose own did not is multiplied by 1
-#pragma unroll
-        for (int n = 0; n < NCB; ++n)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) o[rb][n][r] *= corr;
-      }
-      float psum = 0.f;
-      u32x4_t hw, lw;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        // hi = the weight's upper 16 bits (truncated), lo = the upper 16 bits of the exact rest:
-        // hi + lo differs from the fp32 weight by less than 2^-16 of it, with no rounding arithmetic.
-#pragma unroll
-        for (int r = 0; r < 4; r += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(sc[rb][kb][r] - mref);
-          const float p1 = __builtin_amdgcn_exp2f(sc[rb][kb][r + 1] - mref);
-          psum += p0 + p1;
-          const uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
-          const uint32_t r0 = __float_as_uint(p0 - __uint_as_float(u0 & 0xffff0000u));
-          const uint32_t r1 = __float_as_uint(p1 - __uint_as_float(u1 & 0xffff0000u));
-          hw[kb * 2 + (r >> 1)] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // the upper halves of both
-          lw[kb * 2 + (r >> 1)] = __builtin_amdgcn_perm(r1, r0, 0x07060302u);
-        }
-      }
-      pah[rb] = __builtin_bit_cast(bf16x8_t, hw);
-      pal[rb] = __builtin_bit_cast(bf16x8_t, lw);
-      l[rb] = l[rb] * corr + row_sum(psum);
-      m[rb] = mn;
+        weigh<NCB, true>(a[rb], scale2, myslope[rb], slopes != nullptr, plain, k0 + kq * 8, mylen[rb], mylo[rb], mywlo[rb], keep, sm[rb],
+                   o[rb], pah[rb], pal[rb]);
     }
 #pragma unroll
     for (int n0 = 0; n0 < NCB; n0 += 4) {
@@ -1000,9 +1035,10 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
   const bool fours = (vdim & 3) == 0;
   if (nsplit > 1) {  // RB == 1 (the host splits decode-only steps, whose items have at most 64 rows)
     const int64_t prow = (((int64_t)item * Hkv + g) * nsplit + blockIdx.z) * 64 + wave * 16 + r16;
+    const float l = row_sum(sm[0].l);
     if (kq == 0) {
-      part_ml[prow * 2] = m[0];
-      part_ml[prow * 2 + 1] = l[0];
+      part_ml[prow * 2] = sm[0].top();
+      part_ml[prow * 2 + 1] = l;
     }
 #pragma unroll
     for (int n = 0; n < NCB; ++n) {
@@ -1019,8 +1055,8 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
   }
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
+    const float inv = 1.f / row_sum(sm[rb].l);
     if ((rb * 4 + wave) * 16 + r16 >= ntok * G) continue;
-    const float inv = 1.f / l[rb];
     bf16_t* dst = out + ((int64_t)mytok[rb] * Hq + myhead[rb]) * vdim;
     const bf16_t* gt = gate ? gate + (int64_t)mytok[rb] * gate_stride + myhead[rb] * vdim : nullptr;
 #pragma unroll
@@ -1047,18 +1083,20 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
 }
 
 // Prompts of the usual sizes (dim = 32 NKS and vdim = 16 NCB exactly, pages of whole tiles): the products, masks and softmax
-// of grouped_attention_mfma with less around them. Tiles are copied straight to LDS, the next one into the other buffer while
-// this one is multiplied, so a tile costs no registers, conversions or LDS writes; places of the copies are computed once.
-// A key row's 16-byte pieces lie in the order c ^ (the lane that reads the row), a value column's in c ^ (column / 4), so
-// the lanes of a read meet all banks. Keys enter every sum in the general form's order, so that both give the same bits and the
-// page size of a call does not decide which expert a near tie further on goes to: a lane holds keys 4 kq .. 4 kq + 3 of both
-// halves. It reads one piece of 16 bytes of a value column, eight neighbours, and lanes 16 apart exchange halves (two reads of
-// 8 bytes instead: 91 us where this takes 82). Only a sequence's last tile may hold keys that were never written: its value
-// columns are cleared there. 2048 tokens, 32 heads x 128 over 4 kv heads, window 1024: 67 us;
-// 3 portions of 787 to 901 tokens after 333: 75 us. With a reference that moved only when a row of the wave passed it by 2^8
-// (a row's rounding then depended on the 15 rows beside it) and eight neighbouring keys per lane: the general form 87 / 103 us,
-// this one 57 / 69, two blocks of 16 rows per wave (half the LDS reads) 70 / 76.
-template <int NKS, int NCB>
+// of grouped_attention_mfma with less around them, and the same bits. Tiles are copied straight to LDS, the next one into the other
+// buffer while this one is multiplied, so a tile costs no registers, conversions or LDS writes; places of the copies are computed once.
+// A key row's 16-byte pieces lie in the order c ^ (the lane that reads the row), a value column's in c ^ (-(column / 4) & 3): lanes
+// 0 .. 3 and 12 .. 15 of a read of 16 bytes meet the banks together with lanes 4 .. 11 of the quarter beside theirs, and none meet in one.
+// Only a sequence's last tile may hold keys that were never written: its value columns are cleared there.
+// What bounds it: the waves' own latency (QK, softmax, PV in a row; four waves per SIMD), then the copies' way through the L1.
+// Tiles that every row sees whole and that move no row's reference, nearly all of them, run without masks and corrections.
+// us of 32 heads x 128 over 4 kv heads, window 1024, before (a maximum across lanes and a correction in every tile; waits for the
+// query in the loop, which waited for the copies too; two-way conflicts in the values' reads) and now: 2048 tokens 67.7 / 53.3, without
+// the window 78.2 / 63.6; 3 portions of 787 to 901 tokens after 333 76.3 / 61.2; 635 after 764 41.3 / 32.6; 200 10.7 / 8.8. The general
+// form, the same 2048 tokens on pages of 16: 122 / 110 and 131 / 125.
+// Taken back (same order, 2048 tokens / 635 after 764): two blocks of 16 rows per wave 57.7 / 41.6, eight waves on a tile 59.6 / 36.7,
+// two tiles per barrier 62.2 / 31.5, three and four buffers no different.
+template <int NKS, int NCB, bool SLOPED>
 __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache, const int* __restrict__ tables, int W, int bs,
     const int* __restrict__ items, const int* __restrict__ row_len, float scale, int Hq, int Hkv,
@@ -1080,9 +1118,9 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
   const int mylen = ok ? row_len[mytok] : 0;
   const int mylo = (chunk > 0 && mylen > 0) ? ((mylen - 1) / chunk) * chunk : 0;  // first key of the row's chunk
   const int mywlo = window > 0 ? max(0, mylen - window) : 0;                             // first key of the row's window
-  const float myslope = slopes ? slopes[myhead] * 1.44269504088896341f : 0.f;
-  float m = sinks ? sinks[myhead] * 1.44269504088896341f : -INFINITY;  // a sink is a score that is already counted
-  float l = sinks ? 1.f : 0.f;
+  const float myslope = SLOPED ? slopes[myhead] * 1.44269504088896341f : 0.f;
+  RowSoftmax sm;
+  sm.start(sinks, myhead, kq);
   f32x4_t o[NCB];
 #pragma unroll
   for (int n = 0; n < NCB; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -1104,9 +1142,6 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
   auto key_of = [&](int v) { return v + (v >= keepT ? gap : 0); };
   const int* bt = tables + (int64_t)seq * W;
   const float scale2 = scale * 1.44269504088896341f;
-  const bool pow2 = (bs & (bs - 1)) == 0;
-  const int sh = __builtin_ctz(bs);
-  auto page_of = [&](int v) { return v < vlen ? bt[pow2 ? key_of(v) >> sh : key_of(v) / bs] : 0; };
 
   // copies: key rows in whole, value columns of 64 bytes
   int krow[NK];
@@ -1115,123 +1150,95 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
   for (int i = 0; i < NK; ++i) {
     const int e = (wave + 4 * i) * 64 + lane, row = e / PR;
     krow[i] = row;
-    const int f = NKS == 2 ? (row & 15) >> 1 : row & 15;
-    kpiece[i] = ((e % PR) ^ f) * 16;
+    const int f = (row >> 3) * 4 + (row & 3);  // the lane that reads it
+    kpiece[i] = ((e % PR) ^ (NKS == 2 ? f >> 1 : f)) * 16;
   }
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int e = (wave + 4 * i) * 64 + lane, col = e >> 2;
-    vplace[i] = col * bs * 2 + ((e & 3) ^ (col >> 2 & 3)) * 16;
+    vplace[i] = col * bs * 2 + ((e & 3) ^ (-(col >> 2) & 3)) * 16;
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)tile + wave * 1024;
-  int page = page_of(kbase);
-  auto copy = [&](int v0, int buf) {
-    const int k0 = key_of(v0), off = pow2 ? k0 & (bs - 1) : k0 % bs;
+  // the next tile to copy: its position, key, place in the page, and the page, looked up a tile ahead
+  int cv = kbase, ckey = key_of(kbase), coff = ckey % bs, cpi = ckey / bs;
+  int page = kbase < vlen ? bt[cpi] : 0;
+  auto copy = [&](int buf) {
     const char* base = reinterpret_cast<const char*>(cache + ((int64_t)page * Hkv + g) * bs * (dim + vdim));
-    page = page_of(v0 + MKT);
+    const char *kb = base + coff * RBy, *vb = base + bs * RBy + coff * 2;
     const uint32_t at = lds0 + buf * (KB + VB);
+    const int last = maxlen - 1 - ckey;
+    cv += MKT, ckey += MKT, coff += MKT;
+    if (coff == bs) coff = 0, ++cpi;
+    if (cv == keepT && gap > 0) ckey += gap, coff = ckey % bs, cpi = ckey / bs;
+    if (cv < vlen) page = bt[cpi];
 #pragma unroll
     for (int i = 0; i < NK; ++i)  // rows past the end: the last one again (a page's unwritten rest may hold anything)
-      copy_1k(base + off * RBy, min(krow[i], maxlen - 1 - k0) * RBy + kpiece[i], at + i * 4096);
+      copy_1k(kb, min(krow[i], last) * RBy + kpiece[i], at + i * 4096);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) copy_1k(base + bs * RBy + off * 2, vplace[i], at + KB + i * 4096);
+    for (int i = 0; i < NV; ++i) copy_1k(vb, vplace[i], at + KB + i * 4096);
   };
-  auto arrive = [] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-  // reads: the key row that lane r16 multiplies (block kb: 16 rows further), pieces of columns 16 n + r16
+  // reads: the key row that lane r16 multiplies (block kb: four rows further), pieces of columns 16 n + r16
   int ka[NKS <= 4 ? NKS : 4];
 #pragma unroll
   for (int ks = 0; ks < (NKS <= 4 ? NKS : 4); ++ks)
-    ka[ks] = r16 * RBy + ((4 * ks + kq) ^ (NKS == 2 ? r16 >> 1 : r16)) * 16;
-  const int va = KB + r16 * 64 + ((kq >> 1 | (kq & 1) << 1) ^ r16 >> 2) * 16;
+    ka[ks] = dealt_key(r16, 0) * RBy + ((4 * ks + kq) ^ (NKS == 2 ? r16 >> 1 : r16)) * 16;
+  const int va = KB + r16 * 64 + (kq ^ (-(r16 >> 2) & 3)) * 16;
 
-  if (kbase < vlen) copy(kbase, 0);
-  arrive();
+  if (kbase < vlen) copy(0);
+  // (a wait that hipcc sees, though not the copies: where the query might be pending at the loop's entry it would wait for all in the loop)
+  __builtin_amdgcn_s_waitcnt(0);
+  __builtin_amdgcn_s_barrier();
   int cur = 0;
   for (int v0 = kbase; v0 < vlen; v0 += MKT, cur ^= 1) {
     const int k0 = key_of(v0);
-    char* const t = tile + cur * (KB + VB);
-    if (v0 + MKT < vlen) {
-      copy(v0 + MKT, cur ^ 1);  // read by nobody since the barrier of the previous tile
-    } else if (k0 + MKT > maxlen) {
-      for (int e = threadIdx.x; e < vdim * MKT; e += NT) {
-        const int col = e >> 5, key = e & 31;
-        if (k0 + key >= maxlen)
-          *reinterpret_cast<bf16_t*>(t + KB + col * 64 + ((key >> 3) ^ (col >> 2 & 3)) * 16 + (key & 7) * 2) = 0;
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    }
+    const char* const t = tile + cur * (KB + VB);
+    if (cv < vlen) copy(cur ^ 1);  // read by nobody since the barrier of the previous tile
     const bool plain = k0 >= full_lo && k0 + MKT <= full_hi;  // every key visible to every row: no masks
-    float sc[8];  // scores of this lane's row against keys k0 + 16 kb + 4 kq + r
-    {
-      f32x4_t a[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    f32x4_t a[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks)
+    for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-          const bf16x8_t k = *reinterpret_cast<const bf16x8_t*>(t + ka[ks & 3] + (ks >> 2) * 256 + kb * 16 * RBy);
-          a[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qf[ks], a[kb], 0, 0, 0);
-        }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) sc[i] = a[i >> 2][i & 3] * scale2;
-    }
-    if (!plain) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int key = k0 + (i >> 2) * 16 + kq * 4 + (i & 3);
-        const bool in = (key < mylen) & (key >= mylo) & ((key >= mywlo) | (key < keep));
-        sc[i] = in ? sc[i] - myslope * (float)(mylen - 1 - key) : -INFINITY;
+      for (int kb = 0; kb < 2; ++kb) {
+        const bf16x8_t k = *reinterpret_cast<const bf16x8_t*>(t + ka[ks & 3] + (ks >> 2) * 256 + kb * 4 * RBy);
+        a[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qf[ks], a[kb], 0, 0, 0);
       }
-    } else if (slopes != nullptr) {
-      const float dist = (float)(mylen - 1 - k0 - kq * 4);
+    bf16x8_t pah, pal;
+    auto products = [&](auto value) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) sc[i] -= myslope * (dist - (float)((i >> 2) * 16 + (i & 3)));
-    }
-    float mx = sc[0];
+      for (int n0 = 0; n0 < NCB; n0 += 4) {
+        bf16x8_t v[4];
 #pragma unroll
-    for (int i = 1; i < 8; ++i) mx = fmaxf(mx, sc[i]);
-    mx = row_max(mx);
-    const float mn = fmaxf(m, mx), mref = mn == -INFINITY ? 0.f : mn;  // a row with no key yet
-    const float corr = __builtin_amdgcn_exp2f(m - mref);
-    if (__any(corr != 1.f)) {  // some row's maximum moved; a row whose own did not is multiplied by 1
+        for (int n = 0; n < 4; ++n) v[n] = value(*reinterpret_cast<const bf16x8_t*>(t + va + (n0 + n) * 1024));
 #pragma unroll
-      for (int n = 0; n < NCB; ++n)
+        for (int n = 0; n < 4; ++n) o[n0 + n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[n], pah, o[n0 + n], 0, 0, 0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[n][r] *= corr;
-    }
-    float psum = 0.f;
-    u32x4_t hw, lw;  // the weights in two bf16 parts, as in grouped_attention_mfma
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      const float p0 = __builtin_amdgcn_exp2f(sc[i] - mref), p1 = __builtin_amdgcn_exp2f(sc[i + 1] - mref);
-      psum += p0 + p1;
-      const uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
-      const uint32_t r0 = __float_as_uint(p0 - __uint_as_float(u0 & 0xffff0000u));
-      const uint32_t r1 = __float_as_uint(p1 - __uint_as_float(u1 & 0xffff0000u));
-      hw[i >> 1] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-      lw[i >> 1] = __builtin_amdgcn_perm(r1, r0, 0x07060302u);
-    }
-    const bf16x8_t pah = __builtin_bit_cast(bf16x8_t, hw), pal = __builtin_bit_cast(bf16x8_t, lw);
-    l = l * corr + row_sum(psum);
-    m = mn;
-#pragma unroll
-    for (int n0 = 0; n0 < NCB; n0 += 4) {
-      bf16x8_t v[4];
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        const u32x4_t w = *reinterpret_cast<const u32x4_t*>(t + va + (n0 + n) * 1024);
-        const auto x = __builtin_amdgcn_permlane16_swap(w[0], w[2], false, false);
-        const auto y = __builtin_amdgcn_permlane16_swap(w[1], w[3], false, false);
-        v[n] = __builtin_bit_cast(bf16x8_t, u32x4_t{x[0], y[0], x[1], y[1]});
+        for (int n = 0; n < 4; ++n) o[n0 + n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[n], pal, o[n0 + n], 0, 0, 0);
       }
-#pragma unroll
-      for (int n = 0; n < 4; ++n) o[n0 + n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[n], pah, o[n0 + n], 0, 0, 0);
-#pragma unroll
-      for (int n = 0; n < 4; ++n) o[n0 + n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[n], pal, o[n0 + n], 0, 0, 0);
+    };
+    bool calm = false;
+    if (plain) {
+      float x[8];
+      row_scores(a, scale2, myslope, SLOPED, mylen - 1 - k0 - kq * 8, sm.ref, x);
+      calm = !__any(top8(x) > sm.rise);
+      if (calm) {
+        row_weights(x, sm, pah, pal);
+        products([](bf16x8_t v) { return v; });
+      }
     }
-    arrive();
+    if (!calm) {
+      weigh<NCB, false>(a, scale2, myslope, SLOPED, plain, k0 + kq * 8, mylen, mylo, mywlo, keep, sm, o, pah, pal);
+      u32x4_t seen;  // not the values of keys that were never written
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int left = maxlen - k0 - kq * 8 - 2 * i;
+        seen[i] = left >= 2 ? 0xffffffffu : left == 1 ? 0xffffu : 0u;
+      }
+      products([&](bf16x8_t v) { return __builtin_bit_cast(bf16x8_t, __builtin_bit_cast(u32x4_t, v) & seen); });
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
-  if (wave * 16 + r16 >= ntok * G) return;
-  const float inv = 1.f / l;
+  const float inv = 1.f / row_sum(sm.l);
+  if (!ok) return;
   bf16_t* dst = out + ((int64_t)mytok * Hq + myhead) * vdim;
   const bf16_t* gt = gate ? gate + (int64_t)mytok * gate_stride + myhead * vdim : nullptr;
 #pragma unroll
@@ -2006,13 +2013,17 @@ int sm_grouped_attention_mfma(const void* q, const void* cache, const int* table
   }
   if (nsplit == 1 && rb == 1 && dim == vdim && (dim == 64 || dim == 128 || dim == 256) && bs % MKT == 0 &&
       (((uintptr_t)q | (uintptr_t)cache | (uintptr_t)out) & 15) == 0) {
-#define SM_GP(NKS, NCB)                                                                                               \
-  hipLaunchKernelGGL((grouped_prompt_kernel<NKS, NCB>), dim3(Hkv, n_items), dim3(NT), 0, stream, (const bf16_t*)q,    \
+#define SM_GP(NKS, NCB, SLOPED)                                                                                     \
+  hipLaunchKernelGGL((grouped_prompt_kernel<NKS, NCB, SLOPED>), dim3(Hkv, n_items), dim3(NT), 0, stream, (const bf16_t*)q, \
                      (const bf16_t*)cache, tables, W, bs, items, row_len, scale, Hq, Hkv, (const bf16_t*)gate,        \
                      gate_stride, (bf16_t*)out, slopes, chunk, sinks, window, keep)
-    if (dim == 64) SM_GP(2, 4);
-    else if (dim == 128) SM_GP(4, 8);
-    else SM_GP(8, 16);
+#define SM_GP2(NKS, NCB)               \
+  if (slopes) SM_GP(NKS, NCB, true);   \
+  else SM_GP(NKS, NCB, false)
+    if (dim == 64) { SM_GP2(2, 4); }
+    else if (dim == 128) { SM_GP2(4, 8); }
+    else { SM_GP2(8, 16); }
+#undef SM_GP2
 #undef SM_GP
     return 0;
   }

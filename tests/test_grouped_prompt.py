@@ -87,3 +87,35 @@ def test_bits_do_not_depend_on_the_form(dim, opts):
                 c[:, bs * dim:] = values[i, :, p * bs:(p + 1) * bs].transpose(1, 2).reshape(Hkv, -1)
         out.append(sm.grouped_attention(q, cache.cuda(), dim, dim, dim ** -0.5, m, **kw))
     assert all(torch.equal(out[0], o) for o in out[1:])
+
+
+@pytest.mark.parametrize("bs", [64, 16])  # whole sizes, general form
+@pytest.mark.parametrize("opts", [{}, {"sinks": 1}, {"slopes": True}], ids=["plain", "sink", "slopes"])
+def test_scores_that_climb(bs, opts):
+    """Scores that rise along the keys by less and by more than the weights' reference lets stand, that lie far below and far above zero
+    from the first key on, and sinks far above and below all of them."""
+    from llmd_amd.ops import seqmix as sm
+
+    n, Hq, Hkv, dim = 230, 8, 2, 128
+    g = torch.Generator().manual_seed(3)
+    m, pages = _meta([(0, n)], bs, "cpu")
+    # every key: a first coordinate that climbs with its position; every head: how much of it its queries take, in units of log2
+    climb = torch.tensor([0.0, 0.02, 0.3, 3.0, -0.3, -3.0, 0.05, 0.0])
+    base = torch.tensor([0.0, -900.0, 40.0, -200.0, 700.0, 0.0, -30.0, 300.0])
+    q = torch.randn(n, Hq, dim, generator=g).bfloat16()
+    q[:, :, 0], q[:, :, 1] = (climb * dim ** 0.5).bfloat16(), (base * dim ** 0.5 / 256).bfloat16()
+    keys, values = (torch.randn(Hkv, pages * bs, dim, generator=g).bfloat16() for _ in range(2))
+    cache = torch.zeros(pages, Hkv, bs, 2 * dim).bfloat16()
+    for p in range(-(-n // bs)):
+        k = keys[:, p * bs:(p + 1) * bs].clone()
+        k[..., 0], k[..., 1] = torch.arange(p * bs, (p + 1) * bs).bfloat16(), 256.0
+        c = cache[int(m.tables[0, p])].view(Hkv, -1)
+        c[:, :bs * dim] = k.reshape(Hkv, -1)
+        c[:, bs * dim:] = values[:, p * bs:(p + 1) * bs].transpose(1, 2).reshape(Hkv, -1)
+    vals = {"sinks": torch.tensor([5.0, -800.0, -1000.0, 400.0, 2000.0, 3.0, 0.0, -50.0]), "slopes": torch.rand(Hq, generator=g) * 0.05}
+    kw = {k: vals[k] for k in opts}
+    want = sm.grouped_attention(q.double(), cache.double(), dim, dim, dim ** -0.5, m, **kw)
+    md, _ = _meta([(0, n)], bs, "cuda")
+    got = sm.grouped_attention(q.cuda(), cache.cuda(), dim, dim, dim ** -0.5, md, **{k: v.cuda() for k, v in kw.items()})
+    # scores of up to about 1000 in fp32 (their products' sums are 2^-24 of that off, a few times): weights off by 2^-11; values up to about 5
+    assert ((got.double().cpu() - want).abs() <= 2 ** -8 * want.abs() + 5e-3).all()
