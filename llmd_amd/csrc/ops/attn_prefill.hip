@@ -345,24 +345,33 @@ __global__ __launch_bounds__(NT, 2) void prefill_v2_kernel(
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ q_start,
     const int* __restrict__ q_len, const int* __restrict__ ctx_len, const int* __restrict__ items,
     int Hq, int Hkv, int G, int HPW, float scale_log2, int window,
-    const float* __restrict__ sinks, uint16_t* __restrict__ out, int64_t out_stride, float vscale, int xcd) {
+    const float* __restrict__ sinks, uint16_t* __restrict__ out, int64_t out_stride, float vscale, int order) {
   constexpr int KS = D / 32, NB = D / 16, RB = 2 * D;  // row bytes
   constexpr int P2_IMG = 64 * RB;                       // one 64-key bf16 image
   constexpr int NI = 64 * (D / 8) / 64;                 // DMA wave-instructions per image (16 / 8)
   __shared__ __attribute__((aligned(1024))) char buf0[2 * P2_IMG];  // K | V of even tiles
   __shared__ __attribute__((aligned(1024))) char buf1[2 * P2_IMG];  // K | V of odd tiles
 
-  // xcd: the dispatcher deals workgroups round-robin over the 8 XCDs; remap so
-  // each XCD runs a contiguous (head group, item) range - one KV head's K/V
-  // (5000 tokens: 2.5 MB) stays in that XCD's 4 MB L2 instead of every XCD
-  // streaming all heads' tiles. Measured (profiles/attn_prefill_r2_lanelocal.txt):
-  // ISL 5000 776 -> 833 TF/s, 8k 932 -> 1016; a one-wave grid (5000 x 512
-  // chunk, 256 workgroups) loses 2 %, so the host enables it from 1024 workgroups
+  // order: which item and head group a workgroup takes, for grids that give CUs more than one. The dispatcher deals workgroups
+  // round-robin over the 8 XCDs and within one over its 32 CUs, and two run on a CU, so a grid of up to 512 is resident at once and a
+  // CU's time is that of its two. Items come longest first. An XCD's list holds its own head groups' items (a kv head's K / V stay
+  // in its L2), or where their number is no multiple of 8 every eighth item, longest first over all of them; in a grid of one
+  // round its second 32 go in reverse, so that the longest item shares a CU with the shortest. us, 32 heads over 4: 2048 tokens 63.8
+  // (both rounds gave a CU items of one length) / 53.2, 3000 112 (head group by head group, the last one's long items at the end) / 86,
+  // 731 and 674 tokens after 1024 54.7 / 49.8, 5000 214 / 208; 64 over 8: 1024 35.5 / 29.7, 5000 377 / 372; 20 over 4: 8000 383 / 328.
   int bx = blockIdx.x, by = blockIdx.y;
-  if (xcd) {
-    const int l = xcd_remap(by * gridDim.x + bx, gridDim.x * gridDim.y);
-    bx = l % gridDim.x;
-    by = l / gridDim.x;
+  if (order) {
+    const int ny = gridDim.y, n = gridDim.x * ny, l = by * gridDim.x + bx, xcd = l & 7;
+    const int nx = (n - xcd + 7) >> 3;
+    int j = l >> 3;
+    if (n <= 512 && j >= 32) j = nx - 1 - (j - 32);
+    if (ny % 8 == 0) {
+      const int m = ny >> 3;
+      bx = j / m, by = xcd * m + j % m;
+    } else {
+      const int p = 8 * j + xcd;
+      bx = p / ny, by = p % ny;
+    }
   }
   const int seq = items[2 * bx], qb = items[2 * bx + 1];
   const int NHG = G / HPW;
@@ -1559,7 +1568,7 @@ extern "C" int llmd_paged_prefill(const void* q, int64_t q_stride, const void* k
     hipLaunchKernelGGL(kern, grid, blk, 0, st, (const uint16_t*)q, q_stride, (const uint16_t*)kc,
                        (const uint16_t*)vc, block_stride, bs, block_tables, bt_stride, q_start, q_len, ctx_len,
                        items, Hq, Hkv, G, HPW, scale_log2, window, sinks, (uint16_t*)out, out_stride, v_scale,
-                       xcd_map && (int64_t)n_items * grid.y >= 1024 ? 1 : 0);
+                       xcd_map && (int64_t)n_items * grid.y > 256 ? 1 : 0);
   } else if (D == 128) {
     if (fp8) LAUNCH(128, true); else LAUNCH(128, false);
   } else if (D == 64) {
