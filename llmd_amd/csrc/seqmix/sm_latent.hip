@@ -286,12 +286,12 @@ struct TileFetch {
 };
 
 // The wide form (Dk = 32 NKS = 512 or 576 exactly, R <= 512, pages of whole tiles): the accumulators and the query leave no
-// registers for a tile in flight, so the next tile is copied straight to the other LDS buffer while this one is multiplied. A
-// buffer holds 128 bytes of all 32 rows, then the next 128; eight pieces of 16 bytes lie in the order c ^ f(row), f different
-// in the 16 rows whose pieces are read together (rows two apart share banks), neighbouring pairs staying together, which is
-// what a transposed read takes. The second product comes out as
-// O^T, in the lanes that own the rows (see grouped_attention_mfma). 2048 tokens, 16 heads, latent 512 + 64: 299 us with the
-// general form below (a tile's loads were waited for in the loop; items in order of their length), now 151 us.
+// buffer holds 128 bytes of all 32 rows, then the next 128; eight pieces of 16 bytes lie in the order c ^ f(row). f is even, so that
+// the pairs of pieces that a transposed read takes stay together, and neither of the two kinds of reads meets in a bank: lanes 0 .. 3
+// and 12 .. 15 of a 16-byte read go with lanes 4 .. 11 of the quarter beside theirs, a transposed one takes eight neighbouring rows.
+// The second product comes out as O^T, in the lanes that own the rows (see grouped_attention_mfma). 2048 tokens, 16 heads, latent
+// 512 + 64: 299 us with the general form below (a tile's loads were waited for in the loop; items in order of their length), 149 with
+// the query waited for in the loop, and the next tile with it, and conflicts in a third of the transposed reads' cycles, now 142.
 template <int NKS>
 __global__ __launch_bounds__(NT, 2) void latent_prompt_kernel(
     const bf16_t* __restrict__ q_abs, const bf16_t* __restrict__ cache, const int* __restrict__ tables, int W, int bs,
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(NT, 2) void latent_prompt_kernel(
   constexpr int Dk = 32 * NKS, NCB = 32, RB = 2 * Dk, NG = RB / 128;  // bytes of a row, its parts of 128
   static_assert(NKS % 2 == 0, "whole parts");
   __shared__ __attribute__((aligned(1024))) char tile[2 * MKT * RB];
-  auto f = [](int row) { return (row >> 1 & 3) << 1 | (row >> 3 & 1); };
+  auto f = [](int row) { return row & 6; };
   const int seq = items[blockIdx.x * 3], tok0 = items[blockIdx.x * 3 + 1], ntok = items[blockIdx.x * 3 + 2];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r16 = lane & 15, kq = lane >> 4;
@@ -351,7 +351,9 @@ __global__ __launch_bounds__(NT, 2) void latent_prompt_kernel(
   };
   auto arrive = [] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
   if (kbeg < kend) copy(kbeg, 0);
-  arrive();
+  // (a wait that hipcc sees, though not the copies: where the query might be pending at the loop's entry it would wait for all in the loop)
+  __builtin_amdgcn_s_waitcnt(0);
+  __builtin_amdgcn_s_barrier();
   int cur = 0;
   for (int k0 = kbeg; k0 < kend; k0 += MKT, cur ^= 1) {
     const char* const t = tile + cur * (MKT * RB);
