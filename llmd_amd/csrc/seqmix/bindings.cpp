@@ -24,6 +24,9 @@ int sm_latent_attention(const void*, const void*, const int*, int, int, const in
 int sm_latent_attention_mfma(const void*, const void*, const int*, int, int, const int*, int, const int*, float, int,
                              int, int, void*, int, int, float*, float*, const void*, int64_t, int, int, const int*,
                              hipStream_t);
+void sm_latent_gather(const void*, const int*, int, int, const int*, int, int, int, int, int, void*, void*, hipStream_t);
+void sm_latent_own(const void*, int64_t, const void*, int64_t, int64_t, const void*, const void*, const int*, const int*, int, const int*,
+                   float, int, void*, const void*, int64_t, hipStream_t);
 void sm_embed_norm(const int64_t*, const void*, int64_t, const void*, float, float*, void*, int, int, int, hipStream_t);
 void sm_rms_norm_rows(const void*, int64_t, const void*, float, void*, int, int, int, hipStream_t);
 void sm_relu2(const void*, void*, int64_t, int, hipStream_t);
@@ -296,6 +299,49 @@ bool latent_attention_mfma(Tensor q_abs, Tensor cache, Tensor tables, Tensor ite
                                   (float)scale, H, R, Dk, out.data_ptr(), nsplit, split_keys, po, pm,
                                   gate ? gate->data_ptr() : nullptr, gate ? gate->stride(0) : 0, window, rows,
                                   longest_of(longest), cur()) == 0;
+}
+
+// lat [keys, R], rot [keys, dr] <- the cached rows of sequences first .. ; base [sequences + 1]: their places, the number of keys at the end
+void latent_gather(Tensor cache, Tensor tables, Tensor base, int64_t first, int64_t longest, Tensor lat, Tensor rot) {
+  const c10::hip::OptionalHIPGuard g(dev_of(cache));
+  TORCH_CHECK(cache.is_cuda() && cache.scalar_type() == torch::kBFloat16 && cache.dim() == 3 && cache.is_contiguous(), "cache bf16");
+  CHECK_ACT(lat, cache);
+  CHECK_ACT(rot, cache);
+  CHECK_I32(tables);
+  CHECK_I32(base);
+  const int64_t R = lat.size(1), dr = rot.size(1), bs = cache.size(1);
+  TORCH_CHECK(tables.dim() == 2 && base.numel() == tables.size(0) + 1 && first >= 0 && first <= tables.size(0), "sequences");
+  TORCH_CHECK(lat.dim() == 2 && rot.dim() == 2 && lat.is_contiguous() && rot.is_contiguous() && lat.size(0) == rot.size(0), "rows");
+  TORCH_CHECK(R % 8 == 0 && dr % 8 == 0 && R + dr == cache.size(2) && ((uintptr_t)cache.data_ptr() & 15) == 0, "whole 16-byte pieces");
+  TORCH_CHECK(longest >= 0 && longest <= tables.size(1) * bs && longest * ((R + dr) / 8) < (1ll << 31), "keys of a sequence");
+  sm_latent_gather(cache.data_ptr(), tables.data_ptr<int>(), tables.size(1), bs, base.data_ptr<int>(), first, tables.size(0) - first, longest,
+                   R, dr, lat.data_ptr(), rot.data_ptr(), cur());
+}
+
+// the step's rows that ``items`` (up to 64 tokens each) name, over keys and values of their own
+void latent_own(Tensor q, Tensor q_abs, int64_t R, Tensor kv, Tensor rot, Tensor base, Tensor items, Tensor row_len, double scale, Tensor out,
+                std::optional<Tensor> gate) {
+  const c10::hip::OptionalHIPGuard g(dev_of(q));
+  TORCH_CHECK(q.is_cuda() && q.scalar_type() == torch::kBFloat16 && q_abs.dim() == 3 && q_abs.is_contiguous(), "q bf16, q_abs [T, H, Dk]");
+  CHECK_ACT(q_abs, q);
+  CHECK_ACT(kv, q);
+  CHECK_ACT(rot, q);
+  CHECK_ACT(out, q);
+  CHECK_I32(base);
+  CHECK_I32(items);
+  CHECK_I32(row_len);
+  const int64_t T = q_abs.size(0), H = q_abs.size(1), Dk = q_abs.size(2);
+  TORCH_CHECK(q.dim() == 2 && q.size(0) == T && q.size(1) == H * 192 && q.stride(1) == 1 && q.stride(0) % 8 == 0 &&
+              ((uintptr_t)q.data_ptr() & 15) == 0, "q [T, H (128 + 64)]");
+  TORCH_CHECK(R % 8 == 0 && Dk == R + 64 && rot.dim() == 2 && rot.size(1) == 64 && rot.is_contiguous() && kv.dim() == 2 && kv.is_contiguous() &&
+              kv.size(0) == rot.size(0) && kv.size(1) == H * 256 && H * 512 * 32 < (1ll << 31), "keys and values [n, H (128 + 128)], [n, 64]");
+  TORCH_CHECK(((((uintptr_t)q_abs.data_ptr()) | (uintptr_t)kv.data_ptr() | (uintptr_t)rot.data_ptr() | (uintptr_t)out.data_ptr()) & 15) == 0, "alignment");
+  TORCH_CHECK(items.dim() == 2 && items.size(1) == 3 && items.size(0) <= 65535 && row_len.numel() == T, "items");
+  TORCH_CHECK(out.is_contiguous() && out.numel() == T * H * 128, "out [T, H, 128]");
+  check_head_gate(gate, q_abs);
+  sm_latent_own(q.data_ptr(), q.stride(0), (const char*)q_abs.data_ptr() + R * 2, H * Dk, Dk, kv.data_ptr(), rot.data_ptr(), base.data_ptr<int>(),
+                items.data_ptr<int>(), items.size(0), row_len.data_ptr<int>(), (float)scale, H, out.data_ptr(),
+                gate ? gate->data_ptr() : nullptr, gate ? gate->stride(0) : 0, cur());
 }
 
 void causal_conv_silu(Tensor xz, int64_t C, Tensor w, Tensor b, Tensor state, Tensor seq_start, Tensor seq_slot,
@@ -1163,6 +1209,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("relu2", &relu2);
   m.def("input_conv", &input_conv);
   m.def("hgrn2_scan", &hgrn2_scan);
+  m.def("latent_gather", &latent_gather);
+  m.def("latent_own", &latent_own);
   m.def("gated_add_norm", &gated_add_norm);
   m.def("poly_norm", &poly_norm);
   m.def("retention", &retention);

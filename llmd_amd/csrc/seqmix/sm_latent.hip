@@ -15,6 +15,7 @@
 // window > 0: query i sees key j <= i only if i - j < window; the tiles before the first window of a
 //   work item are not visited (tiles start at multiples of the tile size from position 0). dr may be 0: a
 //   latent without a rotated part.
+#include "row_softmax.h"
 #include "seqmix_common.h"
 
 using namespace sm;
@@ -197,20 +198,16 @@ __global__ __launch_bounds__(NT) void latent_attention_kernel(
 // the weights P enter the second product as a bf16 pair (hi + lo, two MFMAs), which keeps 16 mantissa
 // bits of the fp32 weight. DkP = 32 NKS >= Dk >= R are the padded sizes (zeros in LDS and in the
 // query fragments); columns past R are computed from whatever the row holds there and not stored.
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x8_t __attribute__((ext_vector_type(8)));
 
-constexpr int MKT = 32;  // keys per tile
 constexpr float LOG2E = 1.44269504088896341f;
 
-// Eight keys of one column for a lane: four from ``p`` on and four from 16 rows further down.
-template <int KS>
+// Eight keys of one column for a lane: four from ``p`` on and four from ROWS rows further down.
+template <int KS, int ROWS = 16>
 __device__ __forceinline__ bf16x8_t column_keys(const bf16_t* p) {
   const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)p);
-  const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p + 16 * KS));
+  const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_t*)(p + ROWS * KS));
   return __builtin_bit_cast(bf16x8_t, s16x8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
 }
 
@@ -435,6 +432,123 @@ __global__ __launch_bounds__(NT, 2) void latent_prompt_kernel(
         if (col + r < R) st(dst + col + r, o[n][r] * w);
     }
   }
+}
+
+// Prompts with keys and values of their own. A prompt's rows meet so many keys that the heads' keys W_uk c and values W_uv c are
+// cheaper made once than absorbed into every query: 192 + 128 columns per head and key instead of 576 + 512. The latents of the
+// prompts' sequences are gathered out of their pages, one product makes [key | value] of every head, and the rotated part stays shared.
+// The tiles lie in LDS as in latent_prompt_kernel, in parts of 128 bytes of all 32 keys: two of the head's key, the rotated part, two of
+// the values; key rows are dealt as in grouped_prompt_kernel (f(row): no bank conflicts for either kind of read in that order), whose
+// softmax this is. What bounds it: the waves' latency (QK, softmax, PV in a row, three to four waves per SIMD).
+// 2048 tokens, 16 heads, latent 512 + 64, values 128, us: the absorbed form's kernel and the products before and behind it 19 + 142 + 16,
+// here gather, product, kernel 4 + 20 + 64; 0.0023 off 64 bits (0.0024).
+constexpr int OWN_K = 128, OWN_ROT = 64, OWN_V = 128;
+__global__ __launch_bounds__(NT, 4) void latent_own_kernel(
+    const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ q_rot, int64_t rot_stride, int64_t rot_head,
+    const bf16_t* __restrict__ kv, const bf16_t* __restrict__ rot, const int* __restrict__ base, const int* __restrict__ items,
+    const int* __restrict__ row_len, float scale, int H, bf16_t* __restrict__ out, const bf16_t* __restrict__ gate, int64_t gate_stride) {
+  constexpr int NKS = (OWN_K + OWN_ROT) / 32, NCB = OWN_V / 16, PART = MKT * 128, TB = 5 * PART;
+  __shared__ __attribute__((aligned(1024))) char tile[2 * TB];
+  auto f = [](int row) { return (row & 2) | (row >> 1 & 4); };
+  const int h = blockIdx.x;
+  const int seq = items[blockIdx.y * 3], tok0 = items[blockIdx.y * 3 + 1], ntok = items[blockIdx.y * 3 + 2];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r16 = lane & 15, kq = lane >> 4;
+  const int myrow = wave * 16 + r16;
+  const bool ok = myrow < ntok;
+  const int mytok = tok0 + (ok ? myrow : 0);
+  const int mylen = ok ? row_len[mytok] : 0;
+  const int kend = row_len[tok0 + ntok - 1], full = row_len[tok0];  // tiles below ``full`` are visible to every row
+
+  bf16x8_t qf[NKS];
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks)
+    qf[ks] = *reinterpret_cast<const bf16x8_t*>(ks < OWN_K / 32 ? q + mytok * q_stride + h * (OWN_K + OWN_ROT) + ks * 32 + kq * 8
+                                                                : q_rot + mytok * rot_stride + h * rot_head + (ks - OWN_K / 32) * 32 + kq * 8);
+  RowSoftmax sm;
+  sm.start(nullptr, 0, kq);
+  f32x4_t o[NCB];
+#pragma unroll
+  for (int n = 0; n < NCB; ++n) o[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const float scale2 = scale * LOG2E;
+
+  // a wave copies eight rows of every part, eight lanes per row
+  const int crow = wave * 8 + (lane >> 3), cpiece = ((lane & 7) ^ f(crow)) * 16;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)tile + wave * 1024;
+  const int64_t pitch = (int64_t)H * (OWN_K + OWN_V) * 2;  // bytes of a row of kv
+  const char* const kv0 = reinterpret_cast<const char*>(kv) + base[seq] * pitch + h * (OWN_K + OWN_V) * 2;
+  const char* const rot0 = reinterpret_cast<const char*>(rot) + (int64_t)base[seq] * (OWN_ROT * 2);
+  auto copy = [&](int k0, int buf) {
+    const int row = min(crow, kend - 1 - k0);  // rows past the end: the last one again
+    const uint32_t off = (uint32_t)(row * pitch) + cpiece, at = lds0 + buf * TB;
+    const char* const b = kv0 + k0 * pitch;
+    copy_1k(b, off, at);
+    copy_1k(b + 128, off, at + PART);
+    copy_1k(rot0 + k0 * (OWN_ROT * 2), row * (OWN_ROT * 2) + cpiece, at + 2 * PART);
+    copy_1k(b + OWN_K * 2, off, at + 3 * PART);
+    copy_1k(b + OWN_K * 2 + 128, off, at + 4 * PART);
+  };
+  int ka[2], va[4];
+  const int krow = dealt_key(r16, 0), vrow = 8 * kq + (r16 >> 2);
+#pragma unroll
+  for (int e = 0; e < 2; ++e) ka[e] = krow * 128 + ((e * 4 + kq) ^ f(krow)) * 16;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) va[j] = 3 * PART + vrow * 128 + ((r16 >> 1 & 1) ^ f(vrow) ^ 2 * j) * 16 + (r16 & 1) * 8;
+  copy(0, 0);
+  // (a wait that hipcc sees, though not the copies: where the query might be pending at the loop's entry it would wait for all in the loop)
+  __builtin_amdgcn_s_waitcnt(0);
+  __builtin_amdgcn_s_barrier();
+  int cur = 0;
+  for (int k0 = 0; k0 < kend; k0 += MKT, cur ^= 1) {
+    const char* const t = tile + cur * TB;
+    if (k0 + MKT < kend) copy(k0 + MKT, cur ^ 1);  // read by nobody since the barrier of the previous tile
+    f32x4_t a[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const bf16x8_t k = *reinterpret_cast<const bf16x8_t*>(t + ka[ks & 1] + (ks >> 1) * PART + kb * 4 * 128);
+        a[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qf[ks], a[kb], 0, 0, 0);
+      }
+    bf16x8_t pah, pal;
+    weigh<NCB, true>(a, scale2, 0.f, false, k0 + MKT <= full, k0 + kq * 8, mylen, 0, 0, 0, sm, o, pah, pal);
+#pragma unroll
+    for (int n0 = 0; n0 < NCB; n0 += 4) {
+      bf16x8_t v[4];
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        v[n] = column_keys<64, 4>(reinterpret_cast<const bf16_t*>(t + va[n] + (n0 >> 2) * PART));
+#pragma unroll
+      for (int n = 0; n < 4; ++n) o[n0 + n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[n], pah, o[n0 + n], 0, 0, 0);
+#pragma unroll
+      for (int n = 0; n < 4; ++n) o[n0 + n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[n], pal, o[n0 + n], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+  const float l = row_sum(sm.l);
+  if (!ok) return;
+  float w = 1.f / l;
+  if (gate) w *= 1.f / (1.f + expf(-ld(gate + (int64_t)mytok * gate_stride + h)));
+  bf16_t* dst = out + ((int64_t)mytok * H + h) * OWN_V;
+#pragma unroll
+  for (int n = 0; n < NCB; ++n) {
+    ushort4 b;
+    st(&b.x, o[n][0] * w); st(&b.y, o[n][1] * w); st(&b.z, o[n][2] * w); st(&b.w, o[n][3] * w);
+    *reinterpret_cast<ushort4*>(dst + n * 16 + kq * 4) = b;
+  }
+}
+
+// Cached rows [R | dr] of the sequences ``seq`` .. (blockIdx.y further), back to back from base[seq] on: the latents and the rotated
+// parts apart. base has one number more than there are sequences.
+__global__ __launch_bounds__(NT) void latent_gather_kernel(const bf16_t* __restrict__ cache, const int* __restrict__ tables, int W, int bs,
+                                                           const int* __restrict__ base, int first, int R, int dr,
+                                                           bf16_t* __restrict__ lat, bf16_t* __restrict__ rot) {
+  const int seq = first + blockIdx.y, b = base[seq], n = base[seq + 1] - b, pieces = (R + dr) >> 3;
+  const int e = blockIdx.x * NT + threadIdx.x, key = e / pieces, c = (e - key * pieces) * 8;
+  if (key >= n) return;
+  const u32x4_t v = *reinterpret_cast<const u32x4_t*>(cache + ((int64_t)tables[(int64_t)seq * W + key / bs] * bs + key % bs) * (R + dr) + c);
+  bf16_t* dst = c < R ? lat + (int64_t)(b + key) * R + c : rot + (int64_t)(b + key) * dr + c - R;
+  *reinterpret_cast<u32x4_t*>(dst) = v;
 }
 
 // 16 rows per wave, every wave over all columns. Two tile buffers: the next tile is written while the
@@ -882,6 +996,25 @@ void sm_latent_rope_cache(const void* q, int64_t q_stride, const void* kv, int64
     hipLaunchKernelGGL((latent_rope_cache_kernel<bf16_t>), dim3(T), dim3(NT), 0, stream, (const bf16_t*)q, q_stride,
                        (const bf16_t*)kv, kv_stride, (const bf16_t*)norm_w, eps, positions, cos_sin, H, dn, dr,
                        rot_dims, R, slots, (bf16_t*)cache, (bf16_t*)q_abs, interleaved);
+}
+
+// Latents and rotated parts of sequences first .. first + n - 1, at most ``longest`` keys each.
+void sm_latent_gather(const void* cache, const int* tables, int W, int bs, const int* base, int first, int n, int longest, int R, int dr,
+                      void* lat, void* rot, hipStream_t stream) {
+  if (n == 0 || longest == 0) return;
+  hipLaunchKernelGGL(latent_gather_kernel, dim3((unsigned)(((int64_t)longest * ((R + dr) / 8) + NT - 1) / NT), n), dim3(NT), 0, stream,
+                     (const bf16_t*)cache, tables, W, bs, base, first, R, dr, (bf16_t*)lat, (bf16_t*)rot);
+}
+
+// q [T, H, 128 + 64] rows q_stride apart, of which the first 128; the rotated 64 at q_rot + row * rot_stride + head * rot_head; items of up
+// to 64 tokens; kv [keys, H, 128 + 128], rot [keys, 64] of the gathered sequences; out [T, H, 128] (rows of the items).
+void sm_latent_own(const void* q, int64_t q_stride, const void* q_rot, int64_t rot_stride, int64_t rot_head, const void* kv, const void* rot,
+                   const int* base, const int* items, int n_items, const int* row_len, float scale, int H, void* out, const void* gate,
+                   int64_t gate_stride, hipStream_t stream) {
+  if (n_items == 0) return;
+  hipLaunchKernelGGL(latent_own_kernel, dim3(H, n_items), dim3(NT), 0, stream, (const bf16_t*)q, q_stride, (const bf16_t*)q_rot, rot_stride,
+                     rot_head, (const bf16_t*)kv, (const bf16_t*)rot, base, items, row_len, scale, H, (bf16_t*)out, (const bf16_t*)gate,
+                     gate_stride);
 }
 
 // Returns 0, or 1 when the sizes do not fit the kernel (R > 1024 or rows too wide for LDS).

@@ -31,12 +31,29 @@ class SeqMeta:
     q_lens: Optional[list] = None    # host copy of the run lengths
     ctx_lens: Optional[list] = None  # host copy of each sequence's context length after the step
     longest: Optional[torch.Tensor] = None  # [1] int32, captured steps: longest context of the replay (<= max_len)
-    _items: Optional[dict] = None    # (tokens per item, balance) -> [n, 3] int32 work items (attention_items)
+    _items: Optional[dict] = None    # (tokens per item, balance, runs) -> [n, 3] int32 work items (attention_items)
+    _keys: Optional[tuple] = None    # (first sequence, its key_rows)
     _chunks: Optional[dict] = None   # chunk length -> (table, number of chunks) (scan_chunks)
 
-    def attention_items(self, tokens_per_item: int, balance: int = 0) -> torch.Tensor:
+    def singles(self) -> int:
+        """Runs of one token that the step begins with."""
+        return next((i for i, n in enumerate(self.q_lens) if n != 1), len(self.q_lens))
+
+    def key_rows(self, first: int):
+        """Places of the keys of sequences ``first`` on, back to back: (bounds [n + 1] int32, all zero before ``first``; their
+        number; the longest sequence's). Built once per step (needs ``ctx_lens``)."""
+        if self._keys is None or self._keys[0] != first:
+            ctx = np.asarray(self.ctx_lens, dtype=np.int64).reshape(-1).copy()
+            ctx[:first] = 0
+            bounds = torch.from_numpy(np.concatenate([[0], np.cumsum(ctx)]).astype(np.int32))
+            if self.tables.is_cuda:
+                bounds = bounds.pin_memory().to(self.tables.device, non_blocking=True)
+            self._keys = first, (bounds, int(ctx.sum()), int(ctx.max()))
+        return self._keys[1]
+
+    def attention_items(self, tokens_per_item: int, balance: int = 0, runs: Optional[tuple] = None) -> torch.Tensor:
         """Work items (sequence, first token row, tokens) of the matrix-core attention kernel: every
-        run cut into pieces of at most ``tokens_per_item`` tokens. Built once per step and size.
+        run cut into pieces of at most ``tokens_per_item`` tokens. Built once per step and size. ``runs`` (a, b): of runs a .. b - 1 only.
 
         ``balance`` > 0 (needs ``ctx_lens``): a causal item's work grows with its position in the
         prompt, and the workgroups of a step are all resident at once, dealt to the CUs in order. The
@@ -45,12 +62,14 @@ class SeqMeta:
         one of every block - sum to about the same number of key tiles."""
         if self._items is None:
             self._items = {}
-        key = (tokens_per_item, balance if self.ctx_lens is not None else 0)
+        key = (tokens_per_item, balance if self.ctx_lens is not None else 0, runs)
         it = self._items.get(key)
         if it is None:
             # numpy throughout: a stack of several attention kinds with a prompt of 2048 tokens waited for the host here
             ql = np.asarray(self.q_lens, dtype=np.int64).reshape(-1)
             per = -(-ql // tokens_per_item)                       # items of each run
+            if runs is not None:
+                per[:runs[0]] = per[runs[1]:] = 0
             seq = np.repeat(np.arange(len(ql)), per)
             a = (np.arange(len(seq)) - np.repeat(np.cumsum(per) - per, per)) * tokens_per_item  # within the run
             c = np.minimum(tokens_per_item, ql[seq] - a)

@@ -151,15 +151,16 @@ class LatentAttention(torch.nn.Module):
         self.o = ColumnLinear(heads * vdim, d_model, shard=False, device=device, dtype=dtype)
         self.register_buffer("cos_sin", rope_table(rot_dims, rot_base, max_pos if rot_dims else 1, device, rot_scaling),
                              persistent=False)
-        self.cache = self.uv_t = self.uk_t = None
+        self.cache = self.uv_t = self.uk_t = self.w_kv = None
         # what the runner's generic bookkeeping reads
         self.Hq, self.Hkv, self.D, self.window, self.sinks = heads, 1, kv_rank + rot_dim, 0, None
 
     def finalize(self):
         """W_uv per head as [R, vdim]: the read-out's batched product takes its right operand row-major; W_uk as [R, dim] for the
-        kernel of a few rows, which takes it by columns."""
+        kernel of a few rows, which takes it by columns; both together, head by head, for prompts that make keys and values."""
         self.uv_t = self.uv.data.view(self.H, self.dv, self.R).transpose(1, 2).contiguous()
         self.uk_t = self.uk.data.view(self.H, self.dn, self.R).transpose(1, 2).contiguous()
+        self.w_kv = torch.cat([self.uk.data.view(self.H, self.dn, self.R), self.uv.data.view(self.H, self.dv, self.R)], 1).view(-1, self.R)
 
     @property
     def owns_cache(self) -> bool:
@@ -191,15 +192,20 @@ class LatentAttention(torch.nn.Module):
         q_abs = torch.empty(T, H, R + dr, dtype=h.dtype, device=h.device)
         sm.latent_rope_cache(q, kv, self.dkv_norm if kv is not None else None, self.eps, meta.positions, self.cos_sin,
                              H, dn, dr, self.rot_dims, R, meta.slot_mapping, cache, q_abs, self.interleaved)
-        # absorb W_uk into the query: scores against the latent itself
-        qn = q.reshape(T, H, dn + dr)[:, :, :dn]
-        if not sm.head_product(qn, self.uk_t, q_abs[:, :, :R]):                                       # written where it is read
-            torch.bmm(qn.transpose(0, 1), self.uk.view(H, dn, R), out=q_abs[:, :, :R].transpose(0, 1))
-        o_lat = sm.latent_attention(q_abs, cache, s.tables, s.row_seq, s.row_len, self.scale, R,
-                                    rows_per_group=4 if s.max_q > 1 else 1, seq=s, gate=gate, window=self.win)
         o = torch.empty(T, H, self.dv, dtype=h.dtype, device=h.device)
-        if not sm.head_product(o_lat, self.uv.view(H, self.dv, R), o):
-            torch.bmm(o_lat.transpose(0, 1), self.uv_t, out=o.transpose(0, 1))
+        own = sm.latent_own_from(s, H, dn, dr, self.dv, R, h.dtype, self.win)
+        if own is not None:
+            sm.latent_own(q, q_abs, cache, self.w_kv, self.scale, R, s, own, gate, o)
+        n = T if own is None else own  # rows that absorb W_uk into the query: scores against the latent itself
+        if n:
+            qn = q[:n].reshape(n, H, dn + dr)[:, :, :dn]
+            if not sm.head_product(qn, self.uk_t, q_abs[:n, :, :R]):                                       # written where it is read
+                torch.bmm(qn.transpose(0, 1), self.uk.view(H, dn, R), out=q_abs[:n, :, :R].transpose(0, 1))
+            o_lat = sm.latent_attention(q_abs[:n], cache, s.tables, s.row_seq[:n], s.row_len[:n], self.scale, R,
+                                        rows_per_group=4 if s.max_q > 1 else 1, seq=s, gate=None if gate is None else gate[:n],
+                                        window=self.win, singles=own or 0)
+            if not sm.head_product(o_lat, self.uv.view(H, self.dv, R), o[:n]):
+                torch.bmm(o_lat.transpose(0, 1), self.uv_t, out=o[:n].transpose(0, 1))
         return self.o(o.view(T, H * self.dv))
 
 

@@ -26,6 +26,7 @@ from __future__ import annotations
 import importlib
 import os
 
+import numpy as np
 import torch
 
 from . import seqmix_ref as ref
@@ -108,9 +109,10 @@ MFMA_ATTENTION = os.environ.get("LLMD_LATENT_MFMA", "1") == "1"
 
 
 def latent_attention(q_abs, cache, tables, row_seq, row_len, scale: float, R: int, rows_per_group: int = 1,
-                     seq=None, gate=None, window: int = 0):
+                     seq=None, gate=None, window: int = 0, singles: int = 0):
     """Causal softmax attention of absorbed queries [T, H, R + dr] over the paged latent cache
-    [blocks, bs, R + dr]; row t sees the first row_len[t] keys of sequence row_seq[t].
+    [blocks, bs, R + dr]; row t sees the first row_len[t] keys of sequence row_seq[t]. ``singles`` > 0: the rows are the first
+    ``singles`` sequences' of ``seq``, which bring one token each, as a step of their own.
     Returns the latent outputs [T, H, R]. ``gate`` [T, H] (a column view of a projection): head h's
     output is multiplied by sigmoid(gate[t, h]). ``window`` > 0: query i sees key j <= i only if
     i - j < window (positions in the sequence); earlier key tiles are not visited.
@@ -124,11 +126,12 @@ def latent_attention(q_abs, cache, tables, row_seq, row_len, scale: float, R: in
     if not q_abs.is_cuda:
         return ref.latent_attention(q_abs, cache, tables, row_seq, row_len, scale, R, out, gate, window)
     if MFMA_ATTENTION and seq is not None and q_abs.dtype == torch.bfloat16 and H <= 64:
+        max_q, max_len = (1, max(seq.ctx_lens[:singles])) if singles else (seq.max_q, seq.max_len)
         # ids 256 apart share a CU: long and short items together
-        items = seq.attention_items(max(1, 64 // H), balance=256 if seq.max_q > 1 else 0)
+        items = seq.attention_items(max(1, 64 // H), balance=256 if max_q > 1 else 0, runs=(0, singles) if singles else None)
         nsplit, split, po, pm = 1, 0, None, None
-        rows = H if seq.max_q == 1 else 0   # decode-only step: one token per item, its rows shared by the waves
-        span = min(seq.max_len, window + 64) if window else seq.max_len   # keys a row's tiles hold at most
+        rows = H if max_q == 1 else 0   # decode-only step: one token per item, its rows shared by the waves
+        span = min(max_len, window + 64) if window else max_len   # keys a row's tiles hold at most
         if rows and span > 64:
             # cut the keys into ranges so that items x row blocks x ranges fill the chip: of one tile up to 32 of them (as a captured
             # step does, whatever it was captured for: the same bits), else of two
@@ -146,6 +149,47 @@ def latent_attention(q_abs, cache, tables, row_seq, row_len, scale: float, R: in
     native().latent_attention(q_abs, cache, tables, row_seq, row_len, float(scale), R, int(rows_per_group), out, gate,
                               int(window))
     return out
+
+
+LATENT_OWN = os.environ.get("LLMD_LATENT_OWN", "1") == "1"
+LATENT_OWN_KEYS = 1 << 16  # keys made at once: 0.5 GB of keys and values with 16 heads
+
+
+def latent_own_from(seq, H: int, dn: int, dr: int, dv: int, R: int, dtype, window: int = 0):
+    """The first of a step's sequences whose rows attend over keys and values of their own (``latent_own``), or None: the ones behind
+    the step's single tokens, where their rows meet enough keys."""
+    if not (LATENT_OWN and MFMA_ATTENTION and dtype == torch.bfloat16 and (dn, dr, dv) == (128, 64, 128) and R % 64 == 0 and not window
+            and seq.max_q > 1 and seq.ctx_lens is not None and seq.tables.is_cuda):
+        return None
+    first = seq.singles()
+    n, ctx = np.asarray(seq.q_lens[first:], dtype=np.float64), np.asarray(seq.ctx_lens[first:], dtype=np.float64)
+    rows, keys = float(n.sum()), float(ctx.sum())
+    if keys > LATENT_OWN_KEYS or float(np.ceil(n / 64).sum()) > 65535:
+        return None
+    # us of both on 16 and more heads: making keys and values against absorbing and the two products around it; a tile of 32
+    # keys in the longest row's chain, or all pairs of rows and keys. Measured, own / absorbed: 16 heads, 64 rows 15 / 11, 128 20 / 23, 2048
+    # 89 / 172, 4000 163 / 409, 64 after 1000 50 / 75, 1024 after 4000 189 / 316; 64 heads, 64 after 4000 189 / 237, 2048 179 / 481
+    k, longest, pairs = H / 16, float(ctx.max()), float((n * (ctx - n / 2)).sum())
+    own = 12 + 0.006 * keys * k + max(0.9 * longest / 32, 15e-6 * pairs * k)
+    absorbed = (14 if rows > 64 else 6) + 0.017 * rows * k + max(1.75 * longest / 32, 68e-6 * pairs * k)
+    return first if own < absorbed else None
+
+
+def latent_own(q, q_abs, cache, w_kv, scale: float, R: int, seq, first: int, gate, out):
+    """Attention of the rows behind the first ``first`` single tokens over keys and values made once per head, the same function as
+    absorbing W_uk into the query and applying W_uv to the read-out: q [T, H (128 + 64)], its rotated parts in q_abs [T, H, R + 64],
+    w_kv [H (128 + 128), R] (every head's rows of W_uk, then of W_uv), cache [blocks, bs, R + 64]; out [T, H, 128], of which those
+    rows are written."""
+    from . import linear
+
+    bounds, keys, longest = seq.key_rows(first)
+    lat = torch.empty(keys, R, dtype=cache.dtype, device=cache.device)
+    rot = torch.empty(keys, cache.shape[2] - R, dtype=cache.dtype, device=cache.device)
+    native().latent_gather(cache, seq.tables, bounds, first, longest, lat, rot)
+    H = out.shape[1]
+    # ids 256 apart share a CU: long and short items together
+    items = seq.attention_items(64, balance=max(1, 256 // H), runs=(first, len(seq.q_lens)))
+    native().latent_own(q, q_abs, R, linear(lat, w_kv), rot, bounds, items, seq.row_len, float(scale), out, gate)
 
 
 def causal_conv_silu(xz, C, w, b, conv_state, seq_start, seq_slot, seq_init, max_q: int):
