@@ -24,6 +24,9 @@ int sm_latent_attention(const void*, const void*, const int*, int, int, const in
 int sm_latent_attention_mfma(const void*, const void*, const int*, int, int, const int*, int, const int*, float, int,
                              int, int, void*, int, int, float*, float*, const void*, int64_t, int, int, const int*,
                              hipStream_t);
+int sm_latent_f32_range();
+int sm_latent_f32(const void*, const void*, const int*, int, int, const int*, int, const int*, float, int, int, int, void*, const void*, int64_t,
+                  int, int, float*, float*, hipStream_t);
 void sm_latent_gather(const void*, const int*, int, int, const int*, int, int, int, int, int, void*, void*, hipStream_t);
 void sm_latent_own(const void*, int64_t, const void*, int64_t, int64_t, const void*, const void*, const int*, const int*, int, const int*,
                    float, int, void*, const void*, int64_t, hipStream_t);
@@ -299,6 +302,37 @@ bool latent_attention_mfma(Tensor q_abs, Tensor cache, Tensor tables, Tensor ite
                                   (float)scale, H, R, Dk, out.data_ptr(), nsplit, split_keys, po, pm,
                                   gate ? gate->data_ptr() : nullptr, gate ? gate->stride(0) : 0, window, rows,
                                   longest_of(longest), cur()) == 0;
+}
+
+// fp32 on the matrix cores; nsplit > 1 (single tokens): ranges of latent_f32_range keys apart. False: not these sizes
+bool latent_f32(Tensor q_abs, Tensor cache, Tensor tables, Tensor items, Tensor row_len, double scale, int64_t R, Tensor out, int64_t nsplit,
+                c10::optional<Tensor> part_o, c10::optional<Tensor> part_ml, std::optional<Tensor> gate, int64_t window) {
+  const c10::hip::OptionalHIPGuard g(dev_of(q_abs));
+  TORCH_CHECK(q_abs.is_cuda() && q_abs.scalar_type() == torch::kFloat32 && q_abs.dim() == 3 && q_abs.is_contiguous(), "q_abs [T, H, Dk] fp32");
+  const int64_t T = q_abs.size(0), H = q_abs.size(1), Dk = q_abs.size(2), HG = (H + 15) / 16;
+  CHECK_ACT(cache, q_abs);
+  TORCH_CHECK(cache.dim() == 3 && cache.is_contiguous() && cache.size(2) == Dk && R >= 1 && R <= Dk, "cache");
+  CHECK_I32(tables);
+  CHECK_I32(items);
+  CHECK_I32(row_len);
+  TORCH_CHECK(tables.dim() == 2 && row_len.numel() == T && items.dim() == 2 && items.size(1) == 3, "tables");
+  CHECK_ACT(out, q_abs);
+  TORCH_CHECK(out.is_contiguous() && out.numel() == T * H * R, "out [T, H, R]");
+  check_head_gate(gate, q_abs);
+  TORCH_CHECK(nsplit >= 1 && nsplit <= (1 << 20) && window >= 0 && window < (1ll << 30), "ranges, window");
+  float *po = nullptr, *pm = nullptr;
+  if (nsplit > 1) {
+    TORCH_CHECK(part_o.has_value() && part_ml.has_value(), "ranges apart without workspace");
+    CHECK_F32(*part_o);
+    CHECK_F32(*part_ml);
+    const int64_t rows = items.size(0) * HG * nsplit * 16;
+    TORCH_CHECK(part_o->numel() >= rows * R && part_ml->numel() >= rows * 2, "workspace too small");
+    po = part_o->data_ptr<float>();
+    pm = part_ml->data_ptr<float>();
+  }
+  return sm_latent_f32(q_abs.data_ptr(), cache.data_ptr(), tables.data_ptr<int>(), tables.size(1), cache.size(1), items.data_ptr<int>(),
+                       items.size(0), row_len.data_ptr<int>(), (float)scale, H, R, Dk, out.data_ptr(), gate ? gate->data_ptr() : nullptr,
+                       gate ? gate->stride(0) : 0, window, nsplit, po, pm, cur()) == 0;
 }
 
 // lat [keys, R], rot [keys, dr] <- the cached rows of sequences first .. ; base [sequences + 1]: their places, the number of keys at the end
@@ -1210,6 +1244,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("input_conv", &input_conv);
   m.def("hgrn2_scan", &hgrn2_scan);
   m.def("latent_gather", &latent_gather);
+  m.def("latent_f32", &latent_f32);
+  m.def("latent_f32_range", &sm_latent_f32_range);
   m.def("latent_own", &latent_own);
   m.def("gated_add_norm", &gated_add_norm);
   m.def("poly_norm", &poly_norm);

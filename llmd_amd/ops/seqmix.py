@@ -146,6 +146,21 @@ def latent_attention(q_abs, cache, tables, row_seq, row_len, scale: float, R: in
         if native().latent_attention_mfma(q_abs, cache, tables, items, row_len, float(scale), R, out, nsplit, split,
                                           po, pm, gate, int(window), rows, seq.longest):
             return out
+    if MFMA_ATTENTION and seq is not None and q_abs.dtype == torch.float32 and R == 512 and not singles:
+        C = native()
+        items = seq.attention_items(max(1, 16 // H))
+        # fixed ranges in every step: dealt to several workgroups where one per item leaves CUs idle, with the same bits either way
+        n, FR = items.shape[0] * -(-H // 16), C.latent_f32_range()
+        nsplit, po, pm = -(-seq.max_len // FR), None, None
+        if window:  # keys from a multiple of 32 on
+            nsplit = min(nsplit, (window + 31 + 2 * FR - 33) // FR)
+        if seq.max_q > 1 or n >= LATENT_DECODE_WGS or n * nsplit * 16 * R > 1 << 28:
+            nsplit = 1
+        if nsplit > 1:
+            po = torch.empty(n * nsplit * 16 * R, dtype=torch.float32, device=q_abs.device)
+            pm = torch.empty(n * nsplit * 32, dtype=torch.float32, device=q_abs.device)
+        if C.latent_f32(q_abs, cache, tables, items, row_len, float(scale), R, out, nsplit, po, pm, gate, int(window)):
+            return out
     native().latent_attention(q_abs, cache, tables, row_seq, row_len, float(scale), R, int(rows_per_group), out, gate,
                               int(window))
     return out
