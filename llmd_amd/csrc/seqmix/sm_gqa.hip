@@ -185,7 +185,7 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_kernel(
 // vector cache: angles are read once for all heads of a thread, weights 16 bytes at a time. 2048 tokens of 32 + 4 heads of 128
 // with bias, weights before the rotation and keys as values: 33 us with the partner's values, bias and weights read again,
 // now 17.7; without any of them 12.4.
-// blockIdx.y < gh: the heads of token blockIdx.x. The other workgroups take the values, a column per
+// gh of blockIdx.y: the heads of token blockIdx.x. The other workgroups take the values, a column per
 // thread and tg (1 or 8) tokens: the values of a page are transposed, so eight consecutive tokens of a
 // sequence whose first lands on a multiple of eight are one 16-byte store (a prompt's inner tokens).
 __device__ __forceinline__ void ld8(const bf16_t* p, float (&v)[8]) {
@@ -221,7 +221,10 @@ __device__ __forceinline__ void st8(float* p, const float (&v)[8], float mul) {
   *reinterpret_cast<float4*>(p + 4) = make_float4(v[4] * mul, v[5] * mul, v[6] * mul, v[7] * mul);
 }
 
-// The values of tg (1 or 8) tokens, a column per thread; ``unit`` numbers the workgroups of this part.
+// The values of tg (1 or 8) tokens, a column per thread; ``unit`` numbers the workgroups of this part. Eight tokens whose places in a page
+// are eight whole ones are one store of 16 bytes per column, wherever they begin in the step: the workgroup in whose tokens they begin
+// takes them, the others leave them out. 2532 tokens, three portions after 333, 36 heads and 512 value columns, us, when they had to begin
+// where a workgroup's eight tokens do / now: norms over whole projections 21.7 / 16.8, none 17.5 / 13.8; 2048 whole ones 15.2 / 15.1, 12.0 / 12.1.
 template <typename T, int TAPS>
 __device__ __forceinline__ void value_part(int unit, const T* __restrict__ qkv, int64_t stride,
                                            const float* __restrict__ bias, const int64_t* __restrict__ positions, int Hq,
@@ -230,36 +233,39 @@ __device__ __forceinline__ void value_part(int unit, const T* __restrict__ qkv, 
                                            int v_from_k, const ConvArgs<T>& cv, int tg, int ntok) {
   const int nv = Hkv * vdim, vcol0 = v_from_k ? Hq * dim : (Hq + Hkv) * dim, nvb = (nv + NT - 1) / NT;
   const int e = (unit % nvb) * NT + threadIdx.x, t0 = unit / nvb * tg;
-  if (t0 >= ntok || e >= nv) return;
-  const int col = vcol0 + e, g = e / vdim, c = e - g * vdim;
+  if (t0 >= ntok) return;
+  // lane l: the place of token t0 - 7 + l; bit l of ``next``: the token behind it has the next place
+  int64_t place = -1;
+  uint64_t next = 0;
+  if (tg == 8 && (bs & 7) == 0) {
+    const int lane = threadIdx.x & 63, t = t0 - 7 + lane;
+    if (lane < 23 && t >= 0 && t < ntok) place = slots[t];
+    const int64_t behind = __shfl_down(place, 1, 64);
+    next = __ballot(place >= 0 && behind == place + 1);
+  }
+  const int col = vcol0 + min(e, nv - 1), ec = min(e, nv - 1), g = ec / vdim, c = ec - g * vdim;
   const float vb = bias ? bias[col] : 0.f;
   const int64_t vbase = (int64_t)g * bs * (dim + vdim) + (int64_t)bs * dim + (int64_t)c * bs;  // within a page
   const int64_t page = (int64_t)Hkv * bs * (dim + vdim);
   float w[TAPS > 0 ? TAPS : 1];
 #pragma unroll
   for (int j = 0; j < TAPS; ++j) w[j] = ld(cv.w + (int64_t)col * TAPS + j);
-  const int64_t s0 = slots[t0];
-  bool eight = tg == 8 && t0 + 8 <= ntok && s0 >= 0 && (s0 & 7) == 0 && (bs & 7) == 0;
-  if (eight) {
-#pragma unroll
-    for (int i = 1; i < 8; ++i) eight &= slots[t0 + i] == s0 + i;  // none that is not to be written among them
-  }
-  if (eight) {  // one page, hence one sequence
+  auto eight = [&](int t1, int64_t s0) {  // one page, hence one sequence
     constexpr int PAST = TAPS > 1 ? TAPS - 1 : 0;
     float u[8 + PAST];
     if constexpr (PAST > 0) {
-      const int s = cv.row_seq[t0], run0 = t0 - cv.seq_start[s];
-      const int64_t pos0 = positions[t0];
+      const int s = cv.row_seq[t1], run0 = t1 - cv.seq_start[s];
+      const int64_t pos0 = positions[t1];
       const T* past = cv.state + (int64_t)cv.seq_slot[s] * PAST * cv.C;
 #pragma unroll
       for (int k = 0; k < PAST; ++k) {
         const int back = PAST - k;
         u[k] = pos0 < back ? 0.f
-                           : ld(run0 >= back ? qkv + (t0 - back) * stride + col : past + (int64_t)(k + run0) * cv.C + col) + vb;
+                           : ld(run0 >= back ? qkv + (t1 - back) * stride + col : past + (int64_t)(k + run0) * cv.C + col) + vb;
       }
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) u[PAST + i] = ld(qkv + (t0 + i) * stride + col) + vb;
+    for (int i = 0; i < 8; ++i) u[PAST + i] = ld(qkv + (t1 + i) * stride + col) + vb;
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -270,13 +276,12 @@ __device__ __forceinline__ void value_part(int unit, const T* __restrict__ qkv, 
       } else {
         v[i] = u[i];
       }
-      if (v_mode == 1) v_first[(int64_t)(t0 + i) * nv + e] = v[i];
-      else if (v_mode == 2) v[i] = (1.f - lam) * v[i] + lam * v_first[(int64_t)(t0 + i) * nv + e];
+      if (v_mode == 1) v_first[(int64_t)(t1 + i) * nv + e] = v[i];
+      else if (v_mode == 2) v[i] = (1.f - lam) * v[i] + lam * v_first[(int64_t)(t1 + i) * nv + e];
     }
     st8(cache + s0 / bs * page + vbase + s0 % bs, v, 1.f);
-    return;
-  }
-  for (int t = t0; t < min(t0 + tg, ntok); ++t) {
+  };
+  auto single = [&](int t) {
     const T* row = qkv + t * stride;
     float v = ld(row + col) + vb;
     if constexpr (TAPS > 0) v *= w[TAPS - 1];
@@ -300,6 +305,18 @@ __device__ __forceinline__ void value_part(int unit, const T* __restrict__ qkv, 
     else if (v_mode == 2) v = (1.f - lam) * v + lam * v_first[(int64_t)t * nv + e];
     const int64_t slot = slots[t];
     if (slot >= 0) st(cache + slot / bs * page + vbase + slot % bs, v);
+  };
+  if (e >= nv) return;
+  for (int i = 0; i < min(tg, ntok - t0); ++i) {
+    bool whole = false;
+    int64_t s0 = -1;
+    if (next != 0) {
+      // (readlane: a wave's last lanes may have no column)
+      s0 = (int64_t)__builtin_amdgcn_readlane((int)(place >> 32), 7 + i) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)place, 7 + i);
+      whole = s0 >= 0 && (next >> (7 + i - (int)(s0 & 7)) & 0x7f) == 0x7f;
+    }
+    if (!whole) single(t0 + i);
+    else if ((s0 & 7) == 0) eight(t0 + i, s0);
   }
 }
 
@@ -311,8 +328,10 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_vec_kernel(
     const int64_t* __restrict__ slots, T* __restrict__ cache, int bs, T* __restrict__ q_out,
     const float* __restrict__ qk_w, int norm_first, int v_from_k, ConvArgs<T> cv,
     int gh, int tg, int ntok, const float* __restrict__ q_scale) {
-  if ((int)blockIdx.y >= gh) {
-    value_part<T, TAPS>(((int)blockIdx.y - gh) * gridDim.x + blockIdx.x, qkv, stride, bias, positions, Hq, Hkv, dim, vdim,
+  // the values first: theirs is the longer wait (where they are keys, behind the heads, which read the same columns: 19.2 us, in front 21)
+  const int vy = v_from_k ? (int)blockIdx.y - gh : (int)blockIdx.y, hy = v_from_k ? (int)blockIdx.y : (int)(blockIdx.y + gh - gridDim.y);
+  if (v_from_k ? vy >= 0 : hy < 0) {
+    value_part<T, TAPS>(vy * gridDim.x + blockIdx.x, qkv, stride, bias, positions, Hq, Hkv, dim, vdim,
                      v_first, v_mode, lam, slots, cache, bs, v_from_k, cv, tg, ntok);
     return;
   }
@@ -342,7 +361,7 @@ __global__ __launch_bounds__(NT) void qkv_rope_cache_vec_kernel(
     add8(cs + (first ? c * 8 : c * 8 - half), cc);
     add8(cs + half + (first ? c * 8 : c * 8 - half), sn);
   }
-  for (int h0 = blockIdx.y * hpp; h0 < Hq + Hkv; h0 += gh * hpp) {
+  for (int h0 = hy * hpp; h0 < Hq + Hkv; h0 += gh * hpp) {
     const int hd = h0 + hl;
     const bool on = hd < Hq + Hkv;
     const int col = hd * dim + c * 8;  // q heads, then k heads, back to back in the projection
@@ -448,8 +467,8 @@ __global__ __launch_bounds__(NT) void qkv_wide_cache_vec_kernel(
     int rot_dims, float eps, float* __restrict__ v_first, int v_mode, float lam, const int64_t* __restrict__ slots,
     T* __restrict__ cache, int bs, T* __restrict__ q_out, const float* __restrict__ qk_w,
     ConvArgs<T> cv, int tg, int ntok, const float* __restrict__ q_scale) {
-  if (blockIdx.y > 0) {
-    value_part<T, 0>(((int)blockIdx.y - 1) * gridDim.x + blockIdx.x, qkv, stride, bias, positions, Hq, Hkv, dim, vdim,
+  if (blockIdx.y + 1 < gridDim.y) {  // the values first: theirs is the longer wait
+    value_part<T, 0>((int)blockIdx.y * gridDim.x + blockIdx.x, qkv, stride, bias, positions, Hq, Hkv, dim, vdim,
                   v_first, v_mode, lam, slots, cache, bs, 0, cv, tg, ntok);
     return;
   }
