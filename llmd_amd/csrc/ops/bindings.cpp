@@ -74,6 +74,8 @@ int64_t llmd_pgemm_ws_bytes(int, int, int, int, int);
 int llmd_tgemm_plan(int, int, int, int);
 int llmd_tgemm(const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, float, int, const void*, void*,
                hipStream_t);
+int llmd_router_form(int, int, int, int);
+int llmd_router_product(const void*, int64_t, const void*, int64_t, int, int, int, const void*, int, void*, int, hipStream_t);
 int llmd_fgemm_plan(int, int, int);
 int llmd_fgemm(const void*, int64_t, const void*, int64_t, void*, int64_t, int, int, int, int, const void*, void*, hipStream_t);
 int llmd_pgemm_fp8(const void*, int64_t, const float*, const void*, int64_t, const float*, void*, int64_t, int, int,
@@ -669,6 +671,31 @@ std::optional<torch::Tensor> tgemm(const torch::Tensor& x, const torch::Tensor& 
                             (int)K, (int)act, (float)limit, code, bias ? bias->data_ptr() : nullptr,
                             ws.defined() ? ws.data_ptr() : nullptr, cur_stream());
   TORCH_CHECK(rc == 0, "tgemm failed: ", rc);
+  return y;
+}
+
+// A router's product x w^T (+ bias) of bf16 operands, in fp32 (f32) or bf16 (csrc/ops/router.hip), in the form that llmd_router_form
+// has for these sizes, or in `form`; nothing where it has none or the operands are not what the kernel reads
+std::optional<torch::Tensor> router_product(const torch::Tensor& x, const torch::Tensor& w, const std::optional<torch::Tensor>& bias,
+                                            bool f32, int64_t form) {
+  if (!x.is_cuda() || x.device() != w.device() || x.dim() != 2 || w.dim() != 2 || x.scalar_type() != at::kBFloat16 ||
+      w.scalar_type() != at::kBFloat16)
+    return std::nullopt;
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  const auto off = [](const torch::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 != 0; };
+  if (w.size(1) != K || M > (1 << 24) || N > (1 << 16) || K > (1 << 24) || x.stride(1) != 1 || w.stride(1) != 1 ||
+      x.stride(0) % 8 || w.stride(0) % 8 || x.stride(0) < 0 || w.stride(0) < 0 || off(x) || off(w))
+    return std::nullopt;
+  if (bias && (bias->scalar_type() != at::kBFloat16 || bias->device() != x.device() || bias->dim() != 1 || bias->size(0) != N ||
+               (N > 1 && bias->stride(0) != 1)))
+    return std::nullopt;
+  if (form < 0) form = llmd_router_form((int)M, (int)N, (int)K, f32 ? 1 : 0);
+  if (form < 0) return std::nullopt;
+  const c10::hip::OptionalHIPGuard device_guard(dev_of(x));
+  torch::Tensor y = torch::empty({M, N}, f32 ? x.options().dtype(torch::kFloat) : x.options());
+  const int rc = llmd_router_product(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), (int)M, (int)N, (int)K,
+                                     bias ? bias->data_ptr() : nullptr, f32 ? 1 : 0, y.data_ptr(), (int)form, cur_stream());
+  TORCH_CHECK(rc == 0, "router_product failed: ", rc);
   return y;
 }
 
@@ -1481,6 +1508,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {  // _C, or _C_debug (llmd_amd/build.p
   m.def("mgemm_add_rmsnorm", &mgemm_add_rmsnorm, "decode o / down projection with residual-add + RMSNorm in its split-K reduce");
   m.def("pgemm_fp8", &pgemm_fp8, "prefill fp8 W8A8 GEMM (256x256 LDS-DMA tiles on 16x16x128 f8f6f4 MFMA), "
         "per-token x per-channel scales, optional fused SiLU-and-mul");
+  m.def("router_product", &router_product, "a router's x w^T (+ bias), fp32 or bf16, or None", py::arg("x"), py::arg("w"),
+        py::arg("bias") = py::none(), py::arg("f32") = false, py::arg("form") = -1);
+  m.def("router_form", &llmd_router_form, "form of router_product for (M, N, K, f32), or -1");
   m.def("tgemm", &tgemm, "bf16 GEMM of prompt-sized steps on the tile that fits, or None", py::arg("x"), py::arg("w"),
         py::arg("bias") = std::nullopt, py::arg("act") = 0, py::arg("tile") = 0, py::arg("limit") = 0.0);
   m.def("tgemm_plan", &llmd_tgemm_plan, "tile of tgemm for (M, N, K, silu): mi * 100 + ni * 10 + ranges of K, or 0");

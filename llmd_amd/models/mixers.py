@@ -536,7 +536,7 @@ class ScoreMoE(torch.nn.Module):
         self.router32, self.correction32 = self.router.data.float(), self.correction.data.float()
 
     def forward(self, h):
-        logits = sm.router_logits(h, self.router.data)
+        logits = ops.router_product(h, self.router.data)
         if logits is None:
             logits = F.linear(h.float(), self.router32)
         ids, w = sm.moe_route_scores(logits, self.correction32, self.k, self.groups, self.keep, self.scale)
@@ -658,7 +658,7 @@ class SigmoidMoE(torch.nn.Module):
         self.router32 = self.router.data.float()
 
     def forward(self, h):
-        logits = sm.router_logits(h, self.router.data)
+        logits = ops.router_product(h, self.router.data)
         if logits is None:
             logits = F.linear(h.float(), self.router32)
         ids, w = sm.moe_route(logits, self.k, sigmoid=True)

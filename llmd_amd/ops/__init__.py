@@ -1471,9 +1471,20 @@ def fgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None)
 
 
 def router_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """A router's logits: prompts on ``tgemm`` (2048 x (128, 2048) hipBLASLt 12.4 us, here 7), the rest on the library."""
-    y = tgemm(x, w, bias) if x.dim() == 2 and x.shape[0] > 64 else None
+    """A router's logits in x's dtype: few columns on the kernel of csrc/ops/router.hip (which holds the rule; 64 x (128, 2048) 5.5 us on the
+    library, 3.3 there), large prompts on ``tgemm``, the rest on the library."""
+    if not _gpu(x) or not _plain(x, w):
+        return torch.nn.functional.linear(x, w, bias)
+    y = native().router_product(x, w, bias)
+    if y is None and x.dim() == 2 and x.shape[0] > 64:
+        y = tgemm(x, w, bias)
     return torch.nn.functional.linear(x, w, bias) if y is None else y
+
+
+def router_product(x: torch.Tensor, w: torch.Tensor):
+    """x w^T in fp32 of bfloat16 x [M, K] and w [N, K] (csrc/ops/router.hip), whose products are exact in fp32, or None. No further from
+    64 bits than a float product of widened copies; a row's numbers do not depend on the others."""
+    return native().router_product(x, w, None, True) if _gpu(x) and _plain(x, w) else None
 
 
 def pgemm_pack_gate_up(w: torch.Tensor) -> torch.Tensor:
