@@ -10,7 +10,8 @@
 //                   once (16-byte pieces, a thread keeps its columns), and norms and gates the read-out.
 // Longer runs are cut into chunks of at most C = 64 tokens. A chunk of n tokens that starts from S gives
 //   o_i = decay^(i+1) S^T q_i + sum_{j <= i} decay^(i-j) (q_i . k_j) v_j,   S' = decay^n S + sum_j decay^(n-1-j) k_j v_j^T
-// so all products are matrix products. They run on v_mfma_f32_16x16x4_f32: operands and sums are fp32.
+// so all products are matrix products. They run on v_mfma_f32_16x16x4_f32: operands and sums are fp32. bf16 rows of the usual head sizes
+// take the kernels *_parts further down instead.
 // retention_chunk : every chunk's own part of its final state, L = sum_j decay^(n-1-j) k_j v_j^T.
 // retention_link  : walks a sequence's chunks in order, S_(c+1) = decay^n S_c + L_c; leaves every chunk's start
 //                   state where its L was and the run's final state in the slot.
@@ -19,6 +20,7 @@
 //                   workgroup holds all of a head's columns, else retention_norm follows.
 // In all of them the contraction index is dealt so that an operand's four consecutive elements belong to one lane:
 // step e of a group of 16 takes element 4 kq + e from lane group kq, on both sides.
+#include "moe_tile.h"
 #include "seqmix_common.h"
 #include <algorithm>
 
@@ -487,12 +489,427 @@ __global__ __launch_bounds__(NT) void retention_norm_kernel(const float* __restr
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same two products on v_mfma_f32_16x16x32_bf16, for bf16 rows: numbers that are fp32 (rotated q and k, weights, the state) as
+// three bf16 parts, times 2^24 (moe_tile.h says why); v is bf16 as it is, so its products take three instructions and are exact, those of
+// two fp32 numbers six. Sums that are not finite (infinities, NaN, numbers that overflow so scaled) are done again
+// number by number. The contraction index is dealt to the lane groups in eights; a lane's eight are one 16-byte piece in LDS.
+// Bound by the chunks' states (a head's 128 KB written once and read twice per 64 tokens) and by the chain of loads and barriers of a
+// workgroup; the fp32 instructions alone had taken half of the time, loads one after the other most of the rest.
+// us, chunk + out, 16 heads of 128 x 256: 901 + 844 + 787 tokens 65 + 100 -> 38 + 53. States off 64 bits: less than before (exact
+// products, a sixteenth of the roundings).
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+constexpr float UP1 = 0x1p-24f;  // of sums with one factor times 2^24
+struct Parts {
+  u32x4_t p[3];  // 8 elements: largest part first
+};
+// (As vectors of two: hipcc rounds scalar casts twice, and what asm writes it hands to the matrix units too early.)
+__device__ __forceinline__ Parts split_vals(const float (&a)[4], const float (&b)[4]) {
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  f32x2_t x[4] = {{a[0], a[1]}, {a[2], a[3]}, {b[0], b[1]}, {b[2], b[3]}};
+  Parts r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    x[j] *= moe_tile::SPLIT_UP;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(x[j], bf16x2_t));
+      x[j][0] -= __uint_as_float(w << 16), x[j][1] -= __uint_as_float(w & 0xffff0000u);
+      r.p[i][j] = w;
+    }
+  }
+  return r;
+}
+
+__device__ __forceinline__ f32x4_t mfma_bf(const u32x4_t& a, const u32x4_t& b, const f32x4_t& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4_t mfma_six(const u32x4_t (&a)[3], const u32x4_t (&b)[3], f32x4_t c) {
+  c = mfma_bf(a[2], b[0], c);
+  c = mfma_bf(a[0], b[2], c);
+  c = mfma_bf(a[1], b[1], c);
+  c = mfma_bf(a[1], b[0], c);
+  c = mfma_bf(a[0], b[1], c);
+  return mfma_bf(a[0], b[0], c);
+}
+// Eight rows of W columns (rows[i]: the columns' first bits) to W pieces of eight rows each
+__device__ __forceinline__ uint32_t pick(uint32_t a, uint32_t b, bool high) {
+  return high ? (a >> 16) | (b & 0xffff0000u) : (a & 0xffffu) | (b << 16);
+}
+template <int W>
+__device__ __forceinline__ u32x4_t column(const uint32_t (&rows)[8][W / 2], int i) {
+  u32x4_t r;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) r[x] = pick(rows[2 * x][i / 2], rows[2 * x + 1][i / 2], i & 1);
+  return r;
+}
+// Places of column c's piece where a lane writes W consecutive columns: eight lanes' pieces in banks of their own
+template <int W>
+__device__ __forceinline__ int place(int c) {
+  return W == 4 ? (c & ~3) | ((c + (c >> 3)) & 3) : c ^ ((c >> 3) & 1);
+}
+// W columns of eight tokens, token(i) the place of the i-th one in the chunk; zeros past n. rv: the chunk's values, col: the first column.
+// SHARED: a wave's tokens are the same, their places go beside the address that all lanes share (as pointers hipcc keeps all eight in
+// registers and spills).
+template <int W, bool SHARED, typename F>
+__device__ __forceinline__ void load_v(__amdgpu_buffer_rsrc_t rv, int64_t stride, int col, int n, F token, uint32_t (&rows)[8][W / 2]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int j = token(i), at = min(j, n - 1) * (int)stride * 2;
+    if constexpr (W == 4) {
+      const auto t = __builtin_amdgcn_raw_buffer_load_b64(rv, col * 2 + (SHARED ? 0 : at), SHARED ? at : 0, 0);
+      rows[i][0] = t[0], rows[i][1] = t[1];
+    } else {
+      rows[i][0] = __builtin_amdgcn_raw_buffer_load_b32(rv, col * 2 + (SHARED ? 0 : at), SHARED ? at : 0, 0);
+    }
+#pragma unroll
+    for (int x = 0; x < W / 2; ++x) rows[i][x] = j < n ? rows[i][x] : 0;
+  }
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000);
+}
+
+// Four elements of a row and what their rotation takes. Loads come first and from clamped places, so that those of many calls are in
+// flight together; without a rotation (dims 0) cos_sin points at any sixteen bytes.
+struct Raw4 {
+  uint2 x, p;
+  float4 c, s;
+};
+__device__ __forceinline__ Raw4 load_raw(const bf16_t* row, int e, int dk, const float* cs, int half) {
+  const int ec = min(e, dk - 4), f = ec < half ? ec : ec < 2 * half ? ec - half : 0;
+  Raw4 r;
+  r.x = *reinterpret_cast<const uint2*>(row + ec);
+  r.p = *reinterpret_cast<const uint2*>(row + (ec < half ? ec + half : ec < 2 * half ? ec - half : ec));
+  r.c = *reinterpret_cast<const float4*>(cs + f);
+  r.s = *reinterpret_cast<const float4*>(cs + half + f);
+  return r;
+}
+__device__ __forceinline__ void rotate(const Raw4& r, int e, int dk, int half, float (&v)[4]) {
+  const float x[4] = {__uint_as_float(r.x.x << 16), __uint_as_float(r.x.x & 0xffff0000u), __uint_as_float(r.x.y << 16), __uint_as_float(r.x.y & 0xffff0000u)};
+  const float p[4] = {__uint_as_float(r.p.x << 16), __uint_as_float(r.p.x & 0xffff0000u), __uint_as_float(r.p.y << 16), __uint_as_float(r.p.y & 0xffff0000u)};
+  const float c[4] = {r.c.x, r.c.y, r.c.z, r.c.w}, s[4] = {r.s.x, r.s.y, r.s.z, r.s.w};
+  const int ec = min(e, dk - 4);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float sn = ec < half ? -s[i] : s[i], y = x[i] * c[i] + p[i] * sn;
+    v[i] = ec < 2 * half ? y : x[i];
+    v[i] = e < dk ? v[i] : 0.f;
+  }
+}
+
+// retention_chunk for blockIdx.z: 128 key rows x 128 of the dv columns. A thread rotates four dimensions of eight tokens.
+constexpr int PD = 128, PC = 128;
+__global__ __launch_bounds__(NT, 2) void retention_chunk_parts_kernel(const bf16_t* __restrict__ p, int64_t stride, int H, int dk, int dv,
+                                                                      Rot rot, const float* __restrict__ powers, int pw_stride,
+                                                                      const int* __restrict__ c_start, int c0, float* __restrict__ c_state) {
+  __shared__ __attribute__((aligned(16))) u32x4_t sK[3][8][PD], sV[8][PC];  // a piece: eight tokens of a dimension, of a column
+  const int c = blockIdx.x, h = blockIdx.y, ncb = dv / PC;
+  const int d0 = (int)(blockIdx.z / ncb) * PD, col0 = (int)(blockIdx.z % ncb) * PC;
+  const int64_t t0 = c_start[c0 + c];
+  const int n = c_start[c0 + c + 1] - (int)t0, half = rot.dims >> 1;
+  const float kscale = 1.f / sqrtf((float)dk);
+  const float* pw = powers + (int64_t)h * pw_stride;
+  const bf16_t* keys = p + t0 * stride + (H + h) * dk;
+  const bf16_t* vals = p + t0 * stride + 2 * H * dk + h * dv + col0;
+  int64_t pos0;
+  {
+    const int g = threadIdx.x & 31, jg = threadIdx.x >> 5;
+    uint32_t rows[8][2];
+    load_v<4, false>(buffer(vals), stride, 4 * g, n, [&](int i) { return 8 * jg + i; }, rows);
+    float w[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] = pw[max(n - 1 - (8 * jg + i), 0)];
+    pos0 = rot.positions[t0];
+    Raw4 raw[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int jc = min(8 * jg + i, n - 1);
+      raw[i] = load_raw(keys + jc * stride, d0 + 4 * g, dk, rot.cos_sin + (pos0 + jc) * rot.dims, half);
+    }
+    float k[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      rotate(raw[i], d0 + 4 * g, dk, half, k[i]);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) k[i][x] = 8 * jg + i < n ? k[i][x] * (kscale * w[i]) : 0.f;
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int at = place<4>(4 * g + x);
+      sV[jg][at] = column<4>(rows, x);
+      const float a[4] = {k[0][x], k[1][x], k[2][x], k[3][x]}, b[4] = {k[4][x], k[5][x], k[6][x], k[7][x]};
+      const Parts s = split_vals(a, b);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) sK[i][jg][at] = s.p[i];
+    }
+  }
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
+  f32x4_t acc[2][8] = {};  // columns 32 wave + 16 m + 4 kq .., dimension 16 b + r16
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (32 * t >= n) break;
+    u32x4_t a[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) a[m] = sV[4 * t + kq][place<4>(32 * wave + 16 * m + r16)];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      if (d0 + 16 * b >= dk) break;
+#pragma unroll
+      for (int i = 2; i >= 0; --i) {
+        const u32x4_t k = sK[i][4 * t + kq][place<4>(16 * b + r16)];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) acc[m][b] = mfma_bf(a[m], k, acc[m][b]);
+      }
+    }
+  }
+  float* dst = c_state + ((int64_t)c * H + h) * dk * dv + col0;
+  bool bad = false;
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const int d = d0 + 16 * b + r16;
+    if (d >= dk) break;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      const f32x4_t v = acc[m][b] * UP1;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bad |= !(fabsf(v[e]) <= 3.4028235e38f);
+      *reinterpret_cast<f32x4_t*>(dst + (int64_t)d * dv + 32 * wave + 16 * m + 4 * kq) = v;
+    }
+  }
+  if (!__syncthreads_or(bad)) return;
+  for (int e = threadIdx.x; e < PD * PC; e += NT) {
+    const int d = d0 + e / PC, col = e % PC;
+    if (d >= dk) break;
+    float s = 0.f;
+    for (int j = 0; j < n; ++j)
+      s += rot1(keys + j * stride, d, rot.cos_sin + (pos0 + j) * rot.dims, half) * (kscale * pw[n - 1 - j]) * ld(vals + j * stride + col);
+    dst[(int64_t)d * dv + col] = s;
+  }
+}
+
+// retention_out for heads of 32 NKD dimensions and 16 NCB columns: all keys are rotated and split at once (their loads fly together), then
+// the weights' product with the values, then the state's, 32 dimensions x 128 columns at a time in two buffers, two pieces ahead in registers.
+template <int NKD, int NCB>
+__global__ __launch_bounds__(NT, 3) void retention_out_parts_kernel(const bf16_t* __restrict__ p, int64_t stride, int H, int gate, Rot rot,
+                                                                    const float* __restrict__ powers, int pw_stride, float eps,
+                                                                    const int* __restrict__ c_start, int c0,
+                                                                    const float* __restrict__ c_state, bf16_t* __restrict__ out) {
+  constexpr int dk = 32 * NKD, dv = 16 * NCB, NH = dv / 128, W = NCB / 4;  // W: columns of a thread where values are staged
+  constexpr int KS = C + 2;                                                // pieces of a lane group's keys, and two: banks of their own
+  constexpr int PIECE = 3 * 4 * 128, PIECES = NKD * NH;
+  constexpr int LDS = std::max(3 * NKD * 4 * KS, std::max(2 * 4 * dv, 2 * PIECE));
+  __shared__ __attribute__((aligned(16))) u32x4_t sL[LDS];
+  __shared__ float sP[C + 1], red[NT / 64];
+  static_assert(C * C * 4 <= (int)sizeof(sL) && PIECES >= 2, "");
+  const int c = blockIdx.x, h = blockIdx.y;
+  const int64_t t0 = c_start[c0 + c];
+  const int n = c_start[c0 + c + 1] - (int)t0, half = rot.dims >> 1;
+  const float kscale = 1.f / sqrtf((float)dk);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
+  if (threadIdx.x <= C) sP[threadIdx.x] = powers[(int64_t)h * pw_stride + threadIdx.x];
+  const float* S0 = c_state + ((int64_t)c * H + h) * dk * dv;
+  const int64_t pos0 = rot.positions[t0];
+  const bf16_t* keys = p + t0 * stride + (H + h) * dk;
+  const bf16_t* vals = p + t0 * stride + 2 * H * dk + h * dv;
+  const int qi = wave * 16 + r16, qc = min(qi, n - 1), kj = threadIdx.x >> 2, kc = min(kj, n - 1), ks = threadIdx.x & 3;
+  float q[NKD][8];  // this lane's query, dimensions 32 pc + 8 kq ..
+  {
+    Raw4 raw[NKD][2];
+    const bf16_t* row = p + (t0 + qc) * stride + h * dk;
+    const float* cs = rot.cos_sin + (pos0 + qc) * rot.dims;
+#pragma unroll
+    for (int pc = 0; pc < NKD; ++pc)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) raw[pc][x] = load_raw(row, 32 * pc + 8 * kq + 4 * x, dk, cs, half);
+#pragma unroll
+    for (int pc = 0; pc < NKD; ++pc)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        float v[4];
+        rotate(raw[pc][x], 32 * pc + 8 * kq + 4 * x, dk, half, v);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[pc][4 * x + i] = v[i];
+      }
+  }
+  const auto query = [&](int pc) {
+    const float a[4] = {q[pc][0], q[pc][1], q[pc][2], q[pc][3]}, b[4] = {q[pc][4], q[pc][5], q[pc][6], q[pc][7]};
+    return split_vals(a, b);
+  };
+  {
+    Raw4 raw[NKD][2];
+    const float* cs = rot.cos_sin + (pos0 + kc) * rot.dims;
+#pragma unroll
+    for (int pc = 0; pc < NKD; ++pc)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) raw[pc][x] = load_raw(keys + kc * stride, 32 * pc + 8 * ks + 4 * x, dk, cs, half);
+#pragma unroll
+    for (int pc = 0; pc < NKD; ++pc) {
+      float a[4], b[4];
+      rotate(raw[pc][0], 32 * pc + 8 * ks, dk, half, a);
+      rotate(raw[pc][1], 32 * pc + 8 * ks + 4, dk, half, b);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] *= kscale, b[i] *= kscale;
+      const Parts kp = split_vals(a, b);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) sL[((i * NKD + pc) * 4 + ks) * KS + kj] = kp.p[i];
+    }
+  }
+  const __amdgpu_buffer_rsrc_t rs = buffer(S0), rv = buffer(vals);
+  uint32_t rows[2][8][W / 2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+    load_v<W, true>(rv, stride, W * lane, n, [&](int i) { return 32 * t + 16 * (i >> 2) + 4 * wave + (i & 3); }, rows[t]);
+  __syncthreads();
+  f32x4_t o[NCB], w[4];  // o[m][r]: column 16 m + 4 kq + r of query r16 of the wave; w[jb][r]: key 16 jb + 4 kq + r of that query
+#pragma unroll
+  for (int m = 0; m < NCB; ++m) o[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int jb = 0; jb < 4; ++jb) w[jb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int pc = 0; pc < NKD; ++pc) {
+    const Parts qp = query(pc);
+#pragma unroll
+    for (int jb = 0; jb < 4; ++jb) {
+      if (jb > wave) break;  // keys after every query of this wave
+      u32x4_t f[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) f[i] = sL[((i * NKD + pc) * 4 + kq) * KS + 16 * jb + r16];
+      w[jb] = mfma_six(f, qp.p, w[jb]);
+    }
+  }
+#pragma unroll
+  for (int jb = 0; jb < 4; ++jb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int dist = qi - (jb * 16 + kq * 4 + r);
+      w[jb][r] = dist >= 0 ? w[jb][r] * moe_tile::SPLIT_DOWN * sP[max(dist, 0)] : 0.f;
+    }
+  __syncthreads();  // the keys are read
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int x = 0; x < W; ++x) sL[(4 * t + wave) * dv + place<W>(W * lane + x)] = column<W>(rows[t], x);
+  float2 s[2][8];  // eight dimensions of two columns, of the next two pieces
+  const auto load_s = [&](int piece) {
+    const int src = ((piece / NH * 32 + 8 * wave) * dv + piece % NH * 128) * 4;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      s[piece & 1][i] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(rs, 8 * lane, src + i * dv * 4, 0));
+  };
+  load_s(0);
+  load_s(1);
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (2 * t > wave) break;
+    const float lo[4] = {w[2 * t][0], w[2 * t][1], w[2 * t][2], w[2 * t][3]}, hi[4] = {w[2 * t + 1][0], w[2 * t + 1][1], w[2 * t + 1][2], w[2 * t + 1][3]};
+    const Parts wp = split_vals(lo, hi);
+#pragma unroll
+    for (int m = 0; m < NCB; ++m) {
+      const u32x4_t f = sL[(4 * t + kq) * dv + place<W>(16 * m + r16)];
+#pragma unroll
+      for (int i = 2; i >= 0; --i) o[m] = mfma_bf(f, wp.p[i], o[m]);
+    }
+  }
+  // the state's part: the row's decay goes into its query; sums times 2^48 like the products that follow
+#pragma unroll
+  for (int m = 0; m < NCB; ++m) o[m] *= 1.f / UP1;
+  const float decay = sP[qi + 1];
+#pragma unroll
+  for (int pc = 0; pc < NKD; ++pc)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[pc][i] *= decay;
+  __syncthreads();  // the values are read
+  uint2 g[NCB] = {};
+  Parts qp;
+#pragma unroll
+  for (int piece = 0; piece < PIECES; ++piece) {
+    u32x4_t* buf = sL + (piece & 1) * PIECE;  // (read two pieces ago, with a barrier since)
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      float u[4], v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) u[i] = x ? s[piece & 1][i].y : s[piece & 1][i].x, v[i] = x ? s[piece & 1][4 + i].y : s[piece & 1][4 + i].x;
+      const Parts sp = split_vals(u, v);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) buf[(4 * i + wave) * 128 + place<2>(2 * lane + x)] = sp.p[i];
+    }
+    if (piece + 2 < PIECES) load_s(piece + 2);
+    if (piece + 1 == PIECES && gate) {
+      const bf16_t* grow = p + (t0 + qc) * stride + 2 * H * dk + H * dv + h * dv;
+#pragma unroll
+      for (int m = 0; m < NCB; ++m) g[m] = *reinterpret_cast<const uint2*>(grow + 16 * m + 4 * kq);
+    }
+    if (piece % NH == 0) qp = query(piece / NH);
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < 8; ++m) {
+      u32x4_t f[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) f[i] = buf[(4 * i + kq) * 128 + place<2>(16 * m + r16)];
+      o[piece % NH * 8 + m] = mfma_six(f, qp.p, o[piece % NH * 8 + m]);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int m = 0; m < NCB; ++m)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      o[m][r] *= moe_tile::SPLIT_DOWN;
+      ss += o[m][r] * o[m][r];
+    }
+  ss = row_sum(ss);
+  const float inv = 1.f / sqrtf(ss / (float)dv + eps);
+  if (qi < n) {
+    bf16_t* row = out + ((t0 + qi) * H + h) * dv;
+#pragma unroll
+    for (int m = 0; m < NCB; ++m) {
+      if (gate) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[m][r] *= Fn<bf16_t>::silu(__uint_as_float(r & 1 ? (r < 2 ? g[m].x : g[m].y) & 0xffff0000u : (r < 2 ? g[m].x : g[m].y) << 16));
+      }
+      bf16_t v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) st(&v[r], o[m][r] * inv);
+      *reinterpret_cast<uint2*>(row + 16 * m + 4 * kq) = make_uint2(v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16);
+    }
+  }
+  if (!__syncthreads_or(qi < n && !(ss <= 3.4028235e38f))) return;
+  float* sW = reinterpret_cast<float*>(sL);
+  for (int e = threadIdx.x; e < n * C; e += NT) {
+    const int i = e / C, j = e % C;
+    float a = 0.f;
+    if (j <= i)
+      for (int d = 0; d < dk; ++d)
+        a += rot1(p + (t0 + i) * stride + h * dk, d, rot.cos_sin + (pos0 + i) * rot.dims, half) *
+             (rot1(keys + j * stride, d, rot.cos_sin + (pos0 + j) * rot.dims, half) * kscale);
+    sW[e] = j <= i ? a * sP[i - j] : 0.f;
+  }
+  __syncthreads();
+  for (int i = 0; i < n; ++i) {
+    const int col = min((int)threadIdx.x, dv - 1);
+    const int64_t t = t0 + i;
+    float a = 0.f;
+    for (int d = 0; d < dk; ++d)
+      a += rot1(p + t * stride + h * dk, d, rot.cos_sin + (pos0 + i) * rot.dims, half) * S0[(int64_t)d * dv + col];
+    a *= sP[i + 1];
+    for (int j = 0; j <= i; ++j) a += sW[i * C + j] * ld(vals + j * stride + col);
+    const float norm = 1.f / sqrtf(block_sum<NT>((int)threadIdx.x < dv ? a * a : 0.f, red) / (float)dv + eps);
+    if (gate) a *= Fn<bf16_t>::silu(ld(p + t * stride + 2 * H * dk + H * dv + h * dv + col));
+    if ((int)threadIdx.x < dv) st(out + (t * H + h) * dv + col, a * norm);
+  }
+}
+
 template <typename T>
 int launch(const T* p, int64_t stride, int H, int dk, int dv, int gate, const Rot& rot, const float* powers, int pw_stride,
            float eps, float* state, const int* seq_start, const int* seq_slot, const int* seq_init, T* out, int T_rows,
            int nseq, int nd, int nc, const int* c_start, const int* s_chunk0, float* c_state, float* o_raw,
            hipStream_t stream) {
-  const size_t es = sizeof(T);
+  constexpr size_t es = sizeof(T);
   if (nd > 0) {
     const bool v4 = dv % 4 == 0 && ((uintptr_t)state & 15) == 0;
     const int cols = v4 ? dv / 4 : dv, ncg = std::min(cols, NT), RG = std::min(NT / ncg, dk);
@@ -522,7 +939,20 @@ int launch(const T* p, int64_t stride, int H, int dk, int dv, int gate, const Ro
     hipLaunchKernelGGL((retention_chunk_kernel<T, NCB, VEC>), grid, dim3(NT), lds, stream, p, stride, H, dk, dv, rot, \
                        powers, pw_stride, c_start, nd, c_state);                                                      \
   }
-  if (dv <= 64 && vec) SM_CHUNK(4, true)
+  // bf16 rows on the bf16 units. Heads of 64 or 128 x 128 or 256, whose keys fit three workgroups' LDS on a CU; rows whose 64 tokens lie within
+  // 31 bits
+  bool parts = false;
+  Rot any = rot;  // without a rotation the loads of its table go somewhere
+  if (rot.dims == 0) any.cos_sin = powers;
+  if constexpr (es == 2) {
+    parts = vec && stride <= 1 << 23 && (dk == 64 || dk == 128) && (dv == 128 || dv == 256) && ((uintptr_t)c_state & 15) == 0 &&
+            ((uintptr_t)out & 7) == 0 && H * pw_stride >= 4;
+    if (parts)
+      hipLaunchKernelGGL(retention_chunk_parts_kernel, dim3(n, H, (dk + PD - 1) / PD * (dv / PC)), dim3(NT), 0, stream, p, stride, H, dk, dv, any,
+                         powers, pw_stride, c_start, nd, c_state);
+  }
+  if (parts) {
+  } else if (dv <= 64 && vec) SM_CHUNK(4, true)
   else if (dv <= 64) SM_CHUNK(4, false)
   else if (vec) SM_CHUNK(8, true)
   else SM_CHUNK(8, false)
@@ -538,6 +968,18 @@ int launch(const T* p, int64_t stride, int H, int dk, int dv, int gate, const Ro
     hipLaunchKernelGGL((retention_link_kernel<1>), dim3((unsigned)((per_head * H + NT - 1) / NT), nseq - nd), dim3(NT), 0,
                        stream, c_state, c_start, s_chunk0, nd, nd, H, per_head, powers, pw_stride, state, seq_slot,
                        seq_init);
+  if constexpr (es == 2) {
+    if (parts) {
+      const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(n, H), dim3(NT), 0, stream, p, stride, H, gate, any, powers, pw_stride, eps, c_start, nd, c_state, out);
+      };
+      if (dk == 64 && dv == 128) go(retention_out_parts_kernel<2, 8>);
+      else if (dk == 64) go(retention_out_parts_kernel<2, 16>);
+      else if (dv == 128) go(retention_out_parts_kernel<4, 8>);
+      else go(retention_out_parts_kernel<4, 16>);
+      return 0;
+    }
+  }
 #define SM_OUT(NCB, VEC)                                                                                              \
   {                                                                                                                   \
     const size_t lds = (size_t)(C * OS + OB * (16 * NCB + 4)) * sizeof(float);                                        \
