@@ -432,11 +432,13 @@ struct Parts {
   u32x4_t p[3];  // 8 elements: largest part first
 };
 constexpr float SPLIT_UP = 0x1p24f, SPLIT_DOWN = 0x1p-48f;
-// part i of four elements to (lo, hi); x: what is left of them
+// part i of four elements to (lo, hi); x: what is left of them. (As vectors of two: hipcc rounds scalar casts twice, and does not keep
+// the distance that the matrix units need from what asm writes.)
 __device__ __forceinline__ void take_part(f32x4_t& x, uint32_t& lo, uint32_t& hi) {
-  // (as casts, hipcc rounds every element twice: once for its pair, once to subtract it)
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(lo) : "v"(x[0]), "v"(x[1]));
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(hi) : "v"(x[2]), "v"(x[3]));
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{x[0], x[1]}, bf16x2_t));
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{x[2], x[3]}, bf16x2_t));
   x[0] -= __uint_as_float(lo << 16), x[1] -= __uint_as_float(lo & 0xffff0000u);
   x[2] -= __uint_as_float(hi << 16), x[3] -= __uint_as_float(hi & 0xffff0000u);
 }
