@@ -181,6 +181,90 @@ __global__ __launch_bounds__(NT) void input_conv_vec_kernel(const bf16_t* __rest
   }
 }
 
+// The same for steps with longer runs: a workgroup takes ICR tokens of one run, from a place that ICR divides (the other tokens'
+// workgroups leave), so that weights and earlier inputs are loaded once for all of them. The one at the run's start, the only
+// reader of the run's old state (TAPS - 1 <= ICR), also rolls it: no second launch. Sums in the order of the form above.
+// Bound by loads per CU: a token took TAPS rows and as many pieces of weights, now (ICR + 2 TAPS - 1) / ICR. us, 2048 tokens x 2048 channels,
+// 4 taps: 8.4 and 3.9 for the states -> 6.6.
+constexpr int ICR = 4;
+template <int TAPS, bool PAIR>
+__global__ __launch_bounds__(NT) void input_conv_run_kernel(const bf16_t* __restrict__ h, int C, const bf16_t* __restrict__ w,
+                                                           const bf16_t* __restrict__ w2, bf16_t* state,
+                                                           const int* __restrict__ row_seq, const int* __restrict__ seq_start,
+                                                           const int* __restrict__ seq_slot, const int* __restrict__ seq_init,
+                                                           bf16_t* __restrict__ out, bf16_t* __restrict__ out2, int T) {
+  static_assert(TAPS > 1 && TAPS - 1 <= ICR, "");
+  const int c = (blockIdx.y * NT + threadIdx.x) * 8;
+  // neighbouring workgroups are ICR tokens apart: those that stay are on all XCDs
+  const int groups = gridDim.x / ICR, t = blockIdx.x % groups * ICR + blockIdx.x / groups;
+  if (t >= T || c >= C) return;
+  const int s = row_seq[t], lo = seq_start[s], p = t - lo;
+  if (p % ICR != 0) return;
+  const int hi = seq_start[s + 1];
+  const bool init = seq_init[s] != 0;
+  bf16_t* st_ = state + (int64_t)seq_slot[s] * (TAPS - 1) * C + c;
+  // inputs of the tokens p - (TAPS - 1) ..: one load each from wherever it lies, all in flight together
+  auto input = [&](int pp) {
+    const bf16_t* from = pp < 0 && init ? st_ + (TAPS - 1 + pp) * C : h + (int64_t)(lo + min(max(pp, 0), hi - lo - 1)) * C + c;
+    return *reinterpret_cast<const uint4*>(from);
+  };
+  auto known = [&](int pp, const uint4& v) {
+    const bool yes = pp >= 0 || init;
+    return make_uint4(yes ? v.x : 0, yes ? v.y : 0, yes ? v.z : 0, yes ? v.w : 0);
+  };
+  uint4 x[TAPS - 1 + ICR];
+#pragma unroll
+  for (int i = 0; i < TAPS - 1 + ICR; ++i) x[i] = input(p - (TAPS - 1) + i);
+#pragma unroll
+  for (int i = 0; i < TAPS - 1; ++i) x[i] = known(p - (TAPS - 1) + i, x[i]);
+  auto wide = [](const uint4& q, float (&v)[8]) {
+    v[0] = __uint_as_float(q.x << 16); v[1] = __uint_as_float(q.x & 0xffff0000u);
+    v[2] = __uint_as_float(q.y << 16); v[3] = __uint_as_float(q.y & 0xffff0000u);
+    v[4] = __uint_as_float(q.z << 16); v[5] = __uint_as_float(q.z & 0xffff0000u);
+    v[6] = __uint_as_float(q.w << 16); v[7] = __uint_as_float(q.w & 0xffff0000u);
+  };
+  auto pack = [](float lo_, float hi_) {
+    const __bf16 l16 = (__bf16)lo_, h16 = (__bf16)hi_;
+    return (uint32_t)__builtin_bit_cast(uint16_t, l16) | ((uint32_t)__builtin_bit_cast(uint16_t, h16) << 16);
+  };
+  auto filter = [&](const bf16_t* wp, bf16_t* to) {
+    float wr[8 * TAPS];  // channel i, tap j at i * TAPS + j
+#pragma unroll
+    for (int i = 0; i < TAPS; ++i) {
+      float v[8];
+      wide(*reinterpret_cast<const uint4*>(wp + (int64_t)c * TAPS + 8 * i), v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) wr[8 * i + e] = v[e];
+    }
+#pragma unroll
+    for (int k = 0; k < ICR; ++k) {
+      float a[8], v[8];
+      wide(x[TAPS - 1 + k], v);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) a[i] = v[i] + wr[i * TAPS + TAPS - 1] * v[i];
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j) {
+        wide(x[k + j], v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a[i] += wr[i * TAPS + j] * v[i];
+      }
+      if (t + k < hi)
+        *reinterpret_cast<uint4*>(to + (int64_t)(t + k) * C + c) =
+            make_uint4(pack(a[0], a[1]), pack(a[2], a[3]), pack(a[4], a[5]), pack(a[6], a[7]));
+    }
+  };
+  filter(w, out);
+  if constexpr (PAIR) filter(w2, out2);
+  if (p == 0) {
+    // entry j's input; before the run that is entry hi - lo + j of the old state
+    uint4 v[TAPS - 1];
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) v[j] = input(hi - lo - (TAPS - 1) + j);
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) *reinterpret_cast<uint4*>(st_ + j * C) = known(hi - lo - (TAPS - 1) + j, v[j]);
+  }
+}
+
 // NL lanes per channel (power of two <= 64), SPL states per lane.
 template <typename T, int SPL>
 __global__ __launch_bounds__(NT) void selective_scan_kernel(
@@ -435,7 +519,7 @@ void sm_conv_state(const void* x, int64_t x_stride, int C, int taps, void* state
                        (bf16_t*)state, seq_start, seq_slot, seq_init, skip_single);
 }
 
-// max_q: the longest run of the step; runs of one token roll their state in the first kernel, so a
+// max_q: the longest run of the step; runs of one token, and with up to ICR + 1 taps all of them, roll their state in the first kernel, so a
 // decode-only step needs no second launch. w2 / out2: a second filter over the same inputs, or null.
 void sm_input_conv(const void* h, int C, const void* w, const void* w2, int taps, void* state, const int* row_seq,
                    const int* seq_start, const int* seq_slot, const int* seq_init, void* out, void* out2, int T,
@@ -444,11 +528,22 @@ void sm_input_conv(const void* h, int C, const void* w, const void* w2, int taps
   const dim3 g1(T, (C + NT - 1) / NT);
   if (!f32 && C % 8 == 0 && taps <= ICV_MAX_TAPS &&
       (((uintptr_t)h | (uintptr_t)out | (uintptr_t)out2 | (uintptr_t)state | (uintptr_t)w | (uintptr_t)w2) & 15) == 0) {
-    const dim3 gv(T, (C / 8 + NT - 1) / NT);
+    const dim3 gv(T, (C / 8 + NT - 1) / NT), gr((T + ICR - 1) / ICR * ICR, gv.y);
 #define SM_ICV2(N, P)                                                                                                 \
   hipLaunchKernelGGL((input_conv_vec_kernel<N, P>), gv, dim3(NT), 0, stream, (const bf16_t*)h, C, (const bf16_t*)w,   \
                      (const bf16_t*)w2, (bf16_t*)state, row_seq, seq_start, seq_slot, seq_init, (bf16_t*)out,        \
                      (bf16_t*)out2)
+#define SM_ICR(N)                                                                                                      \
+  case N:                                                                                                             \
+    if (w2)                                                                                                           \
+      hipLaunchKernelGGL((input_conv_run_kernel<N, true>), gr, dim3(NT), 0, stream, (const bf16_t*)h, C, (const bf16_t*)w, (const bf16_t*)w2, \
+                         (bf16_t*)state, row_seq, seq_start, seq_slot, seq_init, (bf16_t*)out, (bf16_t*)out2, T);     \
+    else                                                                                                              \
+      hipLaunchKernelGGL((input_conv_run_kernel<N, false>), gr, dim3(NT), 0, stream, (const bf16_t*)h, C, (const bf16_t*)w, (const bf16_t*)w2, \
+                         (bf16_t*)state, row_seq, seq_start, seq_slot, seq_init, (bf16_t*)out, (bf16_t*)out2, T);     \
+    return
+    if (max_q > 1) switch (taps) { SM_ICR(2); SM_ICR(3); SM_ICR(4); SM_ICR(5); }
+#undef SM_ICR
 #define SM_ICV(N)                 \
   case N:                         \
     if (w2) SM_ICV2(N, true);     \
