@@ -42,6 +42,7 @@ from llmd_amd.utils import markers
 from .attn_meta import AttnMeta, SeqMeta
 from .config import EngineConfig
 from .scheduler import ScheduledReq, SchedulerOutput
+from .step_graph import StepGraph
 
 log = logging.getLogger("llmd.runner")
 
@@ -1050,8 +1051,8 @@ class ModelRunner:
                     h = self.model(self.g_ids[:B], meta)
                     lg = self.model.compute_logits(h)
             torch.cuda.current_stream().wait_stream(s)
-            g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g, pool=pool):
+            g = StepGraph()
+            with g.capture(pool):
                 h = self.model(self.g_ids[:B], meta)
                 lg = self.model.compute_logits(h)
             self.graphs[B] = (g, lg)
@@ -1063,8 +1064,8 @@ class ModelRunner:
                 with torch.cuda.stream(s):
                     self.model(self.g_ids[:B], meta)
                 torch.cuda.current_stream().wait_stream(s)
-                g = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(g, pool=pool):
+                g = StepGraph()
+                with g.capture(pool):
                     h = self.model(self.g_ids[:B], meta)
                     lg = self.model.compute_logits(h)
                 self.cgraphs[B] = (g, lg)
@@ -1104,8 +1105,8 @@ class ModelRunner:
                 for _ in range(2):  # builds the attention layers' work items, which the capture then finds in ``seq``
                     self.model(buf[:B], meta)
             torch.cuda.current_stream().wait_stream(s)
-            g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g, pool=pool):
+            g = StepGraph()
+            with g.capture(pool):
                 h = self.model(buf[:B], meta)
             self.graphs[B] = (g, h, buf, meta)
         self._graph_constants = self._graph_warned = self._seq_constants
@@ -1213,8 +1214,8 @@ class ModelRunner:
                 for _ in range(2):
                     self._dbo_forward(B, metas, streams)
             torch.cuda.current_stream().wait_stream(s)
-            g = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(g, pool=pool):
+            g = StepGraph()
+            with g.capture(pool):
                 lg = self._dbo_forward(B, metas, streams)
             self.dbo_graphs[B] = (g, lg)
 
