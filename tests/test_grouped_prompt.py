@@ -119,3 +119,30 @@ def test_scores_that_climb(bs, opts):
     got = sm.grouped_attention(q.cuda(), cache.cuda(), dim, dim, dim ** -0.5, md, **{k: v.cuda() for k, v in kw.items()})
     # scores of up to about 1000 in fp32 (their products' sums are 2^-24 of that off, a few times): weights off by 2^-11; values up to about 5
     assert ((got.double().cpu() - want).abs() <= 2 ** -8 * want.abs() + 5e-3).all()
+
+
+# portions in whole sizes and in the general form, one and two blocks of rows per wave, key ranges apart (single tokens, pages of 16), and
+# the kernel of single tokens
+@pytest.mark.parametrize("runs,bs,dim", [([(0, 230)], 64, 128), ([(0, 230)], 16, 128), ([(50, 90), (700, 1)], 16, 40), ([(900, 1), (40, 1)], 16, 128),
+                                         ([(900, 1), (40, 1)], 64, 128)])
+def test_sinks_far_below_all_scores(runs, bs, dim):
+    """A sink of minus infinity, or so low that its multiple by log2(e) is, counts nothing, and no sink spoils the scores above it,
+    however far above they are."""
+    from llmd_amd.ops import seqmix as sm
+
+    Hq, Hkv = 8, 2
+    g = torch.Generator().manual_seed(dim)
+    m, pages = _meta(runs, bs, "cpu")
+    T = sum(n for _, n in runs)
+    q, cache = torch.randn(T, Hq, dim, generator=g).bfloat16(), torch.randn(pages, Hkv, bs, 2 * dim, generator=g).bfloat16()
+    # scores of about +-150 in odd heads: in base 2 beyond what an fp32 weight relative to zero can be
+    q[:, 1::2] *= 40
+    low, inf = torch.finfo, float("inf")
+    sinks = torch.tensor([-inf, -inf, low(torch.bfloat16).min, low(torch.float32).min, -1e30, -1e30, -1e10, -1e10])
+    args = (dim, dim, dim ** -0.5)
+    md, _ = _meta(runs, bs, "cuda")
+    for sk in (sinks, sinks.flip(0), torch.tensor([-1e4, 0.0, -inf, 1e10, 300.0, -1e6, 1e4, -3e7])):
+        want = sm.grouped_attention(q.double(), cache.double(), *args, m, sinks=sk)
+        got = sm.grouped_attention(q.cuda(), cache.cuda(), *args, md, sinks=sk.cuda()).double().cpu()
+        # as in test_scores_that_climb: scores of up to about 1000 in fp32
+        assert ((got - want).abs() <= 2 ** -8 * want.abs() + 5e-3).all()
