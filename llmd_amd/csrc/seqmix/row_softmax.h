@@ -15,7 +15,8 @@ constexpr int MKT = 32;  // keys per tile
 // The weights are exp2(score - ref), and a row's ref moves only when one of its own scores passes it by 2^RISE: after a row's
 // first tiles a step has neither a maximum across lanes nor products with the accumulators. Every row decides for itself (one that
 // stays is multiplied by 1), so its bits do not depend on the rows beside it. The sums stay with the lanes until the end.
-constexpr float RISE = 8.f, FAR = 512.f;  // (2^-512: no fp32 sum holds it)
+constexpr float RISE = 8.f;
+constexpr float LOW_SINK = -0x1p20f;  // (base 2; above it a reference is off by a sixteenth at most)
 
 // (fmaxf takes an instruction more for each operand)
 __device__ __forceinline__ float max3(float a, float b, float c) {
@@ -28,13 +29,26 @@ struct RowSoftmax {
   float ref;   // what the weights are relative to; 0 before the first key
   float rise;  // ref moves when a score passes it by more: -infinity before the first key
   float l;     // this lane's part of the sum of weights
-  // a sink is a score that is already counted; one of -infinity, or whose product with log2(e) is, counts nothing
+  // a sink is a score that is already counted, or one that is counted behind all keys: far below them it would take the digits of the
+  // reference that follows it (ref + mx is -1e10 + 1e10), and -infinity has no difference from itself
   __device__ __forceinline__ void start(const float* sinks, int head, int kq) {
     const float sink = sinks ? sinks[head] * 1.44269504088896341f : -INFINITY;
-    const bool none = sink == -INFINITY;
-    ref = none ? 0.f : sink;
-    rise = none ? -INFINITY : RISE;
-    l = !none && kq == 0 ? 1.f : 0.f;
+    const bool later = sink <= LOW_SINK;
+    ref = later ? 0.f : sink;
+    rise = later ? -INFINITY : RISE;
+    l = !later && kq == 0 ? 1.f : 0.f;
+  }
+  template <int NCB>
+  __device__ __forceinline__ void finish(const float* sinks, int head, int kq, f32x4_t (&o)[NCB]) {
+    asm volatile("" : "+v"(head));  // loaded again: no register is kept for it
+    const float sink = sinks ? sinks[head] * 1.44269504088896341f : -INFINITY;
+    if (!(sink <= LOW_SINK) || sink == -INFINITY) return;
+    const bool above = rise < 0.f || sink > ref;
+    const float corr = rise < 0.f || !above ? 1.f : __builtin_amdgcn_exp2f(ref - sink);
+#pragma unroll
+    for (int n = 0; n < NCB; ++n) o[n] *= corr;
+    l = l * corr + (kq > 0 ? 0.f : above ? 1.f : __builtin_amdgcn_exp2f(sink - ref));
+    if (above) ref = sink, rise = RISE;
   }
   __device__ __forceinline__ float top() const { return rise < 0.f ? -INFINITY : ref; }
 };
@@ -87,11 +101,9 @@ __device__ __forceinline__ void weigh(const f32x4_t (&a)[2], float scale2, float
   auto scores = [&](float ref) {
     row_scores(a, scale2, slope, sloped, mylen - 1 - key0, ref, x);
     if (!plain) {
-      int first = key0;
-      asm volatile("" : "+v"(first));  // the masks are made again in each pass: there are no registers to keep them
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int key = first + i;
+        const int key = key0 + i;
         const bool in = (key < mylen) & (key >= mylo) & ((key >= mywlo) | (key < keep));
         x[i] = in ? x[i] : -INFINITY;
       }
@@ -99,23 +111,19 @@ __device__ __forceinline__ void weigh(const f32x4_t (&a)[2], float scale2, float
   };
   scores(s.ref);
   float mx = top8(x);
-  // Twice where a maximum lies far above ref (a sink far below all scores): ref + mx keeps nothing of it then, -1e10 + 1e10. What is
-  // summed is 0 beside it, so the row begins again.
-#pragma unroll 1
-  for (int pass = 0; pass < 2 && __any(mx > s.rise); ++pass) {
+  if (__any(mx > s.rise)) {
     mx = row_max(mx);
-    const bool up = mx > s.rise, far = up && s.rise > 0.f && mx > FAR;
-    const float ref = far ? 0.f : up ? s.ref + mx : s.ref;
-    const float corr = far ? 0.f : s.rise < 0.f ? 1.f : __builtin_amdgcn_exp2f(s.ref - ref);  // (nothing summed yet: nothing to correct)
+    const bool up = mx > s.rise;
+    const float ref = up ? s.ref + mx : s.ref;
+    const float corr = s.rise < 0.f ? 1.f : __builtin_amdgcn_exp2f(s.ref - ref);  // (nothing summed yet: nothing to correct)
 #pragma unroll
     for (int n = 0; n < NCB; ++n)
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[n][r] *= corr;
     s.l *= corr;
     s.ref = ref;
-    if (up) s.rise = far ? -INFINITY : RISE;
+    if (up) s.rise = RISE;
     scores(ref);
-    mx = top8(x);
   }
   row_weights(x, s, pah, pal);
 }

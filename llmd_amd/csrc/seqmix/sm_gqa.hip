@@ -943,6 +943,8 @@ __global__ __launch_bounds__(NT, NKS <= 4 && RB == 1 ? 3 : 1) void grouped_atten
       __syncthreads();
     }
   }
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) sm[rb].finish(blockIdx.z == 0 ? sinks : nullptr, myhead[rb], kq, o[rb]);
   const bool fours = (vdim & 3) == 0;
   if (nsplit > 1) {  // RB == 1 (the host splits decode-only steps, whose items have at most 64 rows)
     const int64_t prow = (((int64_t)item * Hkv + g) * nsplit + blockIdx.z) * 64 + wave * 16 + r16;
@@ -1148,10 +1150,13 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
+  sm.finish(sinks, myhead, kq, o);
   const float inv = 1.f / row_sum(sm.l);
   if (!ok) return;
-  bf16_t* dst = out + ((int64_t)mytok * Hq + myhead) * vdim;
-  const bf16_t* gt = gate ? gate + (int64_t)mytok * gate_stride + myhead * vdim : nullptr;
+  int tok = mytok;
+  asm volatile("" : "+v"(tok));  // the row's place is made again, not kept from the query's over the loop
+  bf16_t* dst = out + ((int64_t)tok * Hq + myhead) * vdim;
+  const bf16_t* gt = gate ? gate + (int64_t)tok * gate_stride + myhead * vdim : nullptr;
 #pragma unroll
   for (int n = 0; n < NCB; ++n) {
     const int col = n * 16 + kq * 4;

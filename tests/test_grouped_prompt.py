@@ -146,3 +146,27 @@ def test_sinks_far_below_all_scores(runs, bs, dim):
         got = sm.grouped_attention(q.cuda(), cache.cuda(), *args, md, sinks=sk.cuda()).double().cpu()
         # as in test_scores_that_climb: scores of up to about 1000 in fp32
         assert ((got - want).abs() <= 2 ** -8 * want.abs() + 5e-3).all()
+
+
+@pytest.mark.parametrize("runs,bs", [([(0, 100)], 64), ([(0, 100)], 16), ([(900, 1), (40, 1)], 16)])
+def test_low_sinks_among_low_scores(runs, bs):
+    """Sinks that are counted behind the keys, below, among and above scores of about -2^20."""
+    from llmd_amd.ops import seqmix as sm
+
+    Hq, Hkv, dim, base = 8, 2, 64, -2.0 ** 20
+    g = torch.Generator().manual_seed(bs)
+    m, pages = _meta(runs, bs, "cpu")
+    T = sum(n for _, n in runs)
+    # sums of whole numbers, exact in fp32, times 1/8
+    q = torch.randint(-1, 2, (T, Hq, dim), generator=g).bfloat16()
+    q[:, :, 0] = 1024
+    cache = torch.randn(pages, Hkv, bs, 2 * dim, generator=g).bfloat16()
+    k = cache.view(pages, Hkv, -1)[:, :, :bs * dim].view(pages, Hkv, bs, dim)
+    k.copy_(torch.randint(-1, 2, k.shape, generator=g))
+    k[..., 0] = -8192
+    sinks = torch.tensor([base + d for d in (-300.0, -30.0, -2.0, 0.0, 3.0, 6.0, 30.0, 300.0)])
+    md, _ = _meta(runs, bs, "cuda")
+    want = sm.grouped_attention(q.double(), cache.double(), dim, dim, dim ** -0.5, m, sinks=sinks)
+    got = sm.grouped_attention(q.cuda(), cache.cuda(), dim, dim, dim ** -0.5, md, sinks=sinks.cuda()).double().cpu()
+    # log2(e) and the sink's multiple by it, 1.5e6, rounded to fp32: the sink's weight is 2^0.15 off
+    assert ((got - want).abs() <= 0.12 * want.abs() + 2e-3).all()
