@@ -232,8 +232,9 @@ __device__ __forceinline__ void value_part(int unit, const T* __restrict__ qkv, 
                                            const int64_t* __restrict__ slots, T* __restrict__ cache, int bs,
                                            int v_from_k, const ConvArgs<T>& cv, int tg, int ntok) {
   const int nv = Hkv * vdim, vcol0 = v_from_k ? Hq * dim : (Hq + Hkv) * dim, nvb = (nv + NT - 1) / NT;
-  const int e = (unit % nvb) * NT + threadIdx.x, t0 = unit / nvb * tg;
-  if (t0 >= ntok) return;
+  // lanes behind the last column take it too (the same numbers, stored by one instruction): a wave has all its lanes, which hold places
+  const int e = min((unit % nvb) * NT + (int)threadIdx.x, nv - 1), t0 = unit / nvb * tg;
+  if (t0 >= ntok || (unit % nvb) * NT + (int)(threadIdx.x & ~63u) >= nv) return;
   // lane l: the place of token t0 - 7 + l; bit l of ``next``: the token behind it has the next place
   int64_t place = -1;
   uint64_t next = 0;
@@ -243,7 +244,7 @@ __device__ __forceinline__ void value_part(int unit, const T* __restrict__ qkv, 
     const int64_t behind = __shfl_down(place, 1, 64);
     next = __ballot(place >= 0 && behind == place + 1);
   }
-  const int col = vcol0 + min(e, nv - 1), ec = min(e, nv - 1), g = ec / vdim, c = ec - g * vdim;
+  const int col = vcol0 + e, g = e / vdim, c = e - g * vdim;
   const float vb = bias ? bias[col] : 0.f;
   const int64_t vbase = (int64_t)g * bs * (dim + vdim) + (int64_t)bs * dim + (int64_t)c * bs;  // within a page
   const int64_t page = (int64_t)Hkv * bs * (dim + vdim);
@@ -306,12 +307,10 @@ __device__ __forceinline__ void value_part(int unit, const T* __restrict__ qkv, 
     const int64_t slot = slots[t];
     if (slot >= 0) st(cache + slot / bs * page + vbase + slot % bs, v);
   };
-  if (e >= nv) return;
   for (int i = 0; i < min(tg, ntok - t0); ++i) {
     bool whole = false;
     int64_t s0 = -1;
     if (next != 0) {
-      // (readlane: a wave's last lanes may have no column)
       s0 = (int64_t)__builtin_amdgcn_readlane((int)(place >> 32), 7 + i) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)place, 7 + i);
       whole = s0 >= 0 && (next >> (7 + i - (int)(s0 & 7)) & 0x7f) == 0x7f;
     }
