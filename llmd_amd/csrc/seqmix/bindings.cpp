@@ -29,7 +29,7 @@ int sm_latent_f32(const void*, const void*, const int*, int, int, const int*, in
                   int, int, float*, float*, hipStream_t);
 void sm_latent_gather(const void*, const int*, int, int, const int*, int, int, int, int, int, void*, void*, hipStream_t);
 void sm_latent_own(const void*, int64_t, const void*, int64_t, int64_t, const void*, const void*, const int*, const int*, int, const int*,
-                   float, int, void*, const void*, int64_t, hipStream_t);
+                   float, int, void*, int64_t, const void*, int64_t, hipStream_t);
 void sm_embed_norm(const int64_t*, const void*, int64_t, const void*, float, float*, void*, int, int, int, hipStream_t);
 void sm_rms_norm_rows(const void*, int64_t, const void*, float, void*, int, int, int, hipStream_t);
 void sm_relu2(const void*, void*, int64_t, int, hipStream_t);
@@ -352,9 +352,9 @@ void latent_gather(Tensor cache, Tensor tables, Tensor base, int64_t first, int6
                    R, dr, lat.data_ptr(), rot.data_ptr(), cur());
 }
 
-// the step's rows that ``items`` (up to 64 tokens each) name, over keys and values of their own
+// the step's rows that ``items`` (up to 64 tokens each) name, over keys and values of their own: those of heads h0 .. that kv holds
 void latent_own(Tensor q, Tensor q_abs, int64_t R, Tensor kv, Tensor rot, Tensor base, Tensor items, Tensor row_len, double scale, Tensor out,
-                std::optional<Tensor> gate) {
+                std::optional<Tensor> gate, int64_t h0) {
   const c10::hip::OptionalHIPGuard g(dev_of(q));
   TORCH_CHECK(q.is_cuda() && q.scalar_type() == torch::kBFloat16 && q_abs.dim() == 3 && q_abs.is_contiguous(), "q bf16, q_abs [T, H, Dk]");
   CHECK_ACT(q_abs, q);
@@ -364,18 +364,20 @@ void latent_own(Tensor q, Tensor q_abs, int64_t R, Tensor kv, Tensor rot, Tensor
   CHECK_I32(base);
   CHECK_I32(items);
   CHECK_I32(row_len);
-  const int64_t T = q_abs.size(0), H = q_abs.size(1), Dk = q_abs.size(2);
+  const int64_t T = q_abs.size(0), H = q_abs.size(1), Dk = q_abs.size(2), n = kv.dim() == 2 ? kv.size(1) / 256 : 0;
   TORCH_CHECK(q.dim() == 2 && q.size(0) == T && q.size(1) == H * 192 && q.stride(1) == 1 && q.stride(0) % 8 == 0 &&
               ((uintptr_t)q.data_ptr() & 15) == 0, "q [T, H (128 + 64)]");
   TORCH_CHECK(R % 8 == 0 && Dk == R + 64 && rot.dim() == 2 && rot.size(1) == 64 && rot.is_contiguous() && kv.dim() == 2 && kv.is_contiguous() &&
-              kv.size(0) == rot.size(0) && kv.size(1) == H * 256 && H * 512 * 32 < (1ll << 31), "keys and values [n, H (128 + 128)], [n, 64]");
+              kv.size(0) == rot.size(0) && kv.size(1) == n * 256 && n * 512 * 32 < (1ll << 31), "keys and values [k, n (128 + 128)], [k, 64]");
+  TORCH_CHECK(n >= 1 && h0 >= 0 && h0 + n <= H, "heads");
   TORCH_CHECK(((((uintptr_t)q_abs.data_ptr()) | (uintptr_t)kv.data_ptr() | (uintptr_t)rot.data_ptr() | (uintptr_t)out.data_ptr()) & 15) == 0, "alignment");
   TORCH_CHECK(items.dim() == 2 && items.size(1) == 3 && items.size(0) <= 65535 && row_len.numel() == T, "items");
   TORCH_CHECK(out.is_contiguous() && out.numel() == T * H * 128, "out [T, H, 128]");
   check_head_gate(gate, q_abs);
-  sm_latent_own(q.data_ptr(), q.stride(0), (const char*)q_abs.data_ptr() + R * 2, H * Dk, Dk, kv.data_ptr(), rot.data_ptr(), base.data_ptr<int>(),
-                items.data_ptr<int>(), items.size(0), row_len.data_ptr<int>(), (float)scale, H, out.data_ptr(),
-                gate ? gate->data_ptr() : nullptr, gate ? gate->stride(0) : 0, cur());
+  const auto at = [](const void* p, int64_t elements) { return (const char*)p + elements * 2; };
+  sm_latent_own(at(q.data_ptr(), h0 * 192), q.stride(0), at(q_abs.data_ptr(), h0 * Dk + R), H * Dk, Dk, kv.data_ptr(), rot.data_ptr(),
+                base.data_ptr<int>(), items.data_ptr<int>(), items.size(0), row_len.data_ptr<int>(), (float)scale, n,
+                (void*)at(out.data_ptr(), h0 * 128), H * 128, gate ? at(gate->data_ptr(), h0) : nullptr, gate ? gate->stride(0) : 0, cur());
 }
 
 void causal_conv_silu(Tensor xz, int64_t C, Tensor w, Tensor b, Tensor state, Tensor seq_start, Tensor seq_slot,

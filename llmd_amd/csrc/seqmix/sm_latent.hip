@@ -446,7 +446,8 @@ constexpr int OWN_K = 128, OWN_ROT = 64, OWN_V = 128;
 __global__ __launch_bounds__(NT, 4) void latent_own_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ q_rot, int64_t rot_stride, int64_t rot_head,
     const bf16_t* __restrict__ kv, const bf16_t* __restrict__ rot, const int* __restrict__ base, const int* __restrict__ items,
-    const int* __restrict__ row_len, float scale, int H, bf16_t* __restrict__ out, const bf16_t* __restrict__ gate, int64_t gate_stride) {
+    const int* __restrict__ row_len, float scale, int H, bf16_t* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ gate,
+    int64_t gate_stride) {
   constexpr int NKS = (OWN_K + OWN_ROT) / 32, NCB = OWN_V / 16, PART = MKT * 128, TB = 5 * PART;
   __shared__ __attribute__((aligned(1024))) char tile[2 * TB];
   auto f = [](int row) { return (row & 2) | (row >> 1 & 4); };
@@ -529,7 +530,7 @@ __global__ __launch_bounds__(NT, 4) void latent_own_kernel(
   if (!ok) return;
   float w = 1.f / l;
   if (gate) w *= 1.f / (1.f + expf(-ld(gate + (int64_t)mytok * gate_stride + h)));
-  bf16_t* dst = out + ((int64_t)mytok * H + h) * OWN_V;
+  bf16_t* dst = out + mytok * out_stride + h * OWN_V;
 #pragma unroll
   for (int n = 0; n < NCB; ++n) {
     ushort4 b;
@@ -1007,14 +1008,15 @@ void sm_latent_gather(const void* cache, const int* tables, int W, int bs, const
 }
 
 // q [T, H, 128 + 64] rows q_stride apart, of which the first 128; the rotated 64 at q_rot + row * rot_stride + head * rot_head; items of up
-// to 64 tokens; kv [keys, H, 128 + 128], rot [keys, 64] of the gathered sequences; out [T, H, 128] (rows of the items).
+// to 64 tokens; kv [keys, H, 128 + 128], rot [keys, 64] of the gathered sequences; out [T, H, 128] (rows of the items), tokens out_stride apart:
+// H heads of more may be asked for.
 void sm_latent_own(const void* q, int64_t q_stride, const void* q_rot, int64_t rot_stride, int64_t rot_head, const void* kv, const void* rot,
-                   const int* base, const int* items, int n_items, const int* row_len, float scale, int H, void* out, const void* gate,
-                   int64_t gate_stride, hipStream_t stream) {
+                   const int* base, const int* items, int n_items, const int* row_len, float scale, int H, void* out, int64_t out_stride,
+                   const void* gate, int64_t gate_stride, hipStream_t stream) {
   if (n_items == 0) return;
   hipLaunchKernelGGL(latent_own_kernel, dim3(H, n_items), dim3(NT), 0, stream, (const bf16_t*)q, q_stride, (const bf16_t*)q_rot, rot_stride,
-                     rot_head, (const bf16_t*)kv, (const bf16_t*)rot, base, items, row_len, scale, H, (bf16_t*)out, (const bf16_t*)gate,
-                     gate_stride);
+                     rot_head, (const bf16_t*)kv, (const bf16_t*)rot, base, items, row_len, scale, H, (bf16_t*)out, out_stride,
+                     (const bf16_t*)gate, gate_stride);
 }
 
 // Returns 0, or 1 when the sizes do not fit the kernel (R > 1024 or rows too wide for LDS).

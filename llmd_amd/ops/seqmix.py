@@ -154,7 +154,7 @@ def latent_attention(q_abs, cache, tables, row_seq, row_len, scale: float, R: in
         nsplit, po, pm = -(-seq.max_len // FR), None, None
         if window:  # keys from a multiple of 32 on
             nsplit = min(nsplit, (window + 31 + 2 * FR - 33) // FR)
-        if seq.max_q > 1 or n >= LATENT_DECODE_WGS or n * nsplit * 16 * R > 1 << 28:
+        if seq.max_q > 1 or n >= LATENT_DECODE_WGS or n * nsplit * 16 * R > 1 << 28:  # (1 GiB, of the 2 GiB that the cache's budget spares)
             nsplit = 1
         if nsplit > 1:
             po = torch.empty(n * nsplit * 16 * R, dtype=torch.float32, device=q_abs.device)
@@ -167,7 +167,10 @@ def latent_attention(q_abs, cache, tables, row_seq, row_len, scale: float, R: in
 
 
 LATENT_OWN = os.environ.get("LLMD_LATENT_OWN", "1") == "1"
-LATENT_OWN_KEYS = 1 << 16  # keys made at once: 0.5 GB of keys and values with 16 heads
+LATENT_OWN_KEYS = 1 << 16  # keys of a step at most
+# Keys and values made at once, a key's of one head 512 bytes: so many heads at a time. They are no part of the activations that the cache's
+# budget has measured (a step's contexts are longer than its tokens), whose spare is 2 GiB.
+LATENT_OWN_BYTES = 1 << 29
 
 
 def latent_own_from(seq, H: int, dn: int, dr: int, dv: int, R: int, dtype, window: int = 0):
@@ -202,9 +205,11 @@ def latent_own(q, q_abs, cache, w_kv, scale: float, R: int, seq, first: int, gat
     rot = torch.empty(keys, cache.shape[2] - R, dtype=cache.dtype, device=cache.device)
     native().latent_gather(cache, seq.tables, bounds, first, longest, lat, rot)
     H = out.shape[1]
+    n = -(-H // -(-H // min(H, max(1, LATENT_OWN_BYTES // (keys * 512)))))  # heads at a time: as many as fit, in groups of about one size
     # ids 256 apart share a CU: long and short items together
-    items = seq.attention_items(64, balance=max(1, 256 // H), runs=(first, len(seq.q_lens)))
-    native().latent_own(q, q_abs, R, linear(lat, w_kv), rot, bounds, items, seq.row_len, float(scale), out, gate)
+    items = seq.attention_items(64, balance=max(1, 256 // n), runs=(first, len(seq.q_lens)))
+    for h in range(0, H, n):
+        native().latent_own(q, q_abs, R, linear(lat, w_kv[h * 256:(h + n) * 256]), rot, bounds, items, seq.row_len, float(scale), out, gate, h)
 
 
 def causal_conv_silu(xz, C, w, b, conv_state, seq_start, seq_slot, seq_init, max_q: int):

@@ -79,3 +79,25 @@ def test_layer(runs, own):
         outs.append(l(h.to(dev, dt), AttnMeta(num_tokens=T, positions=pos.to(dev), slot_mapping=slots.long().to(dev), seq=m)).float().cpu())
     # bf16 throughout: about ten roundings of 2^-9 in a row
     assert (outs[1] - outs[0]).norm() <= 10 * 2 ** -9 * outs[0].norm()
+
+
+@pytest.mark.parametrize("H,at_once", [(5, 2), (64, 24), (64, 64), (3, 1)])
+def test_heads_in_groups(H, at_once, monkeypatch):
+    """Keys and values of some heads at a time, where those of all would take too much memory."""
+    from llmd_amd.ops import seqmix as sm
+
+    runs, R, bs = [(40, 1), (3, 70), (0, 33)], 128, 64
+    g = torch.Generator().manual_seed(H)
+    rand = lambda *s: torch.randn(*s, generator=g).bfloat16()  # noqa: E731
+    meta, pages = _meta(runs, bs, "cpu")
+    T = sum(n for _, n in runs)
+    q, q_abs, cache, gate = rand(T, H * 192), rand(T, H, R + 64), rand(pages, bs, R + 64), rand(T, H)
+    uk, uv = rand(H, 128, R) * R ** -0.5, rand(H, 128, R) * R ** -0.5
+    want = _exact(q.double().view(T, H, 192)[:, :, :128], q_abs.double()[:, :, R:], cache.double(), uk.double(), uv.double(), 0.07, meta, gate.double())
+    m, _ = _meta(runs, bs, "cuda")
+    monkeypatch.setattr(sm, "LATENT_OWN_BYTES", 106 * 512 * at_once + 511)
+    out = torch.full((T, H, 128), float("nan"), dtype=torch.bfloat16, device="cuda")
+    sm.latent_own(q.cuda(), q_abs.cuda(), cache.cuda(), torch.cat([uk, uv], 1).reshape(-1, R).cuda(), 0.07, R, m, 1, gate.cuda(), out)
+    got, want = out.cpu()[1:], want[1:]
+    assert out[:1].isnan().all()
+    assert (got.double() - want).norm() <= 3 * 2 ** -9 * want.norm() and ((got - want).abs() <= 2 ** -5 * want.abs().clamp(min=1)).all()
