@@ -184,9 +184,15 @@ def latent_own_from(seq, H: int, dn: int, dr: int, dv: int, R: int, dtype, windo
     rows, keys = float(n.sum()), float(ctx.sum())
     if keys > LATENT_OWN_KEYS or float(np.ceil(n / 64).sum()) > 65535:
         return None
-    # us of both on 16 and more heads: making keys and values against absorbing and the two products around it; a tile of 32
-    # keys in the longest row's chain, or all pairs of rows and keys. Measured, own / absorbed: 16 heads, 64 rows 15 / 11, 128 20 / 23, 2048
-    # 89 / 172, 4000 163 / 409, 64 after 1000 50 / 75, 1024 after 4000 189 / 316; 64 heads, 64 after 4000 189 / 237, 2048 179 / 481
+    # us of both with 16 and more heads over a latent of 512: making keys and values against absorbing and the two products around it; a
+    # tile of 32 keys in the longest row's chain, or all pairs of rows and keys. Whole layers, own / absorbed, 16 heads: 64 rows 40 / 49, 128
+    # 41 / 58, 2048 118 / 192, 64 after 1000 76 / 102, 512 after 4000 184 / 289; 64 heads: 64 55 / 67, 2048 246 / 560, 64 after 4000 220 / 274; one
+    # head: 128 32 / 47, 2048 88 / 153, 64 after 4000 141 / 252. Smaller latents: 256, 16 heads, 128 rows 39 / 64, 64 after 4000 158 / 342; 64, 16
+    # heads 38 / 48, 159 / 200; 64, 64 heads 51 / 59, 64 after 1000 99 / 97. Of 228 such pairs (1 - 64 heads, latents 64 - 512) the rule takes
+    # the slower form where own gains 1.1 - 1.4 in single rounds of few rows (64 rows, 16 after 500 on 64 heads) and that last one.
+    # Beyond 64 heads the absorbed form has a lane per key: 128 heads, 64 after 1000 140 / 10076.
+    if H > 64:
+        return first
     k, longest, pairs = H / 16, float(ctx.max()), float((n * (ctx - n / 2)).sum())
     own = 12 + 0.006 * keys * k + max(0.9 * longest / 32, 15e-6 * pairs * k)
     absorbed = (14 if rows > 64 else 6) + 0.017 * rows * k + max(1.75 * longest / 32, 68e-6 * pairs * k)
@@ -197,7 +203,9 @@ def latent_own(q, q_abs, cache, w_kv, scale: float, R: int, seq, first: int, gat
     """Attention of the rows behind the first ``first`` single tokens over keys and values made once per head, the same function as
     absorbing W_uk into the query and applying W_uv to the read-out: q [T, H (128 + 64)], its rotated parts in q_abs [T, H, R + 64],
     w_kv [H (128 + 128), R] (every head's rows of W_uk, then of W_uv), cache [blocks, bs, R + 64]; out [T, H, 128], of which those
-    rows are written."""
+    rows are written. Keys and values are rounded to the cache's type where the absorbed form rounds queries and read-outs, and which
+    form a row takes depends on the sizes of its whole step (``latent_own_from``): a token's last bits depend on how its prompt was
+    cut and on what shares the step."""
     from . import linear
 
     bounds, keys, longest = seq.key_rows(first)

@@ -81,7 +81,7 @@ def test_layer(runs, own):
     assert (outs[1] - outs[0]).norm() <= 10 * 2 ** -9 * outs[0].norm()
 
 
-@pytest.mark.parametrize("H,at_once", [(5, 2), (64, 24), (64, 64), (3, 1)])
+@pytest.mark.parametrize("H,at_once", [(5, 2), (64, 24), (64, 64), (3, 1), (128, 128)])
 def test_heads_in_groups(H, at_once, monkeypatch):
     """Keys and values of some heads at a time, where those of all would take too much memory."""
     from llmd_amd.ops import seqmix as sm
@@ -101,3 +101,12 @@ def test_heads_in_groups(H, at_once, monkeypatch):
     got, want = out.cpu()[1:], want[1:]
     assert out[:1].isnan().all()
     assert (got.double() - want).norm() <= 3 * 2 ** -9 * want.norm() and ((got - want).abs() <= 2 ** -5 * want.abs().clamp(min=1)).all()
+
+
+@pytest.mark.parametrize("H,R,runs,own", [(16, 512, [(0, 128)], 0), (1, 512, [(4000, 64)], 0), (64, 64, [(0, 2048)], 0), (64, 512, [(4000, 9)], 0),
+                                          (16, 512, [(9, 1), (0, 20)], None), (128, 512, [(9, 1), (500, 16)], 1), (128, 512, [(9, 1)], None),
+                                          (16, 96, [(0, 128)], None)])
+def test_form(H, R, runs, own):
+    from llmd_amd.ops import seqmix as sm
+
+    assert sm.latent_own_from(_meta(runs, 64, "cuda")[0], H, 128, 64, 128, R, torch.bfloat16) == own
