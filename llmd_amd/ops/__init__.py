@@ -1443,10 +1443,11 @@ def pgemm_silu(x: torch.Tensor, w: torch.Tensor, variant: int = 3, out: Optional
     return pgemm(x, w, epi=3, out=out, variant=variant, split_k=False)
 
 
-def _plain(x: torch.Tensor, w: torch.Tensor) -> bool:
+def _plain(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
     """A call that nobody differentiates, batches, traces or watches: one whose library product a kernel may stand in for."""
     return (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter)
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+            and (bias is None or type(bias) in (torch.Tensor, torch.nn.Parameter))
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)))
             and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.maybe_current_level() is None
             and torch._C._get_tracing_state() is None and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._len_torch_function_stack() == 0)
@@ -1457,7 +1458,7 @@ def tgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     act: silu(x wg^T) * (x wu^T) for w = [gate; up], 1: of the fp32 sums as ``pgemm_silu`` variant 6, 2: of the sums in bf16, the bits
     of the product (one range of K) + ``gated_act``; 3: max(0, x w^T)^2 of the sums in bf16; 4: the clamped units of act 2's operands,
     the bits of the product + ``seqmix.gated_act``."""
-    if PGEMM_AUTO == "0" or not _gpu(x) or not _plain(x, w):
+    if PGEMM_AUTO == "0" or not _gpu(x) or not _plain(x, w, bias):
         return None
     return native().tgemm(x, w, bias, act, 0, limit)
 
@@ -1465,7 +1466,7 @@ def tgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
 def fgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None):
     """fp32 x w^T (+ bias) on the bf16 matrix units, three parts of every number (csrc/ops/fgemm.hip, which holds the rule), or
     None where it is not taken. No further from 64 bits than the library's fp32 product."""
-    if not _gpu(x) or not _plain(x, w):
+    if not _gpu(x) or not _plain(x, w, bias):
         return None
     return native().fgemm(x, w, bias)
 
@@ -1473,7 +1474,7 @@ def fgemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None)
 def router_linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """A router's logits in x's dtype: few columns on the kernel of csrc/ops/router.hip (which holds the rule; 64 x (128, 2048) 5.5 us on the
     library, 3.3 there), large prompts on ``tgemm``, the rest on the library."""
-    if not _gpu(x) or not _plain(x, w):
+    if not _gpu(x) or not _plain(x, w, bias):
         return torch.nn.functional.linear(x, w, bias)
     y = native().router_product(x, w, bias)
     if y is None and x.dim() == 2 and x.shape[0] > 64:

@@ -56,6 +56,23 @@ def test_router_linear_takes_other_calls_as_before():
     assert torch.equal(ops.router_linear(xc, wc), torch.nn.functional.linear(xc, wc))
 
 
+@pytest.mark.parametrize("rows,dtype", [(9, torch.bfloat16), (1000, torch.bfloat16), (8192, torch.bfloat16), (300, torch.float32)])
+def test_a_bias_that_is_differentiated(rows, dtype):
+    """The library's product, which has a backward, whatever the rows: a router's, and a dense one's on the tiles."""
+    N = 128 if dtype == torch.bfloat16 else 4096
+    x, w, b = _rand(rows, 2048).to(dtype), _rand(N, 2048, seed=1).to(dtype), _rand(N, seed=2).to(dtype).requires_grad_()
+    for f in (ops.router_linear, lambda x, w, b: ops.fgemm(x, w, b) if dtype == torch.float32 else ops.tgemm(x, w, b)):
+        with torch.enable_grad():
+            y = f(x, w, b)
+            if y is None:  # left to the library
+                continue
+            y.sum().backward()
+        assert torch.equal(b.grad, torch.full_like(b, float(rows)).to(dtype))
+        b.grad = None
+        with torch.no_grad():
+            assert not f(x, w, b).requires_grad
+
+
 def test_capture():
     x, w = _rand(64, 2048), _rand(132, 2048, seed=1)
     want = ops.router_product(x, w)
