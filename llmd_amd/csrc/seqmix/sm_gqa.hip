@@ -1100,6 +1100,7 @@ __global__ __launch_bounds__(NT, NKS <= 4 ? 4 : 2) void grouped_prompt_kernel(
   // (a wait that hipcc sees, though not the copies: where the query might be pending at the loop's entry it would wait for all in the loop)
   __builtin_amdgcn_s_waitcnt(0);
   __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");  // (neither is a fence for hipcc: reads of the tile stay below)
   int cur = 0;
   for (int v0 = kbase; v0 < vlen; v0 += MKT, cur ^= 1) {
     const int k0 = key_of(v0);

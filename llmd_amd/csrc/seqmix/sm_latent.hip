@@ -351,6 +351,7 @@ __global__ __launch_bounds__(NT, 2) void latent_prompt_kernel(
   // (a wait that hipcc sees, though not the copies: where the query might be pending at the loop's entry it would wait for all in the loop)
   __builtin_amdgcn_s_waitcnt(0);
   __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");  // (neither is a fence for hipcc: reads of the tile stay below)
   int cur = 0;
   for (int k0 = kbeg; k0 < kend; k0 += MKT, cur ^= 1) {
     const char* const t = tile + cur * (MKT * RB);
@@ -499,6 +500,7 @@ __global__ __launch_bounds__(NT, 4) void latent_own_kernel(
   // (a wait that hipcc sees, though not the copies: where the query might be pending at the loop's entry it would wait for all in the loop)
   __builtin_amdgcn_s_waitcnt(0);
   __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");  // (neither is a fence for hipcc: reads of the tile stay below)
   int cur = 0;
   for (int k0 = 0; k0 < kend; k0 += MKT, cur ^= 1) {
     const char* const t = tile + cur * TB;
