@@ -54,3 +54,43 @@ def test_rows_are_the_same_in_every_step(H, window):
     assert torch.equal(out, torch.cat([run(0, 77), run(77, 200), run(200, n)]))
     for t in (0, 31, 127, 128, 129, 300, 399):
         assert torch.equal(out[t:t + 1], run(t, t + 1))  # a step of one token: ranges apart
+
+
+def test_more_ranges_than_workgroups():
+    """Ranges apart, more of them than a token's workgroups: each walks several. 30 tokens, 40 ranges: 34 workgroups a token."""
+    from llmd_amd.ops import seqmix as sm
+
+    runs, H, Dk = [(5000, 1), (4500, 1)] + [(40 * i, 1) for i in range(28)], 16, 576
+    g = torch.Generator().manual_seed(0)
+    m, pages = _meta(runs, 64, "cuda")
+    q, cache = torch.randn(len(runs), H, Dk, generator=g), torch.randn(pages, 64, Dk, generator=g)
+    got = sm.latent_attention(q.cuda(), cache.cuda(), m.tables, m.row_seq, m.row_len, 0.05, 512, 1, seq=m)
+    m.max_q = 2  # one workgroup for all ranges, joined in the same order
+    assert torch.equal(got, sm.latent_attention(q.cuda(), cache.cuda(), m.tables, m.row_seq, m.row_len, 0.05, 512, 1, seq=m))
+    want = _exact(q, cache, _meta(runs, 64, "cpu")[0], 0.05, 512, None, 0)
+    assert ((got.double().cpu() - want).abs() <= 2e-5 * want.abs().clamp(min=1)).all()  # (as above)
+
+
+def test_captured_step():
+    """Ranges planned for the longest context, lengths that change between the replays."""
+    from llmd_amd.ops import seqmix as sm
+
+    H, Dk, n = 16, 576, 5
+    g = torch.Generator().manual_seed(0)
+    m, pages = _meta([(999, 1)] * n, 64, "cuda")
+    q, cache, gate = torch.randn(n, H, Dk, generator=g).cuda(), torch.randn(pages, 64, Dk, generator=g).cuda(), torch.randn(n, H, generator=g).cuda()
+    go = lambda: sm.latent_attention(q, cache, m.tables, m.row_seq, m.row_len, 0.05, 512, 1, seq=m, gate=gate)  # noqa: E731
+    go()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = go()
+    for lens in ([1, 1, 1, 1, 1], [1000, 128, 129, 1, 700], [31, 32, 33, 640, 127]):
+        m.row_len.copy_(torch.tensor(lens, dtype=torch.int32))
+        q.copy_(torch.randn(n, H, Dk, generator=g))
+        short, _ = _meta([(k - 1, 1) for k in lens], 64, "cuda")
+        short.tables = m.tables
+        want = sm.latent_attention(q, cache, m.tables, short.row_seq, short.row_len, 0.05, 512, 1, seq=short, gate=gate)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)

@@ -110,3 +110,37 @@ def test_form(H, R, runs, own):
     from llmd_amd.ops import seqmix as sm
 
     assert sm.latent_own_from(_meta(runs, 64, "cuda")[0], H, 128, 64, 128, R, torch.bfloat16) == own
+
+
+def test_layer_with_anothers_cache():
+    """A layer that reads an earlier layer's latents makes keys and values of them with its own weights."""
+    from llmd_amd.engine.attn_meta import AttnMeta
+    from llmd_amd.models.mixers import LatentAttention
+    from llmd_amd.ops import seqmix as sm
+
+    torch.manual_seed(1)
+    runs, T = [(70, 1), (40, 150), (0, 77)], 228
+    args = (256, 16, 128, 64, 128, 512, 192 ** -0.5, 64, 10000.0, 1e-6, 1024, "cpu", torch.bfloat16)
+    first = LatentAttention(*args, q_rank=128)
+    second = LatentAttention(*args, q_rank=128, gate=True, kv_source=first)
+    both = torch.nn.ModuleList([first, second])
+    for p in both.parameters():
+        p.data.normal_(0, 0.05) if p.dim() > 1 else p.data.uniform_(0.8, 1.2)
+    h, outs = torch.randn(T, 256).bfloat16(), []
+    for dev, dt in (("cpu", torch.float32), ("cuda", torch.bfloat16)):
+        m, pages = _meta(runs, 64, dev)
+        pos = torch.cat([torch.arange(e, e + n) for e, n in runs])
+        slots = torch.cat([m.tables[i].cpu()[torch.arange(e, e + n) // 64] * 64 + torch.arange(e, e + n) % 64 for i, (e, n) in enumerate(runs)])
+        a, b = copy.deepcopy(both).to(dev, dt)
+        for layer in (a, b):
+            layer.cos_sin = first.cos_sin.to(dev)  # stays fp32
+            layer.finalize()
+        assert b._src[0] is a
+        a.bind_cache(torch.randn(pages, 1, 1, 64, 576, generator=torch.Generator().manual_seed(2)).bfloat16().to(dev, dt))
+        if dev == "cuda":
+            assert sm.latent_own_from(m, 16, 128, 64, 128, 512, dt) == 1
+        meta = AttnMeta(num_tokens=T, positions=pos.to(dev), slot_mapping=slots.long().to(dev), seq=m)
+        x = h.to(dev, dt)
+        outs.append([y.float().cpu() for y in (a(x, meta), b(x, meta))])
+    for got, want in zip(outs[1], outs[0]):  # (as in test_layer)
+        assert (got - want).norm() <= 10 * 2 ** -9 * want.norm()
