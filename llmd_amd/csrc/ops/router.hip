@@ -5,7 +5,8 @@
 // until the four sums of each number are added up, in the waves' order. That order is the same for every size, so a row's numbers
 // do not depend on how many rows a step has.
 // Bound by the copies into one CU, 24 cycles per KB: (MB + NB) * K * 32 bytes a workgroup, whence the rule in plan() below.
-// us, 64 / 1000 / 2048 / 8192 rows; fp32 against the float product of widened copies that stood in its place, and the form of few rows
+// us over and over, operands in the caches (in a prompt's step of 2048 behind the kernels before it 8.5 in fp32, 7.5 in bf16; of 64 rows
+// 4.9); 64 / 1000 / 2048 / 8192 rows; fp32 against the float product of widened copies that stood in its place, and the form of few rows
 // (sm_moe.hip router_kernel): (132, 2048) 10.8, 7.2 / 20.8 / 30.8 / 58 -> 3.3 / 5.1 / 6.4 / 15; (256, 7168) 19 / 44 / 71 / 256 -> 7.1 / 13 / 22 /
 // 90. Off 64 bits, rms over sums of variance 1: 1.7e-7, 3.9e-7 (long sums of 2048 rows) -> 1.3e-7; K 7168 3.6e-7, 8.7e-7 -> 2.5e-7.
 // bf16 against the library / tgemm: (128, 2048) 64 rows 5.5 -> 3.3, 1000 8.3 / 8.8 -> 5.2, 2048 8.8 / 9.1 -> 5.7.

@@ -494,9 +494,11 @@ __global__ __launch_bounds__(NT) void retention_norm_kernel(const float* __restr
 // three bf16 parts, times 2^24 (moe_tile.h says why); v is bf16 as it is, so its products take three instructions and are exact, those of
 // two fp32 numbers six. Sums that are not finite (infinities, NaN, numbers that overflow so scaled) are done again
 // number by number. The contraction index is dealt to the lane groups in eights; a lane's eight are one 16-byte piece in LDS.
-// Bound by the chunks' states (a head's 128 KB written once and read twice per 64 tokens) and by the chain of loads and barriers of a
+// Bound by the chunks' states (a head's 128 KB written twice and read twice per 64 tokens: here, by retention_link in between and by
+// retention_out) and by the chain of loads and barriers of a
 // workgroup; the fp32 instructions alone had taken half of the time, loads one after the other most of the rest.
-// us, chunk + out, 16 heads of 128 x 256: 901 + 844 + 787 tokens 65 + 100 -> 38 + 53. States off 64 bits: less than before (exact
+// us, chunk + out, 16 heads of 128 x 256: 901 + 844 + 787 tokens 65 + 100 -> 38 + 53 over and over, 42 + 58 in a step behind its other
+// kernels. States off 64 bits: less than before (exact
 // products, a sixteenth of the roundings).
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
