@@ -521,7 +521,8 @@ def gated_act(gu, Fh: int, kind: str, limit: float = 0.0):
 
 def router_logits(x, w):
     """x w^T in fp32 for bfloat16 x [T, d] and w [N, d] (csrc/seqmix/sm_moe.hip router_kernel), or None. In the
-    order of a float product of copies; ``ops.router_product`` has one of its own and is two to five times as fast."""
+    order of a float product of copies, for callers who want its bits: the layers take ``ops.router_product``, which has an order of its own and
+    is two to five times as fast."""
     return native().router_logits(x, w) if x.is_cuda and x.dtype == torch.bfloat16 else None
 
 
